@@ -31,6 +31,7 @@ KERNEL_UNITS = [
     ("fused_dtype_kernels.hip", "fused_kernels_f32.o", ["-DFTK_FUSED_DT=0"]),
     ("fused_kernels.hip", "fused_kernels.o", []),
     ("topp_kernels.hip", "topp_kernels.o", []),
+    ("topp_sample_kernels.hip", "topp_sample_kernels.o", []),
     ("topk_kernels.hip", "topk_kernels.o", []),
     ("logprob_kernels.hip", "logprob_kernels_f32.o", ["-DFTK_LP_DT=0"]),
     ("logprob_kernels.hip", "logprob_kernels_f16.o", ["-DFTK_LP_DT=1"]),

@@ -31,13 +31,18 @@ struct RowDivisor {
     __device__ __forceinline__ float divide(float n) const
     {
         if (n >= 7.888609052210118e-31f || n == 0.0f) {
-            const float q0 = n * r;
-            const float m0 = __builtin_fmaf(-d, q0, n);
-            const float q1 = __builtin_fmaf(m0, r, q0);
-            const float m1 = __builtin_fmaf(-d, q1, n);
-            return __builtin_fmaf(m1, r, q1);
+            return divide_normal(n);
         }
         return n / d;
+    }
+    // the same for a numerator in [2^-100, 1]
+    __device__ __forceinline__ float divide_normal(float n) const
+    {
+        const float q0 = n * r;
+        const float m0 = __builtin_fmaf(-d, q0, n);
+        const float q1 = __builtin_fmaf(m0, r, q0);
+        const float m1 = __builtin_fmaf(-d, q1, n);
+        return __builtin_fmaf(m1, r, q1);
     }
 };
 
@@ -74,6 +79,15 @@ __device__ __forceinline__ int lane_id()
 __device__ __forceinline__ int wave_id()
 {
     return (int)(threadIdx.x >> 6);
+}
+
+// Workgroup barrier for code that only communicates through LDS: global loads issued earlier stay
+// in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // ---- wave / block reductions ----------------------------------------------------------------
@@ -462,6 +476,41 @@ __device__ __forceinline__ float rng_next_uniform(RngState* st)
     philox4x32_10((uint32_t)off, (uint32_t)(off >> 32), 0u, 0u, (uint32_t)st->seed, (uint32_t)(st->seed >> 32), o);
     st->offset = off + 1;
     return (float)o[0] * 2.3283064365386963e-10f + 1.16415321826934814453125e-10f;
+}
+
+// One flag of a bool array at an index that is the same for the whole workgroup, read through the aligned
+// 32-bit word that holds it: a scalar load, which does not queue behind the vector loads in flight (a byte
+// load would, and its consumer would wait for all of them).
+__device__ __forceinline__ bool uniform_flag(const bool* flags, int index)
+{
+    const bool*    flag = flags + index;
+    const uint32_t mis  = (uint32_t)(reinterpret_cast<uintptr_t>(flag) & 3u);
+    const uint32_t word = *reinterpret_cast<const uint32_t*>(flag - mis);  // stays inside the flag's own word
+    return ((word >> (8u * mis)) & 0xFFu) != 0u;
+}
+
+// Per-row arguments are optional arrays. Reading them behind their null checks makes a chain of loads that
+// each wait for the one before; these helpers always load - from the array when it exists, from `safe` (any
+// valid 4-byte aligned address, the row's end id) when it does not - so that all of a row's arguments are
+// requested together and cost one trip to memory.
+template<typename V>
+__device__ __forceinline__ V row_arg_or(const V* array, int row, const void* safe, V otherwise)
+{
+    static_assert(sizeof(V) == 4, "32-bit arguments");
+    const V* from = array != nullptr ? array + row : reinterpret_cast<const V*>(safe);
+    const V  v    = *from;
+    return array != nullptr ? v : otherwise;
+}
+__device__ __forceinline__ bool row_flag_or(const bool* flags, int row, const void* safe, bool otherwise)
+{
+    const bool* from = flags != nullptr ? flags + row : reinterpret_cast<const bool*>(safe);
+    const bool  v    = uniform_flag(from, 0);
+    return flags != nullptr ? v : otherwise;
+}
+
+__device__ __forceinline__ float uniform_f(float x)
+{
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
 }
 
 // What a row's draw is made from, requested ahead of time without control flow (`safe`: any valid 4-byte aligned

@@ -54,44 +54,6 @@ __device__ __forceinline__ uint32_t* fused_lds_bitmap()
     return words;
 }
 
-// BMW > 0: the history bitmap is a window of BMW words in LDS, built by prepare().
-// BMW == 0: whole-row bitmaps in global memory (built by history_bitmap_kernel, or by
-//           prepare_whole_row() for the literal replay).
-// One flag of a bool array at an index that is the same for the whole workgroup, read through the aligned
-// 32-bit word that holds it: a scalar load, which does not queue behind the vector loads in flight (a byte
-// load would, and its consumer would wait for all of them).
-__device__ __forceinline__ bool uniform_flag(const bool* flags, int index)
-{
-    const bool*    flag = flags + index;
-    const uint32_t mis  = (uint32_t)(reinterpret_cast<uintptr_t>(flag) & 3u);
-    const uint32_t word = *reinterpret_cast<const uint32_t*>(flag - mis);  // stays inside the flag's own word
-    return ((word >> (8u * mis)) & 0xFFu) != 0u;
-}
-
-// Per-row arguments are optional arrays. Reading them behind their null checks makes a chain of loads that
-// each wait for the one before; these helpers always load - from the array when it exists, from `safe` (any
-// valid 4-byte aligned address, the row's end id) when it does not - so that all of a row's arguments are
-// requested together and cost one trip to memory.
-template<typename V>
-__device__ __forceinline__ V row_arg_or(const V* array, int row, const void* safe, V otherwise)
-{
-    static_assert(sizeof(V) == 4, "32-bit arguments");
-    const V* from = array != nullptr ? array + row : reinterpret_cast<const V*>(safe);
-    const V  v    = *from;
-    return array != nullptr ? v : otherwise;
-}
-__device__ __forceinline__ bool row_flag_or(const bool* flags, int row, const void* safe, bool otherwise)
-{
-    const bool* from = flags != nullptr ? flags + row : reinterpret_cast<const bool*>(safe);
-    const bool  v    = uniform_flag(from, 0);
-    return flags != nullptr ? v : otherwise;
-}
-
-__device__ __forceinline__ float uniform_f(float x)
-{
-    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
-}
-
 // A row's per-row arguments, requested in one block without control flow so that they share one trip to memory
 // (the arithmetic on them, which waits for the values, comes afterwards).
 struct FusedRowArgs {
@@ -165,6 +127,9 @@ struct FusedRowDerived {
     int   flags;  // bit 0: keep_pads, bit 1: up_ok
 };
 
+// BMW > 0: the history bitmap is a window of BMW words in LDS, built by prepare().
+// BMW == 0: whole-row bitmaps in global memory (built by history_bitmap_kernel, or by
+//           prepare_whole_row() for the literal replay).
 template<int DT, int BMW>
 struct FusedRow {
     static constexpr int  LDS_WORDS = BMW > 0 ? BMW : 1;

@@ -104,15 +104,6 @@ inline TopkPlan topk_plan(int vocab_padded, int batch, int max_top_k, int elem_b
     return p;
 }
 
-// Workgroup barrier for code that only communicates through LDS: global loads issued earlier stay
-// in flight across it.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // -------------------------------------------------------------------------------------------
 // Row accessors: turn (column, raw storage value) into the value the reference would hand to top-k
 // (an fp32 image of a `T`). PlainRow is the identity (stand-alone entry point); the fused decode

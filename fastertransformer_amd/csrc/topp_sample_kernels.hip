@@ -1,0 +1,2141 @@
+// The top-p step that samples straight from logits (ftk_fused_topp_sample_step, ftk_fused_topp_penalty_step).
+//
+// What TopPSamplingLayer runs per step - temperature, repetition / presence penalty and minimum length
+// (src/fastertransformer/layers/sampling_layers/BaseSamplingLayer.cc:302-352), softmax, nucleus sampling and decay
+// (layers/sampling_layers/TopPSamplingLayer.cu:256-343) - without writing penalised logits or probabilities to the
+// caller's buffer. Results are bit for bit those of the kernel sequence. Three launches (four for fp32):
+//
+//   stage  reads the logits once: the values y after temperature, penalties and masks (kept in the workspace when there
+//          are any), the row's maximum, whether there is a NaN, and, 16-bit types: the maximum of every block of 512
+//          columns, fp32: a histogram of y;
+//   sum    reads y: e = T(exp(y - max)) summed in the order of the reference's softmax
+//          (sampling_topp_kernels.cu:1308-1344: thread t of 1024 adds columns t, t + 1024, ... one after the other, then
+//          xor butterflies). A workgroup owns whole summation chains, so that a row can spread over several workgroups
+//          and the sum keeps the reference's bits. On the way
+//            16-bit types: counts how often every value of e occurs (there are few: at most 3970 / 15361);
+//            fp32: the histogram of the stage says where the draw must lie; what is at or above that cut goes to
+//            its bucket's place in the ordered prefix;
+//   sort   (fp32) long prefixes, in segments dealt out over the launch;
+//   pick   one workgroup per row replays the reference's scan and emits the token.
+//
+// 16-bit types need no sort: the counts are the sorted row in run-length form, the scan reads its values from the
+// runs, and the one id that is emitted is looked up in the row: the n-th column, in order of ids, whose value is the
+// picked one. Long runs of equal values, which 16-bit logits have everywhere, cost nothing.
+#include <algorithm>
+#include <type_traits>
+
+#include "ftk_topp.cuh"
+#include "ftk_sampling.h"
+#include "ftk_topp_sample.h"
+
+namespace ftk {
+
+constexpr int   TSP_STAGE   = 256;        // threads of a stage workgroup
+constexpr int   TSP_SUM16   = 1024;       // threads of a sum workgroup, 16-bit types
+constexpr int   TSP_SUM32   = 256;        // fp32
+constexpr int   TSP_CHAINS  = 1024;       // summation chains of a row (the reference's block)
+constexpr int   TSP_SPLITS  = 64;         // most workgroups per row of the 16-bit stage
+constexpr int   TSP_BLOCK   = 512;        // columns whose maximum the 16-bit stage keeps: one 16-byte vector per lane
+constexpr int   TSP_WINDOW  = 5120 + 4;   // words of the history bitmap of a workgroup
+constexpr int   TSP_BUCKETS = 2048;       // fp32: buckets of y, 1/64 wide, downwards from TSP_ABOVE over the reference
+constexpr float TSP_SCALE   = 64.0f;
+constexpr float TSP_ABOVE   = 8.0f;
+constexpr float TSP_LOWEST  = -3.402823466e+38f;
+
+struct ToppStep {
+    const void*  logits;
+    const void*  bias;
+    int          n, Vp, rows;  // columns of the vocabulary, pitch of a row
+    void*        y;            // [rows][y_pitch], or null: y is the logits themselves
+    int          y_pitch;
+    const float* temperatures;
+    const float* penalties;
+    int          penalty_type;  // 2: none
+    const int*   min_lengths;
+    const int*   end_ids;
+    const int*   input_lengths;
+    const int*   history;  // element (t, row) at history[t * batch_size + row]
+    const int*   sequence_length;
+    int          batch_size, step, max_input_length;
+    const bool*  finished;
+    const bool*  skip;
+    const RngState* rng;
+    const float* uniforms;
+    float        top_p;
+    const float* top_ps;
+    int          splits, chunk;  // 16-bit stage: workgroups per row and columns of one
+    int          parts;          // sum (and the fp32 stage): workgroups per row
+    int          blocks;         // blocks of TSP_BLOCK columns per row
+    float2*      pmax;           // [rows][TSP_SPLITS]: maximum of a stage workgroup, and 1 when it saw a NaN
+    float*       block_max;      // [rows][blocks]
+    float*       ref;            // [rows]
+    float*       gsum;           // [rows][32]
+    uint32_t*    counts;         // 16-bit: [rows][counters]; fp32: [rows][parts][TSP_BUCKETS]
+    ToppRowMeta* meta;
+    uint32_t*    segs;           // [rows][TPB_NB] ends of segments
+    uint32_t*    queue;          // [0]: segments left to the sort's workgroups, then the segments (row * TPB_NB + number)
+    unsigned long long* sorted;
+};
+
+// Counters of the 16-bit types. binary16: one per value of e up to 1. bfloat16: one per value from 2^-31 to 1; a draw
+// that falls among smaller ones takes the exact fallback. LUT_*: the values of y whose e a workgroup of the sum looks up
+// in a table, 2 x LUT_N of them: magnitudes from LUT_LOW on (2^-8 .. 2^8 / 2^6).
+template<int DT>
+struct ToppCode;
+template<>
+struct ToppCode<DT_F16> {
+    static constexpr int COUNTERS = 16384, USED = 15361, BASE = 0;
+    static constexpr int LUT_LOW = 7 << 10, LUT_N = 14 << 10;
+};
+template<>
+struct ToppCode<DT_BF16> {
+    static constexpr int COUNTERS = 4096, BASE = ((127 - 31) << 7) - 1, USED = 127 * 128 - BASE + 1;
+    static constexpr int LUT_LOW = (127 - 8) << 7, LUT_N = 16 << 7;
+};
+static_assert(ToppCode<DT_BF16>::USED <= ToppCode<DT_BF16>::COUNTERS, "bfloat16 counters");
+
+// The value a column has after temperature, penalties and the minimum length, as the kernel sequence leaves it.
+template<int DT>
+struct ToppTransform {
+    TemperatureCtx<DT> temperature;
+    bool               temperature_active;
+    float              penalty;
+    int                penalty_type, masked_end;
+    const typename Storage<DT>::T* bias;
+    // (every load is requested before the first value is used)
+    __device__ __forceinline__ ToppTransform(const ToppStep& s, int row): ToppTransform(s, Args(s, row), row) {}
+
+private:
+    struct Args {
+        float temperature, penalty;
+        int   min_length, length, end_id;
+        __device__ __forceinline__ Args(const ToppStep& s, int row)
+        {
+            const void* safe = s.gsum;
+            temperature      = row_arg_or(s.temperatures, row, safe, 1.0f);
+            penalty          = row_arg_or(s.penalties, row, safe, 0.0f);
+            min_length       = row_arg_or(s.min_lengths, row, safe, 0);
+            length           = row_arg_or(s.min_lengths != nullptr ? s.sequence_length : nullptr, row, safe, 0);
+            end_id           = row_arg_or(s.min_lengths != nullptr ? s.end_ids : nullptr, row, safe, -1);
+        }
+    };
+    __device__ __forceinline__ ToppTransform(const ToppStep& s, const Args& a, int):
+        temperature(a.temperature, s.n, s.Vp, false)
+    {
+        temperature_active = s.temperatures != nullptr;
+        bias               = (const typename Storage<DT>::T*)s.bias;
+        penalty_type       = s.penalties != nullptr ? s.penalty_type : 2;
+        penalty            = a.penalty;
+        masked_end = s.min_lengths != nullptr && min_length_masks(a.length, s.max_input_length, a.min_length) ? a.end_id : -1;
+    }
+
+public:
+    __device__ __forceinline__ float operator()(int v, float x, bool in_history) const
+    {
+        if (temperature_active) {
+            x = temperature.value(x, bias != nullptr, bias != nullptr ? Storage<DT>::ld(bias[v]) : 0.0f);
+        }
+        if (in_history) {
+            x = round_t<DT>(repetition_value(x, penalty, penalty_type));
+        }
+        return v == masked_end ? -Storage<DT>::max_t() : x;
+    }
+};
+
+// Calls mark(id) for the tokens of a row's history that the penalty counts. Every id is a cache line of its own: eight
+// in flight per thread.
+template<class Mark>
+__device__ __forceinline__ void topp_walk_history(const ToppStep& s, int row, Mark&& mark)
+{
+    constexpr int H   = 8;
+    const int     len = s.input_lengths != nullptr ? s.input_lengths[row] : s.max_input_length;
+    for (int t0 = threadIdx.x; t0 < s.step; t0 += H * TSP_STAGE) {
+        int ids[H];
+#pragma unroll
+        for (int u = 0; u < H; ++u) {
+            const int at = t0 + u * TSP_STAGE;
+            // (the padding between a short prompt and max_input_length does not count)
+            ids[u] = at < s.step && !(at >= len && at < s.max_input_length) ? s.history[(size_t)at * s.batch_size + row] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < H; ++u) {
+            mark(ids[u]);
+        }
+    }
+}
+
+__device__ __forceinline__ bool topp_row_idle(const ToppStep& s, int row)
+{
+    const void* safe = s.pmax;
+    const bool  skip = row_flag_or(s.skip, row, safe, false);
+    const bool  fin  = row_flag_or(s.finished, row, safe, false);
+    return skip || fin;
+}
+
+// Eight neighbouring 16-bit columns from any column on: one access where the memory allows.
+__device__ __forceinline__ uint4 topp_load8(const uint16_t* from)
+{
+    uint4 raw;
+    __builtin_memcpy(&raw, from, 16);
+    return raw;
+}
+
+// ---- stage, 16-bit types ------------------------------------------------------------------------------------------
+// (rows x splits) workgroups, each over a run of blocks of 512 columns, a block per wave at a time. Memory-bound. The
+// counters that several workgroups of the sum add to are cleared on the way. 64 x 128256 bfloat16 with temperature and
+// penalty: 14.7 us, bound by latency (flags, history, rows); 128 x 152064: 18 us for 39 MB read and 39 MB written.
+template<int DT, bool TRANSFORM>
+__global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
+{
+    typedef Storage<DT>   S;
+    typedef typename S::T T;
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    constexpr int         EPV = 8, U = 4, NW = TSP_STAGE / WAVE;
+    constexpr uint32_t    INF16 = DT == DT_F16 ? 0x7C00u : 0x7F80u;
+    __shared__ uint32_t   window[TRANSFORM ? TSP_WINDOW : 1];
+    __shared__ float      red[16];
+    __shared__ uint32_t   any_nan;
+    const int             row = blockIdx.x, j = blockIdx.y, t = threadIdx.x;
+    const int lo   = min(s.n, j * s.chunk);
+    const int hi   = min(s.n, lo + s.chunk);
+    const int nblk = (hi - lo + TSP_BLOCK - 1) / TSP_BLOCK;
+    const T*  rowp = (const T*)s.logits + (size_t)row * s.Vp;
+    // the first blocks and everything about the row are requested together
+    uint4 raw[U];
+    auto  load = [&](int b0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // (a vector that runs over the end is put right when it is used)
+            const int v = lo + (b0 + u * NW) * TSP_BLOCK + lane_id() * EPV;
+            raw[u]      = topp_load8(rowp + max(0, min(v, s.n - EPV)));
+        }
+    };
+    load(wave_id());
+    const bool              idle = topp_row_idle(s, row);
+    const ToppTransform<DT> f(s, row);
+    const bool              hist = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
+    if (idle) {
+        return;
+    }
+    T*        y    = (T*)s.y + (size_t)row * s.y_pitch;
+    float*    bmax = s.block_max + (size_t)row * s.blocks;
+    const float mul = f.temperature_active ? f.temperature.inv : 1.0f;
+    if (s.parts > 1) {
+        uint4* counters = reinterpret_cast<uint4*>(s.counts + (size_t)row * ToppCode<DT>::COUNTERS);
+        for (int i = j * TSP_STAGE + t; i < ToppCode<DT>::COUNTERS / 4; i += s.splits * TSP_STAGE) {
+            counters[i] = make_uint4(0u, 0u, 0u, 0u);
+        }
+    }
+    if (t == 0) {
+        any_nan = 0u;
+    }
+    if (hist) {
+        const int words = (hi - lo + 31) / 32 + 1;
+        for (int i = t; i < words; i += TSP_STAGE) {
+            window[i] = 0u;
+        }
+        lds_barrier();
+        topp_walk_history(s, row, [&](int id) {
+            if (id >= lo && id < hi) {
+                atomicOr(&window[(id - lo) >> 5], 1u << ((id - lo) & 31));
+            }
+        });
+    }
+    lds_barrier();
+    float mx   = TSP_LOWEST;
+    u16x2 seen = {0, 0};  // largest magnitude bits (a NaN has the largest)
+    for (int b0 = wave_id(); b0 < nblk; b0 += U * NW) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int b = b0 + u * NW;
+            if (b < nblk) {
+                const int v  = lo + b * TSP_BLOCK + lane_id() * EPV;
+                float     vm = TSP_LOWEST;
+                T*        e  = reinterpret_cast<T*>(&raw[u]);
+                if (v + EPV > s.n) {
+                    for (int c = 0; c < EPV; ++c) {
+                        e[c] = v + c < s.n ? rowp[v + c] : (T)0;
+                    }
+                }
+                if constexpr (TRANSFORM) {
+                    const int      rel  = v - lo;
+                    const uint32_t bits = hist && v < hi ? (window[rel >> 5] >> (rel & 31)) & 0xFFu : 0u;
+                    const uint32_t end  = (uint32_t)(f.masked_end - v);
+                    if (f.bias != nullptr) {
+#pragma unroll
+                        for (int c = 0; c < EPV; ++c) {
+                            e[c] = v + c < hi ? S::st(f(v + c, S::ld(e[c]), ((bits >> c) & 1u) != 0u)) : (T)0;
+                        }
+                    }
+                    else {
+#pragma unroll
+                        for (int c = 0; c < EPV; ++c) {
+                            e[c] = S::st(S::ld(e[c]) * mul);
+                        }
+                        // columns of the history and a masked end id: few lanes
+                        if (bits != 0u || end < (uint32_t)EPV) {
+#pragma unroll
+                            for (int c = 0; c < EPV; ++c) {
+                                if ((bits >> c) & 1u) {
+                                    e[c] = S::st(repetition_value(S::ld(e[c]), f.penalty, f.penalty_type));
+                                }
+                                if (end == (uint32_t)c) {
+                                    e[c] = S::st(-S::max_t());
+                                }
+                            }
+                        }
+                    }
+                    if (v < hi) {
+                        *reinterpret_cast<uint4*>(y + v) = raw[u];  // (rows of y are padded to whole vectors)
+                    }
+                }
+                const uint32_t* w = reinterpret_cast<const uint32_t*>(&raw[u]);
+#pragma unroll
+                for (int c = 0; c < EPV / 2; ++c) {
+                    seen = __builtin_elementwise_max(seen, __builtin_bit_cast(u16x2, w[c] & 0x7FFF7FFFu));
+                }
+                if (v + EPV <= hi) {
+#pragma unroll
+                    for (int c = 0; c < EPV; ++c) {
+                        vm = __builtin_fmaxf(vm, S::ld(e[c]));
+                    }
+                }
+                else {
+                    for (int c = 0; c < EPV; ++c) {
+                        vm = __builtin_fmaxf(vm, v + c < hi ? S::ld(e[c]) : TSP_LOWEST);
+                    }
+                }
+                mx = __builtin_fmaxf(mx, vm);
+                vm = wave_reduce_unordered(vm, [](float a, float c) { return __builtin_fmaxf(a, c); });
+                if (lane_id() == 0) {
+                    bmax[lo / TSP_BLOCK + b] = vm;
+                }
+            }
+        }
+        if (b0 + U * NW < nblk) {
+            load(b0 + U * NW);
+        }
+    }
+    if (max((uint32_t)seen.x, (uint32_t)seen.y) > INF16) {
+        any_nan = 1u;
+    }
+    mx = block_max<float, NW>(mx, red, TSP_LOWEST);  // (barriers)
+    if (t == 0) {
+        s.pmax[(size_t)row * TSP_SPLITS + j] = make_float2(mx, any_nan != 0u ? 1.0f : 0.0f);
+    }
+}
+
+// ---- stage, fp32 --------------------------------------------------------------------------------------------------
+__device__ __forceinline__ int topp_y_bucket(float y, float top)
+{
+    return (int)__builtin_amdgcn_fmed3f((top - y) * TSP_SCALE, 0.0f, (float)(TSP_BUCKETS - 1));
+}
+
+// (rows x parts) workgroups; a workgroup reads the columns of its summation chains, 1024 / parts neighbouring columns
+// out of every 1024, so that its histogram says how many entries of every bucket the sum's workgroup of the same part
+// will place. Rows are the fast index of the grid: the parts of a row read interleaved stretches of one kilobyte or
+// less, and neighbouring workgroups go to different XCDs; with the parts as the fast index every XCD would see the same
+// quarter of every 4 KB and use a quarter of its L2's channels.
+template<bool TRANSFORM>
+__global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
+{
+    __shared__ uint32_t hist[TSP_BUCKETS];
+    __shared__ uint32_t window[TRANSFORM ? TSP_WINDOW : 1];
+    __shared__ float    red[16];
+    __shared__ uint32_t any_nan;
+    const int           row = blockIdx.x, j = blockIdx.y, t = threadIdx.x;
+    if (row == 0 && j == 0 && t == 0) {
+        s.queue[0] = 0u;
+    }
+    if (topp_row_idle(s, row)) {
+        return;
+    }
+    const float* rowp  = (const float*)s.logits + (size_t)row * s.Vp;
+    float*       y     = (float*)s.y + (size_t)row * s.y_pitch;
+    const int    C     = TSP_CHAINS / s.parts;
+    const int    shift = __builtin_ctz((unsigned)C);
+    const int    c0    = j * C;
+    const int    nit   = (s.n + TSP_CHAINS - 1) / TSP_CHAINS;
+    // the origin of the buckets: the largest plain value among the first 1024 columns, the same for every part
+    float first = TSP_LOWEST;
+#pragma unroll
+    for (int u = 0; u < TSP_CHAINS / TSP_STAGE; ++u) {
+        first = __builtin_fmaxf(first, rowp[t + u * TSP_STAGE]);
+    }
+    for (int i = t; i < TSP_BUCKETS; i += TSP_STAGE) {
+        hist[i] = 0u;
+    }
+    if (t == 0) {
+        any_nan = 0u;
+    }
+    const bool                  marks = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
+    const ToppTransform<DT_F32> f(s, row);
+    if (TRANSFORM && marks) {
+        const int words = (nit * C + 31) / 32 + 1;
+        for (int i = t; i < words; i += TSP_STAGE) {
+            window[i] = 0u;
+        }
+    }
+    first = block_max<float, TSP_STAGE / WAVE>(first, red, TSP_LOWEST);  // (two barriers: both tables are clear)
+    if (TRANSFORM && f.temperature_active) {
+        first = first * f.temperature.inv;
+    }
+    if (!(__builtin_fabsf(first) < 1e30f)) {
+        first = 0.0f;
+    }
+    const float top = first + TSP_ABOVE;
+    if (TRANSFORM && marks) {
+        topp_walk_history(s, row, [&](int id) {
+            const int c = (id & (TSP_CHAINS - 1)) - c0;
+            if (id >= 0 && id < s.n && c >= 0 && c < C) {
+                const int at = ((id / TSP_CHAINS) << shift) + c;
+                atomicOr(&window[at >> 5], 1u << (at & 31));
+            }
+        });
+        __syncthreads();
+    }
+    float mx  = TSP_LOWEST;
+    bool  nan = false;
+    auto  one = [&](int it, int c, float x) -> float {  // column it * 1024 + c0 + c
+        if constexpr (TRANSFORM) {
+            const int  at     = (it << shift) + c;
+            const bool marked = marks && ((window[at >> 5] >> (at & 31)) & 1u) != 0u;
+            x                 = f(it * TSP_CHAINS + c0 + c, x, marked);
+        }
+        mx  = __builtin_fmaxf(mx, x);
+        nan = nan || x != x;
+        atomicAdd(&hist[topp_y_bucket(x, top)], 1u);
+        return x;
+    };
+    const int quads = C / 4, qshift = shift - 2;  // 16-byte vectors of a workgroup in one stretch of 1024 columns
+    int       it0   = 0;
+    if ((s.Vp & 3) == 0 && ((uintptr_t)s.logits & 15u) == 0u) {
+        constexpr int U     = 8;
+        const int     nfull = s.n / TSP_CHAINS;  // stretches that lie inside the vocabulary
+        const int     total = nfull * quads;     // vectors
+        for (int i0 = t; i0 < total; i0 += U * TSP_STAGE) {
+            float4 raw[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = min(i0 + u * TSP_STAGE, total - 1);
+                raw[u]      = *reinterpret_cast<const float4*>(rowp + (size_t)(i >> qshift) * TSP_CHAINS + c0 + (i & (quads - 1)) * 4);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + u * TSP_STAGE;
+                if (i < total) {
+                    const int it = i >> qshift;
+                    const int c  = (i & (quads - 1)) * 4;
+                    float4    r  = raw[u];
+                    r.x          = one(it, c, r.x);
+                    r.y          = one(it, c + 1, r.y);
+                    r.z          = one(it, c + 2, r.z);
+                    r.w          = one(it, c + 3, r.w);
+                    if constexpr (TRANSFORM) {
+                        *reinterpret_cast<float4*>(y + (size_t)it * TSP_CHAINS + c0 + c) = r;
+                    }
+                }
+            }
+        }
+        it0 = nfull;
+    }
+    {
+        constexpr int U     = 8;
+        const int     total = (nit - it0) << shift;
+        for (int i0 = t; i0 < total; i0 += U * TSP_STAGE) {
+            float raw[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i = i0 + u * TSP_STAGE;
+                const int v = (it0 + (i >> shift)) * TSP_CHAINS + c0 + (i & (C - 1));
+                raw[u]      = i < total && v < s.n ? rowp[v] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int i  = i0 + u * TSP_STAGE;
+                const int it = it0 + (i >> shift), c = i & (C - 1);
+                const int v  = it * TSP_CHAINS + c0 + c;
+                if (i < total && v < s.n) {
+                    const float x = one(it, c, raw[u]);
+                    if constexpr (TRANSFORM) {
+                        y[v] = x;
+                    }
+                }
+            }
+        }
+    }
+    for (int v = s.n + t; v < s.Vp; v += TSP_STAGE) {  // pads lie in the lowest bucket
+        const int c = (v & (TSP_CHAINS - 1)) - c0;
+        if (c >= 0 && c < C) {
+            atomicAdd(&hist[TSP_BUCKETS - 1], 1u);
+        }
+    }
+    if (nan) {
+        any_nan = 1u;
+    }
+    mx = block_max<float, TSP_STAGE / WAVE>(mx, red, TSP_LOWEST);
+    uint32_t* out = s.counts + ((size_t)row * s.parts + j) * TSP_BUCKETS;
+    for (int i = t; i < TSP_BUCKETS / 4; i += TSP_STAGE) {
+        reinterpret_cast<uint4*>(out)[i] = reinterpret_cast<const uint4*>(hist)[i];
+    }
+    if (t == 0) {
+        s.pmax[(size_t)row * TSP_SPLITS + j] = make_float2(mx, any_nan != 0u ? 1.0f : 0.0f);
+        if (j == 0) {
+            s.ref[row] = first;
+        }
+    }
+}
+
+// The maximum of a row from what the stage's workgroups left (every lane of the wave gets it); a NaN when a sum over
+// the row would be one: there is a NaN among the values, or the maximum is infinite.
+struct ToppRowMax {
+    float2 mine;
+    __device__ __forceinline__ ToppRowMax(const ToppStep& s, int row, int n_partial)
+    {
+        const int l = min(lane_id(), n_partial - 1);
+        mine        = s.pmax[(size_t)row * TSP_SPLITS + l];  // (requested here, used in the call below)
+    }
+    template<int DT>
+    __device__ __forceinline__ float get(const ToppStep& s) const
+    {
+        float mx = mine.x;
+        if (s.Vp > s.n) {
+            mx = __builtin_fmaxf(mx, -Storage<DT>::max_t());
+        }
+        mx             = wave_reduce_unordered(mx, [](float a, float b) { return __builtin_fmaxf(a, b); });
+        const bool nan = __ballot(mine.y != 0.0f) != 0ull || mx == __builtin_inff();
+        return nan ? __builtin_nanf("") : mx;
+    }
+};
+
+// exp of d <= 0 as det_expf_nonpos gives it, for numbers; below -86 something between 0 and 1e-37 instead of the exact
+// value, which no sum over a row that holds a 1 can tell apart (its terms are far below half a unit of any such sum,
+// and the group sums without the 1 vanish against it the same way). The integer part of the argument stays in the low
+// bits of the sum with 3 * 2^22, from where it goes straight into the exponent.
+__device__ __forceinline__ float topp_exp(float d)
+{
+    d               = __builtin_fmaxf(d, -86.0f);
+    const float t   = d * 1.44269502162933349609375f + 12582912.0f;
+    const float n   = t - 12582912.0f;
+    float       r   = fma_rn(n, -0.693145751953125f, d);
+    r               = fma_rn(n, -1.428606765330187045e-06f, r);
+    float p         = 1.9875691500e-4f;
+    p               = fma_rn(p, r, 1.3981999507e-3f);
+    p               = fma_rn(p, r, 8.3334519073e-3f);
+    p               = fma_rn(p, r, 4.1665795894e-2f);
+    p               = fma_rn(p, r, 1.6666665459e-1f);
+    p               = fma_rn(p, r, 5.0000001201e-1f);
+    const float z   = r * r;
+    const float y   = fma_rn(p, z, r) + 1.0f;
+    return u2f(f2u(y) + (f2u(t) << 23));
+}
+
+// Four neighbouring lanes hold consecutive terms of one summation chain: added in their order, in every lane.
+__device__ __forceinline__ float topp_chain_add(float sum, float e)
+{
+    sum += dpp_from<0x00>(e);
+    sum += dpp_from<0x55>(e);
+    sum += dpp_from<0xAA>(e);
+    sum += dpp_from<0xFF>(e);
+    return sum;
+}
+
+// Walks the columns of a workgroup's summation chains: LPC lanes share a chain and take its columns in turn.
+// visit(v, raw) returns e; the chain's sum comes back. Batches of U columns per thread, the next batch requested before
+// the current one is used (a uniform base and a 32-bit offset per lane: one load instruction per column and no address
+// arithmetic in vector registers). `pad` is what the columns behind the vocabulary hold.
+template<class T, int LPC, int U, class Visit>
+__device__ __forceinline__ float topp_walk_chains(const T* __restrict__ y, int n, int Vp, int chain, int q, T pad, Visit&& visit)
+{
+    constexpr int  STRIDE = LPC * TSP_CHAINS;
+    float          sum    = 0.0f;
+    const uint32_t lane   = (uint32_t)(chain + q * TSP_CHAINS);
+    const int      nb     = n / (U * STRIDE);  // batches that every lane of the workgroup holds in full
+    T              buf[2][U];
+    auto           load = [&](T* raw, int b) {
+        const T* base = y + (size_t)b * (U * STRIDE);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            raw[u] = (base + u * STRIDE)[lane];
+        }
+    };
+    auto add = [&](float e) {
+        if constexpr (LPC == 1) {
+            sum += e;
+        }
+        else {
+            sum = topp_chain_add(sum, e);
+        }
+    };
+    auto use = [&](const T* raw, int b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            add(visit((int)lane + (b * U + u) * STRIDE, raw[u]));
+        }
+    };
+    if (nb > 0) {
+        load(buf[0], 0);
+    }
+    for (int b = 0; b < nb; b += 2) {
+        load(buf[1], min(b + 1, nb - 1));
+        use(buf[0], b);
+        load(buf[0], min(b + 2, nb - 1));
+        if (b + 1 < nb) {
+            use(buf[1], b + 1);
+        }
+    }
+    // what does not fill a batch (columns beyond the row count as nothing)
+    for (int v0 = nb * U * STRIDE; v0 < Vp; v0 += U * STRIDE) {
+        T raw[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int v = v0 + u * STRIDE + (int)lane;
+            raw[u]      = y[min(v, n - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int v = v0 + u * STRIDE + (int)lane;
+            if (v0 + u * STRIDE < Vp) {  // (the same for every lane)
+                add(v < Vp ? visit(v, v < n ? raw[u] : pad) : 0.0f);
+            }
+        }
+    }
+    return sum;
+}
+
+// The xor butterflies inside 32-lane groups over the chain sums of the workgroup; the sums of the groups go to memory.
+template<int THREADS, int LPC>
+__device__ __forceinline__ void topp_group_sums(const ToppStep& s, int row, int part, float sum, float* chain_sum)
+{
+    constexpr int C = THREADS / LPC;
+    const int     t = threadIdx.x;
+    if (LPC == 1 || (t % LPC) == 0) {
+        chain_sum[t / LPC] = sum;
+    }
+    __syncthreads();
+    if (t < C) {
+        float v = chain_sum[t];
+#pragma unroll
+        for (int m = 16; m > 0; m >>= 1) {
+            v += __shfl_xor(v, m, 32);
+        }
+        if ((t & 31) == 0) {
+            s.gsum[(size_t)row * 32 + part * (C / 32) + (t >> 5)] = v;
+        }
+    }
+}
+
+// ---- sum, 16-bit types ----------------------------------------------------------------------------------------------
+// A workgroup owns C summation chains: C neighbouring columns out of every 1024 (a "stretch"). Its waves share the
+// stretches out, read eight bytes - four chains - per lane and leave the e of a chunk of stretches in LDS, from where
+// one thread per chain adds them up in the reference's order. (One chain per thread straight from memory means two-byte
+// loads and a dependent addition per load: 14 us for 64 x 128256 bfloat16 whatever is done with the values.)
+// e is a function of the 16 bits of y once the maximum is known: with LUT the workgroup first works it out for the values
+// that occur in earnest (4096 for bfloat16, 28672 for binary16) and then looks it up. Values outside the table (tiny or
+// huge magnitudes, -inf) take the exponential.
+template<int DT, int C, bool LUT>
+__global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
+{
+    typedef Storage<DT>   S;
+    typedef typename S::T T;
+    typedef ToppCode<DT>  Code;
+    constexpr int         KI  = 16384 / C;                 // stretches of a chunk: 32 KB of e
+    constexpr int         WS  = C / 4 / WAVE;              // waves side by side in a stretch
+    constexpr int         PAR = TSP_SUM16 / WAVE / WS;     // stretches taken at a time
+    constexpr int         U   = KI / PAR;                  // vectors per lane and chunk
+    __shared__ uint32_t   cnt[Code::USED + WAVE];
+    __shared__ T          lut[LUT ? 2 * Code::LUT_N : 1];
+    __shared__ uint2      e_of[KI * C / 4];
+    const int             row = blockIdx.x, part = blockIdx.y, t = threadIdx.x;
+    const T* y = s.y != nullptr ? (const T*)s.y + (size_t)row * s.y_pitch : (const T*)s.logits + (size_t)row * s.Vp;
+    const int q    = (t & (C / 4 - 1)) * 4 + part * C;  // first of this lane's four chains
+    const int mine = t / (C / 4);                       // its first stretch
+    const int nst  = (s.Vp + TSP_CHAINS - 1) / TSP_CHAINS;
+    // Four vectors of the lane are in flight; the loop that uses them stays a loop (straight-line code of this length
+    // runs once and waits for its own fetch).
+    const int total = (nst + PAR - 1 - mine) / PAR;  // vectors of this lane
+    auto      load  = [&](int k) -> uint2 {          // its k-th one
+        const int v = (mine + min(k, total - 1) * PAR) * TSP_CHAINS + q;
+        uint2     x;
+        // (columns behind the vocabulary are put right where they are used: any four columns of the row will do here)
+        __builtin_memcpy(&x, y + max(0, min(v, s.n - 4)), 8);
+        return x;
+    };
+    uint2 r0 = load(0), r1 = load(1), r2 = load(2), r3 = load(3);
+    if (topp_row_idle(s, row)) {
+        return;
+    }
+    const ToppRowMax rm(s, row, s.splits);
+    for (int i = t; i < Code::USED; i += TSP_SUM16) {
+        cnt[i] = 0u;
+    }
+    const float mx = rm.get<DT>(s);
+    if (!(mx == mx)) {
+        return;  // (the pick sees the same and needs no sum)
+    }
+    if constexpr (LUT) {
+#pragma unroll 1
+        for (int i = t; i < 2 * Code::LUT_N; i += TSP_SUM16) {
+            const T bits = (T)(i < Code::LUT_N ? Code::LUT_LOW + i : 0x8000 + Code::LUT_LOW + (i - Code::LUT_N));
+            lut[i]       = S::st(topp_exp(__builtin_fminf(S::ld(bits) - mx, 0.0f)));
+        }
+    }
+    __syncthreads();
+    // The e of N values, counted: all look-ups are requested before the first one is used, values that are not in the
+    // table are put right together, and what has no counter goes to a word of the lane's own.
+    auto e_bits = [&](const auto& x, auto& b) {
+        constexpr int N = (int)(sizeof(x) / sizeof(x[0]));
+        if constexpr (LUT) {
+            uint32_t out = 0u;
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                const uint32_t mag = (x[c] & 0x7FFFu) - (uint32_t)Code::LUT_LOW;
+                out                = max(out, mag);
+                b[c]               = lut[min(mag, (uint32_t)Code::LUT_N - 1u) + (x[c] >> 15) * (uint32_t)Code::LUT_N];
+            }
+            if (out >= (uint32_t)Code::LUT_N) {
+#pragma unroll 1
+                for (int c = 0; c < N; ++c) {
+                    const uint32_t xc = N == 1 || c == 0 ? x[0] : c == 1 ? x[N > 1 ? 1 : 0] : c == 2 ? x[N > 2 ? 2 : 0] : x[N - 1];
+                    if ((xc & 0x7FFFu) - (uint32_t)Code::LUT_LOW >= (uint32_t)Code::LUT_N) {
+                        const uint32_t e = S::st(topp_exp(S::ld((T)xc) - mx));
+#pragma unroll
+                        for (int k = 0; k < N; ++k) {
+                            b[k] = k == c ? e : b[k];
+                        }
+                    }
+                }
+            }
+        }
+        else {
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                b[c] = S::st(topp_exp(S::ld((T)x[c]) - mx));
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            const int code = (int)b[c] - Code::BASE;
+            atomicAdd(&cnt[code > 0 ? code : Code::USED + lane_id()], 1u);
+        }
+    };
+    const uint32_t pad = S::st(-S::max_t());
+    float          sum = 0.0f;
+    int            at  = 0;
+    for (int i0 = 0; i0 < nst; i0 += KI) {
+#pragma unroll 1
+        for (int u = 0; u < U; ++u, ++at) {
+            const int i = mine + u * PAR;
+            const int v = (i0 + i) * TSP_CHAINS + q;
+            if (i0 + i >= nst) {
+                break;
+            }
+            const uint2 raw = r0;
+            r0 = r1;
+            r1 = r2;
+            r2 = r3;
+            r3 = load(at + 4);
+            uint32_t b[4];
+            if (v + 4 <= s.n) {
+                const uint32_t x[4] = {raw.x & 0xFFFFu, raw.x >> 16, raw.y & 0xFFFFu, raw.y >> 16};
+                e_bits(x, b);
+            }
+            else {
+#pragma unroll 1
+                for (int c = 0; c < 4; ++c) {
+                    uint32_t e = 0u;
+                    if (v + c < s.Vp) {
+                        const uint32_t x[1] = {v + c < s.n ? (uint32_t)y[v + c] : pad};
+                        uint32_t       one[1];
+                        e_bits(x, one);
+                        e = one[0];
+                    }
+                    b[0] = c == 0 ? e : b[0];
+                    b[1] = c == 1 ? e : b[1];
+                    b[2] = c == 2 ? e : b[2];
+                    b[3] = c == 3 ? e : b[3];
+                }
+            }
+            e_of[i * (C / 4) + (t & (C / 4 - 1))] = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+        }
+        lds_barrier();
+        if (t < C) {
+            const T*  e = reinterpret_cast<const T*>(e_of) + t;
+            const int k = min(KI, nst - i0);
+#pragma unroll 8
+            for (int i = 0; i < k; ++i) {
+                sum += S::ld(e[i * C]);
+            }
+        }
+        lds_barrier();
+    }
+    if (t < C) {
+#pragma unroll
+        for (int m = 16; m > 0; m >>= 1) {
+            sum += __shfl_xor(sum, m, 32);
+        }
+        if ((t & 31) == 0) {
+            s.gsum[(size_t)row * 32 + part * (C / 32) + (t >> 5)] = sum;
+        }
+    }
+    uint32_t* counters = s.counts + (size_t)row * Code::COUNTERS;
+    if (gridDim.y == 1) {
+        for (int i = t; i < Code::COUNTERS; i += TSP_SUM16) {
+            counters[i] = i < Code::USED ? cnt[i] : 0u;
+        }
+    }
+    else {
+        for (int i = t; i < Code::USED; i += TSP_SUM16) {
+            const uint32_t c = cnt[i];
+            if (c != 0u) {
+                atomicAdd(&counters[i], c);
+            }
+        }
+    }
+}
+
+// ---- sum, fp32 --------------------------------------------------------------------------------------------------------
+// Where the draw must lie comes from the stage's histogram: a bucket's mass is at least its count times the exponential
+// of its lower edge, the whole row's at most the same with the upper edges. Everything down to the bucket that certainly
+// covers the draw - and two more, so that all entries which share a probability with the last one that can be drawn are
+// there - goes to its bucket's place in the prefix, keyed by e (the division by the denominator keeps the order).
+template<int LPC>
+__global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
+{
+    constexpr int       C  = TSP_SUM32 / LPC;
+    constexpr int       K  = TSP_BUCKETS / TSP_SUM32;
+    constexpr int       NW = TSP_SUM32 / WAVE;
+    __shared__ uint32_t cur[TSP_BUCKETS];
+    __shared__ float    chain_sum[C];
+    __shared__ float    wmass[NW], wupper[NW];
+    __shared__ uint32_t wcnt[NW], wseg[NW];
+    __shared__ uint32_t red32[16];
+    const int           row = blockIdx.x, part = blockIdx.y, t = threadIdx.x;
+    if (topp_row_idle(s, row)) {
+        return;
+    }
+    const void*         safe = s.pmax;
+    const RowDrawSource ds   = row_draw_source(s.rng, s.uniforms, row, safe);
+    const float         p    = row_arg_or(s.top_ps, row, safe, s.top_p);
+    const ToppRowMax    rm(s, row, s.parts);
+    const float         ref = s.ref[row];
+    const float* y    = s.y != nullptr ? (const float*)s.y + (size_t)row * s.y_pitch : (const float*)s.logits + (size_t)row * s.Vp;
+    // thread t owns buckets [K t, K t + K), in descending order of y
+    uint32_t tot[K], before[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        tot[i] = before[i] = 0u;
+    }
+    const uint4* counts = reinterpret_cast<const uint4*>(s.counts + (size_t)row * s.parts * TSP_BUCKETS);
+#pragma unroll 4
+    for (int q = 0; q < 4 * LPC; ++q) {
+#pragma unroll
+        for (int i = 0; i < K / 4; ++i) {
+            const uint4    c    = counts[(q * TSP_BUCKETS + t * K) / 4 + i];
+            const uint32_t w[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                before[i * 4 + k] += q < part ? w[k] : 0u;
+                tot[i * 4 + k] += w[k];
+            }
+        }
+    }
+    const float mx = rm.get<DT_F32>(s);
+    if (!(mx == mx)) {
+        return;  // (the pick sees the same and needs no sum)
+    }
+    uint64_t    next;
+    const float draw = (s.uniforms != nullptr ? ds.injected : row_draw_generate(ds, &next)) * p;
+    const float top  = ref + TSP_ABOVE;
+    const float lead = top - mx;  // y of the first bucket's upper edge, relative to the maximum
+    const int   mx_bucket = topp_y_bucket(mx, top);
+    float       lower[K], lm = 0.0f, lu = 0.0f;
+    uint32_t    lc = 0u;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int   b     = t * K + i;
+        const float up    = b == 0 ? 1.0f : __builtin_amdgcn_exp2f(__builtin_fminf(lead - (float)b / TSP_SCALE, 0.0f) * 1.44269504f);
+        const float below = b == TSP_BUCKETS - 1 ? 0.0f :
+                                                   __builtin_amdgcn_exp2f(__builtin_fminf(lead - (float)(b + 1) / TSP_SCALE, 0.0f) * 1.44269504f);
+        const float n     = (float)tot[i];
+        lower[i]          = tot[i] == 0u ? 0.0f : n * below;
+        lu += tot[i] == 0u ? 0.0f : n * up;
+        if (b == mx_bucket) {
+            lower[i] += 1.0f - below;  // the maximum itself lies here
+        }
+        lm += lower[i];
+        lc += tot[i];
+    }
+    float    im = lm, iu = lu;
+    uint32_t ic = lc;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const float    um = __shfl_up(im, o, WAVE), uu = __shfl_up(iu, o, WAVE);
+        const uint32_t uc = __shfl_up(ic, o, WAVE);
+        if (lane_id() >= o) {
+            im += um;
+            iu += uu;
+            ic += uc;
+        }
+    }
+    if (lane_id() == WAVE - 1) {
+        wmass[wave_id()]  = im;
+        wupper[wave_id()] = iu;
+        wcnt[wave_id()]   = ic;
+    }
+    __syncthreads();
+    float    em = im - lm, upper = 0.0f;
+    uint32_t ec = ic - lc;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        em += w < wave_id() ? wmass[w] : 0.0f;
+        ec += w < wave_id() ? wcnt[w] : 0u;
+        upper += wupper[w];
+    }
+    const float want  = draw * (upper + 1e-6f) * (1.0f + 1.0f / 256.0f);
+    uint32_t    first = 0xFFFFFFFFu;
+    {
+        float m = em;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            m += lower[i];
+            if (m >= want && first == 0xFFFFFFFFu) {
+                first = (uint32_t)(t * K + i);
+            }
+        }
+    }
+    first         = block_min<uint32_t, NW>(first, red32, 0xFFFFFFFFu);
+    const int cut = (int)min(first == 0xFFFFFFFFu ? first : first + 2u, (uint32_t)(TSP_BUCKETS - 1));
+    // (a row whose values are all -inf takes the exact fallback)
+    const bool usable = mx > TSP_LOWEST;
+    uint32_t   off[K + 1];
+    off[0] = ec;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        off[i + 1]     = off[i] + tot[i];
+        cur[t * K + i] = off[i] + before[i];
+    }
+    if (part == 0) {
+        // the prefix in segments of whole buckets for the sort: a bucket closes a segment when a multiple of TPS_SEG
+        // lies inside it or at its end, and the last gathered bucket closes the last one
+        uint32_t n_mine = 0u;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            n_mine += t * K + i <= cut ? tot[i] : 0u;
+        }
+        n_mine = (uint32_t)wave_sum_i((int)n_mine);
+        if (lane_id() == 0) {
+            wseg[wave_id()] = n_mine;
+        }
+        __syncthreads();
+        uint32_t n = 0u;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            n += wseg[w];
+        }
+        uint32_t closes[K], lclose = 0u;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            const bool in = t * K + i <= cut && tot[i] != 0u;
+            closes[i]     = in && (off[i + 1] / TPS_SEG != off[i] / TPS_SEG || off[i + 1] == n) ? off[i + 1] : 0u;
+            lclose += closes[i] != 0u ? 1u : 0u;
+        }
+        uint32_t iclose = lclose;
+#pragma unroll
+        for (int o = 1; o < WAVE; o <<= 1) {
+            const uint32_t up = __shfl_up(iclose, o, WAVE);
+            if (lane_id() >= o) {
+                iclose += up;
+            }
+        }
+        __syncthreads();
+        if (lane_id() == WAVE - 1) {
+            wseg[wave_id()] = iclose;
+        }
+        __syncthreads();
+        uint32_t at = iclose - lclose, nseg = 0u;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            at += w < wave_id() ? wseg[w] : 0u;
+            nseg += wseg[w];
+        }
+        uint32_t* ends = s.segs + (size_t)row * TPB_NB;
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            if (closes[i] != 0u) {
+                ends[at++] = closes[i];
+            }
+        }
+        if (t == 0) {
+            ToppRowMeta m;
+            m.best  = 0ull;
+            m.cut   = cut;
+            m.n     = usable ? (int)n : 0;
+            m.n_pos = (int)s.Vp;  // the prefix is the whole row exactly when it holds this many entries
+            m.nseg  = (int)nseg;
+            m.flags = 0;
+            // (half a bucket under the one that covers the draw: a bucket and a half above what is not gathered)
+            m.safe      = __builtin_amdgcn_exp2f((lead - ((float)cut - 0.5f) / TSP_SCALE) * 1.44269504f);
+            s.meta[row] = m;
+            wseg[0]     = 0u;
+            if (usable && n > (uint32_t)TPS_CAP) {
+                // prefixes that fit its LDS are ordered by the pick kernel itself, longer ones by the sort's workgroups
+                wseg[0] = atomicAdd(s.queue, nseg) + 1u;
+            }
+        }
+        __syncthreads();
+        if (wseg[0] != 0u) {
+            for (uint32_t i = (uint32_t)t; i < nseg; i += TSP_SUM32) {
+                s.queue[wseg[0] + i] = (uint32_t)row * TPB_NB + i;
+            }
+        }
+    }
+    __syncthreads();
+    unsigned long long* A     = s.sorted + (size_t)row * 2 * s.Vp;
+    // nothing under this lies in the gathered buckets (one bucket of margin)
+    const float         y_low = cut >= TSP_BUCKETS - 1 ? -__builtin_inff() : top - (float)(cut + 2) / TSP_SCALE;
+    const float sum = topp_walk_chains<float, LPC, 16>(y, s.n, s.Vp, part * C + t / LPC, t % LPC, -Storage<DT_F32>::max_t(), [&](int v, float x) -> float {
+        const float e = topp_exp(x - mx);
+        if (x >= y_low && usable) {
+            const int b = topp_y_bucket(x, top);
+            if (b <= cut) {
+                const uint32_t slot = atomicAdd(&cur[b], 1u);
+                const float    ex   = x - mx < -86.0f ? det_expf_nonpos(x - mx) : e;
+                A[slot]             = ((unsigned long long)(~order_key_nonneg(ex)) << 32) | (uint32_t)v;
+            }
+        }
+        return e;
+    });
+    topp_group_sums<TSP_SUM32, LPC>(s, row, part, sum, chain_sum);
+}
+
+// ---- sort, fp32: the segments of long prefixes, dealt out over the launch
+__global__ void __launch_bounds__(TP_THREADS) topp_sort_queue_kernel(ToppStep s)
+{
+    __shared__ ToppSortShared ss;
+    const uint32_t            n = s.queue[0];
+    for (uint32_t w = blockIdx.x; w < n; w += gridDim.x) {
+        const uint32_t      at   = s.queue[1 + w];
+        const int           row  = (int)(at / TPB_NB), i = (int)(at % TPB_NB);
+        const uint32_t*     ends = s.segs + (size_t)row * TPB_NB;
+        const int           s0   = i > 0 ? (int)ends[i - 1] : 0;
+        unsigned long long* A    = s.sorted + (size_t)row * 2 * s.Vp;
+        topp_sort_one(ss, A + s0, A + s.Vp + s0, (int)ends[i] - s0);
+        __syncthreads();
+    }
+}
+
+// ---- pick -------------------------------------------------------------------------------------------------------------
+// A pick is a chain of short steps on one row, bound by latency: everything it reads from memory that does not depend on
+// an earlier step is requested at its start, without control flow (256 fp32 rows with short prefixes: 9 us, 31 us with
+// loads where they are used and a sort of every prefix through memory).
+struct ToppPickOut {
+    int*          ids;
+    int*          sequence_length;
+    bool*         finished;
+    float*        cum_log_probs;
+    float*        output_log_probs;
+    RngState*     rng;
+    ToppDecayArgs dec;
+    int           force_deep;
+};
+
+struct ToppPicked {
+    int   id;
+    float prob;
+    bool  sampled;  // false: the draw was never reached; the id is kept, nothing else is updated (:954)
+};
+
+template<int DT>
+struct ToppPickRow {
+    typedef Storage<DT>  S;
+    typedef typename S::T T;
+    int           row;
+    bool          skip, fin;
+    float         p;
+    RowDrawSource draw;
+    ToppRowMax    rm;
+    float         group;  // one group sum of the row
+    int           end_id, length;
+    float         cum, decay_p, decay_initial, decay_factor, decay_min;
+    int           decay_reset;
+    const T*      y;
+    // worked out later
+    float mx, denom, rand_num;
+
+    __device__ __forceinline__ ToppPickRow(const ToppStep& s, const ToppPickOut& o, int row_, int n_partial):
+        row(row_), rm(s, row_, n_partial)
+    {
+        const void* safe = s.gsum;
+        group         = s.gsum[(size_t)row * 32 + (lane_id() & 31)];
+        skip          = row_flag_or(s.skip, row, safe, false);
+        fin           = row_flag_or(s.finished, row, safe, false);
+        p             = row_arg_or(s.top_ps, row, safe, s.top_p);
+        draw          = row_draw_source(s.rng, s.uniforms, row, safe);
+        end_id        = row_arg_or(s.end_ids, row, safe, -1);
+        length        = row_arg_or(o.sequence_length, row, safe, 0);
+        cum           = row_arg_or(o.cum_log_probs, row, safe, 0.0f);
+        decay_p       = row_arg_or(o.dec.runtime_top_p, row, safe, 0.0f);
+        decay_initial = row_arg_or(o.dec.runtime_top_p != nullptr ? o.dec.initial_top_p : nullptr, row, safe, 0.0f);
+        decay_factor  = row_arg_or(o.dec.runtime_top_p != nullptr ? o.dec.decay : nullptr, row, safe, 0.0f);
+        decay_min     = row_arg_or(o.dec.runtime_top_p != nullptr ? o.dec.top_p_min : nullptr, row, safe, 0.0f);
+        decay_reset   = row_arg_or(o.dec.runtime_top_p != nullptr ? o.dec.reset_ids : nullptr, row, safe, 0);
+        y             = s.y != nullptr ? (const T*)s.y + (size_t)row * s.y_pitch : (const T*)s.logits + (size_t)row * s.Vp;
+    }
+    // One wave or more: the draw (its state goes on), the maximum, the denominator: the reference's second butterfly.
+    __device__ __forceinline__ void derive(const ToppStep& s, const ToppPickOut& o)
+    {
+        uint64_t    next = 0;
+        const float u    = s.uniforms != nullptr ? draw.injected : row_draw_generate(draw, &next);
+        if (s.uniforms == nullptr && threadIdx.x == 0) {
+            o.rng[row].offset = next;  // drawn for every row that is not skipped
+        }
+        rand_num = u * p;
+        if (fin) {
+            // a finished row: its end id alone has e = 1, or, when that lies outside the vocabulary, every column has
+            const bool inside = end_id >= 0 && end_id < s.n;
+            mx                = inside ? S::max_t() : -S::max_t();
+            denom             = (inside ? 1.0f : (float)s.Vp) + 1e-6f;
+        }
+        else {
+            mx      = rm.template get<DT>(s);
+            float v = group;
+#pragma unroll
+            for (int m = 16; m > 0; m >>= 1) {
+                v += __shfl_xor(v, m, 32);
+            }
+            denom = v + 1e-6f;  // (both halves of the wave hold the same group sums)
+        }
+    }
+    // A single thread, once: what the row leaves behind, the decay of its p included.
+    __device__ __forceinline__ void finish(const ToppPickOut& o, ToppPicked r) const
+    {
+        o.ids[row] = r.id;
+        if (r.sampled) {
+            if (o.cum_log_probs != nullptr || o.output_log_probs != nullptr) {
+                const float lp = det_logf(r.prob);
+                if (o.cum_log_probs != nullptr) {
+                    o.cum_log_probs[row] = cum + lp;
+                }
+                if (o.output_log_probs != nullptr) {
+                    o.output_log_probs[row] = lp;
+                }
+            }
+            if (o.sequence_length != nullptr && o.finished != nullptr) {
+                o.sequence_length[row] = fin ? length : length + 1;
+                o.finished[row]        = r.id == end_id;
+            }
+        }
+        decay(o, r.id);
+    }
+    __device__ __forceinline__ void decay(const ToppPickOut& o, int id) const
+    {
+        if (o.dec.runtime_top_p != nullptr) {
+            o.dec.runtime_top_p[row] = id == decay_reset ? decay_initial : __builtin_fmaxf(decay_p * decay_factor, decay_min);
+        }
+    }
+    // Rows that need no look at their columns (every thread gets the same answer): a NaN somewhere, so that no
+    // probability is comparable and the reference keeps id 0, or finished with an ordinary end id.
+    __device__ __forceinline__ bool trivial(const ToppStep& s, ToppPicked& r) const
+    {
+        if (!fin && !(mx == mx)) {
+            r = ToppPicked{0, 0.0f, false};
+            return true;
+        }
+        if (fin && end_id >= 0 && end_id < s.n) {
+            const float one = topp_prob_of<DT>(1.0f, RowDivisor(denom), denom);
+            r               = ToppPicked{end_id, one, round_t<DT>(0.0f + one) >= p || rand_num <= one};
+            return true;
+        }
+        return false;
+    }
+};
+
+// What the exact fallback needs of a row (the whole row, ordered): a draw that is not crossed inside what the step has
+// ordered, or a row without anything ordered.
+template<int DT>
+struct ToppWholeRow {
+    const typename Storage<DT>::T* y;
+    int                            n, Vp, end_id;
+    float                          mx, denom, p, rand_num;
+    bool                           fin;
+    unsigned long long*            sorted;
+};
+
+template<int DT>
+__device__ __attribute__((noinline)) ToppPicked topp_pick_whole_row(TopPScan& sc, unsigned long long* digits, ToppWholeRow<DT> r)
+{
+    typedef Storage<DT> S;
+    const RowDivisor    div(r.denom);
+    const ToppRowValues vals{S::max_t(), r.fin, r.end_id, r.n};
+    auto                prob_at = [&](int v) -> float {
+        const float x = vals.masked(v, v < r.n ? S::ld(r.y[v]) : 0.0f);
+        return topp_prob_of<DT>(round_t<DT>(det_expf_nonpos(x - r.mx)), div, r.denom);
+    };
+    const unsigned long long* src  = sort_whole_row(sc, digits, prob_at, r.Vp, r.sorted, r.sorted + r.Vp);
+    const int                 n    = sc.misc[2];
+    const int                 id   = n > 0 ? (int)(uint32_t)src[0] : 0;
+    const float               best = n > 0 ? key64_prob(src[0]) : prob_at(0);
+    if (round_t<DT>(0.0f + best) >= r.p) {
+        return ToppPicked{id, best, true};
+    }
+    const int found = n > 0 ? scan_tiles<1>(sc, (n + TP_TILE - 1) / TP_TILE, r.rand_num,
+                                            [&](int tile, int l, float* x) { tile_load(src, n, tile, l, x); }) :
+                              -1;
+    if (found < 0) {
+        return ToppPicked{id, best, false};
+    }
+    if (found < n) {
+        return ToppPicked{(int)(uint32_t)src[found], key64_prob(src[found]), true};
+    }
+    if (threadIdx.x == 0) {
+        sc.misc[3] = nth_zero_entry(prob_at, r.Vp, found - n);
+    }
+    __syncthreads();
+    const int z = sc.misc[3];
+    return ToppPicked{z, prob_at(z), true};
+}
+
+// The scan of at most as many tiles as the workgroup's first THREADS threads have 32-lane groups, every group with its
+// tile in registers: load(tile, l, x) as for scan_tiles. `agg` holds one float per group, `*found` (set to INT_MAX in
+// front of the call, a barrier in between) gets the position the reference would pick. Two barriers; every thread of the
+// workgroup calls.
+template<int THREADS, class LoadTile>
+__device__ __forceinline__ int scan_few_tiles(float* agg, int* found, int nt, float rand_num, LoadTile&& load)
+{
+    const int t = threadIdx.x, group = t >> 5, l = t & 31;
+    float     x[8], incl = 0.0f;
+    const bool mine = t < THREADS && group < nt;
+    if (mine) {
+        load(group, l, x);
+        incl = tile_scan(x, l);
+        if (l == 31) {
+            agg[group] = incl;
+        }
+    }
+    __syncthreads();
+    if (mine) {
+        float prefix = 0.0f;
+        for (int g = 0; g < group; ++g) {
+            prefix = prefix + agg[g];
+        }
+        const float excl = __shfl_up(incl, 1, 32);
+        float       a    = l == 0 ? prefix : prefix + excl;
+        uint32_t    m8   = 0u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            a = a + x[j];
+            if (rand_num <= a) {
+                m8 |= 1u << j;
+            }
+        }
+        // the reference looks at words of 32 positions, four lanes here: the first that holds a crossing counts
+        // from its end
+        int c = __popc(m8);
+        c += dpp_from<DPP_QUAD_XOR1>(c);
+        c += dpp_from<DPP_QUAD_XOR2>(c);
+        const unsigned long long b     = __ballot(m8 != 0u);
+        const uint32_t           lanes = (uint32_t)(b >> (lane_id() & 32));
+        if (lanes != 0u) {
+            const int first = __builtin_ctz(lanes) >> 2;
+            if (l == first * 4) {
+                atomicMin(found, group * TP_TILE + first * 32 + (32 - c));
+            }
+        }
+    }
+    __syncthreads();
+    return *found == 0x7FFFFFFF ? -1 : *found;
+}
+
+// ---- pick, fp32
+// The prefix is ordered by (e, id). Entries whose e differ can share a probability; the scan's sums do not depend on
+// the order of equal values, only the emitted id does: the reference emits, of the entries that share the probability
+// at position `found`, the one with as many smaller ids as there are entries of the run in front of `found`. Every
+// thread calls and gets the entry.
+template<class Prob>
+__device__ __forceinline__ unsigned long long topp_settle_run(TopPScan& s, const unsigned long long* A, int n, int found,
+                                                              int vocab, Prob&& prob)
+{
+    const int t = threadIdx.x;
+    if (t == 0) {
+        // both ends of the run are looked for outwards from `found` in doubling steps, then by bisection
+        const float here = prob(A[found]);
+        auto        same = [&](int i) { return prob(A[i]) == here; };
+        int         hi = found, lo = 0;  // first position of the run: in [lo, hi], A[hi] belongs to it
+        for (int step = 1;; step <<= 1) {
+            const int probe = hi - step;
+            if (probe < 0) {
+                lo = 0;
+                break;
+            }
+            if (!same(probe)) {
+                lo = probe + 1;
+                break;
+            }
+            hi = probe;
+        }
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (same(mid)) {
+                hi = mid;
+            }
+            else {
+                lo = mid + 1;
+            }
+        }
+        const int a = lo;
+        lo          = found;
+        hi          = n - 1;  // last position of the run: in [lo, hi], A[lo] belongs to it
+        for (int step = 1;; step <<= 1) {
+            const int probe = lo + step;
+            if (probe > n - 1) {
+                hi = n - 1;
+                break;
+            }
+            if (!same(probe)) {
+                hi = probe - 1;
+                break;
+            }
+            lo = probe;
+        }
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (same(mid)) {
+                lo = mid;
+            }
+            else {
+                hi = mid - 1;
+            }
+        }
+        s.misc[4] = a;
+        s.misc[5] = lo;
+        s.misc[6] = (uint32_t)(A[a] >> 32) != (uint32_t)(A[lo] >> 32) ? 1 : 0;
+    }
+    __syncthreads();
+    if (s.misc[6] == 0) {
+        return A[found];  // one numerator: already in order of ids
+    }
+    // the id with exactly (found - a) smaller ids in the run: bisection over the ids, counting with all threads
+    const int a = s.misc[4], b = s.misc[5];
+    const int want = found - a;
+    int       lo = 0, hi = vocab;
+    while (hi - lo > 1) {
+        const int mid = lo + (hi - lo) / 2;
+        if (t == 0) {
+            s.misc[7] = 0;
+        }
+        __syncthreads();
+        int mine = 0;
+        for (int i = a + t; i <= b; i += TP_THREADS) {
+            mine += (int)(uint32_t)A[i] < mid ? 1 : 0;
+        }
+        mine = wave_sum_i(mine);
+        if (lane_id() == 0 && mine != 0) {
+            atomicAdd(&s.misc[7], mine);
+        }
+        __syncthreads();
+        const int below_mid = s.misc[7];
+        __syncthreads();
+        if (below_mid > want) {
+            hi = mid;
+        }
+        else {
+            lo = mid;
+        }
+    }
+    return (A[found] & 0xFFFFFFFF00000000ull) | (uint32_t)lo;
+}
+
+constexpr int TPF_SMALL = 512;  // prefixes up to this many entries are ordered by counting ranks in LDS
+
+__global__ void __launch_bounds__(TP_THREADS) topp_pick_f32_kernel(ToppStep s, ToppPickOut o)
+{
+    __shared__ TopPScan       sc;
+    __shared__ ToppSortShared ss;
+    __shared__ int            sh_found;
+    static_assert(sizeof(ss.buf) >= TP_DIGITS * sizeof(unsigned long long), "digit counters");
+    static_assert(sizeof(ss.buf) >= 2 * TPF_SMALL * sizeof(unsigned long long), "ranks");
+    const int           row = blockIdx.x;
+    const int           t   = threadIdx.x;
+    unsigned long long* A   = s.sorted + (size_t)row * 2 * s.Vp;
+    ToppPickRow<DT_F32> r(s, o, row, s.parts);
+    const ToppRowMeta   m    = s.meta[row];  // (a row without a record: what an earlier launch left, not looked at)
+    unsigned long long  mine = A[min(t, s.Vp - 1)];
+    if (t == 0) {
+        sh_found = 0x7FFFFFFF;
+    }
+    if (r.skip) {
+        if (t == 0) {
+            r.decay(o, o.dec.runtime_top_p != nullptr ? o.ids[row] : 0);
+        }
+        return;
+    }
+    r.derive(s, o);
+    ToppPicked res;
+    if (r.trivial(s, res)) {
+        if (t == 0) {
+            r.finish(o, res);
+        }
+        return;
+    }
+    const RowDivisor div(r.denom);
+    auto prob = [&](unsigned long long entry) { return topp_prob_of<DT_F32>(key64_prob(entry), div, r.denom); };
+    if (!r.fin && !o.force_deep && m.n > 0) {
+        const int                 n   = m.n;
+        const bool                all = n == m.n_pos;
+        const unsigned long long* src = A;
+        if (n <= TPF_SMALL) {
+            // every entry's rank is the number of smaller ones (entries are distinct: ids are)
+            unsigned long long* in  = ss.buf;
+            unsigned long long* out = ss.buf + TPF_SMALL;
+            if (t < n) {
+                in[t] = mine;
+            }
+            __syncthreads();
+            // (a whole number of waves per copy of the list: 1024 / copies threads look at n / copies entries each)
+            const int per    = n <= 64 ? 64 : n <= 128 ? 128 : n <= 256 ? 256 : 512;
+            const int copies = TP_THREADS / per;
+            const int who = t & (per - 1), copy = t / per;
+            uint32_t* rank = ss.hist;
+            if (t < TPF_SMALL) {
+                rank[t] = 0u;
+            }
+            __syncthreads();
+            if (who < n) {
+                const unsigned long long key  = in[who];
+                const int                step = (n + copies - 1) / copies;
+                const int                j0 = copy * step, j1 = min(n, j0 + step);
+                uint32_t                 below = 0u;
+                for (int j = j0; j < j1; ++j) {
+                    below += in[j] < key ? 1u : 0u;
+                }
+                if (below != 0u) {
+                    atomicAdd(&rank[who], below);
+                }
+            }
+            __syncthreads();
+            if (t < n) {
+                out[rank[t]] = mine;
+            }
+            __syncthreads();
+            src = out;
+        }
+        else if (n <= TPS_CAP) {
+            topp_sort_one(ss, A, A, n);
+            __threadfence_block();
+            __syncthreads();
+        }
+        const unsigned long long best   = topp_settle_run(sc, src, n, 0, s.Vp, prob);
+        const float              p_best = prob(best);
+        // whether all entries that share the probability of the one at position i are in the prefix
+        auto whole_run = [&](int i) { return all || key64_prob(src[i]) >= m.safe; };
+        if (p_best > 0.0f && whole_run(0)) {
+            if (0.0f + p_best >= r.p) {
+                // arg-max shortcut of the reference (:842-849)
+                if (t == 0) {
+                    r.finish(o, ToppPicked{(int)(uint32_t)best, p_best, true});
+                }
+                return;
+            }
+            auto load = [&](int tile, int l, float* x) {
+                const int i0 = tile * TP_TILE + l * 8;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    x[k] = i0 + k < n ? prob(src[i0 + k]) : 0.0f;
+                }
+            };
+            const int nt = (n + TP_TILE - 1) / TP_TILE;
+            __syncthreads();
+            const int found = nt <= TP_THREADS / 32 ? scan_few_tiles<TP_THREADS>(sc.agg, &sh_found, nt, r.rand_num, load) :
+                                                      scan_tiles<2>(sc, nt, r.rand_num, load);
+            if (found >= 0 && found < n && whole_run(found)) {
+                __syncthreads();
+                const unsigned long long e = topp_settle_run(sc, src, n, found, s.Vp, prob);
+                if (t == 0) {
+                    r.finish(o, ToppPicked{(int)(uint32_t)e, prob(e), true});
+                }
+                return;
+            }
+            if (found < 0 && all) {
+                if (t == 0) {
+                    r.finish(o, ToppPicked{(int)(uint32_t)best, p_best, false});  // never crossed: the arg-max stays
+                }
+                return;
+            }
+        }
+        __syncthreads();
+    }
+    const ToppWholeRow<DT_F32> w{r.y, s.n, s.Vp, r.end_id, r.mx, r.denom, r.p, r.rand_num, r.fin, A};
+    res = topp_pick_whole_row<DT_F32>(sc, ss.buf, w);
+    if (t == 0) {
+        r.finish(o, res);
+    }
+}
+
+// ---- pick, 16-bit types
+// 16-bit order-preserving image of a value's bits
+__device__ __forceinline__ uint32_t topp_key16(uint32_t bits)
+{
+    return (bits & 0x8000u) ? (~bits & 0xFFFFu) : (bits | 0x8000u);
+}
+
+template<int DT>
+union ToppRunsShared {
+    struct {
+        uint32_t start[ToppCode<DT>::USED + 1];  // entries in front of a run, in descending order of e
+        uint16_t code[ToppCode<DT>::USED + 1];   // a run's value of e
+        uint16_t prob[ToppCode<DT>::USED + 1];   // and its probability, both as stored values of the type
+    };
+    unsigned long long digits[TP_DIGITS];                          // the fallback's radix sort
+    uint8_t            masks[TP_DIGITS * sizeof(unsigned long long)];  // the look-up's matches: a byte per eight columns
+};
+
+template<int DT>
+__global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, ToppPickOut o)
+{
+    typedef Storage<DT>           S;
+    typedef typename S::T         T;
+    typedef ToppCode<DT>          Code;
+    constexpr int                 CPT  = 16;                    // counters per thread
+    constexpr int                 TEAM = Code::COUNTERS / CPT;  // threads that look at counters
+    constexpr int                 TW   = TEAM / WAVE;
+    constexpr int                 NW   = TP_THREADS / WAVE;
+    constexpr int                 FEW  = 256;                   // threads of the short scan: eight tiles
+    __shared__ TopPScan           sc;
+    __shared__ ToppRunsShared<DT> rs;
+    __shared__ uint32_t           wcnt[TW], wrun[TW], wpick[NW];
+    __shared__ float              wmass[TW];
+    __shared__ uint32_t           sh_enough, key_lo, key_hi;
+    __shared__ int                sh_found, code_lo, code_hi, sh_nth, sh_id;
+    const int       row = blockIdx.x;
+    const int       t   = threadIdx.x;
+    ToppPickRow<DT> r(s, o, row, s.splits);
+    // counters of this thread, descending: position d counts entries of code COUNTERS - 1 - d
+    uint32_t c[CPT];
+    {
+        const uint4* from = reinterpret_cast<const uint4*>(s.counts + (size_t)row * Code::COUNTERS + (Code::COUNTERS - (min(t, TEAM - 1) + 1) * CPT));
+#pragma unroll
+        for (int i = 0; i < CPT / 4; ++i) {
+            const uint4 w      = from[i];
+            c[CPT - 1 - 4 * i] = w.x;
+            c[CPT - 2 - 4 * i] = w.y;
+            c[CPT - 3 - 4 * i] = w.z;
+            c[CPT - 4 - 4 * i] = w.w;
+        }
+    }
+    // the maxima of this wave's blocks of columns: a wave takes a contiguous run of them
+    const int    bpw  = (s.blocks + NW - 1) / NW;
+    const int    b0   = min(s.blocks, wave_id() * bpw), b1 = min(s.blocks, b0 + bpw);
+    const float* bmax = s.block_max + (size_t)row * s.blocks;
+    const float  bm   = bmax[min(b0 + lane_id(), s.blocks - 1)];
+    if (t == 0) {
+        sh_enough = 0xFFFFFFFFu;
+        sh_found  = 0x7FFFFFFF;
+        sh_id     = -1;
+    }
+    if (r.skip) {
+        if (t == 0) {
+            r.decay(o, o.dec.runtime_top_p != nullptr ? o.ids[row] : 0);
+        }
+        return;
+    }
+    r.derive(s, o);
+    ToppPicked res;
+    if (r.trivial(s, res)) {
+        if (t == 0) {
+            r.finish(o, res);
+        }
+        return;
+    }
+    const ToppWholeRow<DT> whole{r.y, s.n, s.Vp, r.end_id, r.mx, r.denom, r.p, r.rand_num, r.fin, s.sorted + (size_t)row * 2 * s.Vp};
+    if (r.fin || o.force_deep) {
+        res = topp_pick_whole_row<DT>(sc, rs.digits, whole);
+        if (t == 0) {
+            r.finish(o, res);
+        }
+        return;
+    }
+    const RowDivisor div(r.denom);
+    const bool       quick = __builtin_amdgcn_readfirstlane((int)div.ok) != 0;
+    auto             prob_of_code = [&](int code) -> float {
+        const float e = S::ld((T)(code + Code::BASE));  // (at least 2^-31)
+        return round_t<DT>(quick ? div.divide_normal(e) : e / r.denom);
+    };
+    // ---- the runs: counts, probabilities and places of the values that occur and whose probability is not zero
+    float    pv[CPT];
+    uint32_t lc = 0u, lr = 0u;
+    float    lm = 0.0f;
+    if (t < TEAM) {
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            pv[i] = 0.0f;
+            if (c[i] != 0u) {
+                pv[i] = prob_of_code(Code::COUNTERS - 1 - (t * CPT + i));
+                if (pv[i] > 0.0f) {
+                    lc += c[i];
+                    lr += 1u;
+                    lm += (float)c[i] * pv[i];
+                }
+            }
+        }
+    }
+    uint32_t ic = lc, ir = lr;
+    float    im = lm;
+    if (t < TEAM) {
+#pragma unroll
+        for (int k = 1; k < WAVE; k <<= 1) {
+            const uint32_t uc = __shfl_up(ic, k, WAVE), ur = __shfl_up(ir, k, WAVE);
+            const float    um = __shfl_up(im, k, WAVE);
+            if (lane_id() >= k) {
+                ic += uc;
+                ir += ur;
+                im += um;
+            }
+        }
+        if (lane_id() == WAVE - 1) {
+            wcnt[wave_id()]  = ic;
+            wrun[wave_id()]  = ir;
+            wmass[wave_id()] = im;
+        }
+    }
+    __syncthreads();
+    uint32_t n = 0u, nruns = 0u;
+    uint32_t at = ic - lc, run = ir - lr;
+    float    mass = im - lm;
+#pragma unroll
+    for (int w = 0; w < TW; ++w) {
+        const uint32_t wc = wcnt[w], wr = wrun[w];
+        at += w < wave_id() ? wc : 0u;
+        run += w < wave_id() ? wr : 0u;
+        mass += w < wave_id() ? wmass[w] : 0.0f;
+        n += wc;
+        nruns += wr;
+    }
+    const uint32_t at0 = at, run0 = run;
+    const float    mass0 = mass;
+    // the place behind the run with which the mass certainly covers the draw: the scan need not look further
+    const float want = r.rand_num * (1.0f + 1.0f / 256.0f) + 1e-5f;
+    if (t < TEAM) {
+        uint32_t enough = 0xFFFFFFFFu;
+#pragma unroll
+        for (int i = 0; i < CPT; ++i) {
+            if (pv[i] > 0.0f) {
+                rs.start[run] = at;
+                rs.code[run]  = (uint16_t)(Code::COUNTERS - 1 - (t * CPT + i));
+                rs.prob[run]  = S::st(pv[i]);
+                at += c[i];
+                mass += (float)c[i] * pv[i];
+                run++;
+                if (mass >= want && enough == 0xFFFFFFFFu) {
+                    enough = at;
+                }
+            }
+        }
+        if (enough != 0xFFFFFFFFu && mass0 < want) {  // (one thread as a rule, a few next to it by rounding)
+            atomicMin(&sh_enough, enough);
+        }
+        if (t == 0) {
+            rs.start[nruns] = n;
+        }
+    }
+    __syncthreads();
+    const int enough = (int)min(n, sh_enough);
+
+    // Whether the runs hold every positive probability: binary16's counters resolve all values of e, bfloat16's leave out
+    // what lies below 2^-31.
+    const bool complete = DT == DT_F16 || n == (uint32_t)s.Vp;
+    int        found    = -1;
+    bool       sampled  = true;
+    float      prob     = 0.0f;
+    bool       fallback = n == 0u;
+    if (!fallback) {
+        const float best = S::ld(rs.prob[0]);
+        if (round_t<DT>(0.0f + best) >= r.p) {
+            found = 0;  // arg-max shortcut of the reference (:842-849)
+        }
+        else {
+            // the run of position i: the last one that starts at or before it
+            auto run_at = [&](int i) -> int {
+                int lo = 0, hi = (int)nruns;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if ((int)rs.start[mid] <= i) {
+                        lo = mid;
+                    }
+                    else {
+                        hi = mid;
+                    }
+                }
+                return lo;
+            };
+            // a lane's eight values from position i0 on, which lies in run `lo`; lo goes along
+            auto values_from = [&](int i0, int& lo, float* x) {
+                float v    = S::ld(rs.prob[lo]);
+                int   next = (int)rs.start[lo + 1];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    x[k] = 0.0f;
+                    if (i0 + k < (int)n) {
+                        if (i0 + k >= next) {
+                            do {
+                                ++lo;
+                                next = (int)rs.start[lo + 1];
+                            } while (i0 + k >= next);
+                            v = S::ld(rs.prob[lo]);
+                        }
+                        x[k] = v;
+                    }
+                }
+            };
+            auto load = [&](int tile, int l, float* x) {
+                const int i0 = tile * TP_TILE + l * 8;
+                int       lo = run_at(min(i0, (int)n - 1));
+                values_from(i0, lo, x);
+            };
+            // A 32-lane group takes neighbouring tiles: the next one goes on in the run where the one before stopped,
+            // and whole tiles of one run have one total.
+            auto totals = [&](int base, int count) {
+                const int l   = t & 31, per = (count + TP_THREADS / 32 - 1) / (TP_THREADS / 32);
+                const int t0  = base + min(count, (t >> 5) * per), t1 = min(base + count, t0 + per);
+                float*    agg = sc.agg - base;
+                if (t0 >= t1) {
+                    return;
+                }
+                int   lo    = run_at(min(t0 * TP_TILE + l * 8, (int)n - 1));
+                int   known = -1;  // run whose whole tiles' total is `total`
+                float total = 0.0f;
+                for (int tile = t0; tile < t1; ++tile) {
+                    const int i0 = tile * TP_TILE + l * 8;
+                    while (i0 < (int)n && i0 >= (int)rs.start[lo + 1]) {
+                        ++lo;
+                    }
+                    const int first = __shfl(lo, 0, 32);
+                    if ((int)rs.start[first + 1] >= (tile + 1) * TP_TILE && known == first) {
+                        if (l == 31) {
+                            agg[tile] = total;
+                        }
+                        continue;
+                    }
+                    float x[8];
+                    int   r = lo;
+                    values_from(i0, r, x);
+                    total = tile_scan(x, l);
+                    known = (int)rs.start[first + 1] >= (tile + 1) * TP_TILE ? first : -1;
+                    if (l == 31) {
+                        agg[tile] = total;
+                    }
+                }
+            };
+            const int nt_all = ((int)n + TP_TILE - 1) / TP_TILE;
+            const int nt     = (enough + TP_TILE - 1) / TP_TILE;
+            bool      over   = false;  // the scan has seen every tile
+            if (nt <= FEW / 32) {
+                found = scan_few_tiles<FEW>(sc.agg, &sh_found, nt, r.rand_num, load);
+                over  = nt == nt_all;
+            }
+            else {
+                found = scan_tiles(sc, nt, r.rand_num, load, totals);
+                over  = nt == nt_all;
+            }
+            if (found < 0 && !over) {
+                __syncthreads();
+                found = scan_tiles(sc, nt_all, r.rand_num, load, totals);
+            }
+            __syncthreads();
+            if (found < 0 || found >= (int)n) {
+                if (complete && found < 0) {
+                    found   = 0;  // never crossed: the arg-max stays (:954)
+                    sampled = false;
+                }
+                else {
+                    fallback = true;
+                }
+            }
+        }
+    }
+    if (fallback) {
+        // (a row without a value that the counters resolve, or a draw behind all of them)
+        __syncthreads();
+        res = topp_pick_whole_row<DT>(sc, rs.digits, whole);
+        if (t == 0) {
+            r.finish(o, res);
+        }
+        return;
+    }
+    // ---- the run of position `found`, together with neighbours whose numerators round to the same quotient
+    if (t < TEAM && lc != 0u && found >= (int)at0 && found < (int)(at0 + lc)) {
+        int q = (int)run0;
+        while (found >= (int)rs.start[q + 1]) {
+            ++q;
+        }
+        const uint16_t here = rs.prob[q];
+        int            a = q, b = q;
+        while (a > 0 && rs.prob[a - 1] == here) {
+            --a;
+        }
+        while (b + 1 < (int)nruns && rs.prob[b + 1] == here) {
+            ++b;
+        }
+        code_hi      = (int)rs.code[a];
+        code_lo      = (int)rs.code[b];
+        sh_nth       = found - (int)rs.start[a];
+        sc.fmisc[1]  = S::ld(here);
+    }
+    __syncthreads();
+    // ---- the values of y with these numerators: a range of the order-preserving image, found by two waves in three
+    // rounds of 64 probes (e does not fall as y rises)
+    if (wave_id() < 2) {
+        const uint32_t key_mx  = topp_key16((uint32_t)S::st(r.mx));
+        const uint32_t key_inf = topp_key16((uint32_t)S::st(-__builtin_inff()));
+        auto           code_of = [&](uint32_t key) -> int {
+            if (key >= key_mx) {
+                return Code::USED - 1;
+            }
+            if (key < key_inf) {
+                return 0;
+            }
+            const T bits = (T)((key & 0x8000u) ? (key & 0x7FFFu) : (~key & 0xFFFFu));
+            return max((int)S::st(topp_exp(S::ld(bits) - r.mx)) - Code::BASE, 0);
+        };
+        const bool upper = wave_id() == 1;  // wave 0: the first key with code >= code_lo; wave 1: with code > code_hi
+        const int  level = upper ? code_hi + 1 : code_lo;
+        uint32_t   base  = 0u;  // keys below base have smaller codes
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int      width  = k == 0 ? 1024 : k == 1 ? 16 : 1;
+            const int      probes = k == 2 ? 16 : 64;
+            const uint32_t key    = base + (uint32_t)(lane_id() + 1) * (uint32_t)width - 1u;
+            const bool     less   = lane_id() < probes && key < 65536u && code_of(key) < level;
+            base += (uint32_t)__popcll(__ballot(less)) * (uint32_t)width;
+        }
+        if (lane_id() == 0) {
+            if (upper) {
+                key_hi = base;  // one past the last
+            }
+            else {
+                key_lo = base;
+            }
+        }
+    }
+    __syncthreads();
+    prob = sc.fmisc[1];
+    // ---- the column: the sh_nth one in order of ids whose value lies in that range. Blocks whose maximum lies below it
+    // cannot hold one: a draw near the head of the distribution reads a few blocks only.
+    const uint32_t klo = key_lo, khi = key_hi;
+    const int      nth = sh_nth;
+    auto match = [&](uint32_t bits) -> bool {
+        const uint32_t k = topp_key16(bits);
+        return k >= klo && k < khi;
+    };
+    auto mask_of = [&](int blk) -> uint32_t {  // the matches among this lane's eight columns of a block
+        const int v0 = blk * TSP_BLOCK + lane_id() * 8;
+        uint32_t  m  = 0u;
+        if (v0 + 8 <= s.n) {
+            const uint4    raw  = topp_load8(r.y + v0);
+            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                m |= (match(w[k] & 0xFFFFu) ? 1u : 0u) << (2 * k);
+                m |= (match(w[k] >> 16) ? 1u : 0u) << (2 * k + 1);
+            }
+        }
+        else {
+            for (int k = 0; k < 8; ++k) {
+                if (v0 + k < s.n && match((uint32_t)r.y[v0 + k])) {
+                    m |= 1u << k;
+                }
+            }
+        }
+        return m;
+    };
+    const bool kept = s.blocks <= (int)sizeof(rs.masks) / WAVE;  // the matches of every block fit LDS
+    int        mine = 0;
+    for (int g = b0; g < b1; g += WAVE) {  // (one turn unless the vocabulary has half a million columns)
+        const float gm   = g == b0 ? bm : bmax[min(g + lane_id(), s.blocks - 1)];
+        const bool  may  = g + lane_id() < b1 && topp_key16((uint32_t)S::st(gm)) >= klo;
+        if (kept && g + lane_id() < b1 && !may) {
+            uint4* z = reinterpret_cast<uint4*>(rs.masks + (g + lane_id()) * WAVE);
+            z[0] = z[1] = z[2] = z[3] = make_uint4(0u, 0u, 0u, 0u);
+        }
+        unsigned long long todo = __ballot(may);
+        while (todo != 0ull) {
+            constexpr int U = 8;
+            int           blk[U];
+            uint32_t      m[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                blk[u] = todo != 0ull ? g + __builtin_ctzll(todo) : -1;
+                todo &= todo - 1ull;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                m[u] = mask_of(max(blk[u], 0));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (blk[u] >= 0) {
+                    mine += __popc(m[u]);
+                    if (kept) {
+                        rs.masks[blk[u] * WAVE + lane_id()] = (uint8_t)m[u];
+                    }
+                }
+            }
+        }
+    }
+    mine = wave_sum_i(mine);
+    if (lane_id() == 0) {
+        wpick[wave_id()] = (uint32_t)mine;
+    }
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const int x = (int)wpick[w];
+        before += w < wave_id() ? x : 0;
+        total += x;
+    }
+    if (nth >= before && nth < before + mine) {  // (one wave)
+        int left = nth - before;
+        for (int g = b0; g < b1; g += WAVE) {
+            // lane i counts the matches of block g + i
+            const int blk = g + lane_id();
+            int       own = 0;
+            if (kept && blk < b1) {
+                const uint4* q = reinterpret_cast<const uint4*>(rs.masks + blk * WAVE);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint4 w = q[k];
+                    own += __popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w);
+                }
+            }
+            else if (!kept) {
+                for (int i = g; i < min(b1, g + WAVE); ++i) {
+                    const int x = wave_sum_i(__popc(mask_of(i)));
+                    own         = lane_id() == i - g ? x : own;
+                }
+            }
+            int inc = own;
+#pragma unroll
+            for (int k = 1; k < WAVE; k <<= 1) {
+                const int up = __shfl_up(inc, k, WAVE);
+                if (lane_id() >= k) {
+                    inc += up;
+                }
+            }
+            const unsigned long long hit = __ballot(inc > left);
+            if (hit == 0ull) {
+                left -= __shfl(inc, WAVE - 1, WAVE);
+                continue;
+            }
+            const int which = __builtin_ctzll(hit);
+            left -= __shfl(inc - own, which, WAVE);
+            const uint32_t m = kept ? (uint32_t)rs.masks[(g + which) * WAVE + lane_id()] : mask_of(g + which);
+            int            in = __popc(m);
+            const int      c1 = in;
+#pragma unroll
+            for (int k = 1; k < WAVE; k <<= 1) {
+                const int up = __shfl_up(in, k, WAVE);
+                if (lane_id() >= k) {
+                    in += up;
+                }
+            }
+            int k = left - (in - c1);
+            if (k >= 0 && k < c1) {
+                uint32_t rest = m;
+                while (k-- > 0) {
+                    rest &= rest - 1u;
+                }
+                r.finish(o, ToppPicked{(g + which) * TSP_BLOCK + lane_id() * 8 + (int)__builtin_ctz(rest), prob, sampled});
+            }
+            break;
+        }
+    }
+    else if (nth >= total && t == 0) {
+        // the pad columns follow the vocabulary; they match when their value does
+        r.finish(o, ToppPicked{min(s.n + (nth - total), s.Vp - 1), prob, sampled});
+    }
+}
+
+// ---- host -------------------------------------------------------------------------------------------------------------
+static inline size_t up256(size_t x)
+{
+    return (x + 255) & ~(size_t)255;
+}
+
+struct ToppSamplePlan {
+    int    parts, splits, chunk, blocks, y_pitch, sorters;
+    size_t off_y, off_counts, off_pmax, off_blocks, off_ref, off_gsum, off_segs, off_queue, off_meta, bytes;
+};
+
+static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vocab_padded, bool keeps_y)
+{
+    ToppSamplePlan p;
+    rows = rows > 0 ? rows : 1;
+    // The sum. fp32: 256-thread workgroups, one chain per thread and four workgroups per row where that fills the chip,
+    // sixteen with four lanes to a chain below. 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four
+    // below.
+    p.parts = dtype == DT_F32 ? (rows >= 256 ? 4 : 16) : (rows >= 192 ? 1 : 4);
+    // 16-bit stage: about four workgroups per compute unit, each with at least four blocks of columns (one per wave), and
+    // no more columns than its bitmap of the history covers
+    p.blocks = (vocab + TSP_BLOCK - 1) / TSP_BLOCK;
+    int s    = (1024 + rows - 1) / rows;
+    s        = std::min(s, std::max(1, p.blocks / 4));
+    s        = std::max(s, (p.blocks + (TSP_WINDOW - 4) * 32 / TSP_BLOCK - 1) / ((TSP_WINDOW - 4) * 32 / TSP_BLOCK));
+    p.splits = std::min(s, TSP_SPLITS);
+    p.chunk  = (p.blocks + p.splits - 1) / p.splits * TSP_BLOCK;
+    p.sorters       = (int)std::min<size_t>(512, (size_t)rows * (vocab_padded / TPS_SEG + 1));
+    p.y_pitch       = (int)((vocab_padded + 7) / 8 * 8);
+    const size_t el = dtype == DT_F32 ? 4 : 2;
+    const size_t counters = dtype == DT_F32 ? (size_t)p.parts * TSP_BUCKETS :
+                            dtype == DT_F16 ? (size_t)ToppCode<DT_F16>::COUNTERS :
+                                              (size_t)ToppCode<DT_BF16>::COUNTERS;
+    size_t off = up256((size_t)rows * vocab_padded * 2 * sizeof(unsigned long long));
+    auto   take = [&](size_t bytes) {
+        const size_t at = off;
+        off += up256(bytes);
+        return at;
+    };
+    p.off_counts = take((size_t)rows * counters * sizeof(uint32_t));
+    p.off_pmax   = take((size_t)rows * TSP_SPLITS * sizeof(float2));
+    p.off_blocks = take(dtype == DT_F32 ? 0 : (size_t)rows * p.blocks * sizeof(float));
+    p.off_ref    = take((size_t)rows * sizeof(float));
+    p.off_gsum   = take((size_t)rows * 32 * sizeof(float));
+    p.off_segs   = take((size_t)rows * TPB_NB * sizeof(uint32_t));
+    p.off_queue  = take(((size_t)rows * TPB_NB + 1) * sizeof(uint32_t));
+    p.off_meta   = take((size_t)rows * sizeof(ToppRowMeta));
+    p.off_y      = keeps_y ? take((size_t)rows * p.y_pitch * el) : 0;
+    p.bytes      = off;
+    return p;
+}
+
+size_t topp_sample_bytes(int dtype, int rows, int vocab, size_t vocab_padded, bool keeps_y)
+{
+    return topp_sample_plan(dtype, rows, vocab, vocab_padded, keeps_y).bytes;
+}
+
+bool topp_sample_covers(int dtype, int rows, int vocab, bool history_penalty)
+{
+    if (vocab < TSP_CHAINS) {
+        return false;  // the sum's order follows the softmax's block of min(n, 1024) threads
+    }
+    if (!history_penalty) {
+        return true;
+    }
+    // the bitmap of the history that a stage's workgroup keeps
+    const ToppSamplePlan p    = topp_sample_plan(dtype, rows, vocab, (size_t)vocab, true);
+    const long long      bits = dtype == DT_F32 ? (long long)((vocab + TSP_CHAINS - 1) / TSP_CHAINS) * (TSP_CHAINS / p.parts) : p.chunk;
+    return bits <= (long long)(TSP_WINDOW - 4) * 32;
+}
+
+int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
+{
+    const bool           keeps_y = c.temperatures != nullptr || (c.penalties != nullptr && c.penalty_type != 2) || c.min_lengths != nullptr;
+    const ToppSamplePlan p       = topp_sample_plan(c.dtype, c.rows, c.vocab_size, c.vocab_size_padded, keeps_y);
+    if (c.workspace_size < p.bytes) {
+        return FTK_ERR_WORKSPACE;
+    }
+    char*    ws = (char*)c.workspace;
+    ToppStep s{};
+    s.logits = c.logits;
+    s.bias   = c.bias;
+    s.n      = c.vocab_size;
+    s.Vp     = (int)c.vocab_size_padded;
+    s.rows   = c.rows;
+    s.y      = keeps_y ? ws + p.off_y : nullptr;
+    s.y_pitch          = p.y_pitch;
+    s.temperatures     = c.temperatures;
+    s.penalties        = c.penalties;
+    s.penalty_type     = c.penalty_type;
+    s.min_lengths      = c.min_lengths;
+    s.end_ids          = c.end_ids;
+    s.input_lengths    = c.input_lengths;
+    s.history          = c.history;
+    s.sequence_length  = c.sequence_length;
+    s.batch_size       = c.batch_size;
+    s.step             = c.step;
+    s.max_input_length = c.max_input_length;
+    s.finished         = c.finished;
+    s.skip             = c.skip_decode;
+    s.rng              = (const RngState*)c.rng_state;
+    s.uniforms         = c.uniform_draws;
+    s.top_p            = c.max_top_p;
+    s.top_ps           = c.runtime_top_p;
+    s.splits           = p.splits;
+    s.chunk            = p.chunk;
+    s.parts            = p.parts;
+    s.blocks           = p.blocks;
+    s.pmax             = (float2*)(ws + p.off_pmax);
+    s.block_max        = (float*)(ws + p.off_blocks);
+    s.ref              = (float*)(ws + p.off_ref);
+    s.gsum             = (float*)(ws + p.off_gsum);
+    s.counts           = (uint32_t*)(ws + p.off_counts);
+    s.meta             = (ToppRowMeta*)(ws + p.off_meta);
+    s.segs             = (uint32_t*)(ws + p.off_segs);
+    s.queue            = (uint32_t*)(ws + p.off_queue);
+    s.sorted           = (unsigned long long*)ws;
+    ToppPickOut o{};
+    o.ids              = c.output_ids;
+    o.sequence_length  = c.sequence_length;
+    o.finished         = c.finished;
+    o.cum_log_probs    = c.cum_log_probs;
+    o.output_log_probs = c.output_log_probs;
+    o.rng        = (RngState*)c.rng_state;
+    o.dec        = ToppDecayArgs{c.top_p_decay != nullptr ? c.runtime_top_p : nullptr, c.initial_top_p, c.top_p_decay,
+                                 c.top_p_min, c.top_p_reset_ids};
+    o.force_deep = topp_force_deep();
+
+    const dim3 parts(c.rows, p.parts), splits(c.rows, p.splits);
+    if (c.dtype == DT_F32) {
+        if (keeps_y) {
+            topp_stage_f32_kernel<true><<<parts, TSP_STAGE, 0, st>>>(s);
+        }
+        else {
+            topp_stage_f32_kernel<false><<<parts, TSP_STAGE, 0, st>>>(s);
+        }
+        FTK_LAUNCH_CHECK();
+        if (p.parts == 4) {
+            topp_sum_gather_kernel<1><<<parts, TSP_SUM32, 0, st>>>(s);
+        }
+        else {
+            topp_sum_gather_kernel<4><<<parts, TSP_SUM32, 0, st>>>(s);
+        }
+        FTK_LAUNCH_CHECK();
+        topp_sort_queue_kernel<<<p.sorters, TP_THREADS, 0, st>>>(s);
+        FTK_LAUNCH_CHECK();
+        topp_pick_f32_kernel<<<c.rows, TP_THREADS, 0, st>>>(s, o);
+        FTK_LAUNCH_CHECK();
+        return 0;
+    }
+    auto run = [&](auto type) -> int {
+        constexpr int DT = decltype(type)::value;
+        if (keeps_y) {
+            topp_stage_kernel<DT, true><<<splits, TSP_STAGE, 0, st>>>(s);
+        }
+        else {
+            topp_stage_kernel<DT, false><<<splits, TSP_STAGE, 0, st>>>(s);
+        }
+        FTK_LAUNCH_CHECK();
+        // binary16's table is seven times bfloat16's: it pays only where one workgroup takes a whole long row
+        if (p.parts == 1) {
+            if (DT == DT_BF16 || c.vocab_size >= 65536) {
+                topp_sum_count_kernel<DT, 1024, true><<<parts, TSP_SUM16, 0, st>>>(s);
+            }
+            else {
+                topp_sum_count_kernel<DT, 1024, false><<<parts, TSP_SUM16, 0, st>>>(s);
+            }
+        }
+        else {
+            topp_sum_count_kernel<DT, 256, DT == DT_BF16><<<parts, TSP_SUM16, 0, st>>>(s);
+        }
+        FTK_LAUNCH_CHECK();
+        topp_pick_runs_kernel<DT><<<c.rows, TP_THREADS, 0, st>>>(s, o);
+        FTK_LAUNCH_CHECK();
+        return 0;
+    };
+    if (c.dtype == DT_F16) {
+        return run(std::integral_constant<int, DT_F16>());
+    }
+    return run(std::integral_constant<int, DT_BF16>());
+}
+
+}  // namespace ftk

@@ -63,6 +63,7 @@ _SIGNATURES = {
     "ftk_invoke_stop_words_criterion_rows": [_vp, _vp, _vp, _vp, _sz, _sz, _i, _i, _i, _i, _vp],
     "ftk_invoke_length_criterion": [_vp, _vp, _vp, _vp, _i, _i, _i, _vp],
     "ftk_fused_topk_step": [_vp, _vp],
+    "ftk_fused_topp_penalty_step": [_vp, _vp],
     "ftk_fused_topk_step_static": [_vp, _vp],
     "ftk_measure_plain_read": [_vp, _sz, _vp, _sz, _vp, _vp],
     "ftk_invoke_log_prob_from_logits": [_i, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _sz, _vp, _sz, _vp, _b],

@@ -187,6 +187,73 @@ void BaseSamplingLayer<T>::forward(std::unordered_map<std::string, Tensor>*     
     forward(&output_map, &input_map);
 }
 
+// The per-row arguments of the penalties that are active in this window, the sampling state and the outputs.
+template<typename T>
+ftk_fused_topk_args BaseSamplingLayer<T>::fusedStepArgs(TensorMap* output_tensors, TensorMap* input_tensors)
+{
+    const int batch_size       = output_tensors->at("output_ids").shape[1];
+    const int local_batch_size = input_tensors->at("logits").shape[0];
+    const int ite              = input_tensors->at("ite").template getVal<int>();
+    const int step             = input_tensors->at("step").template getVal<int>();
+    const int max_input_length = input_tensors->at("max_input_length").template getVal<int>();
+    const int off              = ite * local_batch_size;
+
+    ftk_fused_topk_args a{};
+    a.dtype             = FtkDType<T>::value;
+    a.logits            = input_tensors->at("logits").template getPtr<T>();
+    a.embedding_bias    = input_tensors->at("embedding_bias", Tensor()).template getPtr<T>();
+    a.vocab_size        = (int)vocab_size_;
+    a.vocab_size_padded = (int)vocab_size_padded_;
+    a.batch_size        = batch_size;
+    a.local_batch_size  = local_batch_size;
+    a.step              = step;
+    a.max_input_length  = max_input_length;
+
+    const float* temps = temperature_.data() + off;
+    const bool   temp_active =
+        a.embedding_bias != nullptr || !std::all_of(temps, temps + local_batch_size, [](float t) { return t == 1.0f; });
+    a.temperatures = temp_active ? temperature_buf_ + off : nullptr;
+
+    a.penalty_type = FTK_PENALTY_NONE;
+    if (step > 1 && repetition_penalty_type_ != RepetitionPenaltyType::None) {
+        const float  dflt = getDefaultPenaltyValue(repetition_penalty_type_);
+        const float* pens = repetition_penalty_.data() + off;
+        if (!std::all_of(pens, pens + local_batch_size, [&](float x) { return x == dflt; })) {
+            a.penalty_type = toFtkPenalty(repetition_penalty_type_);
+            a.penalties    = repetition_penalty_buf_ + off;
+        }
+        if (has_frequency_penalty_) {
+            const float* fr = frequency_penalty_.data() + off;
+            if (!std::all_of(fr, fr + local_batch_size, [](float x) { return x == 0.0f; })) {
+                // (x - presence - frequency * count: the presence array goes along even when it is all zeros)
+                a.penalty_type        = FTK_PENALTY_ADDITIVE;
+                a.penalties           = repetition_penalty_buf_ + off;
+                a.frequency_penalties = frequency_penalty_buf_ + off;
+            }
+        }
+    }
+    const int  num_generated_tokens = step - max_input_length;
+    const int* min_lengths          = min_lengths_.data() + off;
+    if (std::any_of(min_lengths, min_lengths + local_batch_size,
+                    [&](int m) { return m > num_generated_tokens; })) {
+        FT_CHECK_WITH_INFO(input_tensors->isExist("end_id"), "Need end_id to apply min length penlaty");
+        a.min_lengths = min_lengths_buf_ + off;
+        FT_CHECK(output_tensors->template getPtr<const int>("sequence_length") != nullptr);
+    }
+    a.end_ids       = input_tensors->at("end_id").template getPtr<const int>();
+    a.input_lengths = input_tensors->at("input_lengths", Tensor()).template getPtr<const int>();
+    a.output_ids    = output_tensors->at("output_ids").template getPtrWithOffset<int>(off);
+    a.skip_decode   = skip_decode_buf_ + off;
+    a.rng_state     = curandstate_buf_ + off;
+    a.uniform_draws = input_tensors->at("uniform_draws", Tensor()).template getPtr<const float>();
+    a.ids = output_tensors->at("output_ids").template getPtrWithOffset<int>((size_t)step * batch_size + off);
+    a.sequence_length = output_tensors->at("sequence_length", Tensor()).template getPtr<int>();
+    a.finished        = output_tensors->at("finished", Tensor()).template getPtr<bool>();
+    a.cum_log_probs    = output_tensors->at("cum_log_probs", Tensor()).template getPtr<float>();
+    a.output_log_probs = output_tensors->at("output_log_probs", Tensor()).template getPtr<float>();
+    return a;
+}
+
 // reference: BaseSamplingLayer<T>::forward, layers/sampling_layers/BaseSamplingLayer.cc:255-359
 template<typename T>
 void BaseSamplingLayer<T>::forward(TensorMap* output_tensors, TensorMap* input_tensors)

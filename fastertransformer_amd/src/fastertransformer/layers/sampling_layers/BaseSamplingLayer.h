@@ -60,6 +60,9 @@ protected:
         return false;
     }
 
+    // What a fused step of either layer is given: everything but the layer's own k / p values and the workspace.
+    ftk_fused_topk_args fusedStepArgs(TensorMap* output_tensors, TensorMap* input_tensors);
+
     template<typename V>
     void fillFromArg(std::vector<V>& host, V* device, const Tensor& arg, size_t batch_size);
 

@@ -128,17 +128,75 @@ void TopPSamplingLayer<T>::setup(const size_t batch_size, const size_t beam_widt
     h2d(top_p_reset_ids_buf_, reset.data(), sizeof(int32_t) * batch_size);
     check_hip_error(hipStreamSynchronize(stream_));  // sources are host temporaries
 
-    // fallback-sort workspace (only rows that draw deep into a flat distribution touch it)
     const bool any_row = std::any_of(skip_decode_.begin(), skip_decode_.begin() + batch_size,
                                      [](uint8_t s) { return s == 0; });
     if (any_row) {
         cub_temp_storage_size_ = 0;
-        invokeFusedTopPStep<T>(nullptr, sampling_workspace_size_, nullptr, nullptr, (int)vocab_size_,
-                               vocab_size_padded_, (int)batch_size, nullptr, nullptr, nullptr, nullptr, nullptr,
-                               nullptr, nullptr, nullptr, 0.0f, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
-                               stream_);
-        sampling_workspace_ = allocator_->reMalloc(sampling_workspace_, sampling_workspace_size_, false);
+        size_t need            = 0;
+        invokeFusedTopPStep<T>(nullptr, need, nullptr, nullptr, (int)vocab_size_, vocab_size_padded_, (int)batch_size,
+                               nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0f, nullptr,
+                               nullptr, nullptr, nullptr, nullptr, nullptr, stream_);
+        if (!keep_probabilities_) {
+            // (the step with penalties keeps its own copy of the rows)
+            need = std::max(need, fusedBytes(batch_size));
+        }
+        sampling_workspace_      = allocator_->reMalloc(sampling_workspace_, need, false);
+        sampling_workspace_size_ = need;
     }
+}
+
+// What a fused step over `rows` rows takes at most with the penalties that setup() saw (0: not covered).
+template<typename T>
+size_t TopPSamplingLayer<T>::fusedBytes(size_t rows)
+{
+    const float         placeholder = 0.0f;  // (a size query looks at which arrays there are, not into them)
+    const int           zero        = 0;
+    ftk_fused_topp_args a{};
+    a.row.dtype             = FtkDType<T>::value;
+    a.row.vocab_size        = (int)vocab_size_;
+    a.row.vocab_size_padded = (int)vocab_size_padded_;
+    a.row.local_batch_size  = (int)rows;
+    a.row.temperatures      = &placeholder;
+    a.row.min_lengths       = &zero;
+    a.row.penalty_type      = toFtkPenalty(this->repetition_penalty_type_);
+    a.row.penalties         = this->repetition_penalty_type_ == RepetitionPenaltyType::None ? nullptr : &placeholder;
+    return ftk_fused_topp_penalty_step(&a, stream_) == 0 ? a.row.workspace_size : 0;
+}
+
+// The whole step - penalties, softmax, sampling, decay - in one call that only reads the logits. Not taken when the
+// caller wants the reference's side effects or for what the call does not cover (small vocabularies, the
+// frequency-penalty extension): forward() then goes on with the kernel sequence.
+template<typename T>
+bool TopPSamplingLayer<T>::runFused(TensorMap* output_tensors, TensorMap* input_tensors)
+{
+    if (keep_probabilities_) {
+        return false;
+    }
+    const int           off = input_tensors->at("ite").template getVal<int>() * (int)input_tensors->at("logits").shape[0];
+    ftk_fused_topp_args a{};
+    a.row             = this->fusedStepArgs(output_tensors, input_tensors);
+    a.max_top_p       = runtime_max_top_p_;
+    a.runtime_top_p   = runtime_top_p_buf_ + off;
+    a.initial_top_p   = initial_top_p_buf_ + off;
+    a.top_p_decay     = top_p_decay_buf_ + off;
+    a.top_p_min       = top_p_min_buf_ + off;
+    a.top_p_reset_ids = top_p_reset_ids_buf_ + off;
+    const int query   = ftk_fused_topp_penalty_step(&a, stream_);  // null workspace: the size
+    if (query == FTK_ERR_UNSUPPORTED) {
+        return false;
+    }
+    check_ftk(query);
+    if (a.row.workspace_size > sampling_workspace_size_) {
+        // (the split of a row depends on the number of rows in the call: a window smaller than the setup batch can
+        // need a slightly larger workspace)
+        sampling_workspace_      = allocator_->reMalloc(sampling_workspace_, a.row.workspace_size, false);
+        sampling_workspace_size_ = a.row.workspace_size;
+    }
+    a.row.workspace      = sampling_workspace_;
+    a.row.workspace_size = sampling_workspace_size_;
+    check_ftk(ftk_fused_topp_penalty_step(&a, stream_));
+    sync_check_hip_error();
+    return true;
 }
 
 // reference: TopPSamplingLayer<T>::runSampling, layers/sampling_layers/TopPSamplingLayer.cu:256-343

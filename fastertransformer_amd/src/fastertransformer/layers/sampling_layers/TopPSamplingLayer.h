@@ -19,6 +19,8 @@ class TopPSamplingLayer: public BaseSamplingLayer<T> {
     void allocateBuffer(size_t batch_size, Tensor top_k, Tensor top_p) override;
     void freeBuffer() override;
     void runSampling(TensorMap* output_tensors, TensorMap* input_tensors, T* logits) override;
+    bool runFused(TensorMap* output_tensors, TensorMap* input_tensors) override;
+    size_t fusedBytes(size_t rows);
 
     using BaseSamplingLayer<T>::vocab_size_;
     using BaseSamplingLayer<T>::vocab_size_padded_;

@@ -259,6 +259,25 @@ typedef struct ftk_fused_topk_args {
 /* workspace == NULL in args: writes the required size into args->workspace_size, launches nothing. */
 int ftk_fused_topk_step(ftk_fused_topk_args* args, ftk_stream_t stream);
 
+/* The same for the rows a top-p layer owns: the kernel sequence BaseSamplingLayer<T>::forward +
+ * TopPSamplingLayer<T>::runSampling issue (layers/sampling_layers/TopPSamplingLayer.cu:256-343): temperature(+bias),
+ * repetition / presence penalty, min-length mask, softmax, nucleus sampling and decay, on logits that are only read
+ * (the values after the penalties are kept in the workspace). Results are bit for bit those of the kernel sequence.
+ * `row` carries what the two steps have in common; its top_ks, top_ps and max_top_k are not read. An embedding bias
+ * needs `temperatures`. FTK_ERR_UNSUPPORTED (also from the size query) for fewer than 1024 columns, a frequency
+ * penalty, or a vocabulary of more than a million columns with a history penalty: run the kernel sequence then.
+ * row.workspace == NULL: size query into row.workspace_size. */
+typedef struct ftk_fused_topp_args {
+    ftk_fused_topk_args row;
+    float               max_top_p;     /* every row's p when runtime_top_p is NULL */
+    float*              runtime_top_p; /* [local], decayed in place when top_p_decay is given */
+    const float*        initial_top_p;
+    const float*        top_p_decay; /* NULL: no decay */
+    const float*        top_p_min;
+    const int32_t*      top_p_reset_ids;
+} ftk_fused_topp_args;
+int ftk_fused_topp_penalty_step(ftk_fused_topp_args* args, ftk_stream_t stream);
+
 /* ---- the fused step over vocabulary shards (producer hand-over) --------------------------------------
  * The reference writes a step's logits from its last GEMM - one vocabulary shard per rank under tensor parallelism,
  * gathered afterwards - and reads them back in DynamicDecodeLayer::forward
