@@ -86,3 +86,51 @@ def test_forms_of_the_log_prob_step_agree_bit_for_bit(dt, B, V, Vp, H, k, kind):
         for name, a, b in zip(("ids", "sequence_length", "finished", "cum_log_probs", "output_log_probs"), ref,
                               results[form]):
             assert np.array_equal(a, b), "%s differ between the two-launch form and %d threads per row" % (name, form)
+
+
+PEAKED = [
+    (O.F16, 6, 9001, 9001, 64, "sharp"),    # k-th probability below binary16's normal range
+    (O.F16, 4, 9001, 9008, 128, "sharper"),  # ... below its smallest number: zeros are picked, pads among them
+    (O.F16, 5, 5003, 5003, 40, "plateau"),  # small probabilities in long runs of ties under a large denominator
+    (O.F32, 4, 5003, 5008, 16, "level"),    # nothing but ties; the short first stage (thread numbers below 128)
+    (O.BF16, 4, 3001, 3001, 128, "level"),
+    (O.F32, 4, 2050, 2056, 128, "alone"),   # one column, every other probability exactly zero
+    (O.BF16, 4, 2050, 2050, 100, "few"),    # fewer numbers than k
+]
+
+
+@pytest.mark.parametrize("dt,B,V,Vp,k,kind", PEAKED, ids=["%s-%d-%s" % (DTYPE_NAMES[c[0]], c[2], c[5]) for c in PEAKED])
+def test_rows_whose_candidates_are_gathered_again(dt, B, V, Vp, k, kind):
+    """Rows that one bound on e cannot settle: ids and log-probs of the oracle's full sequence."""
+    from decode_harness import Case, OracleRunner, ProductRunner, compare
+    from helpers import uniforms
+    rng = np.random.default_rng(len(kind) * 1000 + V)
+    H = 12
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=2, runtime_top_k=[k], runtime_top_p=[1.0], temperature=[0.9],
+             repetition_penalty=[1.2], prompt=rng.integers(0, V, (H, B)).astype(np.int32), with_cum=True,
+             with_out_lp=True)
+    p, o = ProductRunner(c), OracleRunner(c)
+    for i in range(2):
+        x = rng.standard_normal((B, Vp)).astype(np.float32)
+        if kind == "sharp":
+            x *= 6.0
+            x[:, 17] = 28.0
+        elif kind == "sharper":
+            x[:, 17] = 40.0
+        elif kind == "plateau":
+            x = np.round(x * 2.0) / 2.0
+            x[:, 100:160] = 14.0
+        elif kind == "level":
+            x[:] = 0.5
+            x[:, 7::701] = 0.75
+        elif kind == "alone":
+            x[:] = -300.0
+            x[:, 1234] = 5.0
+        else:
+            x[:] = -np.inf
+            x[:, ::97] = 1.0
+        x = O.to_storage(x, dt)
+        u = uniforms(rng, B)
+        p.step(H + i, x, u)
+        o.step(H + i, x, u)
+        compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="%s step %d" % (kind, i))
