@@ -194,7 +194,7 @@ __device__ __forceinline__ float beam_element_of(float xv, const typename Storag
 struct BeamPlan {
     int    parts;  // sections per row
     int    section;
-    size_t off_pmax, off_psum, off_pkeys, off_cand_id, off_cand_val, bytes;
+    size_t off_pmax, off_psum, off_pkeys, off_cand_id, off_cand_val, off_before, bytes;
 };
 
 static inline size_t beam_align(size_t x)
@@ -228,8 +228,38 @@ static BeamPlan beam_plan(int rows, int beam_width, int vocab)
     off += beam_align(r * N * sizeof(int));
     p.off_cand_val = off;
     off += beam_align(r * N * sizeof(float));
+    p.off_before = off;
+    off += beam_align(r * sizeof(int2));
     p.bytes = off;
     return p;
+}
+
+// What a finished row offers (:328-336): MAX_T at its end id, -MAX_T elsewhere, so the end id first, then the lowest
+// ids. Element t of that list.
+struct BeamFinishedRow {
+    bool  inside;  // the end id is a column
+    float m, d;    // maximum and sum of exponentials: inside, every other exponential is 0
+};
+template<int DT>
+__device__ __forceinline__ BeamFinishedRow beam_finished_row(int end_id, int vocab)
+{
+    const bool inside = end_id >= 0 && end_id < vocab;
+    return BeamFinishedRow{inside, inside ? Storage<DT>::max_t() : -Storage<DT>::max_t(), inside ? 1.0f : (float)vocab};
+}
+template<int DT>
+__device__ __forceinline__ unsigned long long beam_finished_key(const BeamFinishedRow& f, int end_id, int t)
+{
+    const int   id = f.inside ? (t == 0 ? end_id : (t - 1 < end_id ? t - 1 : t)) : t;
+    const float u  = f.inside && t == 0 ? Storage<DT>::max_t() : -Storage<DT>::max_t();
+    return beam_key(u, (uint32_t)id);
+}
+
+// A row's flag and length as they were before the step: the batch kernel of a step that updates them in the same
+// launch reads those of other entries' rows.
+__device__ __forceinline__ void beam_keep_before(int2* __restrict__ before, const bool* __restrict__ finished,
+                                                 const int* __restrict__ sequence_lengths, int row)
+{
+    before[row] = make_int2(finished[row] ? 1 : 0, sequence_lengths != nullptr ? sequence_lengths[row] : 0);
 }
 
 // (parts x rows) workgroups: the maximum of a section
@@ -362,7 +392,8 @@ __global__ void __launch_bounds__(BM_THREADS)
 beam_row_kernel(const bool* __restrict__ finished, const int* __restrict__ end_ids,
                 const float* __restrict__ cum_log_probs, int vocab, int K, int parts, const float* __restrict__ pmax,
                 const double* __restrict__ psum, const unsigned long long* __restrict__ pkeys,
-                int* __restrict__ cand_id, float* __restrict__ cand_val)
+                int* __restrict__ cand_id, float* __restrict__ cand_val, const int* __restrict__ sequence_lengths,
+                int2* __restrict__ before)
 {
     typedef Storage<DT>   S;
     __shared__ BeamSelect s;
@@ -371,26 +402,16 @@ beam_row_kernel(const bool* __restrict__ finished, const int* __restrict__ end_i
     const int             N    = 2 * K;
     const float           MAXT = S::max_t();
     const float           cum  = cum_log_probs[row];
+    if (t == 0) {
+        beam_keep_before(before, finished, sequence_lengths, row);
+    }
     if (finished[row]) {
-        // MAX_T at the end id, -MAX_T elsewhere (:328-336): the end id first, then the lowest ids
-        const int  end_id = end_ids[row / K];
-        const bool inside = end_id >= 0 && end_id < vocab;
+        const int             end_id = end_ids[row / K];
+        const BeamFinishedRow f      = beam_finished_row<DT>(end_id, vocab);
         if (t < N) {
-            int   id;
-            float u;
-            if (inside) {
-                id = t == 0 ? end_id : (t - 1 < end_id ? t - 1 : t);
-                u  = t == 0 ? MAXT : -MAXT;
-            }
-            else {
-                id = t;
-                u  = -MAXT;
-            }
-            // inside: m = MAX_T, every other exponential is 0, d = 1; otherwise m = -MAX_T and d = vocab
-            const float m    = inside ? MAXT : -MAXT;
-            const float logd = inside ? 0.0f : det_logf((float)vocab);
-            cand_id[(size_t)row * N + t]  = id + row * vocab;
-            cand_val[(size_t)row * N + t] = round_t<DT>((u - m - logd) + cum);
+            const unsigned long long k   = beam_finished_key<DT>(f, end_id, t);
+            cand_id[(size_t)row * N + t] = (int)beam_key_position(k) + row * vocab;
+            cand_val[(size_t)row * N + t] = round_t<DT>((beam_key_value(k) - f.m - det_logf(f.d)) + cum);
         }
         return;
     }
@@ -430,12 +451,86 @@ beam_row_kernel(const bool* __restrict__ finished, const int* __restrict__ end_i
 // run beside the other's exponentials (64 x 8 beams x 152064 fp16: 120 -> 116 us).
 constexpr int BR_THREADS = 1024;
 
+// A value at or below the row's 2K-th largest, from the threads' maxima, and the row's sum from the waves' sums: found
+// by the first wave alone while the others wait at two barriers. Leaves the candidates' count at zero.
+template<int THREADS>
+__device__ __forceinline__ void beam_bound(BeamSelect& s, const double* red, float fmax, int N, double& row_sum,
+                                           uint32_t& floor)
+{
+    const int t = threadIdx.x;
+    // 2K <= 32 needs no more than 64 maxima to choose the 2K-th largest from, 2K <= 64 no more than 128
+    const int n_slots = N <= 32 ? 64 : N <= 64 ? 128 : 256;
+    const int join    = THREADS / n_slots;  // neighbouring threads that join their maxima: 2 to 16
+    fmax              = __builtin_fmaxf(fmax, __shfl_xor(fmax, 1, WAVE));
+    if (join >= 4) {
+        fmax = __builtin_fmaxf(fmax, __shfl_xor(fmax, 2, WAVE));
+    }
+    if (join >= 8) {
+        fmax = __builtin_fmaxf(fmax, __shfl_xor(fmax, 4, WAVE));
+    }
+    if (join == 16) {
+        fmax = __builtin_fmaxf(fmax, __shfl_xor(fmax, 8, WAVE));
+    }
+    uint32_t* slot_key = reinterpret_cast<uint32_t*>(s.slots);
+    if (t % join == 0) {
+        slot_key[t / join] = order_key(fmax);
+    }
+    if (t == 0) {
+        s.n_cand = 0;
+    }
+    __syncthreads();
+    if (wave_id() == 0) {
+        // The 2K-th largest of the maxima is an element with at least 2K elements at or above it: nothing below it
+        // can be among the 2K best; so is any value below that one. (A group that saw no element reports -inf.)
+        uint32_t P = 0u;
+        if (n_slots == WAVE) {
+            // every lane counts the maxima above its own and those at or above it: the 2K-th largest lies between
+            const uint32_t mine  = slot_key[lane_id()];
+            int            above = 0, reach = 0;
+#pragma unroll
+            for (int j = 0; j < WAVE; ++j) {
+                const uint32_t other = __builtin_amdgcn_readlane(mine, j);
+                above += other > mine ? 1 : 0;
+                reach += other >= mine ? 1 : 0;
+            }
+            const unsigned long long at = __ballot(above < N && reach >= N);
+            P = __builtin_amdgcn_readlane(mine, __builtin_ctzll(at));
+        }
+        else {
+            uint32_t kk[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int i = lane_id() + g * WAVE;
+                kk[g]       = i < n_slots ? slot_key[i] : 0u;
+            }
+            for (int bit = 31; bit >= 8; --bit) {
+                const uint32_t cand = P | (1u << bit);
+                int            c    = 0;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    c += (int)__builtin_popcountll(__ballot(kk[g] >= cand));
+                }
+                P = c >= N ? cand : P;
+            }
+        }
+        if (lane_id() == 0) {
+            double tot = 0.0;
+            for (int w = 0; w < THREADS / WAVE; ++w) {
+                tot += red[w];
+            }
+            row_sum = tot;
+            floor   = P;
+        }
+    }
+    __syncthreads();
+}
+
 template<int DT, int THREADS>
 __global__ void __launch_bounds__(THREADS)
 beam_rowwide_kernel(const typename Storage<DT>::T* __restrict__ x, const typename Storage<DT>::T* __restrict__ bias,
                     const bool* __restrict__ finished, const int* __restrict__ end_ids,
                     const float* __restrict__ cum_log_probs, int vocab, int K, int* __restrict__ cand_id,
-                    float* __restrict__ cand_val)
+                    float* __restrict__ cand_val, const int* __restrict__ sequence_lengths, int2* __restrict__ before)
 {
     typedef Storage<DT>   S;
     constexpr int         BR_WAVES = THREADS / WAVE;
@@ -450,25 +545,16 @@ beam_rowwide_kernel(const typename Storage<DT>::T* __restrict__ x, const typenam
     const int             N    = 2 * K;
     const float           MAXT = S::max_t();
     const float           cum  = cum_log_probs[row];
+    if (t == 0) {
+        beam_keep_before(before, finished, sequence_lengths, row);
+    }
     if (finished[row]) {
-        // MAX_T at the end id, -MAX_T elsewhere (:328-336): the end id first, then the lowest ids
-        const int  end_id = end_ids[row / K];
-        const bool inside = end_id >= 0 && end_id < vocab;
+        const int             end_id = end_ids[row / K];
+        const BeamFinishedRow f      = beam_finished_row<DT>(end_id, vocab);
         if (t < N) {
-            int   id;
-            float u;
-            if (inside) {
-                id = t == 0 ? end_id : (t - 1 < end_id ? t - 1 : t);
-                u  = t == 0 ? MAXT : -MAXT;
-            }
-            else {
-                id = t;
-                u  = -MAXT;
-            }
-            const float m    = inside ? MAXT : -MAXT;
-            const float logd = inside ? 0.0f : det_logf((float)vocab);
-            cand_id[(size_t)row * N + t]  = id + row * vocab;
-            cand_val[(size_t)row * N + t] = round_t<DT>((u - m - logd) + cum);
+            const unsigned long long k   = beam_finished_key<DT>(f, end_id, t);
+            cand_id[(size_t)row * N + t] = (int)beam_key_position(k) + row * vocab;
+            cand_val[(size_t)row * N + t] = round_t<DT>((beam_key_value(k) - f.m - det_logf(f.d)) + cum);
         }
         return;
     }
@@ -495,56 +581,7 @@ beam_rowwide_kernel(const typename Storage<DT>::T* __restrict__ x, const typenam
     if (lane_id() == 0) {
         red[wave_id()] = d;
     }
-    // 2K <= 32 needs no more than 64 maxima to choose the 2K-th largest from, 2K <= 64 no more than 128
-    const int n_slots = N <= 32 ? 64 : N <= 64 ? 128 : 256;
-    const int join    = THREADS / n_slots;  // neighbouring threads that join their maxima: 2 to 16
-    fmax              = __builtin_fmaxf(fmax, __shfl_xor(fmax, 1, WAVE));
-    if (join >= 4) {
-        fmax = __builtin_fmaxf(fmax, __shfl_xor(fmax, 2, WAVE));
-    }
-    if (join >= 8) {
-        fmax = __builtin_fmaxf(fmax, __shfl_xor(fmax, 4, WAVE));
-    }
-    if (join == 16) {
-        fmax = __builtin_fmaxf(fmax, __shfl_xor(fmax, 8, WAVE));
-    }
-    uint32_t* slot_key = reinterpret_cast<uint32_t*>(s.slots);
-    if (t % join == 0) {
-        slot_key[t / join] = order_key(fmax);
-    }
-    if (t == 0) {
-        s.n_cand = 0;
-    }
-    __syncthreads();
-    if (wave_id() == 0) {
-        uint32_t kk[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int i = lane_id() + g * WAVE;
-            kk[g]       = i < n_slots ? slot_key[i] : 0u;
-        }
-        // The 2K-th largest of the maxima is an element with at least 2K elements at or above it: nothing below it
-        // can be among the 2K best; so is any value below that one. (A group that saw no element reports -inf.)
-        uint32_t P = 0u;
-        for (int bit = 31; bit >= 8; --bit) {
-            const uint32_t cand = P | (1u << bit);
-            int            c    = 0;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                c += (int)__builtin_popcountll(__ballot(kk[g] >= cand));
-            }
-            P = c >= N ? cand : P;
-        }
-        if (lane_id() == 0) {
-            double tot = 0.0;
-            for (int w = 0; w < BR_WAVES; ++w) {
-                tot += red[w];
-            }
-            row_sum   = tot;
-            row_floor = P;
-        }
-    }
-    __syncthreads();
+    beam_bound<THREADS>(s, red, fmax, N, row_sum, row_floor);
     const uint32_t floor_key = row_floor;
     const float    floor_val = key_to_float(floor_key);
     const bool     all_pass  = floor_key <= order_key(-__builtin_inff());  // then NaN columns are wanted too
@@ -578,6 +615,168 @@ beam_rowwide_kernel(const typename Storage<DT>::T* __restrict__ x, const typenam
     }
 }
 
+// Rows of up to 65536 columns, read once: a thread keeps its vectors in registers through the three passes, and with
+// at most half as many rows as compute units 2, 4 or 8 workgroups share a row. Every workgroup of a row reads all of it
+// for the maximum (100 KB of a row of 50257 fp16, from the XCD's L2 after the first), so they need nothing of each
+// other; the exponentials, which bound the kernel (23 vector instructions and a double addition each), and the
+// candidates are those of its own part. A part leaves its 2K best, largest first, and its sum; beam_batch_kernel merges.
+// 32 x 4 rows of 50257 fp16: 19.6 us with one workgroup per row that reads it three times, 14.9 us here (traced).
+constexpr int BT_COLUMNS   = 65536;
+constexpr int BT_MAX_PARTS = 8;
+
+template<int DT>
+__global__ void __launch_bounds__(BR_THREADS)
+beam_team_kernel(const typename Storage<DT>::T* __restrict__ x, const typename Storage<DT>::T* __restrict__ bias,
+                 const bool* __restrict__ finished, const int* __restrict__ end_ids,
+                 const int* __restrict__ sequence_lengths, int vocab, int K, float* __restrict__ pmax,
+                 double* __restrict__ psum, unsigned long long* __restrict__ pkeys, int2* __restrict__ before)
+{
+    typedef Storage<DT>   S;
+    typedef typename S::T T;
+    constexpr int         EPV   = (int)(16 / sizeof(T));
+    constexpr int         NV    = BT_COLUMNS / EPV / BR_THREADS;  // vectors of a thread: 8, or 16 of floats
+    constexpr int         WAVES = BR_THREADS / WAVE;
+    __shared__ BeamSelect s;
+    __shared__ double     red[WAVES];
+    __shared__ float      redf[WAVES];
+    __shared__ double     part_sum;
+    __shared__ uint32_t   part_floor;
+    const int             row   = blockIdx.x;
+    const int             part  = blockIdx.y;
+    const int             parts = gridDim.y;
+    const int             t     = threadIdx.x;
+    const int             N     = 2 * K;
+    const float           NEG   = -__builtin_inff();
+    const bool            done  = finished[row];
+    // the row: up to seven columns in front of the first 16-byte boundary, vectors, up to seven columns behind the last
+    const T*     rowp  = x + (size_t)row * vocab;
+    const int    head  = min((int)(((16u - ((uintptr_t)rowp & 15u)) & 15u) / sizeof(T)), vocab);
+    const int    nvec  = (vocab - head) / EPV;
+    const int    tail0 = head + nvec * EPV;
+    const uint4* vec   = reinterpret_cast<const uint4*>(rowp + head);
+    const int    lo    = nvec * part / parts;  // this part's vectors: at most NV * BR_THREADS
+    const int    own   = nvec * (part + 1) / parts - lo;
+    uint4        raw[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = t + u * BR_THREADS;
+        raw[u]      = i < own ? vec[lo + i] : make_uint4(0, 0, 0, 0);
+    }
+    // threads 0..6 hold the columns in front, the second wave's first seven those behind
+    const int  edge     = t < head ? t : (t >= WAVE && t - WAVE < vocab - tail0 ? tail0 + t - WAVE : -1);
+    const bool edge_own = edge >= 0 && (edge < head ? part == 0 : part == parts - 1);
+    const float edge_x  = edge >= 0 ? beam_element_of<DT>(S::ld(rowp[edge]), bias, edge) : NEG;
+    if (t == 0 && part == 0) {
+        beam_keep_before(before, finished, sequence_lengths, row);
+    }
+    unsigned long long* keys = pkeys + ((size_t)row * parts + part) * N;
+    if (done) {
+        const int             end_id = end_ids[row / K];
+        const BeamFinishedRow f      = beam_finished_row<DT>(end_id, vocab);
+        if (t < N) {
+            keys[t] = part == 0 ? beam_finished_key<DT>(f, end_id, t) : 0ull;  // (0 is below every element's key)
+        }
+        if (t == 0) {
+            psum[(size_t)row * parts + part] = part == 0 ? (double)f.d : 0.0;
+            if (part == 0) {
+                pmax[row] = f.m;
+            }
+        }
+        return;
+    }
+    auto each_own = [&](auto&& visit) {
+        if (edge_own) {
+            visit(edge, edge_x);
+        }
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int i = t + u * BR_THREADS;
+            if (i < own) {
+                const T*  e = reinterpret_cast<const T*>(&raw[u]);
+                const int v = head + (lo + i) * EPV;
+#pragma unroll
+                for (int j = 0; j < EPV; ++j) {
+                    visit(v + j, beam_element_of<DT>(S::ld(e[j]), bias, v + j));
+                }
+            }
+        }
+    };
+    // the row's maximum, and the thread's own largest element
+    float m    = -S::max_t();
+    float fmax = NEG;
+    // the other parts' vectors, seen only here
+    constexpr int U      = 4;
+    const int     others = nvec - own;
+    for (int o0 = t; o0 < others; o0 += U * BR_THREADS) {
+        uint4 ov[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int o = o0 + u * BR_THREADS;
+            ov[u]       = o < others ? vec[o < lo ? o : o + own] : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int o = o0 + u * BR_THREADS;
+            if (o < others) {
+                const T*  e = reinterpret_cast<const T*>(&ov[u]);
+                const int v = head + (o < lo ? o : o + own) * EPV;
+#pragma unroll
+                for (int j = 0; j < EPV; ++j) {
+                    m = __builtin_fmaxf(m, beam_element_of<DT>(S::ld(e[j]), bias, v + j));
+                }
+            }
+        }
+    }
+    m = __builtin_fmaxf(m, edge_x);
+    each_own([&](int, float e) { fmax = __builtin_fmaxf(fmax, e); });  // (a NaN is never the maximum)
+    m = block_max<float, WAVES>(__builtin_fmaxf(m, fmax), redf, -S::max_t());
+    double d = 0.0;
+    each_own([&](int, float e) { d += (double)det_expf_nonpos(e - m); });
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        d += __shfl_xor(d, o, WAVE);
+    }
+    if (lane_id() == 0) {
+        red[wave_id()] = d;
+    }
+    beam_bound<BR_THREADS>(s, red, fmax, N, part_sum, part_floor);
+    const uint32_t floor_key = part_floor;
+    const float    floor_val = key_to_float(floor_key);
+    const bool     all_pass  = floor_key <= order_key(NEG);  // then NaN columns are wanted too
+    each_own([&](int v, float e) {
+        if (e >= floor_val || all_pass) {
+            const int at = atomicAdd(&s.n_cand, 1);
+            if (at < BM_CAP) {
+                s.cand[at] = beam_key(e, (uint32_t)v);
+            }
+        }
+    });
+    __syncthreads();
+    if (wave_id() >= BM_WAVES) {
+        return;  // the first four waves select
+    }
+    const int passed = s.n_cand;
+    if (passed <= BM_CAP) {
+        beam_select(s, [&](int i) { return s.cand[i]; }, passed, N);
+    }
+    else {
+        // (rows of many equal values) the selection runs over the part itself
+        const int from  = part == 0 ? 0 : head + lo * EPV;
+        const int until = part == parts - 1 ? vocab : head + (lo + own) * EPV;
+        beam_select(s, [&](int i) { return beam_key(beam_element<DT>(rowp, bias, 0, from + i), (uint32_t)(from + i)); },
+                    until - from, N);
+    }
+    if (t < N) {
+        keys[t] = s.out[t];
+    }
+    if (t == 0) {
+        psum[(size_t)row * parts + part] = part_sum;
+        if (part == 0) {
+            pmax[row] = m;
+        }
+    }
+}
+
 struct BeamHypsDevice {
     int*         output_ids_tgt;
     int*         sequence_lengths_tgt;
@@ -599,142 +798,381 @@ struct BeamHypsDevice {
     int          early_stopping;
 };
 
-// one workgroup per batch entry (:99-262)
+// Where the rows' candidates come from: a list per row, ranked and valued (parts == 0), or per part of a row (1 to 8)
+// its best keys in order and its sum, with the row's maximum.
+struct BeamCandidates {
+    const int*                id;
+    const float*              val;
+    int                       parts;
+    const float*              pmax;
+    const double*             psum;
+    const unsigned long long* pkeys;
+    const int2*               before;  // per row: finished and length before the step
+};
+
+// What a whole step does after the beams are chosen (all of it, or nothing: parent_ids == nullptr)
+struct BeamUpdate {
+    bool*      finished;
+    int*       sequence_length;
+    int*       parent_ids;
+    int*       cache_tgt;  // nullptr: the cache indirection is left to a launch of its own
+    const int* cache_src;
+    int        start_step, num_steps, max_seq_len, step;
+};
+
+constexpr int BB_HISTORY = 1024;  // (step, beam) pairs of the history kept in LDS
+constexpr int BB_MERGED  = 1024;  // keys of an entry that are merged here
+constexpr int BB_CACHE   = 4096;  // cache positions of an entry that are copied here: 16 per thread
+
+// One workgroup per batch entry (:99-262). Bound by latency: a few hundred candidates and one thread that walks the
+// best of them. So everything the walk may read is requested before anything is computed - the hypotheses' state and
+// the last BB_HISTORY (step, beam) pairs of tokens, parents and log-probs among it, through which a finished beam is
+// traced in LDS instead of one dependent read per step - and the launches that followed it (token and parent split,
+// flags, lengths, cache indirection: 4.4 and 3.6 us of mostly latency) are its last lines.
+// 32 entries of 4 beams: 16.8 us in three launches, 9.9 us here (traced); the step 34 -> 25 us.
 template<int DT>
 __global__ void __launch_bounds__(BM_THREADS)
-beam_batch_kernel(const int* __restrict__ cand_id, const float* __restrict__ cand_val, int* __restrict__ ids,
-                  float* cum_log_probs, float* __restrict__ output_log_probs, const bool* __restrict__ finished,
-                  const int* __restrict__ sequence_lengths, BeamHypsDevice h, int K, int max_k2, int vocab,
+beam_batch_kernel(BeamCandidates cd, int* ids, float* cum_log_probs, float* __restrict__ output_log_probs,
+                  const int* __restrict__ end_ids, BeamHypsDevice h, BeamUpdate up, int K, int max_k2, int vocab,
                   float length_penalty, float diversity_rate)
 {
     __shared__ BeamSelect s;
     __shared__ float      old_cum[64];
-    __shared__ float      score_of[BM_MAX_N];
-    const int             b = blockIdx.x;
-    const int             t = threadIdx.x;
-    const int             C = K * 2 * K;
-    const int*            x = cand_id + (size_t)b * C;
-    const float*          y = cand_val + (size_t)b * C;
-    if (t < K) {
-        old_cum[t] = cum_log_probs[b * K + t];
+    __shared__ float      normed[BM_MAX_N];
+    __shared__ int        hist_id[BB_HISTORY], hist_parent[BB_HISTORY];
+    __shared__ float      hist_lp[BB_HISTORY];
+    __shared__ int        cand_x[BM_MAX_N], cand_beam[BM_MAX_N], cand_ends[BM_MAX_N];
+    __shared__ float      cand_y[BM_MAX_N], score_of[BM_MAX_N];
+    __shared__ int        chosen[WAVE], counted[WAVE], parent_of[WAVE], live[WAVE];
+    __shared__ int        complete;  // the entry has its beam_width hypotheses
+    __shared__ int        merged_id[BB_MERGED];
+    __shared__ float      merged_val[BB_MERGED];
+    __shared__ int        cached[BB_MERGED];
+    __shared__ double     part_sum[WAVE];  // (2 K K parts <= BB_MERGED: at most 64 sums)
+    __shared__ float      row_max[WAVE];
+    const int             b         = blockIdx.x;
+    const int             t         = threadIdx.x;
+    const int             N         = 2 * K;
+    const int             C         = K * N;
+    const bool            with_hyps = h.num_beams != nullptr;
+    const bool            updates   = up.parent_ids != nullptr;
+    const int             g         = h.ite * h.local_batch_size + b;
+    // ---- what is read, all of it requested before the first value is used (indices of idle threads are clamped: a
+    // branch per thread would make every group of loads wait for the one before)
+    const int   nb0     = with_hyps ? h.num_beams[g] : 0;
+    const int   nb_here = with_hyps ? h.num_beams[b] : 0;
+    const float mn0     = with_hyps ? h.min_normed_scores[g] : 0.0f;
+    const int   end_h   = with_hyps ? h.end_ids[b] : -1;
+    const int   end_u   = end_ids[b];
+    const int2  before  = cd.before[b];
+    const int   own     = b * K + min(t, K - 1);
+    const float r_cum   = cum_log_probs[own];
+    int         r_id = 0, r_len = 0;
+    bool        r_fin = false;
+    if (updates) {
+        r_id  = ids[own];
+        r_len = up.sequence_length[own];
+        r_fin = up.finished[own];
     }
-    const bool with_hyps = h.num_beams != nullptr;
-    const int  g         = h.ite * h.local_batch_size + b;
+    constexpr int      TURNS   = BB_MERGED / BM_THREADS;
+    const int          per_row = cd.parts * N;
+    const int          n_keys  = K * per_row;
+    unsigned long long r_key[TURNS];
+    double             r_sum = 0.0;
+    float              r_max = 0.0f;
+    if (cd.parts > 0) {
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            if (u * BM_THREADS < n_keys) {
+                r_key[u] = cd.pkeys[(size_t)b * n_keys + min(t + u * BM_THREADS, n_keys - 1)];
+            }
+        }
+        r_sum = cd.psum[(size_t)b * K * cd.parts + min(t, K * cd.parts - 1)];
+        r_max = cd.pmax[own];
+    }
+    const int  kept    = with_hyps ? min(h.step, BB_HISTORY / K) : 0;  // steps of the history in LDS: the last ones
+    const bool with_lp = h.log_probs != nullptr && h.log_probs_src != nullptr;
+    float      r_normed = 0.0f;
+    int        r_hid[TURNS], r_hparent[TURNS];
+    float      r_hlp[TURNS];
     if (with_hyps) {
-        const int nb = h.num_beams[g];
-        if (nb == 0 && t == 0) {
-            h.min_normed_scores[g] = 3.402823466e+38f;
-        }
-        else if (nb == K) {
-            return;
-        }
-    }
-    // (:146-156) the batch entry's own flag and length are used for all of its beams, as in the reference
-    float denom = 1.0f;
-    if (length_penalty != 0.0f) {
-        const int length = finished[b] ? sequence_lengths[b] : sequence_lengths[b] + 1;
-        if (length != 1) {
-            denom = round_t<DT>(det_expf(length_penalty * det_logf((float)length)));
-        }
-        else {
-            length_penalty = 0.0f;
+        r_normed = h.normed_scores[(size_t)g * N + min(t, N - 1)];
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            if (u * BM_THREADS < kept * K) {
+                const int    i   = min(t + u * BM_THREADS, kept * K - 1);
+                const size_t src = (size_t)(h.step - kept + i / K) * h.batch_size * K + (size_t)g * K + i % K;
+                r_hid[u]         = h.output_ids_src[src];
+                r_hparent[u]     = h.parent_ids_src[src];
+                r_hlp[u]         = with_lp ? h.log_probs_src[src] : 0.0f;
+            }
         }
     }
-    const float div_t = round_t<DT>(diversity_rate);
-    auto        score = [&](int c) {
-        float elem = y[c];
-        if (length_penalty != 0.0f) {
-            elem = round_t<DT>(elem / denom);
+    const bool cache_here = up.cache_tgt != nullptr && K * up.num_steps <= BB_MERGED;  // its source goes to LDS, too
+    int        r_cache[TURNS];
+    if (cache_here) {
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            if (u * BM_THREADS < K * up.num_steps) {
+                const int i    = min(t + u * BM_THREADS, K * up.num_steps - 1);
+                const int circ = (up.start_step + i % up.num_steps) % up.max_seq_len;
+                r_cache[u]     = up.cache_src[((size_t)b * K + i / up.num_steps) * up.max_seq_len + circ];
+            }
         }
-        return round_t<DT>(elem + round_t<DT>(div_t * round_t<DT>((float)(c % K))));
-    };
-    const int take = max_k2 < C ? max_k2 : C;
-    beam_select(s, [&](int c) { return beam_key(score(c), (uint32_t)c); }, C, take);
-    // what the walk reads about its candidates, fetched by one thread each
-    __shared__ int   cand_x[BM_MAX_N];
-    __shared__ float cand_y[BM_MAX_N];
-    if (t < take) {
-        const int p = (int)beam_key_position(s.out[t]);
-        score_of[t] = score(p);
-        cand_x[t]   = x[p];
-        cand_y[t]   = y[p];
+    }
+    // ---- and kept
+    if (t < K) {
+        old_cum[t] = r_cum;
+        if (updates) {
+            chosen[t]  = r_id;  // (kept where the walk chooses nothing)
+            counted[t] = r_fin ? r_len : r_len + 1;
+        }
+        if (cd.parts > 0) {
+            row_max[t] = r_max;
+        }
+    }
+    if (with_hyps) {
+        if (t < N) {
+            normed[t] = r_normed;
+        }
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            const int i = t + u * BM_THREADS;
+            if (i < kept * K) {
+                hist_id[i]     = r_hid[u];
+                hist_parent[i] = r_hparent[u];
+                hist_lp[i]     = r_hlp[u];
+            }
+        }
+    }
+    if (cache_here) {
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            const int i = t + u * BM_THREADS;
+            if (i < K * up.num_steps) {
+                cached[i] = r_cache[u];
+            }
+        }
+    }
+    const int*   x = cd.id + (size_t)b * C;
+    const float* y = cd.val + (size_t)b * C;
+    if (cd.parts > 0) {
+        if (t < K * cd.parts) {
+            part_sum[t] = r_sum;
+        }
+#pragma unroll
+        for (int u = 0; u < TURNS; ++u) {
+            const int i = t + u * BM_THREADS;
+            if (i < n_keys) {
+                s.cand[i] = r_key[u];
+            }
+        }
+        __syncthreads();
+        for (int i = t; i < n_keys; i += BM_THREADS) {
+            const unsigned long long k     = s.cand[i];
+            const int                r     = i / per_row;
+            const int                at    = i % per_row;
+            int                      place = at % N;  // its own part's keys in front of it
+            for (int p = 0; p < cd.parts; ++p) {
+                if (p != at / N) {
+                    const unsigned long long* other = s.cand + r * per_row + p * N;
+                    for (int j = 0; j < N; ++j) {
+                        place += other[j] > k ? 1 : 0;
+                    }
+                }
+            }
+            // (a finished row's other parts hold zeros, below the first part's 2K keys: they get no place)
+            if (place < N && k != 0ull) {
+                double d = 0.0;
+                for (int p = 0; p < cd.parts; ++p) {
+                    d += part_sum[r * cd.parts + p];
+                }
+                merged_id[r * N + place] = (int)beam_key_position(k) + (b * K + r) * vocab;
+                merged_val[r * N + place] =
+                    round_t<DT>((beam_key_value(k) - row_max[r] - det_logf((float)d)) + old_cum[r]);
+            }
+        }
+        x = merged_id;
+        y = merged_val;
     }
     __syncthreads();
-    if (t != 0) {
+    const bool  skip = with_hyps && nb0 == K;
+    const float none = 3.402823466e+38f;
+    if (!skip) {
+        // (:146-156) the batch entry's own flag and length are used for all of its beams, as in the reference
+        float denom = 1.0f;
+        if (length_penalty != 0.0f) {
+            const int length = before.x != 0 ? before.y : before.y + 1;
+            if (length != 1) {
+                denom = round_t<DT>(det_expf(length_penalty * det_logf((float)length)));
+            }
+            else {
+                length_penalty = 0.0f;
+            }
+        }
+        const float div_t = round_t<DT>(diversity_rate);
+        auto        score = [&](int c) {
+            float elem = y[c];
+            if (length_penalty != 0.0f) {
+                elem = round_t<DT>(elem / denom);
+            }
+            return round_t<DT>(elem + round_t<DT>(div_t * round_t<DT>((float)(c % K))));
+        };
+        const int take = max_k2 < C ? max_k2 : C;
+        beam_select(s, [&](int c) { return beam_key(score(c), (uint32_t)c); }, C, take);
+        // what the walk asks about its candidates, worked out by one thread each
+        if (t < take) {
+            const int p  = (int)beam_key_position(s.out[t]);
+            score_of[t]  = score(p);
+            cand_x[t]    = x[p];
+            cand_y[t]    = y[p];
+            cand_beam[t] = (cand_x[t] / vocab) % K;
+            cand_ends[t] = with_hyps && cand_x[t] % vocab == end_h ? 1 : 0;
+        }
+        __syncthreads();
+        if (t == 0) {
+            float* v        = cum_log_probs + (size_t)b * K;
+            int    selected = 0;
+            int    nb       = nb0;
+            float  mn       = nb0 == 0 ? none : mn0;
+            bool   closed   = false;
+            for (int i = 0; i < take; ++i) {
+                const int   xp = cand_x[i];
+                const float yp = cand_y[i];
+                if (cand_ends[i] != 0) {
+                    if (i < K) {
+                        const float normed_score = score_of[i];
+                        int         beam_idx     = nb;
+                        if (nb == K) {
+                            if (normed_score < mn) {
+                                break;
+                            }
+                            for (int j = 0; j < K; ++j) {
+                                if (normed[j] == mn) {
+                                    beam_idx = j;
+                                    nb--;
+                                    mn        = none;
+                                    normed[j] = normed_score;
+                                    for (int l = 0; l < K; ++l) {
+                                        mn = __builtin_fminf(mn, normed[l]);
+                                    }
+                                    break;
+                                }
+                            }
+                        }
+                        const int    tgt_beam = g * N + beam_idx;
+                        const size_t tgt      = (size_t)tgt_beam * h.max_seq_len;
+                        int          prev_id  = cand_beam[i];
+                        h.output_ids_tgt[tgt + h.step] = end_h;
+                        if (h.log_probs != nullptr) {
+                            h.log_probs[tgt + h.step] = yp - old_cum[prev_id];
+                        }
+                        for (int j = h.step - 1; j >= 0; --j) {
+                            const int back = j - (h.step - kept);
+                            int       id, parent;
+                            float     lp = 0.0f;
+                            // (a parent outside the beams of an entry - the caller's arrays are not checked - is
+                            // looked up in them like before)
+                            if (back >= 0 && prev_id >= 0 && prev_id < K) {
+                                id     = hist_id[back * K + prev_id];
+                                parent = hist_parent[back * K + prev_id];
+                                lp     = hist_lp[back * K + prev_id];
+                            }
+                            else {
+                                const size_t src = (size_t)j * h.batch_size * K + (size_t)g * K + prev_id;
+                                id               = h.output_ids_src[src];
+                                parent           = h.parent_ids_src[src];
+                                if (with_lp) {
+                                    lp = h.log_probs_src[src];
+                                }
+                            }
+                            h.output_ids_tgt[tgt + j] = id;
+                            if (with_lp) {
+                                h.log_probs[tgt + j] = lp;
+                            }
+                            prev_id = parent;
+                        }
+                        h.sequence_lengths_tgt[tgt_beam] = h.step;
+                        h.normed_scores[tgt_beam]        = normed_score;
+                        normed[beam_idx]                 = normed_score;
+                        mn                               = __builtin_fminf(mn, normed_score);
+                        nb++;
+                        h.cum_log_probs[tgt_beam] = yp;
+                    }
+                }
+                else if ((with_hyps && i < N) || (!with_hyps && i < K)) {
+                    if (updates) {
+                        chosen[selected] = xp;
+                    }
+                    else {
+                        ids[(size_t)b * K + selected] = xp;
+                    }
+                    if (output_log_probs != nullptr) {
+                        output_log_probs[b * K + selected] = yp - old_cum[cand_beam[i]];
+                    }
+                    v[selected] = yp;
+                    selected++;
+                }
+                if (selected >= K) {
+                    break;
+                }
+            }
+            if (with_hyps) {
+                if (nb0 == 0 || nb != nb0 || mn != mn0) {
+                    h.min_normed_scores[g] = mn;
+                }
+                if (nb != nb0) {
+                    h.num_beams[g] = nb;
+                }
+                closed         = (g == b ? nb : nb_here) >= K;
+                if (!closed) {
+                    h.is_done[b] = false;
+                }
+                else if (h.early_stopping) {
+                    h.is_done[b] = true;
+                }
+            }
+            complete = with_hyps && nb == K ? 1 : 0;
+        }
+    }
+    else if (t == 0) {
+        complete = 1;
+    }
+    if (!updates) {
         return;
     }
-    int*   z        = ids + (size_t)b * K;
-    float* v        = cum_log_probs + (size_t)b * K;
-    int    selected = 0;
-    const int end_id = with_hyps ? h.end_ids[b] : -1;
-    for (int i = 0; i < take; ++i) {
-        const int   xp = cand_x[i];
-        const float yp = cand_y[i];
-        if (with_hyps && xp % vocab == end_id) {
-            if (i < K) {
-                const float normed_score = score_of[i];
-                const int   num_beam     = h.num_beams[g];
-                int         beam_idx     = num_beam;
-                if (num_beam == K) {
-                    if (normed_score < h.min_normed_scores[g]) {
-                        selected = K;
-                        break;
-                    }
-                    for (int j = 0; j < K; ++j) {
-                        if (h.normed_scores[g * (K * 2) + j] == h.min_normed_scores[g]) {
-                            beam_idx = j;
-                            h.num_beams[g]--;
-                            h.min_normed_scores[g]           = 3.402823466e+38f;
-                            h.normed_scores[g * (K * 2) + j] = normed_score;
-                            for (int l = 0; l < K; ++l) {
-                                h.min_normed_scores[g] =
-                                    __builtin_fminf(h.min_normed_scores[g], h.normed_scores[g * (K * 2) + l]);
-                            }
-                            break;
-                        }
-                    }
-                }
-                const size_t tgt = ((size_t)(b + h.ite * h.local_batch_size) * (K * 2) + beam_idx) * h.max_seq_len;
-                h.output_ids_tgt[tgt + h.step] = end_id;
-                if (h.log_probs != nullptr) {
-                    h.log_probs[tgt + h.step] = yp - old_cum[(xp / vocab) % K];
-                }
-                int prev_id = (xp / vocab) % K;
-                for (int j = h.step - 1; j >= 0; --j) {
-                    const size_t src =
-                        (size_t)j * h.batch_size * K + (size_t)h.ite * h.local_batch_size * K + (size_t)b * K + prev_id;
-                    h.output_ids_tgt[tgt + j] = h.output_ids_src[src];
-                    if (h.log_probs != nullptr && h.log_probs_src != nullptr) {
-                        h.log_probs[tgt + j] = h.log_probs_src[src];
-                    }
-                    prev_id = h.parent_ids_src[src];
-                }
-                const int tgt_beam              = g * (K * 2) + beam_idx;
-                h.sequence_lengths_tgt[tgt_beam] = h.step;
-                h.normed_scores[tgt_beam]        = normed_score;
-                h.min_normed_scores[g] = __builtin_fminf(h.min_normed_scores[g], h.normed_scores[tgt_beam]);
-                h.num_beams[g]++;
-                h.cum_log_probs[tgt_beam] = yp;
-            }
-        }
-        else if ((with_hyps && i < 2 * K) || (!with_hyps && i < K)) {
-            z[selected] = xp;
-            if (output_log_probs != nullptr) {
-                output_log_probs[b * K + selected] = yp - old_cum[(z[selected] / vocab) % K];
-            }
-            v[selected] = yp;
-            selected++;
-        }
-        if (selected >= K) {
-            break;
-        }
+    __syncthreads();
+    // layers/beam_search_layers/OnlineBeamSearchLayer.cu:24-61, as beam_update_kernel
+    if (t < K) {
+        const int  i       = b * K + t;
+        const int  word    = chosen[t];
+        const int  end_id  = end_u;
+        const bool valid   = word >= 0;  // (as there: a slot left untouched holds whatever the buffer held)
+        const int  beam_id = valid ? (word / vocab) % K : t;
+        const int  word_id = valid ? word % vocab : end_id;
+        const bool done    = complete != 0 || word_id == end_id;
+        up.sequence_length[i] = counted[beam_id];
+        up.finished[i]        = done;
+        up.parent_ids[i]      = beam_id;
+        ids[i]                = word_id;
+        parent_of[t]          = beam_id;
+        live[t]               = done ? 0 : 1;
     }
-    if (with_hyps) {
-        if (h.num_beams[b] < K) {
-            h.is_done[b] = false;
-        }
-        else if (h.early_stopping) {
-            h.is_done[b] = true;
+    if (up.cache_tgt == nullptr) {
+        return;
+    }
+    __syncthreads();
+    // layers/beam_search_layers/BaseBeamSearchLayer.cu:22-49, as beam_indir_cache_kernel
+    for (int i = t; i < K * up.num_steps; i += BM_THREADS) {
+        const int beam = i / up.num_steps;
+        if (live[beam] != 0) {
+            const int    time_step = up.start_step + i % up.num_steps;
+            const int    circ      = time_step % up.max_seq_len;
+            const size_t base      = (size_t)b * K * up.max_seq_len + circ;
+            const int    from      = parent_of[beam];
+            const int    value     = cache_here ? cached[from * up.num_steps + i % up.num_steps] :
+                                                  up.cache_src[base + (size_t)from * up.max_seq_len];
+            up.cache_tgt[base + (size_t)beam * up.max_seq_len] = time_step == up.step ? beam : value;
         }
     }
 }
@@ -902,13 +1340,30 @@ extern "C" void ftk_test_set_beam_path(int v)
 }
 #endif
 
-extern "C" {
+// How many workgroups share a row of beam_team_kernel: as many as the compute units allow, as long as every part has at
+// least 4096 columns to itself (below that the read of the whole row is all there is) and an entry's keys fit the
+// merge. Rows too long for the registers, and more rows than compute units, take the other forms (0): of two
+// 512-thread workgroups on a compute unit one reads while the other computes.
+static int beam_team_parts(int rows, int beam_width, int vocab, const BeamPlan& plan)
+{
+    if (vocab > BT_COLUMNS || rows > 256) {
+        return 0;
+    }
+    int parts = 1;
+    while (parts < BT_MAX_PARTS && 2 * parts * rows <= 256 && vocab / (2 * parts) >= 4096 && 2 * parts <= plan.parts) {
+        parts *= 2;
+    }
+    while (parts > 0 && 2 * beam_width * beam_width * parts > BB_MERGED) {
+        parts /= 2;
+    }
+    return parts;
+}
 
-int ftk_invoke_topk_softmax(int dtype, const void* log_probs, const void* bias, const bool* finished,
-                            const int* sequence_lengths, float* cum_log_probs, float* output_log_probs, int* ids,
-                            void* temp_storage, size_t* temp_storage_size, const ftk_beam_hypotheses* beam_hyps,
-                            int batch_size, int beam_width, int vocab_size, const int* end_ids, float diversity_rate,
-                            float length_penalty, ftk_stream_t stream)
+static int beam_step(int dtype, const void* log_probs, const void* bias, const bool* finished,
+                     const int* sequence_lengths, float* cum_log_probs, float* output_log_probs, int* ids,
+                     void* temp_storage, size_t* temp_storage_size, const ftk_beam_hypotheses* beam_hyps,
+                     int batch_size, int beam_width, int vocab_size, const int* end_ids, float diversity_rate,
+                     float length_penalty, BeamUpdate up, ftk_stream_t stream)
 {
     if (dtype < 0 || dtype > 2) {
         return FTK_ERR_DTYPE;
@@ -981,29 +1436,38 @@ int ftk_invoke_topk_softmax(int dtype, const void* log_probs, const void* bias, 
         h.max_seq_len          = beam_hyps->max_seq_len;
         h.early_stopping       = beam_hyps->early_stopping ? 1 : 0;
     }
+    int2*      before = (int2*)(ws + plan.off_before);
     const dim3 sections(plan.parts, rows);
-    // One 1024-thread workgroup per row does the work of the first three launches, except where a few long rows
-    // would leave most compute units idle (measured on MI355X, f16: 32 rows of 128256 take 40 us that way and 34 us
-    // in sections; 64 rows of 50257 27 against 30 us, 256 rows 29 against 36 us, 512 rows of 152064 112 against
+    // A few long rows would leave most compute units idle with one workgroup each: they go in sections (measured on
+    // MI355X, f16: 32 rows of 128256 take 40 us in one launch and 34 us in sections; 512 rows of 152064 112 against
     // 115 us).
+    int  team        = beam_team_parts(rows, beam_width, vocab_size, plan);
     bool one_per_row = vocab_size <= BR_SHORT_ROW || rows >= BR_MANY_ROWS;
     bool half_size   = rows > 256;  // two 512-thread workgroups per compute unit
 #ifdef FTK_TEST_HOOKS
+    team        = g_beam_path == 0 ? team : 0;
     one_per_row = g_beam_path == 0 ? one_per_row : g_beam_path >= 2;
     half_size   = g_beam_path <= 1 ? half_size : g_beam_path == 3;
 #endif
+    const BeamCandidates cd{cand_id, cand_val, team, pmax, psum, pkeys, before};
     FTK_DISPATCH_DTYPE(dtype, {
         typedef Storage<DT>::T T;
-        if (one_per_row && half_size) {
+        if (team > 0) {
+            beam_team_kernel<DT><<<dim3(rows, team), BR_THREADS, 0, st>>>((const T*)log_probs, (const T*)bias, finished,
+                                                                          end_ids, sequence_lengths, vocab_size,
+                                                                          beam_width, pmax, psum, pkeys, before);
+            FTK_LAUNCH_CHECK();
+        }
+        else if (one_per_row && half_size) {
             beam_rowwide_kernel<DT, BR_THREADS / 2><<<rows, BR_THREADS / 2, 0, st>>>(
                 (const T*)log_probs, (const T*)bias, finished, end_ids, cum_log_probs, vocab_size, beam_width, cand_id,
-                cand_val);
+                cand_val, sequence_lengths, before);
             FTK_LAUNCH_CHECK();
         }
         else if (one_per_row) {
             beam_rowwide_kernel<DT, BR_THREADS><<<rows, BR_THREADS, 0, st>>>(
                 (const T*)log_probs, (const T*)bias, finished, end_ids, cum_log_probs, vocab_size, beam_width, cand_id,
-                cand_val);
+                cand_val, sequence_lengths, before);
             FTK_LAUNCH_CHECK();
         }
         else {
@@ -1014,18 +1478,70 @@ int ftk_invoke_topk_softmax(int dtype, const void* log_probs, const void* bias, 
                                                                      vocab_size, plan.section, N, pmax, psum, pkeys);
             FTK_LAUNCH_CHECK();
             beam_row_kernel<DT><<<rows, BM_THREADS, 0, st>>>(finished, end_ids, cum_log_probs, vocab_size, beam_width,
-                                                             plan.parts, pmax, psum, pkeys, cand_id, cand_val);
+                                                             plan.parts, pmax, psum, pkeys, cand_id, cand_val,
+                                                             sequence_lengths, before);
             FTK_LAUNCH_CHECK();
         }
-        beam_batch_kernel<DT><<<batch_size, BM_THREADS, 0, st>>>(cand_id, cand_val, ids, cum_log_probs,
-                                                                 output_log_probs, finished, sequence_lengths, h,
-                                                                 beam_width, 2 * max_k, vocab_size, length_penalty,
+        beam_batch_kernel<DT><<<batch_size, BM_THREADS, 0, st>>>(cd, ids, cum_log_probs, output_log_probs, end_ids, h,
+                                                                 up, beam_width, 2 * max_k, vocab_size, length_penalty,
                                                                  diversity_rate);
         FTK_LAUNCH_CHECK();
     });
     return 0;
 }
 
+extern "C" {
+
+int ftk_invoke_topk_softmax(int dtype, const void* log_probs, const void* bias, const bool* finished,
+                            const int* sequence_lengths, float* cum_log_probs, float* output_log_probs, int* ids,
+                            void* temp_storage, size_t* temp_storage_size, const ftk_beam_hypotheses* beam_hyps,
+                            int batch_size, int beam_width, int vocab_size, const int* end_ids, float diversity_rate,
+                            float length_penalty, ftk_stream_t stream)
+{
+    return beam_step(dtype, log_probs, bias, finished, sequence_lengths, cum_log_probs, output_log_probs, ids,
+                     temp_storage, temp_storage_size, beam_hyps, batch_size, beam_width, vocab_size, end_ids,
+                     diversity_rate, length_penalty, BeamUpdate{}, stream);
+}
+
+int ftk_fused_beam_step(int dtype, const void* log_probs, bool* finished, int* sequence_lengths, float* cum_log_probs,
+                        float* output_log_probs, int* ids, int* parent_ids, int* tgt_indir_cache,
+                        const int* src_indir_cache, void* temp_storage, size_t temp_storage_size,
+                        const ftk_beam_hypotheses* beam_hyps, int batch_size, int beam_width, int vocab_size,
+                        int max_seq_len, int step, const int* end_ids, float diversity_rate, float length_penalty,
+                        ftk_stream_t stream)
+{
+    if (temp_storage == nullptr) {
+        return FTK_ERR_WORKSPACE;
+    }
+    if (max_seq_len < 1 || step < 0
+        || (batch_size > 0
+            && (sequence_lengths == nullptr || parent_ids == nullptr || tgt_indir_cache == nullptr
+                || src_indir_cache == nullptr))) {
+        return FTK_ERR_ARGUMENT;
+    }
+    BeamUpdate up{};
+    up.finished        = finished;
+    up.sequence_length = sequence_lengths;
+    up.parent_ids      = parent_ids;
+    up.max_seq_len     = max_seq_len;
+    up.step            = step;
+    up.start_step      = step + 1 - max_seq_len > 0 ? step + 1 - max_seq_len : 0;
+    up.num_steps       = step + 1 < max_seq_len ? step + 1 : max_seq_len;
+    // a long cache is copied by as many workgroups as it needs, in a launch of its own
+    const bool copies = (long long)beam_width * up.num_steps <= BB_CACHE;
+    if (copies) {
+        up.cache_tgt = tgt_indir_cache;
+        up.cache_src = src_indir_cache;
+    }
+    const int rc = beam_step(dtype, log_probs, nullptr, finished, sequence_lengths, cum_log_probs, output_log_probs, ids,
+                             temp_storage, &temp_storage_size, beam_hyps, batch_size, beam_width, vocab_size, end_ids,
+                             diversity_rate, length_penalty, up, stream);
+    if (rc != 0 || copies) {
+        return rc;
+    }
+    return ftk_invoke_update_indir_cache(tgt_indir_cache, src_indir_cache, parent_ids, finished, batch_size, batch_size,
+                                         beam_width, max_seq_len, step, stream);
+}
 
 int ftk_invoke_add_bias_apply_penalties(int dtype, int step, void* logits, const int* current_ids,
                                         const int* previous_ids, const int* parent_ids, const int* input_lengths,

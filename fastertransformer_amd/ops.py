@@ -74,6 +74,7 @@ _SIGNATURES = {
     "ftk_invoke_topk_softmax": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _f, _f, _vp],
     "ftk_invoke_add_bias_apply_penalties": [_i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp,
                                             _f, _f, _i, _i, _vp],
+    "ftk_fused_beam_step": [_i] + [_vp] * 10 + [_sz, _vp, _i, _i, _i, _i, _i, _vp, _f, _f, _vp],
     "ftk_invoke_beam_update": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp],
     "ftk_invoke_update_indir_cache": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "ftk_fused_topk_shard_gather": [_vp, _vp, _vp],

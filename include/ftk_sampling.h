@@ -457,6 +457,16 @@ int ftk_invoke_update_indir_cache(int* tgt_indir_cache, const int* src_indir_cac
                                   const bool* finished, int batch_dim, int local_batch_size, int beam_width,
                                   int max_seq_len, int step, ftk_stream_t stream);
 
+/* ftk_invoke_topk_softmax, ftk_invoke_beam_update and ftk_invoke_update_indir_cache of one step in two launches, with
+ * the same results: what OnlineBeamSearchLayer runs. Arguments as there; ids = the step's ids, which come out as
+ * tokens; temp_storage is sized by ftk_invoke_topk_softmax and holds nothing between calls. */
+int ftk_fused_beam_step(int dtype, const void* log_probs, bool* finished, int* sequence_lengths, float* cum_log_probs,
+                        float* output_log_probs, int* ids, int* parent_ids, int* tgt_indir_cache,
+                        const int* src_indir_cache, void* temp_storage, size_t temp_storage_size,
+                        const ftk_beam_hypotheses* beam_hyps, int batch_size, int beam_width, int vocab_size,
+                        int max_seq_len, int step, const int* end_ids, float diversity_rate, float length_penalty,
+                        ftk_stream_t stream);
+
 /* ---- per-kernel timing of the fused step (the reference's counterpart is its CudaTimer / NVTX ranges,
  * utils/cuda_utils.h:247-258, utils/nvtx_utils.h:37-49) ------------------------------------------
  * ftk_profile_enable(n) makes the next n fused steps bracket each of their kernels with HIP events on

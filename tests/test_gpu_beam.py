@@ -552,3 +552,66 @@ def test_word_lists_with_beams(dt):
         torch.cuda.synchronize()
         assert np.array_equal(to_numpy(d_fin), fin) and fin.any()
 
+
+
+@pytest.mark.parametrize("batch,K,V,step,max_seq_len,ite", [
+    (3, 4, 50257, 5, 12, 0),      # 8 parts of a row, odd rows
+    (9, 8, 20011, 127, 200, 1),   # 2 parts, the second window of two, the cache through LDS at its limit
+    (33, 4, 9001, 300, 310, 0),   # one part, a history longer than its copy, the cache of an entry read in place
+    (2, 16, 33000, 64, 70, 0),    # 2 parts at the merge's limit
+    (1, 22, 65536, 3, 4, 0),      # one part at the merge's limit, the longest row kept in registers
+    (1, 23, 65537, 3, 4, 0),      # beyond both
+    (2, 2, 8191, 2050, 2048, 0),  # a circular cache, copied inside the step
+    (2, 8, 4097, 700, 800, 0),    # a cache that takes its own launch
+])
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+def test_fused_beam_step_is_its_three_parts(dt, batch, K, V, step, max_seq_len, ite):
+    """ftk_fused_beam_step against ftk_invoke_topk_softmax, ftk_invoke_beam_update and ftk_invoke_update_indir_cache
+    (each compared with the oracle above) on the same inputs: every array bit for bit"""
+    import torch
+    ops, lib = _lib()
+    rng = np.random.default_rng(1000 * K + step + dt)
+    windows, depth = ite + 1, max(max_seq_len, step + 1)
+    c = make_beam_case(rng, dt, batch * windows, K, V, step=min(step, depth - 1), max_seq_len=depth)
+    first = batch * ite
+    c["ids"] = rng.integers(-1, batch * K * V, (batch, K)).astype(np.int32)
+    src = rng.integers(0, K, (batch, K, max_seq_len)).astype(np.int32)
+    x = to_torch(c["log_probs"][first * K:], dt)
+    results = []
+    for fused in (False, True):
+        d = {k: to_torch(c[k][first * K:] if k in ("finished", "sequence_lengths", "cum_log_probs") else
+                         c[k][first:] if k == "end_ids" else c[k][:batch])
+             for k in ("finished", "sequence_lengths", "cum_log_probs", "end_ids", "ids", "output_log_probs")}
+        d["parents"], d["src"] = torch.zeros((batch, K), dtype=torch.int32, device="cuda"), to_torch(src)
+        d["tgt"] = torch.full_like(d["src"], -7)
+        hyps = ops.BeamHypotheses()
+        for name in HYP_ARRAYS:
+            d[name] = to_torch(c["hyps"][name])
+            setattr(hyps, name, d[name].data_ptr())
+        hyps.end_ids = d["end_ids"].data_ptr()
+        hyps.step, hyps.ite, hyps.batch_size, hyps.local_batch_size = c["hyps"]["step"], ite, batch * windows, batch
+        hyps.max_seq_len, hyps.early_stopping = depth, True
+        at = {k: v.data_ptr() for k, v in d.items()}
+        size = C.c_size_t(0)
+        head = (dt, x.data_ptr(), None, at["finished"], at["sequence_lengths"], at["cum_log_probs"],
+                at["output_log_probs"], at["ids"])
+        tail = (C.addressof(hyps), batch, K, V, at["end_ids"], 0.1, 0.7, ops.current_stream())
+        ops.check(lib.ftk_invoke_topk_softmax(*head, None, C.addressof(size), *tail))
+        ws = torch.empty(size.value, dtype=torch.uint8, device="cuda")
+        print("fused beam step", DTYPE_NAMES[dt], batch, K, V, step, max_seq_len, ite, fused, flush=True)
+        if fused:
+            ops.check(lib.ftk_fused_beam_step(
+                dt, x.data_ptr(), at["finished"], at["sequence_lengths"], at["cum_log_probs"], at["output_log_probs"],
+                at["ids"], at["parents"], at["tgt"], at["src"], ws.data_ptr(), size.value, C.addressof(hyps), batch, K,
+                V, max_seq_len, step, at["end_ids"], 0.1, 0.7, ops.current_stream()))
+        else:
+            ops.check(lib.ftk_invoke_topk_softmax(*head, ws.data_ptr(), C.addressof(size), *tail))
+            ops.check(lib.ftk_invoke_beam_update(at["finished"], at["parents"], at["sequence_lengths"], at["ids"],
+                                                 at["ids"], C.addressof(hyps), batch, K, V, at["end_ids"],
+                                                 ops.current_stream()))
+            ops.check(lib.ftk_invoke_update_indir_cache(at["tgt"], at["src"], at["parents"], at["finished"], batch,
+                                                        batch, K, max_seq_len, step, ops.current_stream()))
+        torch.cuda.synchronize()
+        results.append({k: to_numpy(v) for k, v in d.items()})
+    for name, want in results[0].items():
+        assert np.array_equal(want, results[1][name]), name
