@@ -579,9 +579,9 @@ def test_fused_beam_step_is_its_three_parts(dt, batch, K, V, step, max_seq_len, 
     x = to_torch(c["log_probs"][first * K:], dt)
     results = []
     for fused in (False, True):
-        d = {k: to_torch(c[k][first * K:] if k in ("finished", "sequence_lengths", "cum_log_probs") else
+        d = {k: to_torch(c[k][first * K:] if k in ("finished", "sequence_lengths") else
                          c[k][first:] if k == "end_ids" else c[k][:batch])
-             for k in ("finished", "sequence_lengths", "cum_log_probs", "end_ids", "ids", "output_log_probs")}
+             for k in ("finished", "sequence_lengths", "end_ids", "ids", "output_log_probs")}
         d["parents"], d["src"] = torch.zeros((batch, K), dtype=torch.int32, device="cuda"), to_torch(src)
         d["tgt"] = torch.full_like(d["src"], -7)
         hyps = ops.BeamHypotheses()
@@ -591,9 +591,12 @@ def test_fused_beam_step_is_its_three_parts(dt, batch, K, V, step, max_seq_len, 
         hyps.end_ids = d["end_ids"].data_ptr()
         hyps.step, hyps.ite, hyps.batch_size, hyps.local_batch_size = c["hyps"]["step"], ite, batch * windows, batch
         hyps.max_seq_len, hyps.early_stopping = depth, True
+        # (the beams' own log-probs: the hypotheses have an array of the same name, and one buffer for both would have
+        # an entry's beams written over another entry's hypotheses in no fixed order)
+        d["beam_cum_log_probs"] = to_torch(c["cum_log_probs"][first * K:])
         at = {k: v.data_ptr() for k, v in d.items()}
         size = C.c_size_t(0)
-        head = (dt, x.data_ptr(), None, at["finished"], at["sequence_lengths"], at["cum_log_probs"],
+        head = (dt, x.data_ptr(), None, at["finished"], at["sequence_lengths"], at["beam_cum_log_probs"],
                 at["output_log_probs"], at["ids"])
         tail = (C.addressof(hyps), batch, K, V, at["end_ids"], 0.1, 0.7, ops.current_stream())
         ops.check(lib.ftk_invoke_topk_softmax(*head, None, C.addressof(size), *tail))
@@ -601,9 +604,9 @@ def test_fused_beam_step_is_its_three_parts(dt, batch, K, V, step, max_seq_len, 
         print("fused beam step", DTYPE_NAMES[dt], batch, K, V, step, max_seq_len, ite, fused, flush=True)
         if fused:
             ops.check(lib.ftk_fused_beam_step(
-                dt, x.data_ptr(), at["finished"], at["sequence_lengths"], at["cum_log_probs"], at["output_log_probs"],
-                at["ids"], at["parents"], at["tgt"], at["src"], ws.data_ptr(), size.value, C.addressof(hyps), batch, K,
-                V, max_seq_len, step, at["end_ids"], 0.1, 0.7, ops.current_stream()))
+                dt, x.data_ptr(), at["finished"], at["sequence_lengths"], at["beam_cum_log_probs"],
+                at["output_log_probs"], at["ids"], at["parents"], at["tgt"], at["src"], ws.data_ptr(), size.value,
+                C.addressof(hyps), batch, K, V, max_seq_len, step, at["end_ids"], 0.1, 0.7, ops.current_stream()))
         else:
             ops.check(lib.ftk_invoke_topk_softmax(*head, ws.data_ptr(), C.addressof(size), *tail))
             ops.check(lib.ftk_invoke_beam_update(at["finished"], at["parents"], at["sequence_lengths"], at["ids"],
