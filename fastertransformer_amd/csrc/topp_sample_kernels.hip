@@ -809,6 +809,7 @@ __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
     __shared__ float    chain_sum[C];
     __shared__ float    wmass[NW], wupper[NW];
     __shared__ uint32_t wcnt[NW], wseg[NW];
+    __shared__ uint32_t queue_at;  // where the row's segments go in the queue, plus one (0: the pick orders them)
     __shared__ uint32_t red32[16];
     const int           row = blockIdx.x, part = blockIdx.y, t = threadIdx.x;
     if (topp_row_idle(s, row)) {
@@ -977,16 +978,15 @@ __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
             // (half a bucket under the one that covers the draw: a bucket and a half above what is not gathered)
             m.safe      = __builtin_amdgcn_exp2f((lead - ((float)cut - 0.5f) / TSP_SCALE) * 1.44269504f);
             s.meta[row] = m;
-            wseg[0]     = 0u;
-            if (usable && n > (uint32_t)TPS_CAP) {
-                // prefixes that fit its LDS are ordered by the pick kernel itself, longer ones by the sort's workgroups
-                wseg[0] = atomicAdd(s.queue, nseg) + 1u;
-            }
+            // prefixes that fit its LDS are ordered by the pick kernel itself, longer ones by the sort's workgroups
+            // (a word of its own: the other waves may still be reading wseg)
+            queue_at = usable && n > (uint32_t)TPS_CAP ? atomicAdd(s.queue, nseg) + 1u : 0u;
         }
         __syncthreads();
-        if (wseg[0] != 0u) {
+        const uint32_t to = queue_at;
+        if (to != 0u) {
             for (uint32_t i = (uint32_t)t; i < nseg; i += TSP_SUM32) {
-                s.queue[wseg[0] + i] = (uint32_t)row * TPB_NB + i;
+                s.queue[to + i] = (uint32_t)row * TPB_NB + i;
             }
         }
     }

@@ -1,12 +1,14 @@
 """The top-p step with its penalties folded in (ftk_fused_topp_penalty_step, what the top-p layer takes): edges of the
 kernels' tiles and of the rules that split a row, against the oracle's kernel-by-kernel layer. Ids, flags and lengths bit
 for bit; log-probs within the harness's tolerance."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import ft_oracle as O
 from decode_harness import Case, OracleRunner, ProductRunner, compare
-from helpers import DTYPE_NAMES, DTYPES, make_logits, uniforms
+from helpers import DTYPE_NAMES, DTYPES, make_logits, to_numpy, to_torch, uniforms
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +48,53 @@ def test_penalised_nucleus_rows(dt, shape):
         p.step(H + i, x, u)
         o.step(H + i, x, u)
         compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
+
+
+def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None):
+    """One ftk_fused_topp_sample_step over rows of `x`: (ids, finished, lengths, cumulative log-probs). The draws are
+    `draws`, or generated from `states` (advanced in place)."""
+    import torch
+    from fastertransformer_amd import ops
+    lib = ops.ftk()
+    B, Vp = x.shape
+    d_x, d_p, d_end, d_u = to_torch(x, dt), to_torch(p_arr), to_torch(end_ids), to_torch(draws)
+    ids = torch.full((B,), -7, dtype=torch.int32, device="cuda")
+    fin, seq = torch.zeros(B, dtype=torch.bool, device="cuda"), torch.zeros(B, dtype=torch.int32, device="cuda")
+    cum = torch.zeros(B, dtype=torch.float32, device="cuda")
+    size = C.c_size_t(0)
+    ops.check(lib.ftk_fused_topp_sample_step(dt, None, C.addressof(size), None, V, Vp, B, *(None,) * 8, 1.0, *(None,) * 7))
+    ws = torch.empty(size.value, dtype=torch.uint8, device="cuda")
+    ops.check(lib.ftk_fused_topp_sample_step(
+        dt, ws.data_ptr(), C.addressof(size), d_x.data_ptr(), V, Vp, B, d_end.data_ptr(), fin.data_ptr(), seq.data_ptr(),
+        ids.data_ptr(), cum.data_ptr(), None, ops.ptr(states), ops.ptr(d_u), 1.0, d_p.data_ptr(), None, None, None, None,
+        None, ops.current_stream()))
+    torch.cuda.synchronize()
+    return tuple(to_numpy(a) for a in (ids, fin, seq, cum))
+
+
+def _oracle_step(dt, x, V, p_arr, end_ids, draws):
+    B, Vp = x.shape
+    probs, fin, seq = x.copy(), np.zeros(B, np.bool_), np.zeros(B, np.int32)
+    O.add_bias_softmax(dt, probs, None, end_ids, fin, B, Vp, V)
+    ids, cum, out = np.full(B, -7, np.int32), np.zeros(B, np.float32), np.zeros(B, np.float32)
+    O.batch_topp_sampling(dt, probs, ids, seq, fin, cum, out, draws, B, Vp, end_ids, 0.0, p_arr, None)
+    return ids, fin, seq, cum
+
+
+def _same(got, want, dt):
+    for a, b in zip(got[:3], want[:3]):
+        assert np.array_equal(a, b)
+    np.testing.assert_allclose(got[3], want[3], rtol=1e-5 if dt == O.F32 else 2e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("B,V", [(24, 20011), (256, 14000)])   # sixteen and four workgroups per row
+def test_long_fp32_prefixes(B, V):
+    """Draws so deep into flat fp32 rows that the prefix in front of them (most of the row, more than 5632 entries) is
+    ordered in segments that the whole launch shares out."""
+    rng = np.random.default_rng(B + V)
+    x = rng.standard_normal((B, V)).astype(np.float32) * rng.uniform(0.2, 1.0, (B, 1)).astype(np.float32)
+    p_arr, end_ids = np.full(B, 1.0, np.float32), rng.integers(0, V, B).astype(np.int32)
+    for step in range(2):
+        u = rng.uniform(0.8, 0.999, B).astype(np.float32)
+        print("long prefixes", B, V, step, flush=True)
+        _same(_sample_step(O.F32, x, V, p_arr, end_ids, u), _oracle_step(O.F32, x, V, p_arr, end_ids, u), O.F32)
