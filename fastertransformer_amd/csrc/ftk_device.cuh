@@ -532,8 +532,8 @@ __device__ __forceinline__ RowDrawSource row_draw_source(const RngState* rng, co
     d.off_hi   = *(st != nullptr ? st + 3 : from);
     return d;
 }
-// One thread per row: the generated draw (same values as rng_next_uniform) and the counter the row's state goes on
-// with, which the caller stores.
+// The generated draw (same values as rng_next_uniform) and the counter the row's state goes on with, which the caller
+// stores: once per row, and where several waves draw for themselves, behind a barrier after the last one's load.
 __device__ __forceinline__ float row_draw_generate(const RowDrawSource& d, uint64_t* next_offset)
 {
     uint32_t o[4];

@@ -1061,7 +1061,8 @@ struct ToppPickRow {
     int           decay_reset;
     const T*      y;
     // worked out later
-    float mx, denom, rand_num;
+    float    mx, denom, rand_num;
+    uint64_t next_draw;  // what the row's generator goes on with
 
     __device__ __forceinline__ ToppPickRow(const ToppStep& s, const ToppPickOut& o, int row_, int n_partial):
         row(row_), rm(s, row_, n_partial)
@@ -1082,15 +1083,12 @@ struct ToppPickRow {
         decay_reset   = row_arg_or(o.dec.runtime_top_p != nullptr ? o.dec.reset_ids : nullptr, row, safe, 0);
         y             = s.y != nullptr ? (const T*)s.y + (size_t)row * s.y_pitch : (const T*)s.logits + (size_t)row * s.Vp;
     }
-    // One wave or more: the draw (its state goes on), the maximum, the denominator: the reference's second butterfly.
-    __device__ __forceinline__ void derive(const ToppStep& s, const ToppPickOut& o)
+    // One wave or more: the draw, the maximum, the denominator: the reference's second butterfly.
+    __device__ __forceinline__ void derive(const ToppStep& s)
     {
-        uint64_t    next = 0;
-        const float u    = s.uniforms != nullptr ? draw.injected : row_draw_generate(draw, &next);
-        if (s.uniforms == nullptr && threadIdx.x == 0) {
-            o.rng[row].offset = next;  // drawn for every row that is not skipped
-        }
-        rand_num = u * p;
+        next_draw     = 0;
+        const float u = s.uniforms != nullptr ? draw.injected : row_draw_generate(draw, &next_draw);
+        rand_num      = u * p;
         if (fin) {
             // a finished row: its end id alone has e = 1, or, when that lies outside the vocabulary, every column has
             const bool inside = end_id >= 0 && end_id < s.n;
@@ -1105,6 +1103,14 @@ struct ToppPickRow {
                 v += __shfl_xor(v, m, 32);
             }
             denom = v + 1e-6f;  // (both halves of the wave hold the same group sums)
+        }
+    }
+    // The generator's state goes on, for every row that is not skipped. Every wave has read the state for its own
+    // derive(): unless only this thread's draw counts, a barrier lies between that and this.
+    __device__ __forceinline__ void keep_draw(const ToppStep& s, const ToppPickOut& o) const
+    {
+        if (s.uniforms == nullptr && threadIdx.x == 0) {
+            o.rng[row].offset = next_draw;
         }
     }
     // A single thread, once: what the row leaves behind, the decay of its p included.
@@ -1370,14 +1376,17 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_f32_kernel(ToppStep s, T
         }
         return;
     }
-    r.derive(s, o);
+    r.derive(s);
     ToppPicked res;
     if (r.trivial(s, res)) {
+        r.keep_draw(s, o);
         if (t == 0) {
             r.finish(o, res);
         }
         return;
     }
+    __syncthreads();
+    r.keep_draw(s, o);
     const RowDivisor div(r.denom);
     auto prob = [&](unsigned long long entry) { return topp_prob_of<DT_F32>(key64_prob(entry), div, r.denom); };
     if (!r.fin && !o.force_deep && m.n > 0) {
@@ -1539,9 +1548,10 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
         }
         return;
     }
-    r.derive(s, o);
+    r.derive(s);
     ToppPicked res;
     if (r.trivial(s, res)) {
+        r.keep_draw(s, o);
         if (t == 0) {
             r.finish(o, res);
         }
@@ -1549,6 +1559,8 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     }
     const ToppWholeRow<DT> whole{r.y, s.n, s.Vp, r.end_id, r.mx, r.denom, r.p, r.rand_num, r.fin, s.sorted + (size_t)row * 2 * s.Vp};
     if (r.fin || o.force_deep) {
+        __syncthreads();
+        r.keep_draw(s, o);
         res = topp_pick_whole_row<DT>(sc, rs.digits, whole);
         if (t == 0) {
             r.finish(o, res);
@@ -1599,6 +1611,7 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
         }
     }
     __syncthreads();
+    r.keep_draw(s, o);
     uint32_t n = 0u, nruns = 0u;
     uint32_t at = ic - lc, run = ir - lr;
     float    mass = im - lm;

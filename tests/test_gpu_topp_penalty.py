@@ -98,3 +98,30 @@ def test_long_fp32_prefixes(B, V):
         u = rng.uniform(0.8, 0.999, B).astype(np.float32)
         print("long prefixes", B, V, step, flush=True)
         _same(_sample_step(O.F32, x, V, p_arr, end_ids, u), _oracle_step(O.F32, x, V, p_arr, end_ids, u), O.F32)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("B,V", [(40, 14000), (300, 2051)])
+def test_generated_draws_are_the_injected_ones(dt, B, V):
+    """Three steps that draw for themselves from per-row generators against the same draws injected: ids, flags, lengths
+    and log-probs bit for bit, and generators that have gone on by one draw a step."""
+    import torch
+    from fastertransformer_amd import ops
+    hooks = ops.ftk_hooks()
+    rng = np.random.default_rng(V + dt)
+    states = torch.zeros(B * 2, dtype=torch.int64, device="cuda")
+    seeds = to_torch(rng.integers(0, 1 << 62, B).astype(np.uint64))
+    ops.check(hooks.ftk_invoke_curand_batch_initialize(states.data_ptr(), B, seeds.data_ptr(), ops.current_stream()))
+    drawn, ahead = torch.empty(B * 3, dtype=torch.float32, device="cuda"), states.clone()
+    ops.check(hooks.ftk_test_rng_uniform(ahead.data_ptr(), drawn.data_ptr(), B, 3, ops.current_stream()))
+    torch.cuda.synchronize()
+    draws = to_numpy(drawn).reshape(B, 3)
+    p_arr, end_ids = rng.uniform(0.3, 1.0, B).astype(np.float32), rng.integers(0, V, B).astype(np.int32)
+    for i, spread in enumerate((0.3, 2.0, 8.0)):    # from draws deep into flat rows to one token that is all there is
+        x = make_logits(rng, dt, B, V, V, spread)
+        print("generated draws", DTYPE_NAMES[dt], B, V, i, flush=True)
+        own = _sample_step(dt, x, V, p_arr, end_ids, states=states)
+        for a, b in zip(own, _sample_step(dt, x, V, p_arr, end_ids, np.ascontiguousarray(draws[:, i]))):
+            assert np.array_equal(a, b)
+        assert (to_numpy(states).reshape(B, 2)[:, 1] == i + 1).all()
+    assert np.array_equal(to_numpy(states), to_numpy(ahead))
