@@ -58,7 +58,8 @@ HIP_FLAGS = [
 
 
 HOOK_UNITS = [("fused_kernels.hip", "fused_kernels.o"), ("topp_kernels.hip", "topp_kernels.o"),
-              ("criteria_kernels.hip", "criteria_kernels.o"), ("beam_kernels.hip", "beam_kernels.o")]
+              ("topp_sample_kernels.hip", "topp_sample_kernels.o"), ("criteria_kernels.hip", "criteria_kernels.o"),
+              ("beam_kernels.hip", "beam_kernels.o")]
 
 
 def _run(cmd):

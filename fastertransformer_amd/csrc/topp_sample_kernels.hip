@@ -356,11 +356,16 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     const int    shift = __builtin_ctz((unsigned)C);
     const int    c0    = j * C;
     const int    nit   = (s.n + TSP_CHAINS - 1) / TSP_CHAINS;
-    // the origin of the buckets: the largest plain value among the first 1024 columns, the same for every part
-    float first = TSP_LOWEST;
+    // the origin of the buckets: the largest value among 1024 columns, 64 stretches of 16 spread over the row (ids of one
+    // script or of special tokens are neighbours), without the history; the same for every part. Everything 8 or more above
+    // it lies in the first bucket (256 x 128256 with the first 1024 columns masked: 22 ms a step with the first 1024
+    // columns as the sample, 0.12 ms)
+    constexpr int U0 = TSP_CHAINS / TSP_STAGE;
+    auto  sample = [&](int u) { return (u * (TSP_STAGE / 16) + (t >> 4)) * (s.n / 64) + (t & 15); };
+    float plain[U0];
 #pragma unroll
-    for (int u = 0; u < TSP_CHAINS / TSP_STAGE; ++u) {
-        first = __builtin_fmaxf(first, rowp[t + u * TSP_STAGE]);
+    for (int u = 0; u < U0; ++u) {
+        plain[u] = rowp[sample(u)];
     }
     for (int i = t; i < TSP_BUCKETS; i += TSP_STAGE) {
         hist[i] = 0u;
@@ -376,10 +381,12 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
             window[i] = 0u;
         }
     }
-    first = block_max<float, TSP_STAGE / WAVE>(first, red, TSP_LOWEST);  // (two barriers: both tables are clear)
-    if (TRANSFORM && f.temperature_active) {
-        first = first * f.temperature.inv;
+    float first = TSP_LOWEST;
+#pragma unroll
+    for (int u = 0; u < U0; ++u) {
+        first = __builtin_fmaxf(first, TRANSFORM ? f(sample(u), plain[u], false) : plain[u]);
     }
+    first = block_max<float, TSP_STAGE / WAVE>(first, red, TSP_LOWEST);  // (two barriers: both tables are clear)
     if (!(__builtin_fabsf(first) < 1e30f)) {
         first = 0.0f;
     }
@@ -796,8 +803,8 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
 
 // ---- sum, fp32 --------------------------------------------------------------------------------------------------------
 // Where the draw must lie comes from the stage's histogram: a bucket's mass is at least its count times the exponential
-// of its lower edge, the whole row's at most the same with the upper edges. Everything down to the bucket that certainly
-// covers the draw - and two more, so that all entries which share a probability with the last one that can be drawn are
+// of its lower edge and at most the same with its upper edge. Everything down to the bucket that certainly covers the
+// draw - and two more, so that all entries which share a probability with the last one that can be drawn are
 // there - goes to its bucket's place in the prefix, keyed by e (the division by the denominator keeps the order).
 template<int LPC>
 __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
@@ -850,7 +857,7 @@ __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
     const float top  = ref + TSP_ABOVE;
     const float lead = top - mx;  // y of the first bucket's upper edge, relative to the maximum
     const int   mx_bucket = topp_y_bucket(mx, top);
-    float       lower[K], lm = 0.0f, lu = 0.0f;
+    float       lower[K], upper[K], lm = 0.0f, lu = 0.0f;
     uint32_t    lc = 0u;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
@@ -860,47 +867,65 @@ __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
                                                    __builtin_amdgcn_exp2f(__builtin_fminf(lead - (float)(b + 1) / TSP_SCALE, 0.0f) * 1.44269504f);
         const float n     = (float)tot[i];
         lower[i]          = tot[i] == 0u ? 0.0f : n * below;
-        lu += tot[i] == 0u ? 0.0f : n * up;
+        upper[i]          = tot[i] == 0u ? 0.0f : n * up;
         if (b == mx_bucket) {
             lower[i] += 1.0f - below;  // the maximum itself lies here
         }
         lm += lower[i];
+        lu += upper[i];
         lc += tot[i];
     }
-    float    im = lm, iu = lu;
+    float    im = lm, iu = lu;  // running sums: im, ic from the first bucket on, iu from the last one back
     uint32_t ic = lc;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
-        const float    um = __shfl_up(im, o, WAVE), uu = __shfl_up(iu, o, WAVE);
+        const float    um = __shfl_up(im, o, WAVE), uu = __shfl_down(iu, o, WAVE);
         const uint32_t uc = __shfl_up(ic, o, WAVE);
         if (lane_id() >= o) {
             im += um;
-            iu += uu;
             ic += uc;
+        }
+        if (lane_id() + o < WAVE) {
+            iu += uu;
         }
     }
     if (lane_id() == WAVE - 1) {
-        wmass[wave_id()]  = im;
+        wmass[wave_id()] = im;
+        wcnt[wave_id()]  = ic;
+    }
+    if (lane_id() == 0) {
         wupper[wave_id()] = iu;
-        wcnt[wave_id()]   = ic;
     }
     __syncthreads();
-    float    em = im - lm, upper = 0.0f;
+    float em = im - lm, rest = __shfl_down(iu, 1, WAVE);
+    rest     = lane_id() == WAVE - 1 ? 0.0f : rest;
     uint32_t ec = ic - lc;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
         em += w < wave_id() ? wmass[w] : 0.0f;
         ec += w < wave_id() ? wcnt[w] : 0u;
-        upper += wupper[w];
+        rest += w > wave_id() ? wupper[w] : 0.0f;
     }
-    const float want  = draw * (upper + 1e-6f) * (1.0f + 1.0f / 256.0f);
+    // The prefix holds the draw when (mass of the prefix) >= draw * (mass of the row), that is
+    // mass * (1 - draw) >= draw * (mass behind it): with the mass from below on the left and from above on the right this
+    // is sharp where little lies behind the prefix, however wide its buckets are. (Bounds on the whole row's mass differ
+    // by a bucket's width, 1/64, so that draws above 0.98 would always take the whole row. 256 x 128256 N(0, 2.5), p = 0.9,
+    // us a step: 406 with such bounds, 117; with two columns far ahead 601, 66.) The margin is the rounding of the
+    // reference's scan.
+    const float q     = draw * (1.0f + 1.0f / 1024.0f);
     uint32_t    first = 0xFFFFFFFFu;
     {
+        float behind[K];
+        behind[K - 1] = rest;
+#pragma unroll
+        for (int i = K - 1; i > 0; --i) {
+            behind[i - 1] = behind[i] + upper[i];
+        }
         float m = em;
 #pragma unroll
         for (int i = 0; i < K; ++i) {
             m += lower[i];
-            if (m >= want && first == 0xFFFFFFFFu) {
+            if (m > 0.0f && m * (1.0f - q) >= q * (behind[i] + 1e-6f) && first == 0xFFFFFFFFu) {
                 first = (uint32_t)(t * K + i);
             }
         }
@@ -2152,3 +2177,14 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
 }
 
 }  // namespace ftk
+
+#ifdef FTK_TEST_HOOKS
+// Test hook (hooks build of the library only): what the last fp32 step in this workspace gathered of every row.
+extern "C" int ftk_test_topp_prefix_lengths(const void* workspace, int rows, int vocab, size_t pitch, int keeps_y,
+                                            int* lengths)
+{
+    const ftk::ToppSamplePlan p = ftk::topp_sample_plan(ftk::DT_F32, rows, vocab, pitch, keeps_y != 0);
+    return (int)hipMemcpy2D(lengths, sizeof(int), (const char*)workspace + p.off_meta + offsetof(ftk::ToppRowMeta, n),
+                            sizeof(ftk::ToppRowMeta), sizeof(int), rows, hipMemcpyDeviceToHost);
+}
+#endif

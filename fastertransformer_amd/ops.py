@@ -90,6 +90,7 @@ _HOOK_SIGNATURES = {
     "ftk_test_device_math": [_i, _vp, _vp, _sz, _vp],
     "ftk_test_rng_uniform": [_vp, _vp, _i, _i, _vp],
     "ftk_test_set_topp_force_deep": [_i],
+    "ftk_test_topp_prefix_lengths": [_vp, _i, _i, _sz, _i, _vp],
     "ftk_test_set_fused_force_general": [_i],
     "ftk_test_set_fused_two_launches": [_i],
     "ftk_test_last_fused_path": [],

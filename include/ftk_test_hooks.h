@@ -26,6 +26,9 @@ int ftk_test_device_math(int kind, const float* in, float* out, size_t n, ftk_st
 int ftk_test_rng_uniform(ftk_rng_state* states, float* out, int batch_size, int n_draws, ftk_stream_t stream);
 /* non-zero: every top-p row takes the radix-sort fallback (exercises it on small inputs); process-wide */
 void ftk_test_set_topp_force_deep(int enable);
+/* entries in the ordered prefix of each of the `rows` rows (host array) after an fp32 ftk_fused_topp_sample_step
+   (keeps_y 0) or ftk_fused_topp_penalty_step with penalties (1) in this workspace; meaningless for rows without one */
+int ftk_test_topp_prefix_lengths(const void* workspace, int rows, int vocab, size_t pitch, int keeps_y, int* lengths);
 /* non-zero: every fused step takes the general stream, also where the lean gather would run; process-wide */
 void ftk_test_set_fused_force_general(int enable);
 /* non-zero: the fused step keeps gather and selection in two launches also where one workgroup per row could do

@@ -50,12 +50,13 @@ def test_penalised_nucleus_rows(dt, shape):
         compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
 
 
-def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None):
+def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None, gathered=None):
     """One ftk_fused_topp_sample_step over rows of `x`: (ids, finished, lengths, cumulative log-probs). The draws are
-    `draws`, or generated from `states` (advanced in place)."""
+    `draws`, or generated from `states` (advanced in place). `gathered` (fp32; an int32 array) gets the number of entries
+    in each row's ordered prefix."""
     import torch
     from fastertransformer_amd import ops
-    lib = ops.ftk()
+    lib = ops.ftk() if gathered is None else ops.ftk_hooks()
     B, Vp = x.shape
     d_x, d_p, d_end, d_u = to_torch(x, dt), to_torch(p_arr), to_torch(end_ids), to_torch(draws)
     ids = torch.full((B,), -7, dtype=torch.int32, device="cuda")
@@ -69,6 +70,8 @@ def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None):
         ids.data_ptr(), cum.data_ptr(), None, ops.ptr(states), ops.ptr(d_u), 1.0, d_p.data_ptr(), None, None, None, None,
         None, ops.current_stream()))
     torch.cuda.synchronize()
+    if gathered is not None:
+        ops.check(lib.ftk_test_topp_prefix_lengths(ws.data_ptr(), B, V, Vp, 0, gathered.ctypes.data))
     return tuple(to_numpy(a) for a in (ids, fin, seq, cum))
 
 
@@ -125,3 +128,49 @@ def test_generated_draws_are_the_injected_ones(dt, B, V):
             assert np.array_equal(a, b)
         assert (to_numpy(states).reshape(B, 2)[:, 1] == i + 1).all()
     assert np.array_equal(to_numpy(states), to_numpy(ahead))
+
+
+def _prefix_bound(y, draw):
+    """The most entries a row's ordered prefix may need. Buckets are 1/64 wide: the sum bounds a prefix's mass from below
+    and what lies behind it from above by a factor of e^(1/64) each, and takes two more buckets than the one that covers
+    the draw (with the margin of 1/1024 on it). Beyond that, the buckets' open top, 8 above the largest of a sample of
+    1024 columns, may hold columns that the sample missed: 200 are allowed for here."""
+    y = np.sort(y.astype(np.float64))[::-1]
+    mass = np.cumsum(np.exp(y - y[0]))
+    behind = np.maximum(mass[-1] - mass, 0.0) + 1e-6
+    q = draw * (1 + 1 / 1024)
+    if q >= 1:
+        return len(y)
+    enough = np.nonzero(mass * (1 - q) >= 1.001 * np.exp(2 / 64) * q * behind)[0]
+    return len(y) if len(enough) == 0 else int((y >= y[enough[0]] - 4 / 64).sum()) + 200
+
+
+@pytest.mark.parametrize("kind", ["two_ahead", "five_ahead", "masked_head", "cold", "allowed_few", "peaked"])
+@pytest.mark.parametrize("B,V", [(12, 40009), (256, 9001)])   # sixteen and four workgroups per row
+def test_fp32_prefix_is_what_the_draw_needs(B, V, kind):
+    """Rows whose columns are unlike each other: a few tokens far ahead of all others, an id range masked out, a low
+    temperature, nearly everything masked. The prefix that is gathered and ordered follows the draw, not the layout."""
+    rng = np.random.default_rng(V + len(kind))
+    x = (rng.standard_normal((B, V)) * 2.5).astype(np.float32)
+    if kind == "two_ahead":
+        x[:, V // 25], x[:, V * 2 // 3] = 20.0, 19.5
+    elif kind == "five_ahead":
+        x[:, rng.integers(V // 25, V, 5)] = np.float32([20.0, 19.9, 19.8, 19.7, 19.6])
+    elif kind == "masked_head":
+        x[:, :1024] = -1e4
+    elif kind == "cold":
+        x *= 10.0
+    elif kind == "allowed_few":
+        keep = rng.random((B, V)) < 0.01
+        x[~keep] = -1e4
+        x[:, 5] = 3.0
+    else:
+        x[:, V // 2:V // 2 + 50] += 12.0
+    p_arr, end_ids = np.ones(B, np.float32), rng.integers(0, V, B).astype(np.int32)
+    u = rng.uniform(0.05, 0.995, B).astype(np.float32)
+    u[:6] = [0.3, 0.6, 0.85, 0.98, 0.99, 0.995]
+    got = np.zeros(B, np.int32)
+    print("prefix", B, V, kind, flush=True)
+    _same(_sample_step(O.F32, x, V, p_arr, end_ids, u, gathered=got), _oracle_step(O.F32, x, V, p_arr, end_ids, u), O.F32)
+    bound = np.array([_prefix_bound(x[b], float(u[b])) for b in range(B)])
+    assert (got >= 1).all() and (got <= bound).all(), (got[got > bound], bound[got > bound])
