@@ -2005,6 +2005,13 @@ struct ToppSamplePlan {
     size_t off_y, off_counts, off_pmax, off_blocks, off_ref, off_gsum, off_segs, off_queue, off_meta, bytes;
 };
 
+// most columns that the bitmap of the history covers, and the columns of a workgroup of the fp32 stage
+constexpr int TSP_WINDOW_BITS = (TSP_WINDOW - 4) * 32;
+static int topp_part_columns(int vocab, int parts)
+{
+    return (vocab + TSP_CHAINS - 1) / TSP_CHAINS * (TSP_CHAINS / parts);
+}
+
 static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vocab_padded, bool keeps_y)
 {
     ToppSamplePlan p;
@@ -2013,12 +2020,17 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     // sixteen with four lanes to a chain below. 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four
     // below.
     p.parts = dtype == DT_F32 ? (rows >= 256 ? 4 : 16) : (rows >= 192 ? 1 : 4);
+    // (a quarter of more than 655360 columns does not fit the bitmap of the history, a sixteenth does: whether a
+    // vocabulary is covered must not depend on the rows of the call)
+    if (dtype == DT_F32 && keeps_y && topp_part_columns(vocab, p.parts) > TSP_WINDOW_BITS) {
+        p.parts = 16;
+    }
     // 16-bit stage: about four workgroups per compute unit, each with at least four blocks of columns (one per wave), and
     // no more columns than its bitmap of the history covers
     p.blocks = (vocab + TSP_BLOCK - 1) / TSP_BLOCK;
     int s    = (1024 + rows - 1) / rows;
     s        = std::min(s, std::max(1, p.blocks / 4));
-    s        = std::max(s, (p.blocks + (TSP_WINDOW - 4) * 32 / TSP_BLOCK - 1) / ((TSP_WINDOW - 4) * 32 / TSP_BLOCK));
+    s        = std::max(s, (p.blocks + TSP_WINDOW_BITS / TSP_BLOCK - 1) / (TSP_WINDOW_BITS / TSP_BLOCK));
     p.splits = std::min(s, TSP_SPLITS);
     p.chunk  = (p.blocks + p.splits - 1) / p.splits * TSP_BLOCK;
     p.sorters       = (int)std::min<size_t>(512, (size_t)rows * (vocab_padded / TPS_SEG + 1));
@@ -2060,9 +2072,8 @@ bool topp_sample_covers(int dtype, int rows, int vocab, bool history_penalty)
         return true;
     }
     // the bitmap of the history that a stage's workgroup keeps
-    const ToppSamplePlan p    = topp_sample_plan(dtype, rows, vocab, (size_t)vocab, true);
-    const long long      bits = dtype == DT_F32 ? (long long)((vocab + TSP_CHAINS - 1) / TSP_CHAINS) * (TSP_CHAINS / p.parts) : p.chunk;
-    return bits <= (long long)(TSP_WINDOW - 4) * 32;
+    const ToppSamplePlan p = topp_sample_plan(dtype, rows, vocab, (size_t)vocab, true);
+    return (dtype == DT_F32 ? topp_part_columns(vocab, p.parts) : p.chunk) <= TSP_WINDOW_BITS;
 }
 
 int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)

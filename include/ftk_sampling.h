@@ -122,7 +122,7 @@ int ftk_fused_topp_step(int dtype, void* workspace, size_t* workspace_size, void
  * log-probs, lengths, finished flags and decayed top-p values, but `logits` is only read (the reference leaves the
  * probabilities there, layers/sampling_layers/TopPSamplingLayer.cu:287-297; nothing in its decode loop reads them
  * again). Every probability that is needed is worked out from the logits on the way, with the arithmetic of
- * ftk_invoke_add_bias_softmax, so the row is read three times and never written. FTK_ERR_UNSUPPORTED (also from
+ * ftk_invoke_add_bias_softmax, so the row is read twice and never written. FTK_ERR_UNSUPPORTED (also from
  * the size query) when vocab_size < 1024; a step with an embedding bias takes ftk_fused_topp_step.
  * workspace == NULL: size query (ftk_fused_topp_step's). */
 int ftk_fused_topp_sample_step(int dtype, void* workspace, size_t* workspace_size, const void* logits,
@@ -265,8 +265,9 @@ int ftk_fused_topk_step(ftk_fused_topk_args* args, ftk_stream_t stream);
  * (the values after the penalties are kept in the workspace). Results are bit for bit those of the kernel sequence.
  * `row` carries what the two steps have in common; its top_ks, top_ps and max_top_k are not read. An embedding bias
  * needs `temperatures`. FTK_ERR_UNSUPPORTED (also from the size query) for fewer than 1024 columns, a frequency
- * penalty, or a vocabulary of more than a million columns with a history penalty: run the kernel sequence then.
- * row.workspace == NULL: size query into row.workspace_size. */
+ * penalty, or, with a history penalty, a vocabulary of more than 2621440 columns (fp32) or 10485760 (16-bit types): run
+ * the kernel sequence then. The answer does not depend on the number of rows. row.workspace == NULL: size query into
+ * row.workspace_size. */
 typedef struct ftk_fused_topp_args {
     ftk_fused_topk_args row;
     float               max_top_p;     /* every row's p when runtime_top_p is NULL */

@@ -201,3 +201,25 @@ def test_kernel_wrappers_instantiate_and_answer_host_queries(tmp_path):
                            "-Wl,-rpath," + os.path.join(PKG, "lib"), "-Wl,-rpath,/opt/rocm/lib", "-o", exe])
     out = subprocess.run([exe], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+@pytest.mark.parametrize("rows", [1, 95, 96, 191, 192, 255, 256, 1024])
+@pytest.mark.parametrize("dt,most", [(O.F32, 2621440), (O.F16, 10485760), (O.BF16, 10485760)])
+def test_topp_penalty_step_covers_a_vocabulary_for_every_row_count(dt, most, rows):
+    """the limits that include/ftk_sampling.h states, from the size query"""
+    _ensure_built()
+    from fastertransformer_amd import ops
+    row = ops.FusedTopkArgs(dtype=dt, local_batch_size=rows, penalty_type=0, penalties=8)  # (the array is not looked into)
+
+    class Args(C.Structure):
+        _fields_ = [("row", ops.FusedTopkArgs), ("max_top_p", C.c_float)] + [("p%d" % i, C.c_void_p) for i in range(5)]
+
+    def query(vocab):
+        a = Args(row=row)
+        a.row.vocab_size = a.row.vocab_size_padded = vocab
+        return ops.ftk().ftk_fused_topp_penalty_step(C.addressof(a), None), a.row.workspace_size
+
+    for vocab in (1024, 655360, 655361, most):
+        rc, size = query(vocab)
+        assert rc == 0 and size > 0, vocab
+    assert query(1023)[0] == ops.FTK_ERR_UNSUPPORTED and query(most + 1)[0] == ops.FTK_ERR_UNSUPPORTED
