@@ -2016,10 +2016,15 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
 {
     ToppSamplePlan p;
     rows = rows > 0 ? rows : 1;
-    // The sum. fp32: 256-thread workgroups, one chain per thread and four workgroups per row where that fills the chip,
-    // sixteen with four lanes to a chain below. 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four
-    // below.
-    p.parts = dtype == DT_F32 ? (rows >= 256 ? 4 : 16) : (rows >= 192 ? 1 : 4);
+    // The sum. fp32: 256-thread workgroups, one chain per thread and four workgroups per row from 96 rows on, sixteen with
+    // four lanes to a chain below. Sixteen share a short batch out better, but each of them reads the histograms of all
+    // sixteen (128 KB). us a step, zipf rows, p = 0.9, sixteen / four:
+    //   rows      8         64        96        128        255
+    //   8192      29 / 30   39 / 35   44 / 36   50 / 36   116 / 45
+    //   32000     34 / 37   53 / 52   62 / 54   70 / 57   145 / 72
+    //   128256    43 / 56   76 / 82   93 / 86  104 / 90   181 / 114
+    // 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four below.
+    p.parts = dtype == DT_F32 ? (rows >= 96 ? 4 : 16) : (rows >= 192 ? 1 : 4);
     // (a quarter of more than 655360 columns does not fit the bitmap of the history, a sixteenth does: whether a
     // vocabulary is covered must not depend on the rows of the call)
     if (dtype == DT_F32 && keeps_y && topp_part_columns(vocab, p.parts) > TSP_WINDOW_BITS) {
