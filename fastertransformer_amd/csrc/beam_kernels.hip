@@ -822,6 +822,7 @@ struct BeamUpdate {
 
 constexpr int BB_HISTORY = 1024;  // (step, beam) pairs of the history kept in LDS
 constexpr int BB_MERGED  = 1024;  // keys of an entry that are merged here
+constexpr int BB_SHARED  = 512;   // the same where rows are shared: two per thread
 constexpr int BB_CACHE   = 4096;  // cache positions of an entry that are copied here: 16 per thread
 
 // One workgroup per batch entry (:99-262). Bound by latency: a few hundred candidates and one thread that walks the
@@ -848,8 +849,7 @@ beam_batch_kernel(BeamCandidates cd, int* ids, float* cum_log_probs, float* __re
     __shared__ int        merged_id[BB_MERGED];
     __shared__ float      merged_val[BB_MERGED];
     __shared__ int        cached[BB_MERGED];
-    __shared__ double     part_sum[WAVE];  // (2 K K parts <= BB_MERGED: at most 64 sums)
-    __shared__ float      row_max[WAVE];
+    __shared__ float      row_max[WAVE], row_logd[WAVE];
     const int             b         = blockIdx.x;
     const int             t         = threadIdx.x;
     const int             N         = 2 * K;
@@ -887,7 +887,7 @@ beam_batch_kernel(BeamCandidates cd, int* ids, float* cum_log_probs, float* __re
                 r_key[u] = cd.pkeys[(size_t)b * n_keys + min(t + u * BM_THREADS, n_keys - 1)];
             }
         }
-        r_sum = cd.psum[(size_t)b * K * cd.parts + min(t, K * cd.parts - 1)];
+        r_sum = cd.psum[(size_t)b * K * cd.parts + min(t, K * cd.parts - 1)];  // (2 K K parts <= BB_MERGED: one wave has all)
         r_max = cd.pmax[own];
     }
     const int  kept    = with_hyps ? min(h.step, BB_HISTORY / K) : 0;  // steps of the history in LDS: the last ones
@@ -957,8 +957,15 @@ beam_batch_kernel(BeamCandidates cd, int* ids, float* cum_log_probs, float* __re
     const int*   x = cd.id + (size_t)b * C;
     const float* y = cd.val + (size_t)b * C;
     if (cd.parts > 0) {
-        if (t < K * cd.parts) {
-            part_sum[t] = r_sum;
+        if (t < WAVE) {
+            // a row's sums lie in neighbouring lanes; added and turned into a logarithm once per row
+            double d = 0.0;
+            for (int p = 0; p < cd.parts; ++p) {
+                d += __shfl(r_sum, min(t * cd.parts + p, WAVE - 1), WAVE);
+            }
+            if (t < K) {
+                row_logd[t] = det_logf((float)d);
+            }
         }
 #pragma unroll
         for (int u = 0; u < TURNS; ++u) {
@@ -971,25 +978,23 @@ beam_batch_kernel(BeamCandidates cd, int* ids, float* cum_log_probs, float* __re
         for (int i = t; i < n_keys; i += BM_THREADS) {
             const unsigned long long k     = s.cand[i];
             const int                r     = i / per_row;
-            const int                at    = i % per_row;
-            int                      place = at % N;  // its own part's keys in front of it
-            for (int p = 0; p < cd.parts; ++p) {
-                if (p != at / N) {
-                    const unsigned long long* other = s.cand + r * per_row + p * N;
-                    for (int j = 0; j < N; ++j) {
-                        place += other[j] > k ? 1 : 0;
-                    }
+            int                      place = i - r * per_row;
+            if (cd.parts > 1) {
+                // its rank among the row's keys, four looked at at a time
+                const ulonglong2* pairs = reinterpret_cast<const ulonglong2*>(s.cand + r * per_row);
+                place                   = 0;
+#pragma unroll 2
+                for (int j = 0; j < per_row / 4; ++j) {
+                    const ulonglong2 m = pairs[2 * j];
+                    const ulonglong2 n = pairs[2 * j + 1];
+                    place += (m.x > k ? 1 : 0) + (m.y > k ? 1 : 0) + (n.x > k ? 1 : 0) + (n.y > k ? 1 : 0);
                 }
             }
             // (a finished row's other parts hold zeros, below the first part's 2K keys: they get no place)
             if (place < N && k != 0ull) {
-                double d = 0.0;
-                for (int p = 0; p < cd.parts; ++p) {
-                    d += part_sum[r * cd.parts + p];
-                }
                 merged_id[r * N + place] = (int)beam_key_position(k) + (b * K + r) * vocab;
                 merged_val[r * N + place] =
-                    round_t<DT>((beam_key_value(k) - row_max[r] - det_logf((float)d)) + old_cum[r]);
+                    round_t<DT>((beam_key_value(k) - row_max[r] - row_logd[r]) + old_cum[r]);
             }
         }
         x = merged_id;
@@ -1341,9 +1346,15 @@ extern "C" void ftk_test_set_beam_path(int v)
 #endif
 
 // How many workgroups share a row of beam_team_kernel: as many as the compute units allow, as long as every part has at
-// least 4096 columns to itself (below that the read of the whole row is all there is) and an entry's keys fit the
-// merge. Rows too long for the registers, and more rows than compute units, take the other forms (0): of two
-// 512-thread workgroups on a compute unit one reads while the other computes.
+// least 4096 columns to itself and an entry's keys fit the merge. Rows too long for the registers, and more rows than
+// compute units, take the other forms (0). Requests of four steps through the layer, fp16, us, other forms / this one:
+//   32 x 4 x 50257, two parts        124 / 106    (8192 columns, one part: 86 / 87)
+//    8 x 4 x 50257, eight parts      117 / 94     (32000 columns, four parts: 102 / 89)
+//   64 x 4 x 50257, one part         132 / 126    (fp32: 160 / 139)
+//    1 x 8 x 50257, four parts       127 / 106    (8192 columns, two parts: 91 / 91)
+//    8 x 16 x 50257, one part        186 / 180    (8192 columns: 146 / 146)
+// Where rows are shared a merge takes two keys per thread at most: with four, each ranked among the keys of its row, the
+// last two took 18 us and 28 us longer than here.
 static int beam_team_parts(int rows, int beam_width, int vocab, const BeamPlan& plan)
 {
     if (vocab > BT_COLUMNS || rows > 256) {
@@ -1353,7 +1364,7 @@ static int beam_team_parts(int rows, int beam_width, int vocab, const BeamPlan& 
     while (parts < BT_MAX_PARTS && 2 * parts * rows <= 256 && vocab / (2 * parts) >= 4096 && 2 * parts <= plan.parts) {
         parts *= 2;
     }
-    while (parts > 0 && 2 * beam_width * beam_width * parts > BB_MERGED) {
+    while (parts > 0 && 2 * beam_width * beam_width * parts > (parts > 1 ? BB_SHARED : BB_MERGED)) {
         parts /= 2;
     }
     return parts;

@@ -148,6 +148,35 @@ def test_beam_step_both_forms_of_the_row_stage(path):
         hooks.ftk_test_set_beam_path(0)
 
 
+@pytest.mark.parametrize("batch,K,V", [(1, 2, 65536), (2, 5, 50257), (1, 6, 40009), (1, 8, 65536), (2, 11, 33001),
+                                       (1, 12, 33001)], ids=["8", "8odd", "4", "4full", "2", "1"])
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+def test_rows_shared_by_workgroups(dt, batch, K, V):
+    """rows whose candidates come in 8, 4, 2 lists or one (by the number of keys an entry merges), ordinary ones and
+    rows of equal values, masked to -inf but for a few columns, with NaN columns, and with every beam finished"""
+    rng = np.random.default_rng(K * V + dt)
+    _one_case(rng, dt, batch, K, V, True, 0.1, 0.7)
+    for kind in range(4):
+        c = make_beam_case(rng, dt, batch, K, V, step=5, max_seq_len=12, with_hyps=True, finished_frac=0.0)
+        x = O.to_f32(c["log_probs"], dt)
+        if kind == 0:
+            x[:] = 1.5
+        elif kind == 1:
+            x[:] = -np.inf
+            x[:, rng.choice(V, 3 * K, replace=False)] = rng.standard_normal(3 * K)
+        elif kind == 2:
+            x[:, rng.choice(V, 40, replace=False)] = np.nan
+        else:
+            c["finished"][:] = True
+        c["log_probs"] = O.to_storage(x, dt).reshape(c["log_probs"].shape)
+        want = copy_beam_case(c)
+        assert O.topk_softmax(dt, want["log_probs"], None, want["finished"], want["sequence_lengths"],
+                              want["cum_log_probs"], want["output_log_probs"], want["ids"], want["hyps"], batch, K, V,
+                              want["end_ids"], 0.0, 0.5) == 0
+        print("shared rows", DTYPE_NAMES[dt], batch, K, V, kind, flush=True)
+        _compare(c, want, _run_product(c, dt, batch, K, V, 0.0, 0.5), dt)
+
+
 def test_beam_step_degenerate_rows():
     """rows of equal values (ties settled by the lower id at every stage), rows masked to -inf except a few
     columns, every beam finished, hypotheses already complete for every entry"""
