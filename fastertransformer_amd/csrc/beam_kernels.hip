@@ -1353,8 +1353,8 @@ extern "C" void ftk_test_set_beam_path(int v)
 //   64 x 4 x 50257, one part         132 / 126    (fp32: 160 / 139)
 //    1 x 8 x 50257, four parts       127 / 106    (8192 columns, two parts: 91 / 91)
 //    8 x 16 x 50257, one part        186 / 180    (8192 columns: 146 / 146)
-// Where rows are shared a merge takes two keys per thread at most: with four, each ranked among the keys of its row, the
-// last two took 18 us and 28 us longer than here.
+// Where rows are shared a merge takes two keys per thread at most: with four, ranked one by one, the last two took 186 and
+// 211 us.
 static int beam_team_parts(int rows, int beam_width, int vocab, const BeamPlan& plan)
 {
     if (vocab > BT_COLUMNS || rows > 256) {
