@@ -2005,8 +2005,9 @@ struct ToppSamplePlan {
     size_t off_y, off_counts, off_pmax, off_blocks, off_ref, off_gsum, off_segs, off_queue, off_meta, bytes;
 };
 
-// most columns that the bitmap of the history covers, and the columns of a workgroup of the fp32 stage
-constexpr int TSP_WINDOW_BITS = (TSP_WINDOW - 4) * 32;
+constexpr int TSP_MANY_ROWS   = 96;                     // fp32: from here on four workgroups per row, sixteen below
+constexpr int TSP_WINDOW_BITS = (TSP_WINDOW - 4) * 32;  // most columns that the bitmap of the history covers
+// the columns of a workgroup of the fp32 stage
 static int topp_part_columns(int vocab, int parts)
 {
     return (vocab + TSP_CHAINS - 1) / TSP_CHAINS * (TSP_CHAINS / parts);
@@ -2024,7 +2025,7 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     //   32000     34 / 37   53 / 52   62 / 54   70 / 57   145 / 72
     //   128256    43 / 56   76 / 82   93 / 86  104 / 90   181 / 114
     // 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four below.
-    p.parts = dtype == DT_F32 ? (rows >= 96 ? 4 : 16) : (rows >= 192 ? 1 : 4);
+    p.parts = dtype == DT_F32 ? (rows >= TSP_MANY_ROWS ? 4 : 16) : (rows >= 192 ? 1 : 4);
     // (a quarter of more than 655360 columns does not fit the bitmap of the history, a sixteenth does: whether a
     // vocabulary is covered must not depend on the rows of the call)
     if (dtype == DT_F32 && keeps_y && topp_part_columns(vocab, p.parts) > TSP_WINDOW_BITS) {
@@ -2041,16 +2042,17 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     p.sorters       = (int)std::min<size_t>(512, (size_t)rows * (vocab_padded / TPS_SEG + 1));
     p.y_pitch       = (int)((vocab_padded + 7) / 8 * 8);
     const size_t el = dtype == DT_F32 ? 4 : 2;
-    const size_t counters = dtype == DT_F32 ? (size_t)p.parts * TSP_BUCKETS :
-                            dtype == DT_F16 ? (size_t)ToppCode<DT_F16>::COUNTERS :
-                                              (size_t)ToppCode<DT_BF16>::COUNTERS;
+    // (fp32: also as many as a call of fewer rows and more parts takes, so that a window of a batch never needs more)
+    const size_t counters =
+        dtype == DT_F32 ? (size_t)std::max(rows * p.parts, std::min(rows, TSP_MANY_ROWS - 1) * 16) * TSP_BUCKETS :
+                          (size_t)rows * (dtype == DT_F16 ? ToppCode<DT_F16>::COUNTERS : ToppCode<DT_BF16>::COUNTERS);
     size_t off = up256((size_t)rows * vocab_padded * 2 * sizeof(unsigned long long));
     auto   take = [&](size_t bytes) {
         const size_t at = off;
         off += up256(bytes);
         return at;
     };
-    p.off_counts = take((size_t)rows * counters * sizeof(uint32_t));
+    p.off_counts = take(counters * sizeof(uint32_t));
     p.off_pmax   = take((size_t)rows * TSP_SPLITS * sizeof(float2));
     p.off_blocks = take(dtype == DT_F32 ? 0 : (size_t)rows * p.blocks * sizeof(float));
     p.off_ref    = take((size_t)rows * sizeof(float));

@@ -187,8 +187,8 @@ bool TopPSamplingLayer<T>::runFused(TensorMap* output_tensors, TensorMap* input_
     }
     check_ftk(query);
     if (a.row.workspace_size > sampling_workspace_size_) {
-        // (the split of a row depends on the number of rows in the call: a window smaller than the setup batch can
-        // need a slightly larger workspace)
+        // (with penalties setup() reserved enough for every window; without them the size is also the kernel sequence's,
+        // whose chunks per row depend on the rows of the call, see runSampling())
         sampling_workspace_      = allocator_->reMalloc(sampling_workspace_, a.row.workspace_size, false);
         sampling_workspace_size_ = a.row.workspace_size;
     }

@@ -203,23 +203,35 @@ def test_kernel_wrappers_instantiate_and_answer_host_queries(tmp_path):
     assert out.returncode == 0, out.stdout + out.stderr
 
 
+def _topp_penalty_query(dt, rows, vocab):
+    """(code, workspace size) of ftk_fused_topp_penalty_step with a history penalty"""
+    from fastertransformer_amd import ops
+
+    class Args(C.Structure):
+        _fields_ = [("row", ops.FusedTopkArgs), ("max_top_p", C.c_float)] + [("p%d" % i, C.c_void_p) for i in range(5)]
+
+    a = Args(row=ops.FusedTopkArgs(dtype=dt, local_batch_size=rows, vocab_size=vocab, vocab_size_padded=vocab,
+                                   penalty_type=0, penalties=8))  # (a query does not look into the array)
+    return ops.ftk().ftk_fused_topp_penalty_step(C.addressof(a), None), a.row.workspace_size
+
+
 @pytest.mark.parametrize("rows", [1, 95, 96, 191, 192, 255, 256, 1024])
 @pytest.mark.parametrize("dt,most", [(O.F32, 2621440), (O.F16, 10485760), (O.BF16, 10485760)])
 def test_topp_penalty_step_covers_a_vocabulary_for_every_row_count(dt, most, rows):
     """the limits that include/ftk_sampling.h states, from the size query"""
     _ensure_built()
     from fastertransformer_amd import ops
-    row = ops.FusedTopkArgs(dtype=dt, local_batch_size=rows, penalty_type=0, penalties=8)  # (the array is not looked into)
-
-    class Args(C.Structure):
-        _fields_ = [("row", ops.FusedTopkArgs), ("max_top_p", C.c_float)] + [("p%d" % i, C.c_void_p) for i in range(5)]
-
-    def query(vocab):
-        a = Args(row=row)
-        a.row.vocab_size = a.row.vocab_size_padded = vocab
-        return ops.ftk().ftk_fused_topp_penalty_step(C.addressof(a), None), a.row.workspace_size
-
     for vocab in (1024, 655360, 655361, most):
-        rc, size = query(vocab)
+        rc, size = _topp_penalty_query(dt, rows, vocab)
         assert rc == 0 and size > 0, vocab
-    assert query(1023)[0] == ops.FTK_ERR_UNSUPPORTED and query(most + 1)[0] == ops.FTK_ERR_UNSUPPORTED
+    for vocab in (1023, most + 1):
+        assert _topp_penalty_query(dt, rows, vocab)[0] == ops.FTK_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("vocab", [1024, 3001, 50257])
+def test_topp_penalty_step_of_a_window_fits_the_batch_workspace(dt, vocab):
+    """a layer reserves for its batch and may then be called for windows of it: fewer rows never need more"""
+    _ensure_built()
+    sizes = [_topp_penalty_query(dt, rows, vocab)[1] for rows in range(1, 600)]
+    assert sizes == sorted(sizes)
