@@ -51,17 +51,18 @@ def test_penalised_nucleus_rows(dt, shape):
         compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
 
 
-def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None, gathered=None):
+def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None, gathered=None, finished=None, hooks=False):
     """One ftk_fused_topp_sample_step over rows of `x`: (ids, finished, lengths, cumulative log-probs). The draws are
     `draws`, or generated from `states` (advanced in place). `gathered` (fp32; an int32 array) gets the number of entries
     in each row's ordered prefix."""
     import torch
     from fastertransformer_amd import ops
-    lib = ops.ftk() if gathered is None else ops.ftk_hooks()
+    lib = ops.ftk_hooks() if hooks or gathered is not None else ops.ftk()
     B, Vp = x.shape
     d_x, d_p, d_end, d_u = to_torch(x, dt), to_torch(p_arr), to_torch(end_ids), to_torch(draws)
     ids = torch.full((B,), -7, dtype=torch.int32, device="cuda")
-    fin, seq = torch.zeros(B, dtype=torch.bool, device="cuda"), torch.zeros(B, dtype=torch.int32, device="cuda")
+    fin = torch.zeros(B, dtype=torch.bool, device="cuda") if finished is None else to_torch(finished)
+    seq = torch.zeros(B, dtype=torch.int32, device="cuda")
     cum = torch.zeros(B, dtype=torch.float32, device="cuda")
     size = C.c_size_t(0)
     ops.check(lib.ftk_fused_topp_sample_step(dt, None, C.addressof(size), None, V, Vp, B, *(None,) * 8, 1.0, *(None,) * 7))
@@ -76,9 +77,9 @@ def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None, gathered=Non
     return tuple(to_numpy(a) for a in (ids, fin, seq, cum))
 
 
-def _oracle_step(dt, x, V, p_arr, end_ids, draws):
+def _oracle_step(dt, x, V, p_arr, end_ids, draws, finished=None):
     B, Vp = x.shape
-    probs, fin, seq = x.copy(), np.zeros(B, np.bool_), np.zeros(B, np.int32)
+    probs, fin, seq = x.copy(), np.zeros(B, np.bool_) if finished is None else finished.copy(), np.zeros(B, np.int32)
     O.add_bias_softmax(dt, probs, None, end_ids, fin, B, Vp, V)
     ids, cum, out = np.full(B, -7, np.int32), np.zeros(B, np.float32), np.zeros(B, np.float32)
     O.batch_topp_sampling(dt, probs, ids, seq, fin, cum, out, draws, B, Vp, end_ids, 0.0, p_arr, None)
@@ -172,6 +173,98 @@ def test_fp32_prefix_is_what_the_draw_needs(B, V, kind):
     u[:6] = [0.3, 0.6, 0.85, 0.98, 0.99, 0.995]
     got = np.zeros(B, np.int32)
     print("prefix", B, V, kind, flush=True)
-    _same(_sample_step(O.F32, x, V, p_arr, end_ids, u, gathered=got), _oracle_step(O.F32, x, V, p_arr, end_ids, u), O.F32)
+    _same(_sample_step(O.F32, x, V, p_arr, end_ids, u, gathered=got), _oracle_step(O.F32, x, V, p_arr, end_ids, u),
+          O.F32)
     bound = np.array([_prefix_bound(x[b], float(u[b])) for b in range(B)])
     assert (got >= 1).all() and (got <= bound).all(), (got[got > bound], bound[got > bound])
+
+
+# (rows of the batch, of a window, columns, pitch): odd columns, padded and odd pitches, both splits of a row
+@pytest.mark.parametrize("B,window,V,Vp", [(12, 6, 1501, 1504), (12, 6, 2050, 2051), (6, 6, 33001, 33008),
+                                           (200, 100, 1030, 1030), (200, 200, 1025, 1032)])
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+def test_biased_nucleus_rows(dt, B, window, V, Vp):
+    """An embedding bias under every other penalty, rows of both layers, windows of the batch; the second step's bias
+    masks most columns."""
+    rng = np.random.default_rng(V + dt)
+    H = 7
+    ks = np.where(rng.random(B) < 0.3, 4, 0).astype(np.uint32)
+    kind = "repetition_penalty" if V % 2 else "presence_penalty"
+    for masks in (False, True):
+        bias = rng.standard_normal(Vp).astype(np.float32)
+        if masks:
+            bias[rng.random(Vp) < 0.9] = -1e4
+        c = Case(dt, B, V, Vp, max_input_length=H, gen_len=2, local_batch=window, runtime_top_k=ks,
+                 runtime_top_p=rng.uniform(0.2, 1.0, B), temperature=rng.uniform(0.5, 1.5, B),
+                 min_length=rng.integers(0, 3, B), end_ids=rng.integers(0, V, B),
+                 input_lengths=rng.integers(1, H + 1, B), prompt=rng.integers(0, V, (H, B)).astype(np.int32),
+                 embedding_bias=O.to_storage(bias, dt), with_cum=True, with_out_lp=window == B, **{kind: rng.uniform(0.5, 1.5, B)})
+        p, o = ProductRunner(c), OracleRunner(c)
+        for i in range(2):
+            x, u = make_logits(rng, dt, B, V, Vp, 2.0), uniforms(rng, B)
+            for ite in range(B // window):
+                print("biased", DTYPE_NAMES[dt], B, window, V, Vp, masks, i, ite, flush=True)
+                p.step(H + i, x, u, ite=ite)
+                o.step(H + i, x, u, ite=ite)
+                compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d window %d" % (i, ite))
+
+
+def _penalty_step(dt, x, V, p_arr, end_ids, draws, finished, temps, penalties, history):
+    """_sample_step with a temperature and a repetition penalty over `history` [steps, rows]"""
+    import torch
+    from fastertransformer_amd import ops
+
+    class Args(C.Structure):
+        _fields_ = [("row", ops.FusedTopkArgs), ("max_top_p", C.c_float), ("runtime_top_p", C.c_void_p)] + [
+            ("decay%d" % i, C.c_void_p) for i in range(4)]
+
+    lib, (B, Vp) = ops.ftk_hooks(), x.shape
+    d = dict(logits=to_torch(x, dt), temperatures=to_torch(temps), penalties=to_torch(penalties),
+             end_ids=to_torch(end_ids), output_ids=to_torch(history), uniform_draws=to_torch(draws), finished=to_torch(finished),
+             ids=torch.full((B,), -7, dtype=torch.int32, device="cuda"),
+             sequence_length=torch.zeros(B, dtype=torch.int32, device="cuda"),
+             cum_log_probs=torch.zeros(B, dtype=torch.float32, device="cuda"))
+    a = Args(row=ops.FusedTopkArgs(dtype=dt, vocab_size=V, vocab_size_padded=Vp, batch_size=B, local_batch_size=B,
+                                   step=len(history), max_input_length=len(history), penalty_type=1,
+                                   **{k: v.data_ptr() for k, v in d.items()}))
+    d["p"] = to_torch(p_arr)
+    a.max_top_p, a.runtime_top_p = 1.0, d["p"].data_ptr()
+    ops.check(lib.ftk_fused_topp_penalty_step(C.addressof(a), None))
+    ws = torch.empty(a.row.workspace_size, dtype=torch.uint8, device="cuda")
+    a.row.workspace = ws.data_ptr()
+    ops.check(lib.ftk_fused_topp_penalty_step(C.addressof(a), ops.current_stream()))
+    torch.cuda.synchronize()
+    return tuple(to_numpy(d[k]) for k in ("ids", "finished", "sequence_length", "cum_log_probs"))
+
+
+@pytest.mark.parametrize("B,V,Vp", [(7, 1027, 1027), (6, 4096, 4104), (200, 1100, 1101)])
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+def test_whole_row_fallback(dt, B, V, Vp):
+    """The exact way out of the pick, every row sent there by the test build's switch, and without it: plain and
+    penalised rows against the oracle. Among them finished rows with an end id inside and outside of the vocabulary."""
+    from fastertransformer_amd import ops
+    rng = np.random.default_rng(V + 10 * dt)
+    hooks, H = ops.ftk_hooks(), 9
+    end_ids = rng.integers(0, V, B).astype(np.int32)
+    end_ids[1], end_ids[2], end_ids[3] = Vp + 5, -1, V - 1
+    finished = np.zeros(B, np.bool_)
+    finished[1:4] = True
+    temps, pens = (rng.uniform(0.5, 1.5, B).astype(np.float32) for _ in range(2))
+    history = rng.integers(0, V, (H, B)).astype(np.int32)
+    for i, spread in enumerate((0.3, 2.0, 8.0)):
+        x = make_logits(rng, dt, B, V, Vp, spread)
+        p_arr, u = rng.uniform(0.3, 1.0, B).astype(np.float32), uniforms(rng, B)
+        u[0], p_arr[0] = 1.0, 1.0
+        y = x.copy()
+        O.batch_apply_temperature_penalty(dt, y, None, temps, B, V, Vp)
+        O.batch_apply_repetition_penalty(dt, y, pens, history, B, B, Vp, None, H, H, 1)
+        for deep in (1, 0):
+            hooks.ftk_test_set_topp_force_deep(deep)
+            try:
+                print("whole row", DTYPE_NAMES[dt], B, V, Vp, i, deep, flush=True)
+                plain = _sample_step(dt, x, V, p_arr, end_ids, u, finished=finished, hooks=True)
+                penalised = _penalty_step(dt, x, V, p_arr, end_ids, u, finished, temps, pens, history)
+            finally:
+                hooks.ftk_test_set_topp_force_deep(0)
+            _same(plain, _oracle_step(dt, x, V, p_arr, end_ids, u, finished), dt)
+            _same(penalised, _oracle_step(dt, y, V, p_arr, end_ids, u, finished), dt)
