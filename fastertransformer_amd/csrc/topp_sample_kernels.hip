@@ -326,9 +326,9 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
 }
 
 // ---- stage, fp32 --------------------------------------------------------------------------------------------------
-__device__ __forceinline__ int topp_y_bucket(float y, float top)
+__device__ __forceinline__ int topp_y_bucket(float y, float top, float last = (float)(TSP_BUCKETS - 1))
 {
-    return (int)__builtin_amdgcn_fmed3f((top - y) * TSP_SCALE, 0.0f, (float)(TSP_BUCKETS - 1));
+    return (int)__builtin_amdgcn_fmed3f((top - y) * TSP_SCALE, 0.0f, last);
 }
 
 // (rows x parts) workgroups; a workgroup reads the columns of its summation chains, 1024 / parts neighbouring columns
@@ -339,11 +339,14 @@ __device__ __forceinline__ int topp_y_bucket(float y, float top)
 template<bool TRANSFORM>
 __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
 {
-    __shared__ uint32_t hist[TSP_BUCKETS];
+    // The last bucket is open below: masked columns, half of a row perhaps, lie there and would queue for its counter. It
+    // is spread over a counter per lane (256 x 128256, every second column -inf: 153 -> 114 us a step).
+    __shared__ uint32_t hist[TSP_BUCKETS - 1 + WAVE];
     __shared__ uint32_t window[TRANSFORM ? TSP_WINDOW : 1];
     __shared__ float    red[16];
     __shared__ uint32_t any_nan;
     const int           row = blockIdx.x, j = blockIdx.y, t = threadIdx.x;
+    const float         last = (float)(TSP_BUCKETS - 1 + lane_id());
     if (row == 0 && j == 0 && t == 0) {
         s.queue[0] = 0u;
     }
@@ -367,7 +370,7 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     for (int u = 0; u < U0; ++u) {
         plain[u] = rowp[sample(u)];
     }
-    for (int i = t; i < TSP_BUCKETS; i += TSP_STAGE) {
+    for (int i = t; i < TSP_BUCKETS - 1 + WAVE; i += TSP_STAGE) {
         hist[i] = 0u;
     }
     if (t == 0) {
@@ -411,7 +414,7 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
         }
         mx  = __builtin_fmaxf(mx, x);
         nan = nan || x != x;
-        atomicAdd(&hist[topp_y_bucket(x, top)], 1u);
+        atomicAdd(&hist[topp_y_bucket(x, top, last)], 1u);
         return x;
     };
     const int quads = C / 4, qshift = shift - 2;  // 16-byte vectors of a workgroup in one stretch of 1024 columns
@@ -471,10 +474,10 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
             }
         }
     }
-    for (int v = s.n + t; v < s.Vp; v += TSP_STAGE) {  // pads lie in the lowest bucket
+    for (int v = s.n + t; v < s.Vp; v += TSP_STAGE) {  // pads lie in the last bucket
         const int c = (v & (TSP_CHAINS - 1)) - c0;
         if (c >= 0 && c < C) {
-            atomicAdd(&hist[TSP_BUCKETS - 1], 1u);
+            atomicAdd(&hist[TSP_BUCKETS - 1 + lane_id()], 1u);
         }
     }
     if (nan) {
@@ -482,8 +485,13 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     }
     mx = block_max<float, TSP_STAGE / WAVE>(mx, red, TSP_LOWEST);
     uint32_t* out = s.counts + ((size_t)row * s.parts + j) * TSP_BUCKETS;
-    for (int i = t; i < TSP_BUCKETS / 4; i += TSP_STAGE) {
-        reinterpret_cast<uint4*>(out)[i] = reinterpret_cast<const uint4*>(hist)[i];
+    const int low = wave_sum_i((int)hist[TSP_BUCKETS - 1 + lane_id()]);
+#pragma unroll
+    for (int u = 0; u < TSP_BUCKETS / 4 / TSP_STAGE; ++u) {
+        const int i = t + u * TSP_STAGE;
+        uint4     c = reinterpret_cast<const uint4*>(hist)[i];
+        c.w         = i == TSP_BUCKETS / 4 - 1 ? (uint32_t)low : c.w;
+        reinterpret_cast<uint4*>(out)[i] = c;
     }
     if (t == 0) {
         s.pmax[(size_t)row * TSP_SPLITS + j] = make_float2(mx, any_nan != 0u ? 1.0f : 0.0f);
