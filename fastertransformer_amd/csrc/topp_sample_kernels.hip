@@ -359,12 +359,12 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     const int    shift = __builtin_ctz((unsigned)C);
     const int    c0    = j * C;
     const int    nit   = (s.n + TSP_CHAINS - 1) / TSP_CHAINS;
-    // the origin of the buckets: the largest value among 1024 columns, 64 stretches of 16 spread over the row (ids of one
-    // script or of special tokens are neighbours), without the history; the same for every part. Everything 8 or more above
-    // it lies in the first bucket (256 x 128256 with the first 1024 columns masked: 22 ms a step with the first 1024
-    // columns as the sample, 0.12 ms)
+    // the origin of the buckets: the largest value among 1024 columns, 32 lines of 32 spread over the row (ids of one script
+    // or of special tokens are neighbours), without the history; the same for every part. Everything 8 or more above it
+    // lies in the first bucket (256 x 128256 with the first 1024 columns masked: 22 ms a step with those as the sample,
+    // 0.12 ms). More and shorter stretches cost time on every row: 64 of 16, 0.7 us.
     constexpr int U0 = TSP_CHAINS / TSP_STAGE;
-    auto  sample = [&](int u) { return (u * (TSP_STAGE / 16) + (t >> 4)) * (s.n / 64) + (t & 15); };
+    auto  sample = [&](int u) { return (u * (TSP_STAGE / 32) + (t >> 5)) * ((s.n / 32) & ~31) + (t & 31); };
     float plain[U0];
 #pragma unroll
     for (int u = 0; u < U0; ++u) {
