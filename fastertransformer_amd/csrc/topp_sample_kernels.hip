@@ -78,19 +78,16 @@ struct ToppStep {
 };
 
 // Counters of the 16-bit types. binary16: one per value of e up to 1. bfloat16: one per value from 2^-31 to 1; a draw
-// that falls among smaller ones takes the exact fallback. LUT_*: the values of y whose e a workgroup of the sum looks up
-// in a table, 2 x LUT_N of them: magnitudes from LUT_LOW on (2^-8 .. 2^8 / 2^6).
+// that falls among smaller ones takes the exact fallback.
 template<int DT>
 struct ToppCode;
 template<>
 struct ToppCode<DT_F16> {
     static constexpr int COUNTERS = 16384, USED = 15361, BASE = 0;
-    static constexpr int LUT_LOW = 7 << 10, LUT_N = 14 << 10;
 };
 template<>
 struct ToppCode<DT_BF16> {
     static constexpr int COUNTERS = 4096, BASE = ((127 - 31) << 7) - 1, USED = 127 * 128 - BASE + 1;
-    static constexpr int LUT_LOW = (127 - 8) << 7, LUT_N = 16 << 7;
 };
 static_assert(ToppCode<DT_BF16>::USED <= ToppCode<DT_BF16>::COUNTERS, "bfloat16 counters");
 
@@ -645,10 +642,10 @@ __device__ __forceinline__ void topp_group_sums(const ToppStep& s, int row, int 
 // stretches out, read eight bytes - four chains - per lane and leave the e of a chunk of stretches in LDS, from where
 // one thread per chain adds them up in the reference's order. (One chain per thread straight from memory means two-byte
 // loads and a dependent addition per load: 14 us for 64 x 128256 bfloat16 whatever is done with the values.)
-// e is a function of the 16 bits of y once the maximum is known: with LUT the workgroup first works it out for the values
-// that occur in earnest (4096 for bfloat16, 28672 for binary16) and then looks it up. Values outside the table (tiny or
-// huge magnitudes, -inf) take the exponential.
-template<int DT, int C, bool LUT>
+// e is a function of the 16 bits of y once the maximum is known, but a table of it in LDS, made by every workgroup, does
+// not pay: gathers from it cost as much as the exponential (256 x 128256, us a step with a table / so: binary16 95 / 92,
+// bfloat16 76 / 76; every second column masked 98 / 84 and 85 / 72).
+template<int DT, int C>
 __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
 {
     typedef Storage<DT>   S;
@@ -659,7 +656,6 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
     constexpr int         PAR = TSP_SUM16 / WAVE / WS;     // stretches taken at a time
     constexpr int         U   = KI / PAR;                  // vectors per lane and chunk
     __shared__ uint32_t   cnt[Code::USED + WAVE];
-    __shared__ T          lut[LUT ? 2 * Code::LUT_N : 1];
     __shared__ uint2      e_of[KI * C / 4];
     const int             row = blockIdx.x, part = blockIdx.y, t = threadIdx.x;
     const T* y = s.y != nullptr ? (const T*)s.y + (size_t)row * s.y_pitch : (const T*)s.logits + (size_t)row * s.Vp;
@@ -688,45 +684,13 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
     if (!(mx == mx)) {
         return;  // (the pick sees the same and needs no sum)
     }
-    if constexpr (LUT) {
-#pragma unroll 1
-        for (int i = t; i < 2 * Code::LUT_N; i += TSP_SUM16) {
-            const T bits = (T)(i < Code::LUT_N ? Code::LUT_LOW + i : 0x8000 + Code::LUT_LOW + (i - Code::LUT_N));
-            lut[i]       = S::st(topp_exp(__builtin_fminf(S::ld(bits) - mx, 0.0f)));
-        }
-    }
     __syncthreads();
-    // The e of N values, counted: all look-ups are requested before the first one is used, values that are not in the
-    // table are put right together, and what has no counter goes to a word of the lane's own.
+    // The e of N values, counted; what has no counter goes to a word of the lane's own.
     auto e_bits = [&](const auto& x, auto& b) {
         constexpr int N = (int)(sizeof(x) / sizeof(x[0]));
-        if constexpr (LUT) {
-            uint32_t out = 0u;
 #pragma unroll
-            for (int c = 0; c < N; ++c) {
-                const uint32_t mag = (x[c] & 0x7FFFu) - (uint32_t)Code::LUT_LOW;
-                out                = max(out, mag);
-                b[c]               = lut[min(mag, (uint32_t)Code::LUT_N - 1u) + (x[c] >> 15) * (uint32_t)Code::LUT_N];
-            }
-            if (out >= (uint32_t)Code::LUT_N) {
-#pragma unroll 1
-                for (int c = 0; c < N; ++c) {
-                    const uint32_t xc = N == 1 || c == 0 ? x[0] : c == 1 ? x[N > 1 ? 1 : 0] : c == 2 ? x[N > 2 ? 2 : 0] : x[N - 1];
-                    if ((xc & 0x7FFFu) - (uint32_t)Code::LUT_LOW >= (uint32_t)Code::LUT_N) {
-                        const uint32_t e = S::st(topp_exp(S::ld((T)xc) - mx));
-#pragma unroll
-                        for (int k = 0; k < N; ++k) {
-                            b[k] = k == c ? e : b[k];
-                        }
-                    }
-                }
-            }
-        }
-        else {
-#pragma unroll
-            for (int c = 0; c < N; ++c) {
-                b[c] = S::st(topp_exp(S::ld((T)x[c]) - mx));
-            }
+        for (int c = 0; c < N; ++c) {
+            b[c] = S::st(topp_exp(S::ld((T)x[c]) - mx));
         }
 #pragma unroll
         for (int c = 0; c < N; ++c) {
@@ -2179,17 +2143,11 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
             topp_stage_kernel<DT, false><<<splits, TSP_STAGE, 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
-        // binary16's table is seven times bfloat16's: it pays only where one workgroup takes a whole long row
         if (p.parts == 1) {
-            if (DT == DT_BF16 || c.vocab_size >= 65536) {
-                topp_sum_count_kernel<DT, 1024, true><<<parts, TSP_SUM16, 0, st>>>(s);
-            }
-            else {
-                topp_sum_count_kernel<DT, 1024, false><<<parts, TSP_SUM16, 0, st>>>(s);
-            }
+            topp_sum_count_kernel<DT, 1024><<<parts, TSP_SUM16, 0, st>>>(s);
         }
         else {
-            topp_sum_count_kernel<DT, 256, DT == DT_BF16><<<parts, TSP_SUM16, 0, st>>>(s);
+            topp_sum_count_kernel<DT, 256><<<parts, TSP_SUM16, 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
         topp_pick_runs_kernel<DT><<<c.rows, TP_THREADS, 0, st>>>(s, o);
