@@ -620,7 +620,7 @@ beam_rowwide_kernel(const typename Storage<DT>::T* __restrict__ x, const typenam
 // for the maximum (100 KB of a row of 50257 fp16, from the XCD's L2 after the first), so they need nothing of each
 // other; the exponentials, which bound the kernel (23 vector instructions and a double addition each), and the
 // candidates are those of its own part. A part leaves its 2K best, largest first, and its sum; beam_batch_kernel merges.
-// 32 x 4 rows of 50257 fp16: 19.6 us with one workgroup per row that reads it three times, 14.9 us here (traced).
+// 32 x 4 rows of 50257 fp16: 19.6 us with one workgroup per row that reads it three times, 14.5 us here (traced).
 constexpr int BT_COLUMNS   = 65536;
 constexpr int BT_MAX_PARTS = 8;
 
@@ -830,7 +830,7 @@ constexpr int BB_CACHE   = 4096;  // cache positions of an entry that are copied
 // the last BB_HISTORY (step, beam) pairs of tokens, parents and log-probs among it, through which a finished beam is
 // traced in LDS instead of one dependent read per step - and the launches that followed it (token and parent split,
 // flags, lengths, cache indirection: 4.4 and 3.6 us of mostly latency) are its last lines.
-// 32 entries of 4 beams: 16.8 us in three launches, 9.9 us here (traced); the step 34 -> 25 us.
+// 32 entries of 4 beams: 16.8 us in three launches, 9.7 us here (traced); the step 34 -> 25 us.
 template<int DT>
 __global__ void __launch_bounds__(BM_THREADS)
 beam_batch_kernel(BeamCandidates cd, int* ids, float* cum_log_probs, float* __restrict__ output_log_probs,

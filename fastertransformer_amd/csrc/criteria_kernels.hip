@@ -113,8 +113,7 @@ length_criterion_kernel(bool* __restrict__ finished, int* finished_sum, const ui
     __shared__ int smem[16];
     int            count = 0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        // (both are requested at once: with || the limit waits for the flag, 1024 f16 rows of 152064 with log-probs
-        // then take 166.5 us a step instead of 165.0)
+        // (both are requested at once: with || the limit waits for the flag)
         const bool was = finished[i], over = (uint32_t)step >= limit[i / beam_width];
         finished[i]    = was | over;
         count += was | over ? 1 : 0;

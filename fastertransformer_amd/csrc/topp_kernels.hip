@@ -212,7 +212,9 @@ softmax_kernel(typename Storage<DT>::T* __restrict__ logits, const typename Stor
 // A row whose draw is not crossed inside its prefix (it cannot be unless the bound above fails)
 // falls back to a stable radix sort of all its positive entries.
 // Callers that do not need the probabilities afterwards take a second form of the step, which only reads the logits
-// (topp_sample_kernels.hip).// Workspace sections (all offsets multiples of 256 bytes). `sorted` keeps the reference's shape of
+// (topp_sample_kernels.hip).
+
+// Workspace sections (all offsets multiples of 256 bytes). `sorted` keeps the reference's shape of
 // two 64-bit arrays per row; the second one is only touched by the radix sorts.
 struct ToppPlan {
     int    splits;  // chunks per row of the two streaming kernels
@@ -255,6 +257,7 @@ static ToppPlan topp_plan(int batch, size_t vocab)
     p.bytes = off;
     return p;
 }
+
 template<int DT>
 __global__ void __launch_bounds__(TPH_THREADS)
 topp_histogram_kernel(const typename Storage<DT>::T* __restrict__ probs, int vocab, int chunk,

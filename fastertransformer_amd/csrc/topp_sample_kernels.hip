@@ -640,8 +640,8 @@ __device__ __forceinline__ void topp_group_sums(const ToppStep& s, int row, int 
 // ---- sum, 16-bit types ----------------------------------------------------------------------------------------------
 // A workgroup owns C summation chains: C neighbouring columns out of every 1024 (a "stretch"). Its waves share the
 // stretches out, read eight bytes - four chains - per lane and leave the e of a chunk of stretches in LDS, from where
-// one thread per chain adds them up in the reference's order. (One chain per thread straight from memory means two-byte
-// loads and a dependent addition per load: 14 us for 64 x 128256 bfloat16 whatever is done with the values.)
+// one thread per chain adds them up in the reference's order. (One chain per thread straight from memory would mean
+// two-byte loads and a dependent addition per load.) 64 x 128256 bfloat16: 14 us, vector instructions in 0.55 of it.
 // e is a function of the 16 bits of y once the maximum is known, but a table of it in LDS, made by every workgroup, does
 // not pay: gathers from it cost as much as the exponential (256 x 128256, us a step with a table / so: binary16 95 / 92,
 // bfloat16 76 / 76; every second column masked 98 / 84 and 85 / 72).
@@ -1512,7 +1512,7 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     __shared__ uint32_t           wcnt[TW], wrun[TW], wpick[NW];
     __shared__ float              wmass[TW];
     __shared__ uint32_t           sh_enough, key_lo, key_hi;
-    __shared__ int                sh_found, code_lo, code_hi, sh_nth, sh_id;
+    __shared__ int                sh_found, code_lo, code_hi, sh_nth;
     const int       row = blockIdx.x;
     const int       t   = threadIdx.x;
     ToppPickRow<DT> r(s, o, row, s.splits);
@@ -1537,7 +1537,6 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     if (t == 0) {
         sh_enough = 0xFFFFFFFFu;
         sh_found  = 0x7FFFFFFF;
-        sh_id     = -1;
     }
     if (r.skip) {
         if (t == 0) {
@@ -1996,7 +1995,13 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     //   8192      29 / 30   39 / 35   44 / 36   50 / 36   116 / 45
     //   32000     34 / 37   53 / 52   62 / 54   70 / 57   145 / 72
     //   128256    43 / 56   76 / 82   93 / 86  104 / 90   181 / 114
-    // 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four below.
+    // 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four below; one / four:
+    //   rows                64        96        128       160       224
+    //   binary16  32000     38 / 37   38 / 43   39 / 45   40 / 51   40 / 59
+    //             128256    75 / 61   79 / 76   81 / 79   85 / 93   90 / 110
+    //   bfloat16  32000     33 / 31   33 / 32   33 / 33   34 / 36   35 / 38
+    //             128256    63 / 49   66 / 55   67 / 56   70 / 65   74 / 74
+    // (binary16, whose counters take four times the time to merge, would change over at some 130 rows)
     p.parts = dtype == DT_F32 ? (rows >= TSP_MANY_ROWS ? 4 : 16) : (rows >= 192 ? 1 : 4);
     // (a quarter of more than 655360 columns does not fit the bitmap of the history, a sixteenth does: whether a
     // vocabulary is covered must not depend on the rows of the call)
