@@ -401,7 +401,8 @@ softmax_finish_histogram_kernel(typename Storage<DT>::T* __restrict__ logits,
                 y = v == end_id ? MAXT : -MAXT;
             }
             else {
-                y = round_t<DT>(x + S::ld(bias[v]));
+                // (rows without a bias come here, too, when their denominator is no ordinary number)
+                y = round_t<DT>(x + (bias != nullptr ? S::ld(bias[v]) : 0.0f));
             }
             return finish(v, y);
         });

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import ft_oracle as O
-from decode_harness import Case, OracleRunner, ProductRunner, compare
+from decode_harness import Case, OracleRunner, ProductRunner, compare, kernel_sequence
 from helpers import DTYPE_NAMES, DTYPES, make_logits, to_numpy, to_torch, uniforms
 
 pytestmark = pytest.mark.gpu
@@ -268,3 +268,27 @@ def test_whole_row_fallback(dt, B, V, Vp):
                 hooks.ftk_test_set_topp_force_deep(0)
             _same(plain, _oracle_step(dt, x, V, p_arr, end_ids, u, finished), dt)
             _same(penalised, _oracle_step(dt, y, V, p_arr, end_ids, u, finished), dt)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("V,Vp,sequence", [(500, 500, False), (333, 336, False), (2050, 2050, True), (2050, 2056, True),
+                                           (2050, 2050, False)])
+def test_rows_without_an_ordinary_denominator(dt, V, Vp, sequence):
+    """Rows with a NaN, with an infinity, all masked and all at the lowest number, without a bias: through the step that
+    writes the probabilities (fewer than 1024 columns, or asked for) and through the one that does not."""
+    rng = np.random.default_rng(V + dt)
+    B, H = 9, 3
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=2, runtime_top_k=[0], runtime_top_p=rng.uniform(0.2, 1.0, B),
+             end_ids=np.full(B, V - 1), prompt=rng.integers(0, V, (H, B)).astype(np.int32), with_cum=True)
+    with kernel_sequence(sequence):
+        p, o = ProductRunner(c), OracleRunner(c)
+        for i in range(2):
+            x = rng.standard_normal((B, Vp)).astype(np.float32)
+            x[1, rng.integers(0, V)], x[2, rng.integers(0, V)] = np.nan, np.inf
+            x[3], x[4], x[5], x[6] = -np.inf, np.nan, O.max_t(dt) * -1.0, 0.0
+            x = O.to_storage(x, dt)
+            u = uniforms(rng, B)
+            print("denominators", DTYPE_NAMES[dt], V, Vp, sequence, i, flush=True)
+            p.step(H + i, x, u)
+            o.step(H + i, x, u)
+            compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
