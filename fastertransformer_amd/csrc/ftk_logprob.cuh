@@ -1212,6 +1212,23 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                 push(v, e);
             }
         });
+    if (p.V < p.Vp) {
+        // pad columns count once nothing of the vocabulary is far above -MAX_T (rows that are masked throughout)
+        const float pad_e = round_t<DT>(det_expf_nonpos(-S::max_t() - row_max));
+        if (pad_e > 0.0f) {
+#pragma unroll 1
+            for (int v = p.V + ((t - p.V) & (THREADS - 1)); v < p.Vp; v += THREADS) {
+                const int chain = (v & (LP_BLOCK - 1)) / THREADS;
+#pragma unroll
+                for (int c = 0; c < CH; ++c) {
+                    acc[c] = c == chain ? acc[c] + pad_e : acc[c];
+                }
+                if (pad_e >= thr_low) {
+                    push(v, pad_e);
+                }
+            }
+        }
+    }
     LPW_STAMP(5)
     if constexpr (THREADS < LPW_THREADS) {
         __builtin_amdgcn_s_setprio(3);

@@ -134,3 +134,29 @@ def test_rows_whose_candidates_are_gathered_again(dt, B, V, Vp, k, kind):
         p.step(H + i, x, u)
         o.step(H + i, x, u)
         compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="%s step %d" % (kind, i))
+
+
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16], ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("B,V,Vp,k", [(6, 1452, 1459, 5), (300, 1030, 1040, 20), (5, 2100, 3200, 130), (4, 9001, 9008, 8)])
+def test_masked_rows_count_their_pads(dt, B, V, Vp, k):
+    """Rows masked throughout, with -inf or the type's lowest number: the pad columns hold -MAX_T and carry the softmax."""
+    from decode_harness import Case, OracleRunner, ProductRunner, compare
+    from helpers import uniforms
+    rng = np.random.default_rng(V + dt)
+    H = 4
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=2, runtime_top_k=[k], runtime_top_p=[1.0],
+             end_ids=np.full(B, V - 1), prompt=rng.integers(0, V, (H, B)).astype(np.int32), with_cum=True,
+             with_out_lp=True)
+    p, o = ProductRunner(c), OracleRunner(c)
+    for i in range(2):
+        x = rng.standard_normal((B, Vp)).astype(np.float32)
+        x[0] = -np.inf
+        x[1] = -O.max_t(dt)
+        x[2], x[2, rng.integers(0, V, 3)] = -np.inf, -O.max_t(dt)
+        x[3], x[3, rng.integers(0, V, V // 2)] = -O.max_t(dt), -np.inf
+        x, u = O.to_storage(x, dt), uniforms(rng, B)
+        print("masked rows", DTYPE_NAMES[dt], B, V, Vp, k, i, flush=True)
+        p.step(H + i, x, u)
+        o.step(H + i, x, u)
+        compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
+
