@@ -774,6 +774,7 @@ topp_pick_kernel(const typename Storage<DT>::T* __restrict__ probs, int* ids, in
                        -1;
     };
     auto emit_at = [&](const unsigned long long* src, int n, int found) {
+        found = min(found, vocab - 1);  // (the zeros that fill the last tile can hold the crossing)
         if (found < n) {
             const unsigned long long e = src[found];
             emit((int)(uint32_t)e, key64_prob(e));

@@ -1182,12 +1182,13 @@ __device__ __attribute__((noinline)) ToppPicked topp_pick_whole_row(TopPScan& sc
     if (round_t<DT>(0.0f + best) >= r.p) {
         return ToppPicked{id, best, true};
     }
-    const int found = n > 0 ? scan_tiles<1>(sc, (n + TP_TILE - 1) / TP_TILE, r.rand_num,
-                                            [&](int tile, int l, float* x) { tile_load(src, n, tile, l, x); }) :
-                              -1;
+    int found = n > 0 ? scan_tiles<1>(sc, (n + TP_TILE - 1) / TP_TILE, r.rand_num,
+                                      [&](int tile, int l, float* x) { tile_load(src, n, tile, l, x); }) :
+                        -1;
     if (found < 0) {
         return ToppPicked{id, best, false};
     }
+    found = min(found, r.Vp - 1);  // (the zeros that fill the last tile can hold the crossing)
     if (found < n) {
         return ToppPicked{(int)(uint32_t)src[found], key64_prob(src[found]), true};
     }

@@ -292,3 +292,24 @@ def test_rows_without_an_ordinary_denominator(dt, V, Vp, sequence):
             p.step(H + i, x, u)
             o.step(H + i, x, u)
             compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
+
+
+@pytest.mark.parametrize("sequence", [False, True])
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+def test_crossings_behind_the_last_column(dt, sequence):
+    """Draws of 1.0: where rounding lets the running sum reach them only among the zeros that fill the last tile, the last
+    entry in order of probabilities is emitted."""
+    rng = np.random.default_rng(dt)
+    B, V = 300, 1526
+    x = np.round(rng.standard_normal((B, V)) * 5.0).astype(np.float32) / 2
+    x = O.to_storage(x, dt)
+    c = Case(dt, B, V, V, gen_len=1, runtime_top_k=[0], runtime_top_p=[1.0])
+    with kernel_sequence(sequence):
+        p, o = ProductRunner(c), OracleRunner(c)
+        print("behind the last column", DTYPE_NAMES[dt], sequence, flush=True)
+        p.step(0, x, np.ones(B, np.float32))
+        o.step(0, x, np.ones(B, np.float32))
+    compare(p.snapshot(), o.snapshot(), dt, check_logits=False)
+    if dt == O.F32:
+        last = np.argsort(-x, axis=1, kind="stable")[:, -1]
+        assert ((o.snapshot()["output_ids"][0] == last) & (last != V - 1)).any()
