@@ -367,6 +367,23 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     for (int u = 0; u < U0; ++u) {
         plain[u] = rowp[sample(u)];
     }
+    // (and the first vectors of the row, so that they do not wait for the sample's maximum)
+    constexpr int U     = 8;
+    const int     quads = C / 4, qshift = shift - 2;  // 16-byte vectors of a workgroup in one stretch of 1024 columns
+    const int     nfull = s.n / TSP_CHAINS;           // stretches that lie inside the vocabulary
+    const int     total = nfull * quads;              // vectors
+    const bool    vec   = (s.Vp & 3) == 0 && ((uintptr_t)s.logits & 15u) == 0u;
+    float4        raw[U];
+    auto          load = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = min(i0 + u * TSP_STAGE, total - 1);
+            raw[u]      = *reinterpret_cast<const float4*>(rowp + (size_t)(i >> qshift) * TSP_CHAINS + c0 + (i & (quads - 1)) * 4);
+        }
+    };
+    if (vec) {
+        load(t);
+    }
     for (int i = t; i < TSP_BUCKETS - 1 + WAVE; i += TSP_STAGE) {
         hist[i] = 0u;
     }
@@ -414,18 +431,11 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
         atomicAdd(&hist[topp_y_bucket(x, top, last)], 1u);
         return x;
     };
-    const int quads = C / 4, qshift = shift - 2;  // 16-byte vectors of a workgroup in one stretch of 1024 columns
-    int       it0   = 0;
-    if ((s.Vp & 3) == 0 && ((uintptr_t)s.logits & 15u) == 0u) {
-        constexpr int U     = 8;
-        const int     nfull = s.n / TSP_CHAINS;  // stretches that lie inside the vocabulary
-        const int     total = nfull * quads;     // vectors
+    int it0 = 0;
+    if (vec) {
         for (int i0 = t; i0 < total; i0 += U * TSP_STAGE) {
-            float4 raw[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = min(i0 + u * TSP_STAGE, total - 1);
-                raw[u]      = *reinterpret_cast<const float4*>(rowp + (size_t)(i >> qshift) * TSP_CHAINS + c0 + (i & (quads - 1)) * 4);
+            if (i0 != t) {
+                load(i0);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
