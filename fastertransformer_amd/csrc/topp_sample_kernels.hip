@@ -330,9 +330,11 @@ __device__ __forceinline__ int topp_y_bucket(float y, float top, float last = (f
 
 // (rows x parts) workgroups; a workgroup reads the columns of its summation chains, 1024 / parts neighbouring columns
 // out of every 1024, so that its histogram says how many entries of every bucket the sum's workgroup of the same part
-// will place. Rows are the fast index of the grid: the parts of a row read interleaved stretches of one kilobyte or
-// less, and neighbouring workgroups go to different XCDs; with the parts as the fast index every XCD would see the same
-// quarter of every 4 KB and use a quarter of its L2's channels.
+// will place. Rows are the fast index of the grid, and their number is rounded up to a multiple of eight: the parts of a
+// row then run on one XCD, of the stage and of the sum, and its L2 keeps the row's histograms from the one to the other
+// (us a step, as they come / rounded up: 1 x 8192 25.2 / 23.7, 33 x 8192 42 / 36, 95 x 8192 68 / 45; 255 x 128256
+// 113 / 117). With the parts as the fast index every XCD would see the same quarter of every 4 KB and use a quarter of its
+// L2's channels.
 template<bool TRANSFORM>
 __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
 {
@@ -347,7 +349,7 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     if (row == 0 && j == 0 && t == 0) {
         s.queue[0] = 0u;
     }
-    if (topp_row_idle(s, row)) {
+    if (row >= s.rows || topp_row_idle(s, row)) {
         return;
     }
     const float* rowp  = (const float*)s.logits + (size_t)row * s.Vp;
@@ -801,7 +803,7 @@ __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
     __shared__ uint32_t queue_at;  // where the row's segments go in the queue, plus one (0: the pick orders them)
     __shared__ uint32_t red32[16];
     const int           row = blockIdx.x, part = blockIdx.y, t = threadIdx.x;
-    if (topp_row_idle(s, row)) {
+    if (row >= s.rows || topp_row_idle(s, row)) {
         return;
     }
     const void*         safe = s.pmax;
@@ -1987,7 +1989,7 @@ struct ToppSamplePlan {
     size_t off_y, off_counts, off_pmax, off_blocks, off_ref, off_gsum, off_segs, off_queue, off_meta, bytes;
 };
 
-constexpr int TSP_MANY_ROWS   = 96;                     // fp32: from here on four workgroups per row, sixteen below
+constexpr int TSP_MANY_ROWS   = 72;                     // fp32: from here on four workgroups per row, sixteen below
 constexpr int TSP_WINDOW_BITS = (TSP_WINDOW - 4) * 32;  // most columns that the bitmap of the history covers
 // the columns of a workgroup of the fp32 stage
 static int topp_part_columns(int vocab, int parts)
@@ -1999,13 +2001,13 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
 {
     ToppSamplePlan p;
     rows = rows > 0 ? rows : 1;
-    // The sum. fp32: 256-thread workgroups, one chain per thread and four workgroups per row from 96 rows on, sixteen with
+    // The sum. fp32: 256-thread workgroups, one chain per thread and four workgroups per row from 72 rows on, sixteen with
     // four lanes to a chain below. Sixteen share a short batch out better, but each of them reads the histograms of all
     // sixteen (128 KB). us a step, zipf rows, p = 0.9, sixteen / four:
-    //   rows      8         64        96        128        255
-    //   8192      29 / 30   39 / 35   44 / 36   50 / 36   116 / 45
-    //   32000     34 / 37   53 / 52   62 / 54   70 / 57   145 / 72
-    //   128256    43 / 56   76 / 82   93 / 86  104 / 90   181 / 114
+    //   rows      7         47        65        79        95        129       255
+    //   8192      30 / 30   37 / 34   42 / 36   44 / 36   45 / 36   53 / 37   73 / 39
+    //   32000     33 / 36   49 / 50   57 / 52   60 / 53   63 / 54   72 / 57  101 / 68
+    //   128256    43 / 55   68 / 76   80 / 82   86 / 84   93 / 86  103 / 91  158 / 117
     // 16-bit types: 1024-thread workgroups, one per row from 192 rows on, four below; one / four:
     //   rows                64        96        128       160       224
     //   binary16  32000     38 / 37   38 / 43   39 / 45   40 / 51   40 / 59
@@ -2130,18 +2132,19 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
 
     const dim3 parts(c.rows, p.parts), splits(c.rows, p.splits);
     if (c.dtype == DT_F32) {
+        const dim3 grid((c.rows + 7) / 8 * 8, p.parts);
         if (keeps_y) {
-            topp_stage_f32_kernel<true><<<parts, TSP_STAGE, 0, st>>>(s);
+            topp_stage_f32_kernel<true><<<grid, TSP_STAGE, 0, st>>>(s);
         }
         else {
-            topp_stage_f32_kernel<false><<<parts, TSP_STAGE, 0, st>>>(s);
+            topp_stage_f32_kernel<false><<<grid, TSP_STAGE, 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
         if (p.parts == 4) {
-            topp_sum_gather_kernel<1><<<parts, TSP_SUM32, 0, st>>>(s);
+            topp_sum_gather_kernel<1><<<grid, TSP_SUM32, 0, st>>>(s);
         }
         else {
-            topp_sum_gather_kernel<4><<<parts, TSP_SUM32, 0, st>>>(s);
+            topp_sum_gather_kernel<4><<<grid, TSP_SUM32, 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
         topp_sort_queue_kernel<<<p.sorters, TP_THREADS, 0, st>>>(s);

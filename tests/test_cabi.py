@@ -215,7 +215,7 @@ def _topp_penalty_query(dt, rows, vocab):
     return ops.ftk().ftk_fused_topp_penalty_step(C.addressof(a), None), a.row.workspace_size
 
 
-@pytest.mark.parametrize("rows", [1, 95, 96, 191, 192, 255, 256, 1024])
+@pytest.mark.parametrize("rows", [1, 71, 72, 191, 192, 255, 256, 1024])
 @pytest.mark.parametrize("dt,most", [(O.F32, 2621440), (O.F16, 10485760), (O.BF16, 10485760)])
 def test_topp_penalty_step_covers_a_vocabulary_for_every_row_count(dt, most, rows):
     """the limits that include/ftk_sampling.h states, from the size query"""
