@@ -4,10 +4,12 @@
 #include <string.h>
 
 #include "ftk_device.cuh"
+#include "ftk_exp16.cuh"
 #include "ftk_sampling.h"
 #ifdef FTK_TEST_HOOKS
 #include "ftk_test_hooks.h"
 #endif
+#include "ftk_transform.cuh"
 #include "ftk_words.cuh"
 
 namespace ftk {
@@ -158,6 +160,40 @@ __global__ void test_math_kernel(int kind, const float* __restrict__ in, float* 
         }
         out[i] = y;
     }
+}
+
+// Workgroup b: every pair (y, max) with the value of bits b as the maximum and y not above it, or NaN.
+// wrong[0]: results that are not T(det_expf(y - max)); wrong[1]: pairs of values that took det_expf.
+template<int DT>
+__global__ void test_exp_pairs_kernel(unsigned long long* wrong)
+{
+    typedef Storage<DT> S;
+    const float         max = S::ld((typename S::T)blockIdx.x);
+    if (!(max == max)) {
+        return;
+    }
+    const ExpPairs<DT> ex(max);
+    unsigned long long bad = 0ull, again = 0ull;
+    for (uint32_t i = threadIdx.x; i < 32768u; i += blockDim.x) {
+        uint32_t y = 0u;  // two neighbouring values; what lies above the maximum becomes the maximum
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t bits = 2u * i + (uint32_t)h;
+            y |= (uint32_t)(S::ld((typename S::T)bits) > max ? S::st(max) : (typename S::T)bits) << (16 * h);
+        }
+        uint32_t redo = ex.never;
+        uint32_t e    = ex(y, redo);
+        if (ex.undecided(redo)) {
+            e = ex.exact(y);
+            again++;
+        }
+        for (int h = 0; h < 2; ++h) {
+            const float    want = round_t<DT>(det_expf_nonpos(S::ld((typename S::T)(y >> (16 * h))) - max));
+            const float    got  = S::ld((typename S::T)(e >> (16 * h)));
+            bad += want != want ? (got != got ? 0u : 1u) : (f2u(want) != f2u(got) ? 1u : 0u);
+        }
+    }
+    atomicAdd(&wrong[0], bad);
+    atomicAdd(&wrong[1], again);
 }
 
 __global__ void test_rng_kernel(RngState* states, float* out, int batch, int n_draws)
@@ -345,6 +381,21 @@ int ftk_test_device_math(int kind, const float* in, float* out, size_t n, ftk_st
     }
     const int grid = (int)min((size_t)2048, (n + 255) / 256);
     test_math_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(kind, in, out, n);
+    FTK_LAUNCH_CHECK();
+    return 0;
+}
+
+int ftk_test_exp_pairs(int dtype, unsigned long long* wrong, ftk_stream_t stream)
+{
+    if (dtype == FTK_DTYPE_F16) {
+        test_exp_pairs_kernel<DT_F16><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
+    }
+    else if (dtype == FTK_DTYPE_BF16) {
+        test_exp_pairs_kernel<DT_BF16><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
+    }
+    else {
+        return FTK_ERR_DTYPE;
+    }
     FTK_LAUNCH_CHECK();
     return 0;
 }

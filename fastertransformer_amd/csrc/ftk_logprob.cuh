@@ -9,7 +9,7 @@
 //   2. e_v = T(exp(y_v - max)) summed in the order of the reference's softmax
 //      (sampling_topp_kernels.cu:1308-1344: thread t of 1024 adds columns t, t + 1024, ... one after the other;
 //      reduce_kernel_utils.cuh:73-103: xor butterflies 16..1 inside 32-lane groups, then over the 32 group sums),
-//      so the sum has the reference's bits; on the way the candidates of the top-k selection are gathered by e_v,
+//      so the sum has the reference's bits. The candidates of the top-k selection are gathered by e_v,
 //      with a bound lowered by what the division and rounding to T can merge, so that every column whose
 //      probability ties with the k-th largest is among them. The candidates' e_v then become probabilities
 //      T(e_v / (sum + 1e-6)), the reference's tie orders are replayed on them and the row is sampled
@@ -30,6 +30,7 @@
 #pragma once
 #include <type_traits>
 
+#include "ftk_exp16.cuh"
 #include "ftk_lean.cuh"
 
 namespace ftk {
@@ -872,11 +873,12 @@ __global__ void __launch_bounds__(LP_THREADS) lp_row_kernel(FusedParams p, Fused
 
 // ---- one launch: a workgroup per row reads it twice ---------------------------------------------------------------
 // With few rows lp_row_kernel's four waves per row are what bounds the step (about a microsecond per 1024 columns),
-// and most compute units idle. Here THREADS threads share a row, thread t owning summation chains t, t + THREADS, ...
-// of the reference's 1024, so the sum has the reference's order without any regrouping. First pass: the row's maximum
-// after temperature, penalties and masks, and every thread's own largest value, from which the bound of the candidates
-// follows (the k-th largest of 256 joined thread maxima, each of them a column of its own). Second pass (the row
-// comes from the caches this time): e = T(exp(y - max)) summed chain by chain, candidates collected on the way. Then
+// and most compute units idle. Here THREADS threads share a row, thread t owning 1024 / THREADS neighbouring summation
+// chains of the reference's 1024, so the sum has the reference's order without any regrouping. First pass: the row's
+// maximum after temperature, penalties and masks, and every thread's own largest value, from which the bound of the
+// candidates follows (the k-th largest of 256 joined thread maxima, each of them a column of its own). Second pass (the
+// row comes from the caches this time): e = T(exp(y - max)) summed chain by chain. Then the candidates, out of the few
+// groups of vectors whose largest raw value reaches the bound. Then
 // all waves but four leave and those finish like lp_row_kernel (lp_finish).
 // THREADS = 1024 for launches of at most one row per compute unit; with more rows, workgroups of fewer threads share a
 // compute unit and one's first pass (memory) runs beside another's second (arithmetic).
@@ -888,16 +890,49 @@ constexpr int LPW_THREADS = 1024;
 #define LPW_STAMP(i)
 #endif
 
+// element i of an array in registers (the empty asm keeps the compiler from making it an array in memory)
+template<int N, class V>
+__device__ __forceinline__ V lp_pick(const V* from, int i)
+{
+    V x = from[0];
+#pragma unroll
+    for (int q = 1; q < N; ++q) {
+        x = i == q ? from[q] : x;
+        asm("" : "+v"(x));
+    }
+    return x;
+}
+
+// Whether any lane of the wave has it, in a branch that the whole wave takes: what it leads to is out of the way of the
+// straight line (a branch for some lanes would be jumped over by all others, at the cost of a fetch).
+__device__ __forceinline__ bool lp_rare(bool mine)
+{
+    return __builtin_expect(__ballot(mine) != 0ull, 0);
+}
+
+// Bound by the arithmetic of the second pass (vector instructions, and its waits where only eight waves share a compute
+// unit). 1024 x 152064 f16, k = 64: 166 us a step with every column through det_expf, columns one by one and candidates
+// looked for in both passes; 141 us now. 16-bit types hold their values in pairs and take det_expf only where the
+// hardware's exponential leaves the rounding open (ftk_exp16.cuh), the first pass looks at raw values alone, candidates
+// are looked for in some ninety groups of 64 columns, and flags of the history cost a bit test per sixteen columns. Other
+// sizes, us before / now: 256 x 152064 f16 53.7 / 48.7, 512 x 50257 f16 51.9 / 45.2, 1024 x 32000 bf16 56.6 / 43.5, 256 x
+// 128256 f16 with 2000 ids of history 70.8 / 58.1, 8 x 50257 f32 25.2 / 23.1, 400 x 152064 f32 96.0 / 91.7; rows that
+// exceed the last-level cache lose some of it to the second look at the groups (1024 x 152064 f32 206 / 213).
 template<int DT, int BMW, int THREADS>
 __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLaunch l, LogProbLaunch lp)
 {
     typedef Storage<DT>   S;
     typedef typename S::T T;
-    constexpr int         CH = LP_BLOCK / THREADS;  // chains of a thread
-    constexpr int         U  = 8 / CH;              // rounds (1024 columns each) of a thread's batch: 8 columns
-    constexpr int         N  = U * CH;
-    static_assert(THREADS * CH == LP_BLOCK && U * CH == 8 && THREADS % 32 == 0 && THREADS >= TK_THREADS,
+    constexpr bool        WORD16 = DT != DT_F32;
+    constexpr int         CH = LP_BLOCK / THREADS;     // neighbouring chains of a thread
+    constexpr int         N  = WORD16 ? 16 : 8;        // columns of a thread's batch
+    constexpr int         U  = N / CH;                 // ... in rounds of 1024 columns
+    constexpr int         NR = WORD16 && CH > 1 ? N / 2 : N;  // registers a batch is loaded into
+    constexpr int         NY = WORD16 ? N / 2 : N;            // ... and its values, 16-bit types in pairs
+    static_assert(THREADS * CH == LP_BLOCK && U * CH == N && THREADS % 32 == 0 && THREADS >= TK_THREADS,
                   "a workgroup owns all chains of its row");
+    typedef std::conditional_t<WORD16 && CH == 1, uint16_t, uint32_t> Raw;
+    typedef std::conditional_t<WORD16, uint32_t, float>               Val;
     __shared__ TopkShared s;
     __shared__ uint32_t   wide_key[THREADS];
     __shared__ uint32_t   slot_key[TK_THREADS];
@@ -914,8 +949,8 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     if constexpr (THREADS < LPW_THREADS) {
         __builtin_amdgcn_s_setprio(3);
     }
-    // slot j of a batch: round j / CH of the batch, chain (j % CH) * THREADS + t
-    auto offset_of = [](int j) { return (j / CH) * LP_BLOCK + (j % CH) * THREADS; };
+    // slot j of a batch: round j / CH of the batch, chain CH * t + j % CH
+    auto offset_of = [](int j) { return (j / CH) * LP_BLOCK + j % CH; };
     // First pass, for the maximum only: the order of the columns does not matter, so the row comes in as the 16-byte
     // vectors of the memory, thread t taking vectors vlo + t, vlo + t + THREADS, ... (`a` columns of the row's first
     // vector lie in front of the row; what lies in front of vector vlo and behind vector vhi is looked at column by
@@ -930,8 +965,9 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     const int     turns = (nvec + THREADS - 1) / THREADS;
     // (the history before them: its ids are scattered reads that nothing should queue behind)
     constexpr int HU   = 2048 / THREADS;
-    const bool    hist = BMW > 0 && p.bitmaps != nullptr && p.penalties != nullptr;
+    const bool    hist = p.bitmaps != nullptr && p.penalties != nullptr;
     int           hist_ids[HU];
+    T             hist_raw[HU];
     if (hist) {
 #pragma unroll
         for (int i = 0; i < HU; ++i) {
@@ -949,11 +985,12 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     }
     // Second pass: thread t takes columns of its own chains, batches of N
     const int nfull = p.V / (U * LP_BLOCK);  // batches that every thread holds in full
-    T         buf[2][N];
-    auto      load = [&](T* raw, int b) {
+    constexpr int R2 = WORD16 && CH > 1 ? 4 : 2;  // batches in registers, the one in use included
+    Raw       buf[R2][NR];
+    auto      load = [&](Raw* raw, int b) {
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            raw[j] = rowp[b * U * LP_BLOCK + offset_of(j) + t];
+        for (int r = 0; r < U; ++r) {
+            __builtin_memcpy(raw + r * (NR / U), rowp + (b * U + r) * LP_BLOCK + CH * t, CH * sizeof(T));
         }
     };
     const bool            skip = row_flag_or(p.skip_decode, row, p.end_ids + row, false);
@@ -972,22 +1009,36 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         return;
     }
     if (t == 0) {
-        s.n_cand = 0;
+        s.n_cand  = 0;
+        s.misc[1] = 0;  // groups of vectors kept in mind
     }
     const TopkOutputs out =
         topk_outputs(l.ids, l.sequence_length, l.finished, lp.cum_log_probs, lp.output_log_probs, row, p.end_ids);
+    // (the first and last columns of a row, outside its whole vectors, are nobody's: at >= 0 && at < nvec fails)
+    uint32_t own_flags = 0u;  // bit b % 32: a column of the thread's batch b has a value of its own
+    auto     flag_of   = [&](int v) { return 1u << ((v / (U * LP_BLOCK)) & 31); };
+    auto     owner_of  = [&](int v) { return (v & (LP_BLOCK - 1)) / CH; };
     if (hist) {
-        // the row's history bitmap in LDS (launches with a window and a history penalty)
-        uint32_t* window = fused_lds_bitmap<FusedRow<DT, BMW>::LDS_WORDS>();
-        const int words  = min(FusedRow<DT, BMW>::LDS_WORDS, (p.V + 31) / 32 + 1);
-        for (int i = t; i < words; i += THREADS) {
-            window[i] = 0u;
+        // which columns of the row are in its history: a bitmap in LDS (launches with a window; others have one in
+        // memory), and per thread which of its batches hold one
+        wide_key[t] = 0u;
+        if constexpr (BMW > 0) {
+            uint32_t* window = fused_lds_bitmap<FusedRow<DT, BMW>::LDS_WORDS>();
+            const int words  = min(FusedRow<DT, BMW>::LDS_WORDS, (p.V + 31) / 32 + 1);
+            for (int i = t; i < words; i += THREADS) {
+                window[i] = 0u;
+            }
+            rowctx.bm_mode   = 1;
+            rowctx.bm_origin = 0;
         }
         __syncthreads();
         auto mark = [&](int pos, int id) {
             id -= p.col_offset;
             if (id >= 0 && id < p.V && rowctx.history_position_counts(pos)) {
-                atomicOr(&window[id >> 5], 1u << (id & 31));
+                if constexpr (BMW > 0) {
+                    atomicOr(&fused_lds_bitmap<FusedRow<DT, BMW>::LDS_WORDS>()[id >> 5], 1u << (id & 31));
+                }
+                atomicOr(&wide_key[owner_of(id)], flag_of(id));
             }
         };
 #pragma unroll
@@ -999,45 +1050,103 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         for (int pos = t + HU * THREADS; pos < p.step; pos += THREADS) {
             mark(pos, p.output_ids[(size_t)pos * p.batch_size + row]);
         }
-        rowctx.bm_mode   = 1;
-        rowctx.bm_origin = 0;
+#pragma unroll
+        for (int i = 0; i < HU; ++i) {  // what the columns of the history hold, for the maximum
+            hist_raw[i] = rowp[min(max(hist_ids[i] - p.col_offset, 0), p.V - 1)];
+        }
     }
     __syncthreads();
+    if (hist) {
+        own_flags = wide_key[t];
+    }
+    if (rowctx.masked_end_id >= 0 && rowctx.masked_end_id < p.V && owner_of(rowctx.masked_end_id) == t) {
+        own_flags |= flag_of(rowctx.masked_end_id);
+    }
+    // visit(v, raw) for the columns of the history and the masked end id, by whichever thread
+    auto for_special = [&](auto&& visit) {
+        if (hist) {
+#pragma unroll
+            for (int i = 0; i < HU; ++i) {
+                const int id = hist_ids[i] - p.col_offset;
+                if (hist_ids[i] >= 0 && id >= 0 && id < p.V && rowctx.history_position_counts(t + i * THREADS)) {
+                    visit(id, hist_raw[i]);
+                }
+            }
+#pragma unroll 1
+            for (int pos = t + HU * THREADS; pos < p.step; pos += THREADS) {
+                const int id = p.output_ids[(size_t)pos * p.batch_size + row] - p.col_offset;
+                if (id >= 0 && id < p.V && rowctx.history_position_counts(pos)) {
+                    visit(id, rowp[id]);
+                }
+            }
+        }
+        if (t == 0 && rowctx.masked_end_id >= 0 && rowctx.masked_end_id < p.V) {
+            visit(rowctx.masked_end_id, rowp[rowctx.masked_end_id]);
+        }
+    };
     LPW_STAMP(1)
     const uint32_t KMIN    = min_valid_key<DT>();
     const float    NEG_INF = -__builtin_inff();
-    // The values of a batch's columns (v0 = the first one's, t included) after temperature, history penalty and the
-    // min-length mask. A column's history flag is bit t % 32 of word v / 32 of the bitmap. The words of a batch are
-    // read together, and one look tells whether any of its columns needs more than the multiplication.
+    // The values of a batch's columns (v0 = the first one) after temperature, history penalty and the min-length mask.
+    // Batches without a flag need no more than the multiplication. `whole`: all columns lie in the row.
     const bool bitsv = rowctx.has_vector_bits();
-    const int  bsh   = t & 31;
-    auto values = [&](int v0, const T* raw, float* y) {
-        uint32_t w[N];
-        uint32_t any = 0u;
-        if (bitsv) {
+    auto values = [&](auto whole, int v0, const Raw* raw, Val* y) __attribute__((always_inline)) {
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                w[j] = rowctx.bm_word((v0 + offset_of(j)) >> 5);
+        for (int i = 0; i < NY; ++i) {
+            if constexpr (!WORD16) {
+                y[i] = rowctx.fast(u2f(raw[i]));
             }
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                any |= w[j];
-            }
-            any = (any >> bsh) & 1u;
-        }
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            y[j] = rowctx.fast(S::ld(raw[j]));
-        }
-        const uint32_t to_end = (uint32_t)(rowctx.masked_end_id - v0);  // offset_of(j) for the masked end id at slot j
-        if (any != 0u || (to_end < (uint32_t)(U * LP_BLOCK) && (to_end & (THREADS - 1)) == 0u)) {  // rare
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                if (bitsv && ((w[j] >> bsh) & 1u)) {
-                    y[j] = rowctx.flagged(y[j], v0 + offset_of(j));
+            else {
+                uint32_t pair;
+                if constexpr (CH == 1) {
+                    pair = (uint32_t)raw[2 * i] | ((uint32_t)raw[2 * i + 1] << 16);
                 }
-                if (to_end == (uint32_t)offset_of(j)) {
-                    y[j] = -S::max_t();
+                else {
+                    pair = raw[i];
+                }
+                y[i] = ExpPairs<DT>::scale(pair, rowctx.fast_mul);
+            }
+        }
+        if (lp_rare((own_flags & flag_of(v0)) != 0u)) {
+            const uint32_t to_end = (uint32_t)(rowctx.masked_end_id - v0);  // offset_of(j) for the masked end id at slot j
+            const int      bsh    = v0 & 31;  // (a thread's columns of a round are neighbouring bits of one word)
+            uint32_t       special, flags = 0u;
+            if (bitsv) {
+#pragma unroll
+                for (int r = 0; r < U; ++r) {
+                    const int at = (v0 >> 5) + r * (LP_BLOCK / 32);
+                    flags |= ((rowctx.bm_word(decltype(whole)::value ? at : min(at, p.V >> 5)) >> bsh) & ((1u << CH) - 1u))
+                             << (r * CH);
+                }
+            }
+            special = flags;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                special |= to_end == (uint32_t)offset_of(j) ? 1u << j : 0u;
+            }
+            while (special != 0u) {  // (a slot per lane and turn: one or two turns as a rule)
+                const int j = __builtin_ctz(special), v = v0 + offset_of(j);
+                special &= special - 1u;
+                if constexpr (!WORD16) {
+                    float x = lp_pick<N>(y, j);
+                    x       = (flags >> j) & 1u ? rowctx.flagged(x, v) : x;
+                    x       = to_end == (uint32_t)offset_of(j) ? -S::max_t() : x;
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        y[i] = i == j ? x : y[i];
+                    }
+                }
+                else {
+                    const uint32_t pair  = lp_pick<NY>(y, j >> 1);
+                    const int      shift = 16 * (j & 1);
+                    float          x     = S::ld((T)(pair >> shift));
+                    x                    = (flags >> j) & 1u ? rowctx.flagged(x, v) : x;
+                    x                    = to_end == (uint32_t)offset_of(j) ? -S::max_t() : x;
+                    const uint32_t other = (pair & (0xFFFF0000u >> shift)) | ((uint32_t)S::st(x) << shift);
+#pragma unroll
+                    for (int i = 0; i < NY; ++i) {
+                        y[i] = i == j >> 1 ? other : y[i];
+                    }
                 }
             }
         }
@@ -1050,76 +1159,215 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         }
         return v == rowctx.masked_end_id ? -S::max_t() : y;
     };
-    // The second pass over the row: whole batches with the next one's loads issued before the current one is used,
-    // then the columns behind them one by one, loaded together.
-    // use_batch(v0, y) takes a batch's values, use_one(j, v, y) the value of column v at slot j.
-    auto stream = [&](auto&& use_batch, auto&& use_one) {
-        if (nfull > 0) {
-            load(buf[0], 0);
-        }
-        auto batch = [&](const T* raw, int b) {
-            float     y[N];
-            const int v0 = b * U * LP_BLOCK + t;
-            values(v0, raw, y);
-            use_batch(v0, y);
-        };
-        // (every load is issued whatever the batch, one past the last fetches the last again, unused: with the same
-        // number of loads on every path the waits can name the older batch instead of everything in flight)
-        for (int b = 0; b < nfull; b += 2) {
-            load(buf[1], min(b + 1, nfull - 1));
-            batch(buf[0], b);
-            load(buf[0], min(b + 2, nfull - 1));
-            if (b + 1 < nfull) {
-                batch(buf[1], b + 1);
-            }
-        }
-        const int v0 = nfull * U * LP_BLOCK + t;
-        if (v0 < p.V) {
-            T raw[N];
+    // The values of any batch of the row, -inf behind its end.
+    auto some_values = [&](int v0, Val* y) __attribute__((always_inline)) {
+        Raw raw[NR];
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                raw[j] = rowp[min(v0 + offset_of(j), p.V - 1)];
-            }
+        for (int r = 0; r < U; ++r) {
+            T         one[CH];
+            const int v = v0 + r * LP_BLOCK;
+            __builtin_memcpy(one, rowp + min(v, p.V - CH), CH * sizeof(T));
+            if (CH > 1 && v < p.V && v + CH > p.V) {  // (one thread at most)
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                if (v0 + offset_of(j) < p.V) {
-                    use_one(j, v0 + offset_of(j), value(v0 + offset_of(j), raw[j]));
+                for (int c = 0; c < CH; ++c) {
+                    one[c] = rowp[min(v + c, p.V - 1)];
+                }
+            }
+            __builtin_memcpy(raw + r * (NR / U), one, CH * sizeof(T));
+        }
+        values(std::false_type(), v0, raw, y);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            if (v0 + offset_of(j) >= p.V) {
+                if constexpr (!WORD16) {
+                    y[j] = NEG_INF;
+                }
+                else {
+                    const uint32_t none = S::st(NEG_INF);
+                    y[j / 2] = j % 2 == 0 ? (y[j / 2] & 0xFFFF0000u) | none : (y[j / 2] & 0xFFFFu) | (none << 16);
                 }
             }
         }
     };
+    // The second pass over the row: whole batches with the next one's loads issued before the current one is used,
+    // then the columns behind them in a batch that ends with -inf. use_batch(y, rounds) takes a batch's values, as
+    // many rounds of them as there are.
+    auto stream = [&](auto&& use_batch) {
+        if (nfull > 0) {
+#pragma unroll
+            for (int r = 0; r < R2 - 1; ++r) {
+                load(buf[r], min(r, nfull - 1));
+            }
+        }
+        // (every load is issued whatever the batch, one past the last fetches the last again, unused: with the same
+        // number of loads on every path the waits can name the older batch instead of everything in flight)
+        for (int b0 = 0; b0 < nfull; b0 += R2) {
+#pragma unroll
+            for (int r = 0; r < R2; ++r) {
+                load(buf[(r + R2 - 1) % R2], min(b0 + r + R2 - 1, nfull - 1));
+                if (b0 + r < nfull) {
+                    Val       y[NY];
+                    const int v0 = (b0 + r) * U * LP_BLOCK + CH * t;
+                    values(std::true_type(), v0, buf[r], y);
+                    use_batch(y, U);
+                }
+            }
+        }
+        const int rest = p.V - nfull * U * LP_BLOCK;
+        if (rest > 0) {
+            Val       y[NY];
+            const int v0 = nfull * U * LP_BLOCK + CH * t;
+            some_values(v0, y);
+            use_batch(y, (rest + LP_BLOCK - 1) / LP_BLOCK);
+        }
+    };
 
     // ---- first pass: the maximum (pad columns count as -MAX_T), and the thread's own
-    float m = NEG_INF;
-    {
-        const float mul     = rowctx.fast_mul;
-        const bool  ordered = mul > 0.0f && mul < __builtin_inff();  // the plain transform keeps the order
+    // The plain transform keeps the order, so a thread's maximum is that of its raw values - columns of the history and
+    // the masked end id apart, which have values of their own. Looking for them vector by vector costs more than the
+    // maximum itself; instead every history id looks whether its raw value is the largest of the thread that owns its
+    // column. Such a thread says nothing about its columns (nothing follows for the candidates' bound), unless its raw
+    // maximum lies above everything else: then a wave goes through its vectors with the flags at hand.
+    // The maxima of groups of a thread's vectors stay behind in the candidates' array: once the bound is there they tell
+    // which groups to look into for candidates.
+    constexpr int GROUPS = 2 * TK_CCAP / THREADS;  // per thread
+    const float   mul     = rowctx.fast_mul;
+    const bool    ordered = mul > 0.0f && mul < __builtin_inff();  // the plain transform keeps the order
+    int           glog    = 3;                                     // log2 of the turns of a group
+    while ((GROUPS << glog) < turns) {
+        ++glog;
+    }
+    float* group_max = reinterpret_cast<float*>(&s.cand);  // [group][thread]
+    static_assert(sizeof(s.cand) >= GROUPS * THREADS * sizeof(float) && R1 == 8, "a group is a whole number of rings");
+    float m       = NEG_INF;
+    float raw_own = NEG_INF;
+    if (ordered) {
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        float group = NEG_INF;
+        auto  ring_of = [&](auto last, int q0) {  // `last`: not every thread has all of these vectors
+            const _Float16 low  = -__builtin_inff16();
+            f16x2          pair = {low, low};
+            float          most = NEG_INF;
+#pragma unroll
+            for (int r = 0; r < R1; ++r) {
+                if (!decltype(last)::value || (q0 + r) * THREADS + t < nvec) {
+                    const uint4& v = ring[r];
+                    if constexpr (DT == DT_F16) {
+                        const f16x2 x = __builtin_bit_cast(f16x2, v.x), y = __builtin_bit_cast(f16x2, v.y);
+                        const f16x2 z = __builtin_bit_cast(f16x2, v.z), w = __builtin_bit_cast(f16x2, v.w);
+                        pair = __builtin_elementwise_max(
+                            __builtin_elementwise_max(pair, __builtin_elementwise_max(x, y)),
+                            __builtin_elementwise_max(z, w));
+                    }
+                    else {
+                        most = __builtin_fmaxf(most, lean_raw_max<DT>(v));
+                    }
+                }
+                vload(r, q0 + r + R1);
+            }
+            if constexpr (DT == DT_F16) {
+                most = __builtin_fmaxf((float)pair.x, (float)pair.y);
+            }
+            group   = __builtin_fmaxf(group, most);
+            raw_own = __builtin_fmaxf(raw_own, most);
+            if (((q0 + R1) & ((1 << glog) - 1)) == 0 || q0 + R1 >= turns) {
+                group_max[(q0 >> glog) * THREADS + t] = group;
+                group                                 = NEG_INF;
+            }
+        };
+        int q0 = 0;
+        for (; (q0 + R1) * THREADS <= nvec; q0 += R1) {
+            ring_of(std::false_type(), q0);
+        }
+        if (q0 < turns) {
+            ring_of(std::true_type(), q0);
+        }
+    }
+    else {
         for (int q0 = 0; q0 < turns; q0 += R1) {
 #pragma unroll
             for (int r = 0; r < R1; ++r) {
-                const int q = q0 + r;
-                if (q < turns) {
-                    const int   rel = q * THREADS + t;
-                    const float vm  = lp_vector_max<DT, BMW>(rowctx, ring[r], (vlo + min(rel, nvec - 1)) * EPV - a, a,
+                const int rel = (q0 + r) * THREADS + t;
+                if (q0 + r < turns) {
+                    const float vm = lp_vector_max<DT, BMW>(rowctx, ring[r], (vlo + min(rel, nvec - 1)) * EPV - a, a,
                                                             bitsv, ordered);
-                    m               = __builtin_fmaxf(m, rel < nvec ? vm : NEG_INF);
+                    m              = __builtin_fmaxf(m, rel < nvec ? vm : NEG_INF);
                 }
-                vload(r, q + R1);
+                vload(r, q0 + r + R1);
             }
         }
-        // the columns in front of the first whole vector and behind the last
+    }
+    // the columns in front of the first whole vector and behind the last
+    auto for_outer = [&](auto&& visit) {
         for (int v = t; v < min(p.V, vlo * EPV - a); v += THREADS) {
-            m = __builtin_fmaxf(m, value(v, rowp[v]));
+            visit(v);
         }
         for (int v = vhi * EPV - a + t; v < p.V; v += THREADS) {
-            m = __builtin_fmaxf(m, value(v, rowp[v]));
+            visit(v);
+        }
+    };
+    for_outer([&](int v) { m = __builtin_fmaxf(m, value(v, rowp[v])); });
+    float unsure = NEG_INF;  // an upper bound of this thread's columns where no more is known
+    float seen   = m;        // what counts for the row's maximum
+    // the vector of column v, counted from the row's first whole one
+    auto vector_of = [&](int v) { return (v + a) / EPV - vlo; };
+    if (ordered) {
+        wide_key[t] = f2u(raw_own);
+        if (t < THREADS / 32) {
+            slot_key[t] = 0u;  // bit t % 32 of word t / 32: thread t's raw maximum is a column with a value of its own
+        }
+        __syncthreads();
+        for_special([&](int v, T raw) {
+            const int at = vector_of(v), owner = at & (THREADS - 1);
+            if (at >= 0 && at < nvec && S::ld(raw) >= u2f(wide_key[owner])) {
+                atomicOr(&slot_key[owner >> 5], 1u << (owner & 31));
+            }
+            seen = __builtin_fmaxf(seen, value(v, raw));
+        });
+        __syncthreads();
+        const float top = rowctx.fast(raw_own);
+        if ((slot_key[t >> 5] >> (t & 31)) & 1u) {
+            unsure = top;
+        }
+        else {
+            m    = __builtin_fmaxf(m, top);
+            seen = __builtin_fmaxf(seen, top);
         }
     }
     LPW_STAMP(2)
     if (t == 0) {
         s.misc[0] = __float_as_int(row_uniform(l.rng, l.uniforms, row));  // (read behind the barriers of the sum)
     }
-    float row_max = block_max<float, THREADS / WAVE>(m, redf, NEG_INF);
+    seen   = wave_max(seen);
+    unsure = wave_max(unsure);
+    if (lane_id() == 0) {
+        redf[wave_id()]     = seen;
+        warp_sum[wave_id()] = unsure;
+    }
+    __syncthreads();
+    constexpr int NW      = THREADS / WAVE;
+    float         row_max = wave_max(lane_id() < NW ? redf[lane_id()] : NEG_INF);
+    if (wave_max(lane_id() < NW ? warp_sum[lane_id()] : NEG_INF) > row_max) {  // (the same for every wave)
+        // the vectors of the threads in question, one thread's by a wave (lane i looks at the marks of word i)
+        float          found = NEG_INF;
+        int            n     = 0;
+        const uint32_t marks = lane_id() < THREADS / 32 ? slot_key[lane_id()] : 0u;
+        for (unsigned long long words = __ballot(marks != 0u); words != 0ull; words &= words - 1ull) {
+            const int w = __builtin_ctzll(words);
+            for (uint32_t bits = (uint32_t)__shfl((int)marks, w, WAVE); bits != 0u; bits &= bits - 1u) {
+                const int who = w * 32 + __builtin_ctz(bits);
+                if (!(rowctx.fast(u2f(wide_key[who])) > row_max) || n++ % NW != wave_id()) {
+                    continue;
+                }
+                for (int rel = lane_id() * THREADS + who; rel < nvec; rel += WAVE * THREADS) {
+                    found = __builtin_fmaxf(found, lp_vector_max<DT, BMW>(rowctx, base[vlo + rel], (vlo + rel) * EPV - a,
+                                                                         a, bitsv, ordered));
+                }
+            }
+        }
+        __syncthreads();
+        row_max = __builtin_fmaxf(row_max, block_max<float, NW>(found, redf, NEG_INF));
+    }
     LPW_STAMP(3)
     row_max       = __builtin_fmaxf(-3.402823466e+38f, row_max);
     if (p.V < p.Vp) {
@@ -1149,6 +1397,46 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         valid         = true;
     }
 
+    // ---- where the candidates are: groups of vectors with a raw value that the bound does not rule out
+    // (the list lies where the selection keeps its own later on)
+    int*      parked    = s.sel.idx;
+    float     raw_floor = NEG_INF;
+    bool      raises    = false;  // the history penalty raises values
+    if (valid && ordered) {
+        // an unflagged column with e >= thr_low has at least this raw value (e's rounding, the logarithm's, y's)
+        const float rounding = DT == DT_F32 ? 0.99999f : (DT == DT_F16 ? (thr_low < 2.44140625e-04f ? 0.4f : 0.998f) : 0.98f);
+        float       y        = row_max + det_logf(thr_low * rounding);
+        y                    = lean_below_rounding<DT>(y - __builtin_fabsf(row_max) * 1e-6f - 1e-5f) / mul;
+        y                    = y - __builtin_fabsf(y) * 1e-6f;
+        raw_floor            = uniform_f(y < 3.0e38f ? y : NEG_INF);
+        uint32_t mine        = 0u;
+        for (int g = 0; g << glog < turns; ++g) {
+            mine |= (group_max[g * THREADS + t] >= raw_floor ? 1u : 0u) << g;
+        }
+        // (a penalty that raises values: the columns of the history can reach the bound from any raw value)
+        raises = hist && !(p.penalty_type == 0 ? rowctx.penalty >= 0.0f : rowctx.penalty >= 1.0f);
+        if (raises) {
+            __syncthreads();
+            wide_key[t] = mine;
+            __syncthreads();
+            for_special([&](int v, T) {
+                const int at = vector_of(v);
+                if (at >= 0 && at < nvec) {
+                    atomicOr(&wide_key[at & (THREADS - 1)], 1u << ((at / THREADS) >> glog));
+                }
+            });
+            __syncthreads();
+            mine = wide_key[t];
+        }
+        while (mine != 0u) {
+            const int g    = __builtin_ctz(mine);
+            const int slot = atomicAdd(&s.misc[1], 1);
+            if (slot < TK_CCAP) {
+                parked[slot] = (g << glog) * THREADS + t;  // the group's first vector
+            }
+            mine &= mine - 1u;
+        }
+    }
     LPW_STAMP(4)
     if constexpr (THREADS < LPW_THREADS) {
         __builtin_amdgcn_s_setprio(0);
@@ -1166,66 +1454,83 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             s.cand.idx[slot] = (uint32_t)v;
         }
     };
-    stream(
-        [&](int v0, const float* y) {
-            float d[N], e[N];
-            bool  number = true;  // one look for a NaN per pair of columns instead of one per column
+    const auto  ex   = [&] {
+        if constexpr (WORD16) {
+            return ExpPairs<DT>(row_max);
+        }
+        else {
+            return 0;
+        }
+    }();
+    // e of slots [j0, j0 + G) of a batch. 16-bit types: half a batch in a straight line, then one look for pairs that the
+    // hardware's exponential does not decide, and a closer one at four columns each (a wave alone waits for every branch).
+    constexpr int G = WORD16 ? 8 : 4;
+    auto numerators = [&](const Val* y, Val* e, int j0) __attribute__((always_inline)) {
+        if constexpr (!WORD16) {
+            float d[G];
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                d[j] = y[j] - row_max;
+            for (int j = 0; j < G; ++j) {
+                d[j] = y[j0 + j] - row_max;
             }
 #pragma unroll
-            for (int j = 0; j < N; j += 2) {
-                number = number && !__builtin_isunordered(d[j], d[j + 1]);
+            for (int j = 0; j < G; ++j) {
+                e[j0 + j] = det_expf_nonpos_number(d[j]);
             }
-            if (number) {
+            if (lp_rare(__builtin_isunordered(d[0], d[1]) || __builtin_isunordered(d[2], d[3]))) {
 #pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    e[j] = round_t<DT>(det_expf_nonpos_number(d[j]));
+                for (int j = 0; j < G; ++j) {
+                    e[j0 + j] = d[j] != d[j] ? d[j] : e[j0 + j];
                 }
             }
-            else {
+        }
+        else {
+            uint32_t redo[G / 4], any = 0u;
 #pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    e[j] = round_t<DT>(det_expf_nonpos(d[j]));
-                }
+            for (int i = 0; i < G / 4; ++i) {
+                redo[i] = ex.never;
+                e[j0 / 2 + 2 * i]     = ex(y[j0 / 2 + 2 * i], redo[i]);
+                e[j0 / 2 + 2 * i + 1] = ex(y[j0 / 2 + 2 * i + 1], redo[i]);
+                any |= redo[i];
             }
-            float top = e[0];
+            if (lp_rare(ex.undecided(any))) {
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                acc[j % CH] = acc[j % CH] + e[j];  // (slots of a chain in ascending order of their columns)
-                top         = __builtin_fmaxf(top, e[j]);
-            }
-            if (top >= thr_low) {  // (a NaN is no candidate, with or without the maximum)
-#pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    if (e[j] >= thr_low) {
-                        push(v0 + offset_of(j), e[j]);
+                for (int i = 0; i < G / 4; ++i) {
+                    if (lp_rare(ex.undecided(redo[i]))) {
+                        e[j0 / 2 + 2 * i]     = ex.exact(y[j0 / 2 + 2 * i]);
+                        e[j0 / 2 + 2 * i + 1] = ex.exact(y[j0 / 2 + 2 * i + 1]);
                     }
                 }
             }
-        },
-        [&](int j, int v, float y) {
-            const float e = round_t<DT>(det_expf_nonpos(y - row_max));
-            acc[j % CH]   = acc[j % CH] + e;
-            if (e >= thr_low) {
-                push(v, e);
-            }
-        });
-    if (p.V < p.Vp) {
-        // pad columns count once nothing of the vocabulary is far above -MAX_T (rows that are masked throughout)
-        const float pad_e = round_t<DT>(det_expf_nonpos(-S::max_t() - row_max));
-        if (pad_e > 0.0f) {
-#pragma unroll 1
-            for (int v = p.V + ((t - p.V) & (THREADS - 1)); v < p.Vp; v += THREADS) {
-                const int chain = (v & (LP_BLOCK - 1)) / THREADS;
+        }
+    };
+    stream([&](const Val* y, int rounds) {
 #pragma unroll
-                for (int c = 0; c < CH; ++c) {
-                    acc[c] = c == chain ? acc[c] + pad_e : acc[c];
+        for (int j0 = 0; j0 < N; j0 += G) {
+            if (j0 / CH < rounds) {  // (whole batches: always)
+                Val e[NY];
+                numerators(y, e, j0);
+                // (slots of a chain in ascending order of their columns)
+#pragma unroll
+                for (int j = j0; j < j0 + G; ++j) {
+                    if constexpr (!WORD16) {
+                        acc[j % CH] = acc[j % CH] + e[j];
+                    }
+                    else if (j % 2 == 0) {
+                        acc[j % CH]       = ex.add_low(acc[j % CH], e[j / 2]);
+                        acc[(j + 1) % CH] = ex.add_high(acc[(j + 1) % CH], e[j / 2]);
+                    }
                 }
-                if (pad_e >= thr_low) {
-                    push(v, pad_e);
-                }
+            }
+        }
+    });
+    const float pad_e = p.V < p.Vp ? round_t<DT>(det_expf_nonpos(-S::max_t() - row_max)) : 0.0f;
+    if (pad_e > 0.0f) {
+        // pad columns count once nothing of the vocabulary is far above -MAX_T (rows that are masked throughout)
+#pragma unroll 1
+        for (int v0 = (p.V & ~(LP_BLOCK - 1)) + CH * t; v0 < p.Vp; v0 += LP_BLOCK) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                acc[c] = v0 + c >= p.V && v0 + c < p.Vp ? acc[c] + pad_e : acc[c];
             }
         }
     }
@@ -1234,35 +1539,73 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         __builtin_amdgcn_s_setprio(3);
     }
     // the reference's order: xor butterflies inside 32-chain groups, then over the 32 group sums
+    // (chains that are CH or more apart belong to other lanes, nearer ones to the same thread)
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
+    for (int o = 16; o >= 1; o >>= 1) {
+        float other[CH];
 #pragma unroll
-        for (int o = 16; o >= 1; o >>= 1) {
-            acc[c] = acc[c] + __shfl_xor(acc[c], o, 32);
+        for (int c = 0; c < CH; ++c) {
+            other[c] = o >= CH ? __shfl_xor(acc[c], o >= CH ? o / CH : 0, 32) : acc[c ^ (o & (CH - 1))];
         }
-        if ((t & 31) == 0) {
-            warp_sum[(c * THREADS + t) >> 5] = acc[c];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            acc[c] = acc[c] + other[c];
         }
     }
-    __syncthreads();
-    if (t < 32) {
-        float total = warp_sum[t];
-#pragma unroll
-        for (int o = 16; o >= 1; o >>= 1) {
-            total = total + __shfl_xor(total, o, 32);
-        }
-        if (t == 0) {
-            warp_sum[0] = total;
-        }
+    if (((CH * t) & 31) == 0) {
+        warp_sum[(CH * t) >> 5] = acc[0];
     }
     __syncthreads();
-    const float denom = uniform_f(warp_sum[0] + 1e-6f);
+    float total = warp_sum[lane_id() & 31];
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) {
+        total = total + __shfl_xor(total, o, 32);
+    }
+    const float denom = uniform_f(total + 1e-6f);
     const float u     = __int_as_float(s.misc[0]);
-    int         n     = __builtin_amdgcn_readfirstlane(s.n_cand);
-    bool        probs = false;
+    // the candidates: the columns at or above the bound in the groups kept in mind (the whole row where raw values say
+    // nothing), a vector per thread and turn, and those outside the whole vectors
+    const int n_parked = __builtin_amdgcn_readfirstlane(s.misc[1]);
+    if (valid && n_parked <= TK_CCAP) {
+        auto consider = [&](int v) {
+            const float e = round_t<DT>(det_expf_nonpos(value(v, rowp[v]) - row_max));
+            if (e >= thr_low) {  // (a NaN is no candidate)
+                push(v, e);
+            }
+        };
+        const int vectors = ordered ? n_parked << glog : nvec;
+#pragma unroll 1
+        for (int i = t; i < vectors; i += THREADS) {
+            const int rel = ordered ? parked[i >> glog] + (i & ((1 << glog) - 1)) * THREADS : i;
+            if (rel < nvec) {
+                const uint4 v    = base[vlo + rel];
+                uint32_t    hits = 0u;
+#pragma unroll
+                for (int j = 0; j < EPV; ++j) {
+                    hits |= (!(vector_element<DT>(v, j) < raw_floor) ? 1u : 0u) << j;
+                }
+                if (raises) {
+                    hits = (1u << EPV) - 1u;
+                }
+                while (hits != 0u) {
+                    consider((vlo + rel) * EPV - a + __builtin_ctz(hits));
+                    hits &= hits - 1u;
+                }
+            }
+        }
+        for_outer(consider);
+        if (pad_e > 0.0f && pad_e >= thr_low) {
+            for (int v = p.V + t; v < p.Vp; v += THREADS) {
+                push(v, pad_e);
+            }
+        }
+    }
+    __syncthreads();
+    int  n     = __builtin_amdgcn_readfirstlane(s.n_cand);
+    bool probs = false;
     __syncthreads();
     const float e_bound = key_to_float(thr);
-    if (n > TK_CCAP || !valid || !lp_gather_covers<DT>(e_bound, denom)) {
+    if (n_parked > TK_CCAP || n > TK_CCAP || !valid || !lp_gather_covers<DT>(e_bound, denom)) {
         // (fewer than k columns with e > 0: columns of probability zero are picked too, by the reference's tie rules)
         probs = true;
         n     = lp_regather<DT, THREADS>(

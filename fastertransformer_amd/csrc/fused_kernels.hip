@@ -161,12 +161,12 @@ extern "C" int ftk_profile_read(int kernel, double* total_ms, int* launches)
     return 0;
 }
 
-// Threads per row of a log-prob step in one launch (lp_wide_kernel). Measured on MI355X (k = 64, us per step with 1024
-// / 512 / 256 threads per row; the two-launch form in brackets): 256 x 152064 f16 59 / 66 / 96 (129); 512 x 152064 f16
-// 109 / 96 / 110 (153); 1024 x 152064 f16 209 / 174 / 200 (218); 1024 x 128256 f32 206 / 177 / 217 (219); 1024 x 50264
-// f32 114 / 89 / 88 (111); 1024 x 32000 bf16 94 / 72 / 64; 8 x 50264 f32 28 / 33 / 47 (58). One workgroup per compute
-// unit wants all sixteen waves on its row; with more rows than compute units, two workgroups of eight waves overlap
-// one's reading with the other's arithmetic; many short rows do best with four of four.
+// Threads per row of a log-prob step in one launch (lp_wide_kernel). Measured on MI355X (us per step with 1024 / 512 /
+// 256 threads per row): 8 x 50257 f32 23.1 / 24.4 / 30.0; 64 x 32000 f32 23.3 / 23.4 / 28.4; 256 x 128256 f32 55 / 56 /
+// 68; 256 x 152064 f16 48 / 50 / 57; 300 x 32000 f32 41 / 28 / 30; 512 x 50257 f16 60 / 45 / 47; 512 x 50257 f32 68 / 54 /
+// 57; 1024 x 32000 bf16 85 / 54 / 44. One workgroup per compute unit wants all sixteen waves on its row; with more rows
+// than compute units, two workgroups of eight waves overlap one's reading with the other's arithmetic; many short rows do
+// best with four of four.
 static int lp_threads_per_row(int rows, int vocab_size)
 {
     if (rows <= 256) {

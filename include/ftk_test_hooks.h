@@ -22,6 +22,10 @@ void ftk_host_philox4x32_10(const uint32_t counter[4], const uint32_t key[2], ui
  * quotient by the shared-reciprocal sequence of the softmax, out[2j+1] = the ordinary division; n elements on
  * device */
 int ftk_test_device_math(int kind, const float* in, float* out, size_t n, ftk_stream_t stream);
+/* the rounded exponentials of the 16-bit softmax for every pair (y, max) of the type: adds to wrong[0] how many are not
+ * T(det_expf(y - max)) and to wrong[1] how many pairs of values the hardware's exponential did not decide; `wrong` is on
+ * the device */
+int ftk_test_exp_pairs(int dtype, unsigned long long* wrong, ftk_stream_t stream);
 /* draws `n_draws` uniforms per row into out[row*n_draws + i], advancing the states */
 int ftk_test_rng_uniform(ftk_rng_state* states, float* out, int batch_size, int n_draws, ftk_stream_t stream);
 /* non-zero: every top-p row takes the radix-sort fallback (exercises it on small inputs); process-wide */

@@ -85,8 +85,8 @@ def uniforms(rng, n):
 
 
 def run_fused_step(entry, torch, dt, B, V, H, k, logits, history, draws, finished0, seqlen0, lib=None, ws_fill=None,
-                   log_probs=None, Vp=None):
-    """One fused decode step straight through the C ABI (temperature 0.8, repetition penalty 1.1 over `history`,
+                   log_probs=None, Vp=None, penalty=1.1):
+    """One fused decode step straight through the C ABI (temperature 0.8, repetition penalty `penalty` over `history`,
     top-k `k`, top-p 0.9, injected draws). entry: "caller" = ftk_fused_topk_step with a workspace of the queried
     size, "static" = ftk_fused_topk_step_static. Returns (ids, sequence_length, finished, rc, needed bytes, change of
     the device's free memory across the static call). With a dict as `log_probs` the step also keeps log-probs:
@@ -101,7 +101,7 @@ def run_fused_step(entry, torch, dt, B, V, H, k, logits, history, draws, finishe
     finished = finished0.clone()
     seq = seqlen0.clone()
     temps = torch.full((B,), 0.8, device=dev)
-    pens = torch.full((B,), 1.1, device=dev)
+    pens = torch.full((B,), penalty, device=dev)
     end_ids = torch.full((B,), V - 1, dtype=torch.int32, device=dev)
     top_ks = torch.full((B,), k, dtype=torch.int32, device=dev)
     top_ps = torch.full((B,), 0.9, device=dev)

@@ -106,6 +106,19 @@ def test_device_exp_of_non_positive_arguments(env):
     assert np.isnan(to_numpy(out)[0])
 
 
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+def test_rounded_exponentials_of_every_pair(env, dt):
+    """The 16-bit softmax takes the hardware's exponential wherever its error cannot change the rounding to T: for every
+    maximum of the type and every value that is not above it, the bits of T(det_expf(y - max))."""
+    torch, _, ops = env
+    wrong = torch.zeros(2, dtype=torch.int64, device="cuda")
+    ops.check(ops.ftk_hooks().ftk_test_exp_pairs(dt, wrong.data_ptr(), ops.current_stream()))
+    _sync(torch)
+    bad, again = wrong.tolist()
+    assert bad == 0
+    assert 0 < again < (1 << 31)
+
+
 def test_device_division_by_a_shared_reciprocal(env):
     """The softmax divides a row by one denominator with the reciprocal's part of the division computed once:
     bit for bit numpy's IEEE quotient, for numerators over the whole range an exponential can take (zero,

@@ -88,6 +88,42 @@ def test_forms_of_the_log_prob_step_agree_bit_for_bit(dt, B, V, Vp, H, k, kind):
             assert np.array_equal(a, b), "%s differ between the two-launch form and %d threads per row" % (name, form)
 
 
+RAISING = [
+    (O.F16, 300, 33001, 33003, 600, 50, 0.7),   # a penalty that raises: columns of the history reach the bound from below
+    (O.F32, 9, 4999, 5001, 30, 30, 0.6),
+    (O.BF16, 5, 170000, 170000, 16, 64, 0.8),   # the history's bitmaps in memory; groups of sixteen vectors
+    (O.F16, 7, 20000, 20000, 5000, 40, 1.5),    # every fourth column or so in the history, more ids than threads hold
+]
+
+
+@pytest.mark.parametrize("dt,B,V,Vp,H,k,penalty", RAISING,
+                         ids=["%s-%dx%d-%g" % (DTYPE_NAMES[c[0]], c[1], c[2], c[6]) for c in RAISING])
+def test_forms_agree_whatever_the_penalty_does_to_the_largest_values(dt, B, V, Vp, H, k, penalty):
+    """The one-launch form takes a row's maximum from raw values and corrects it for the columns of the history."""
+    import torch
+    from fastertransformer_amd import ops
+    from helpers import run_fused_step
+    hooks = ops.ftk_hooks()
+    logits, history, draws, finished0, seqlen0 = _case(torch, dt, B, V, Vp, H, k, 77 + V, "normal")
+    order = logits[:, :V].float().argsort(dim=1, descending=True)
+    history[:H // 2] = order[:, 1::3][:, :H // 2].t().int()  # among the largest, but not all of them
+    history[0, ::2] = order[::2, 0].int()                    # and in every other row the largest itself
+    results = {}
+    try:
+        for form in FORMS:
+            hooks.ftk_test_set_lp_form(form)
+            lp = {}
+            out = run_fused_step("caller", torch, dt, B, V, H, k, logits, history, draws, finished0, seqlen0,
+                                 lib=hooks, log_probs=lp, Vp=Vp, penalty=penalty)
+            assert out[3] == 0 and hooks.ftk_test_last_fused_path() == 4
+            results[form] = (out[0], out[1], out[2], lp["cum"].view(np.uint32), lp["out"].view(np.uint32))
+    finally:
+        hooks.ftk_test_set_lp_form(0)
+    for form in FORMS[1:]:
+        for a, b in zip(results[FORMS[0]], results[form]):
+            assert np.array_equal(a, b), "%d threads per row" % form
+
+
 PEAKED = [
     (O.F16, 6, 9001, 9001, 64, "sharp"),    # k-th probability below binary16's normal range
     (O.F16, 4, 9001, 9008, 128, "sharper"),  # ... below its smallest number: zeros are picked, pads among them
