@@ -97,6 +97,43 @@ struct ExpPairs {
     {
         return pack(det_expf_nonpos(low(y) - max), det_expf_nonpos(high(y) - max));
     }
+    // e of P pairs, exactly: all of them in a straight line, then one look for pairs that are not decided, in a branch that
+    // the whole wave takes, and a closer one at two pairs each.
+    template<int P>
+    __device__ __forceinline__ void numerators(const uint32_t* y, uint32_t* e) const
+    {
+        static_assert(P % 2 == 0, "two pairs at a time");
+        uint32_t redo[P / 2], any = 0u;
+#pragma unroll
+        for (int i = 0; i < P / 2; ++i) {
+            redo[i]      = never;
+            e[2 * i]     = (*this)(y[2 * i], redo[i]);
+            e[2 * i + 1] = (*this)(y[2 * i + 1], redo[i]);
+            any |= redo[i];
+        }
+        if (__builtin_expect(__ballot(undecided(any)) != 0ull, 0)) {
+#pragma unroll
+            for (int i = 0; i < P / 2; ++i) {
+                if (DT == DT_BF16 && never == 0u) {
+                    // masked columns: -inf has e = 0, whatever the absolute part of the bounds says
+                    const uint32_t a = infinite(y[2 * i]), b = infinite(y[2 * i + 1]);
+                    e[2 * i] &= ~a;
+                    e[2 * i + 1] &= ~b;
+                    redo[i] &= ~(a & b);
+                }
+                if (__ballot(undecided(redo[i])) != 0ull) {
+                    e[2 * i]     = exact(y[2 * i]);
+                    e[2 * i + 1] = exact(y[2 * i + 1]);
+                }
+            }
+        }
+    }
+    // all ones in the halves that are -inf
+    static __device__ __forceinline__ uint32_t infinite(uint32_t y)
+    {
+        const uint32_t x = Storage<DT>::st(-__builtin_inff());
+        return ((y & 0xFFFFu) == x ? 0xFFFFu : 0u) | ((y >> 16) == x ? 0xFFFF0000u : 0u);
+    }
     // sum + the first / second value of a pair, rounded once
     __device__ __forceinline__ float add_low(float sum, uint32_t e) const
     {

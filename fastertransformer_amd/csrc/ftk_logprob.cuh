@@ -1462,8 +1462,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             return 0;
         }
     }();
-    // e of slots [j0, j0 + G) of a batch. 16-bit types: half a batch in a straight line, then one look for pairs that the
-    // hardware's exponential does not decide, and a closer one at four columns each (a wave alone waits for every branch).
+    // e of slots [j0, j0 + G) of a batch. 16-bit types: half a batch in a straight line (a wave waits for every branch).
     constexpr int G = WORD16 ? 8 : 4;
     auto numerators = [&](const Val* y, Val* e, int j0) __attribute__((always_inline)) {
         if constexpr (!WORD16) {
@@ -1484,23 +1483,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             }
         }
         else {
-            uint32_t redo[G / 4], any = 0u;
-#pragma unroll
-            for (int i = 0; i < G / 4; ++i) {
-                redo[i] = ex.never;
-                e[j0 / 2 + 2 * i]     = ex(y[j0 / 2 + 2 * i], redo[i]);
-                e[j0 / 2 + 2 * i + 1] = ex(y[j0 / 2 + 2 * i + 1], redo[i]);
-                any |= redo[i];
-            }
-            if (lp_rare(ex.undecided(any))) {
-#pragma unroll
-                for (int i = 0; i < G / 4; ++i) {
-                    if (lp_rare(ex.undecided(redo[i]))) {
-                        e[j0 / 2 + 2 * i]     = ex.exact(y[j0 / 2 + 2 * i]);
-                        e[j0 / 2 + 2 * i + 1] = ex.exact(y[j0 / 2 + 2 * i + 1]);
-                    }
-                }
-            }
+            ex.template numerators<G / 2>(y + j0 / 2, e + j0 / 2);
         }
     };
     stream([&](const Val* y, int rounds) {
