@@ -445,7 +445,6 @@ struct TopPScan {
     uint32_t           red32[16];
     float              agg[TP_ROUND];
     float              carry[TP_ROUND + 1];
-    uint32_t           tilemask[32][8];
     int                wtot[256];
     int                misc[8];
     float              fmisc[4];
@@ -473,6 +472,26 @@ __device__ __forceinline__ void tile_load(const unsigned long long* __restrict__
     }
 }
 
+// x of the lane `D` lanes below within a 32-lane group, for lanes that have one (others get something): shifts inside
+// rows of 16 lanes, and across rows the other row's value, rotated. Vector instructions, where a shuffle goes through LDS.
+template<int D>
+__device__ __forceinline__ float group_shift_up(float x, int l)
+{
+    static_assert(D == 1 || D == 2 || D == 4 || D == 8 || D == 16, "shifts of the raking");
+    constexpr int ROW_SHR = 0x110, ROW_ROR = 0x120;
+    const int     bits = __float_as_int(x);
+    // (v_permlane16_swap: its first result holds, in odd rows of 16 lanes, the even row in front of them)
+    if constexpr (D == 16) {
+        return __int_as_float((int)__builtin_amdgcn_permlane16_swap((unsigned)bits, (unsigned)bits, false, false)[0]);
+    }
+    else {
+        const int within = __builtin_amdgcn_update_dpp(bits, bits, ROW_SHR + D, 0xF, 0xF, false);
+        const int turned = __builtin_amdgcn_update_dpp(bits, bits, ROW_ROR + D, 0xF, 0xF, false);
+        const int across = (int)__builtin_amdgcn_permlane16_swap((unsigned)turned, (unsigned)turned, false, false)[0];
+        return __int_as_float((l & 15) >= D ? within : across);
+    }
+}
+
 // Inclusive raking scan of the lane totals of a tile.
 __device__ __forceinline__ float tile_scan(const float x[8], int l)
 {
@@ -482,13 +501,18 @@ __device__ __forceinline__ float tile_scan(const float x[8], int l)
         seg = seg + x[j];
     }
     float incl = seg;
-#pragma unroll
-    for (int d = 1; d < 32; d <<= 1) {
-        const float up = __shfl_up(incl, d, 32);
-        if (l >= d) {
+    auto  step = [&](auto d) {
+        constexpr int D  = decltype(d)::value;
+        const float   up = group_shift_up<D>(incl, l);
+        if (l >= D) {
             incl = up + incl;
         }
-    }
+    };
+    step(std::integral_constant<int, 1>());
+    step(std::integral_constant<int, 2>());
+    step(std::integral_constant<int, 4>());
+    step(std::integral_constant<int, 8>());
+    step(std::integral_constant<int, 16>());
     return incl;
 }
 
@@ -510,29 +534,35 @@ __device__ __forceinline__ int scan_tiles(TopPScan& s, int nt, float rand_num, L
         const int ntr = min(TP_ROUND, nt - base);
         totals(base, ntr);
         __syncthreads();
-        if (t == 0) {
-            // the additions depend on each other, the loads do not: eight totals are fetched at a time
+        if (t < WAVE) {
+            // The additions depend on each other, nothing else does: a lane holds a total, the running sum takes them one
+            // after the other out of the lanes (244 tiles: 2 us, 6 us with the totals read and the sums written in memory
+            // by one thread).
             float c  = carry_in;
             int   g0 = -1;
-            for (int g = 0; g < ntr; g += 8) {
-                float a[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    a[j] = s.agg[g + j];  // TP_ROUND is a multiple of 8; entries from ntr on are not used
+            for (int g = 0; g < ntr; g += WAVE) {
+                const bool  mine = g + t < ntr;
+                const float a    = mine ? s.agg[g + t] : 0.0f;
+                const int   n    = min(WAVE, ntr - g);
+                float       before = 0.0f;
+#pragma unroll 8
+                for (int j = 0; j < n; ++j) {
+                    before = t == j ? c : before;
+                    c      = c + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), j));
                 }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if (g + j < ntr) {
-                        s.carry[g + j] = c;
-                        c              = c + a[j];
-                        if (g0 < 0 && c >= near) {
-                            g0 = g + j;
-                        }
-                    }
+                if (mine) {
+                    s.carry[g + t] = before;
+                }
+                const unsigned long long reach = __ballot(mine && before + a >= near);
+                if (g0 < 0 && reach != 0ull) {
+                    g0 = g + __builtin_ctzll(reach);
                 }
             }
-            s.carry[ntr] = c;
-            s.misc[1]    = g0;
+            if (t == 0) {
+                s.carry[ntr] = c;
+                s.misc[0]    = 0x7FFFFFFF;
+                s.misc[1]    = g0;
+            }
         }
         __syncthreads();
         const int g0 = s.misc[1];
@@ -555,25 +585,22 @@ __device__ __forceinline__ int scan_tiles(TopPScan& s, int nt, float rand_num, L
                         }
                     }
                 }
-                reinterpret_cast<unsigned char*>(&s.tilemask[group][0])[l] = (unsigned char)m8;
-                __syncthreads();
-                if (t == 0) {
-                    int found = -1;
-                    for (int q = 0; q < TP_THREADS / 32 && found < 0; ++q) {
-                        for (int w = 0; w < 8; ++w) {
-                            const uint32_t mk = s.tilemask[q][w];
-                            if (mk != 0u) {
-                                found = (base + gs + q) * TP_TILE + w * 32 + (32 - __popc(mk));
-                                break;
-                            }
-                        }
+                // the reference looks at words of 32 positions, four lanes here: the first that holds a crossing counts
+                // from its end
+                int c = __popc(m8);
+                c += dpp_from<DPP_QUAD_XOR1>(c);
+                c += dpp_from<DPP_QUAD_XOR2>(c);
+                const uint32_t lanes = (uint32_t)(__ballot(m8 != 0u) >> (lane_id() & 32));
+                if (lanes != 0u) {
+                    const int first = __builtin_ctz(lanes) >> 2;
+                    if (l == first * 4) {
+                        atomicMin(&s.misc[0], (base + g) * TP_TILE + first * 32 + (32 - c));
                     }
-                    s.misc[0] = found;
                 }
                 __syncthreads();
                 const int found = s.misc[0];
                 __syncthreads();
-                if (found >= 0) {
+                if (found != 0x7FFFFFFF) {
                     return found;
                 }
             }

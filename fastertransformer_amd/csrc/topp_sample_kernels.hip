@@ -1525,7 +1525,7 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     __shared__ uint32_t           wcnt[TW], wrun[TW], wpick[NW];
     __shared__ float              wmass[TW];
     __shared__ uint32_t           sh_enough, key_lo, key_hi;
-    __shared__ int                sh_found, code_lo, code_hi, sh_nth;
+    __shared__ int                sh_found, code_lo, code_hi, sh_nth, sh_mixed;
     const int       row = blockIdx.x;
     const int       t   = threadIdx.x;
     ToppPickRow<DT> r(s, o, row, s.splits);
@@ -1662,7 +1662,6 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     }
     __syncthreads();
     const int enough = (int)min(n, sh_enough);
-
     // Whether the runs hold every positive probability: binary16's counters resolve all values of e, bfloat16's leave out
     // what lies below 2^-31.
     const bool complete = DT == DT_F16 || n == (uint32_t)s.Vp;
@@ -1714,37 +1713,52 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
                 int       lo = run_at(min(i0, (int)n - 1));
                 values_from(i0, lo, x);
             };
-            // A 32-lane group takes neighbouring tiles: the next one goes on in the run where the one before stopped,
-            // and whole tiles of one run have one total.
+            // Tiles inside one run first, a thread each: the scan of 256 equal values ends with 32 times what a lane adds up
+            // (every step of the raking doubles). The others go to 32-lane groups. (128 x 152064 bf16, a draw behind 62437 entries: 29 us
+            // for the scan with tiles dealt out in order and runs walked one by one, 16 us.)
             auto totals = [&](int base, int count) {
-                const int l   = t & 31, per = (count + TP_THREADS / 32 - 1) / (TP_THREADS / 32);
-                const int t0  = base + min(count, (t >> 5) * per), t1 = min(base + count, t0 + per);
-                float*    agg = sc.agg - base;
-                if (t0 >= t1) {
-                    return;
+                const int l = t & 31;
+                if (t == 0) {
+                    sh_mixed = 0;
                 }
-                int   lo    = run_at(min(t0 * TP_TILE + l * 8, (int)n - 1));
-                int   known = -1;  // run whose whole tiles' total is `total`
-                float total = 0.0f;
-                for (int tile = t0; tile < t1; ++tile) {
-                    const int i0 = tile * TP_TILE + l * 8;
-                    while (i0 < (int)n && i0 >= (int)rs.start[lo + 1]) {
-                        ++lo;
-                    }
-                    const int first = __shfl(lo, 0, 32);
-                    if ((int)rs.start[first + 1] >= (tile + 1) * TP_TILE && known == first) {
-                        if (l == 31) {
-                            agg[tile] = total;
+                __syncthreads();
+                if (t < count) {
+                    const int i0    = (base + t) * TP_TILE;
+                    const int first = run_at(i0);
+                    if ((int)rs.start[first + 1] >= i0 + TP_TILE) {
+                        const float v   = S::ld(rs.prob[first]);
+                        float       seg = v;
+#pragma unroll
+                        for (int k = 1; k < 8; ++k) {
+                            seg = seg + v;
                         }
-                        continue;
+                        sc.agg[t] = seg * 32.0f;
+                    }
+                    else {
+                        sc.carry[atomicAdd(&sh_mixed, 1)] = __int_as_float((t << 16) | first);
+                    }
+                }
+                __syncthreads();
+                const int mixed = sh_mixed;
+                for (int m = t >> 5; m < mixed; m += TP_THREADS / 32) {
+                    const int what = __float_as_int(sc.carry[m]);
+                    const int tile = what >> 16, i = (base + tile) * TP_TILE + l * 8;
+                    // (a lane's first entry: of the runs that begin inside the tile)
+                    int lo = what & 0xFFFF, hi = min((int)nruns, lo + TP_TILE);
+                    while (hi - lo > 1) {
+                        const int mid = (lo + hi) >> 1;
+                        if ((int)rs.start[mid] <= i) {
+                            lo = mid;
+                        }
+                        else {
+                            hi = mid;
+                        }
                     }
                     float x[8];
-                    int   r = lo;
-                    values_from(i0, r, x);
-                    total = tile_scan(x, l);
-                    known = (int)rs.start[first + 1] >= (tile + 1) * TP_TILE ? first : -1;
+                    values_from(i, lo, x);
+                    const float total = tile_scan(x, l);
                     if (l == 31) {
-                        agg[tile] = total;
+                        sc.agg[tile] = total;
                     }
                 }
             };
@@ -1843,28 +1857,46 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     prob = sc.fmisc[1];
     // ---- the column: the sh_nth one in order of ids whose value lies in that range. Blocks whose maximum lies below it
     // cannot hold one: a draw near the head of the distribution reads a few blocks only.
-    const uint32_t klo = key_lo, khi = key_hi;
+    // (no value lies above the maximum)
+    const uint32_t klo = key_lo, khi = min(key_hi, topp_key16((uint32_t)S::st(r.mx)) + 1u);
     const int      nth = sh_nth;
     auto match = [&](uint32_t bits) -> bool {
         const uint32_t k = topp_key16(bits);
         return k >= klo && k < khi;
     };
-    auto mask_of = [&](int blk) -> uint32_t {  // the matches among this lane's eight columns of a block
-        const int v0 = blk * TSP_BLOCK + lane_id() * 8;
+    // Matches among a lane's eight columns of a block: bit k is column 2 k, bit 4 + k column 2 k + 1. Two columns at a
+    // time: with a range of one sign the distance of the bits from its first value, otherwise of their images (with a
+    // column at a time a deep draw, whose blocks are nearly all of the row, spent 10 us here at 128256 columns).
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    typedef short          i16x2 __attribute__((ext_vector_type(2)));
+    const bool           positive = klo >= 0x8000u, one_sign = positive || khi <= 0x8000u;
+    const unsigned short origin   = (unsigned short)(!one_sign ? klo : positive ? klo - 0x8000u : 0x10000u - khi);
+    const unsigned short length   = (unsigned short)min(khi - klo, 0xFFFFu);  // (all 65536: a row of one value ends above)
+    const u16x2          from = {origin, origin}, size = {length, length}, unit = {1, 1};
+    auto mask_of = [&](int blk) -> uint32_t {
+        const int b0 = __builtin_amdgcn_readfirstlane(blk) * TSP_BLOCK;  // (the same for the wave)
         uint32_t  m  = 0u;
-        if (v0 + 8 <= s.n) {
-            const uint4    raw  = topp_load8(r.y + v0);
+        if (b0 + TSP_BLOCK <= s.n) {
+            const uint4    raw  = topp_load8(r.y + b0 + lane_id() * 8);
             const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                m |= (match(w[k] & 0xFFFFu) ? 1u : 0u) << (2 * k);
-                m |= (match(w[k] >> 16) ? 1u : 0u) << (2 * k + 1);
+                u16x2 x = __builtin_bit_cast(u16x2, w[k]);
+                if (!one_sign) {
+                    const i16x2 sign = __builtin_bit_cast(i16x2, w[k]) >> 15;
+                    x = __builtin_bit_cast(u16x2, w[k] ^ (__builtin_bit_cast(uint32_t, sign) | 0x80008000u));
+                }
+                const u16x2 in = __builtin_elementwise_min(__builtin_elementwise_sub_sat(size, (u16x2)(x - from)), unit);
+                m |= __builtin_bit_cast(uint32_t, in) << k;
             }
+            m = (m | (m >> 12)) & 0xFFu;
         }
         else {
+            const int v0 = b0 + lane_id() * 8;
+#pragma unroll 1
             for (int k = 0; k < 8; ++k) {
                 if (v0 + k < s.n && match((uint32_t)r.y[v0 + k])) {
-                    m |= 1u << k;
+                    m |= 1u << ((k >> 1) + 4 * (k & 1));
                 }
             }
         }
@@ -1881,7 +1913,7 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
         }
         unsigned long long todo = __ballot(may);
         while (todo != 0ull) {
-            constexpr int U = 8;
+            constexpr int U = 4;  // (eight: a microsecond more on rows with one block, nothing gained on long ones)
             int           blk[U];
             uint32_t      m[U];
 #pragma unroll
@@ -1963,7 +1995,11 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
             }
             int k = left - (in - c1);
             if (k >= 0 && k < c1) {
-                uint32_t rest = m;
+                uint32_t rest = 0u;  // in the order of the columns
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    rest |= (((m >> q) & 1u) | (((m >> (4 + q)) & 1u) << 1)) << (2 * q);
+                }
                 while (k-- > 0) {
                     rest &= rest - 1u;
                 }

@@ -92,6 +92,29 @@ def _same(got, want, dt):
     np.testing.assert_allclose(got[3], want[3], rtol=1e-5 if dt == O.F32 else 2e-3, atol=1e-6)
 
 
+@pytest.mark.parametrize("dt,V,kind", [(O.F16, 20011, "signs"), (O.BF16, 20011, "signs"), (O.F16, 30000, "levels"),
+                                       (O.BF16, 70001, "levels"), (O.BF16, 300000, "levels")])
+def test_deep_draws_into_long_runs(dt, V, kind):
+    """16-bit rows whose draws lie behind whole scan tiles of one value, tiles of many and both in turn, up to more tiles
+    than one round of the scan holds; the column that is picked is one of thousands of equal probabilities, whose logits
+    may be of both signs."""
+    B = 6
+    rng = np.random.default_rng(V + len(kind))
+    if kind == "signs":  # e is 1 / e^3 for all of them, whatever their sign
+        x = (rng.choice([-1.0, 1.0], (B, V)) * 2.0 ** rng.uniform(-22.0, -16.0, (B, V))).astype(np.float32)
+        x[:, ::97] = 3.0
+    else:
+        x = rng.choice(np.array([0.0, -0.25, -0.5, -1.0], np.float32), (B, V))
+        some = rng.random((B, V)) < 0.05
+        x = np.where(some, rng.standard_normal((B, V)) * 0.5 - 0.5, x).astype(np.float32)
+        x[:, :400] = rng.standard_normal((B, 400)) * 1.5 + 1.0
+    x = O.to_storage(x, dt)
+    p = np.array([1.0, 1.0, 0.97, 0.9, 1.0, 0.6], np.float32)
+    draws = np.array([0.05, 0.5, 0.999, 0.7, 0.92, 0.8], np.float32)
+    end_ids = np.full(B, -1, np.int32)
+    _same(_sample_step(dt, x, V, p, end_ids, draws), _oracle_step(dt, x, V, p, end_ids, draws), dt)
+
+
 @pytest.mark.parametrize("B,V", [(24, 20011), (256, 14000)])   # sixteen and four workgroups per row
 def test_long_fp32_prefixes(B, V):
     """Draws so deep into flat fp32 rows that the prefix in front of them (most of the row, more than 5632 entries) is
