@@ -451,15 +451,19 @@ beam_row_kernel(const bool* __restrict__ finished, const int* __restrict__ end_i
 // run beside the other's exponentials (64 x 8 beams x 152064 fp16: 120 -> 116 us).
 constexpr int BR_THREADS = 1024;
 
-// A value at or below the row's 2K-th largest, from the threads' maxima, and the row's sum from the waves' sums: found
-// by the first wave alone while the others wait at two barriers. Leaves the candidates' count at zero.
-template<int THREADS>
-__device__ __forceinline__ void beam_bound(BeamSelect& s, const double* red, float fmax, int N, double& row_sum,
-                                           uint32_t& floor)
+// A value at or below the row's 2K-th largest, from the threads' maxima: the maxima of neighbouring threads joined into
+// slots, in LDS behind the next barrier, and, by one wave behind that barrier, the bound. Leaves the candidates' count at
+// zero.
+__device__ __forceinline__ int beam_n_slots(int N)
 {
-    const int t = threadIdx.x;
     // 2K <= 32 needs no more than 64 maxima to choose the 2K-th largest from, 2K <= 64 no more than 128
-    const int n_slots = N <= 32 ? 64 : N <= 64 ? 128 : 256;
+    return N <= 32 ? 64 : N <= 64 ? 128 : 256;
+}
+template<int THREADS>
+__device__ __forceinline__ void beam_slots(BeamSelect& s, float fmax, int N)
+{
+    const int t       = threadIdx.x;
+    const int n_slots = beam_n_slots(N);
     const int join    = THREADS / n_slots;  // neighbouring threads that join their maxima: 2 to 16
     fmax              = __builtin_fmaxf(fmax, __shfl_xor(fmax, 1, WAVE));
     if (join >= 4) {
@@ -478,41 +482,56 @@ __device__ __forceinline__ void beam_bound(BeamSelect& s, const double* red, flo
     if (t == 0) {
         s.n_cand = 0;
     }
-    __syncthreads();
-    if (wave_id() == 0) {
-        // The 2K-th largest of the maxima is an element with at least 2K elements at or above it: nothing below it
-        // can be among the 2K best; so is any value below that one. (A group that saw no element reports -inf.)
-        uint32_t P = 0u;
-        if (n_slots == WAVE) {
-            // every lane counts the maxima above its own and those at or above it: the 2K-th largest lies between
-            const uint32_t mine  = slot_key[lane_id()];
-            int            above = 0, reach = 0;
+}
+__device__ __forceinline__ uint32_t beam_floor(const BeamSelect& s, int N)
+{
+    const int       n_slots  = beam_n_slots(N);
+    const uint32_t* slot_key = reinterpret_cast<const uint32_t*>(s.slots);
+    // The 2K-th largest of the maxima is an element with at least 2K elements at or above it: nothing below it
+    // can be among the 2K best; so is any value below that one. (A group that saw no element reports -inf.)
+    uint32_t P = 0u;
+    if (n_slots == WAVE) {
+        // every lane counts the maxima above its own and those at or above it: the 2K-th largest lies between
+        const uint32_t mine  = slot_key[lane_id()];
+        int            above = 0, reach = 0;
 #pragma unroll
-            for (int j = 0; j < WAVE; ++j) {
-                const uint32_t other = __builtin_amdgcn_readlane(mine, j);
-                above += other > mine ? 1 : 0;
-                reach += other >= mine ? 1 : 0;
-            }
-            const unsigned long long at = __ballot(above < N && reach >= N);
-            P = __builtin_amdgcn_readlane(mine, __builtin_ctzll(at));
+        for (int j = 0; j < WAVE; ++j) {
+            const uint32_t other = __builtin_amdgcn_readlane(mine, j);
+            above += other > mine ? 1 : 0;
+            reach += other >= mine ? 1 : 0;
         }
-        else {
-            uint32_t kk[4];
+        const unsigned long long at = __ballot(above < N && reach >= N);
+        P = __builtin_amdgcn_readlane(mine, __builtin_ctzll(at));
+    }
+    else {
+        uint32_t kk[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int i = lane_id() + g * WAVE;
+            kk[g]       = i < n_slots ? slot_key[i] : 0u;
+        }
+        for (int bit = 31; bit >= 8; --bit) {
+            const uint32_t cand = P | (1u << bit);
+            int            c    = 0;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int i = lane_id() + g * WAVE;
-                kk[g]       = i < n_slots ? slot_key[i] : 0u;
+                c += (int)__builtin_popcountll(__ballot(kk[g] >= cand));
             }
-            for (int bit = 31; bit >= 8; --bit) {
-                const uint32_t cand = P | (1u << bit);
-                int            c    = 0;
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    c += (int)__builtin_popcountll(__ballot(kk[g] >= cand));
-                }
-                P = c >= N ? cand : P;
-            }
+            P = c >= N ? cand : P;
         }
+    }
+    return P;
+}
+
+// The same and the row's sum from the waves' sums, by the first wave alone while the others wait at two barriers.
+template<int THREADS>
+__device__ __forceinline__ void beam_bound(BeamSelect& s, const double* red, float fmax, int N, double& row_sum,
+                                           uint32_t& floor)
+{
+    beam_slots<THREADS>(s, fmax, N);
+    __syncthreads();
+    if (wave_id() == 0) {
+        const uint32_t P = beam_floor(s, N);
         if (lane_id() == 0) {
             double tot = 0.0;
             for (int w = 0; w < THREADS / WAVE; ++w) {
@@ -639,7 +658,6 @@ beam_team_kernel(const typename Storage<DT>::T* __restrict__ x, const typename S
     __shared__ BeamSelect s;
     __shared__ double     red[WAVES];
     __shared__ float      redf[WAVES];
-    __shared__ double     part_sum;
     __shared__ uint32_t   part_floor;
     const int             row   = blockIdx.x;
     const int             part  = blockIdx.y;
@@ -717,7 +735,10 @@ beam_team_kernel(const typename Storage<DT>::T* __restrict__ x, const typename S
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int o = o0 + u * BR_THREADS;
-            if (o < others) {
+            if (o < others && bias == nullptr) {
+                m = __builtin_fmaxf(m, lean_raw_max<DT>(ov[u]));
+            }
+            else if (o < others) {
                 const T*  e = reinterpret_cast<const T*>(&ov[u]);
                 const int v = head + (o < lo ? o : o + own) * EPV;
 #pragma unroll
@@ -728,29 +749,79 @@ beam_team_kernel(const typename Storage<DT>::T* __restrict__ x, const typename S
         }
     }
     m = __builtin_fmaxf(m, edge_x);
-    each_own([&](int, float e) { fmax = __builtin_fmaxf(fmax, e); });  // (a NaN is never the maximum)
-    m = block_max<float, WAVES>(__builtin_fmaxf(m, fmax), redf, -S::max_t());
+    // (a NaN is never the maximum)
+    if (bias == nullptr) {
+        fmax = __builtin_fmaxf(edge_own ? edge_x : NEG, NEG);
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            if (t + u * BR_THREADS < own) {
+                fmax = __builtin_fmaxf(fmax, lean_raw_max<DT>(raw[u]));
+            }
+        }
+    }
+    else {
+        each_own([&](int, float e) { fmax = __builtin_fmaxf(fmax, e); });
+    }
+    beam_slots<BR_THREADS>(s, fmax, N);
+    m = block_max<float, WAVES>(__builtin_fmaxf(m, fmax), redf, -S::max_t());  // (barriers: the slots are there)
+    if (wave_id() == 0) {
+        const uint32_t P = beam_floor(s, N);  // while the other waves go on
+        if (t == 0) {
+            part_floor = P;
+        }
+    }
     double d = 0.0;
     each_own([&](int, float e) { d += (double)det_expf_nonpos(e - m); });
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        d += __shfl_xor(d, o, WAVE);
-    }
+    d = wave_reduce_unordered(d, [](double p, double q) { return p + q; });
     if (lane_id() == 0) {
         red[wave_id()] = d;
     }
-    beam_bound<BR_THREADS>(s, red, fmax, N, part_sum, part_floor);
+    __syncthreads();
     const uint32_t floor_key = part_floor;
     const float    floor_val = key_to_float(floor_key);
     const bool     all_pass  = floor_key <= order_key(NEG);  // then NaN columns are wanted too
-    each_own([&](int v, float e) {
+    auto push = [&](int v, float e) {
         if (e >= floor_val || all_pass) {
             const int at = atomicAdd(&s.n_cand, 1);
             if (at < BM_CAP) {
                 s.cand[at] = beam_key(e, (uint32_t)v);
             }
         }
-    });
+    };
+    if (bias != nullptr || all_pass) {
+        each_own(push);
+    }
+    else if (fmax >= floor_val) {  // (few threads hold a candidate; short code, since it waits for its own fetch)
+        if (edge_own) {
+            push(edge, edge_x);
+        }
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int i = t + u * BR_THREADS;
+            if (u * BR_THREADS < own && i < own && lean_raw_max<DT>(raw[u]) >= floor_val) {
+                const T* e    = reinterpret_cast<const T*>(&raw[u]);
+                uint32_t hits = 0u;
+#pragma unroll
+                for (int j = 0; j < EPV; ++j) {
+                    hits |= (S::ld(e[j]) >= floor_val ? 1u : 0u) << j;
+                }
+                const uint32_t w[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
+                while (hits != 0u) {
+                    const int      j    = __builtin_ctz(hits);
+                    const uint32_t word = register_pick<4>(w, j * (int)sizeof(T) / 4);
+                    float          x;
+                    if constexpr (sizeof(T) == 4) {
+                        x = u2f(word);
+                    }
+                    else {
+                        x = S::ld((T)(word >> (16 * (j & 1))));
+                    }
+                    push(head + (lo + i) * EPV + j, x);
+                    hits &= hits - 1u;
+                }
+            }
+        }
+    }
     __syncthreads();
     if (wave_id() >= BM_WAVES) {
         return;  // the first four waves select
@@ -770,7 +841,12 @@ beam_team_kernel(const typename Storage<DT>::T* __restrict__ x, const typename S
         keys[t] = s.out[t];
     }
     if (t == 0) {
-        psum[(size_t)row * parts + part] = part_sum;
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            sum += red[w];
+        }
+        psum[(size_t)row * parts + part] = sum;
         if (part == 0) {
             pmax[row] = m;
         }

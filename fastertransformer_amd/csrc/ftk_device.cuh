@@ -551,4 +551,41 @@ __device__ __forceinline__ float row_uniform(RngState* rng, const float* injecte
     return rng_next_uniform(rng + b);
 }
 
+// largest element of a 16-byte vector as stored (no transform); NaN elements are ignored
+template<int DT>
+__device__ __forceinline__ float lean_raw_max(const uint4& v)
+{
+    if constexpr (DT == DT_F32) {
+        return __builtin_fmaxf(__builtin_fmaxf(__uint_as_float(v.x), __uint_as_float(v.y)),
+                               __builtin_fmaxf(__uint_as_float(v.z), __uint_as_float(v.w)));
+    }
+    else if constexpr (DT == DT_F16) {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        const h2         a = __builtin_bit_cast(h2, v.x), b = __builtin_bit_cast(h2, v.y);
+        const h2         c = __builtin_bit_cast(h2, v.z), d = __builtin_bit_cast(h2, v.w);
+        const h2 m = __builtin_elementwise_max(__builtin_elementwise_max(a, b), __builtin_elementwise_max(c, d));
+        return __builtin_fmaxf((float)m.x, (float)m.y);
+    }
+    else {
+        auto pair_max = [](uint32_t w) -> float {
+            return __builtin_fmaxf(__uint_as_float(w << 16), __uint_as_float(w & 0xFFFF0000u));
+        };
+        return __builtin_fmaxf(__builtin_fmaxf(pair_max(v.x), pair_max(v.y)),
+                               __builtin_fmaxf(pair_max(v.z), pair_max(v.w)));
+    }
+}
+
+// element i of an array in registers (the empty asm keeps the compiler from making it an array in memory)
+template<int N, class V>
+__device__ __forceinline__ V register_pick(const V* from, int i)
+{
+    V x = from[0];
+#pragma unroll
+    for (int q = 1; q < N; ++q) {
+        x = i == q ? from[q] : x;
+        asm("" : "+v"(x));
+    }
+    return x;
+}
+
 }  // namespace ftk

@@ -88,30 +88,6 @@ __device__ __forceinline__ uint32_t lean_kth_of_slots(const uint32_t* keys, int 
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)P);
 }
 
-// largest element of a 16-byte vector as stored (no transform); NaN elements are ignored
-template<int DT>
-__device__ __forceinline__ float lean_raw_max(const uint4& v)
-{
-    if constexpr (DT == DT_F32) {
-        return __builtin_fmaxf(__builtin_fmaxf(__uint_as_float(v.x), __uint_as_float(v.y)),
-                               __builtin_fmaxf(__uint_as_float(v.z), __uint_as_float(v.w)));
-    }
-    else if constexpr (DT == DT_F16) {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        const h2         a = __builtin_bit_cast(h2, v.x), b = __builtin_bit_cast(h2, v.y);
-        const h2         c = __builtin_bit_cast(h2, v.z), d = __builtin_bit_cast(h2, v.w);
-        const h2 m = __builtin_elementwise_max(__builtin_elementwise_max(a, b), __builtin_elementwise_max(c, d));
-        return __builtin_fmaxf((float)m.x, (float)m.y);
-    }
-    else {
-        auto pair_max = [](uint32_t w) -> float {
-            return __builtin_fmaxf(__uint_as_float(w << 16), __uint_as_float(w & 0xFFFF0000u));
-        };
-        return __builtin_fmaxf(__builtin_fmaxf(pair_max(v.x), pair_max(v.y)),
-                               __builtin_fmaxf(pair_max(v.z), pair_max(v.w)));
-    }
-}
-
 // A value that an unrounded product must reach before its rounding to T can reach `x`.
 template<int DT>
 __device__ __forceinline__ float lean_below_rounding(float x)

@@ -890,19 +890,6 @@ constexpr int LPW_THREADS = 1024;
 #define LPW_STAMP(i)
 #endif
 
-// element i of an array in registers (the empty asm keeps the compiler from making it an array in memory)
-template<int N, class V>
-__device__ __forceinline__ V lp_pick(const V* from, int i)
-{
-    V x = from[0];
-#pragma unroll
-    for (int q = 1; q < N; ++q) {
-        x = i == q ? from[q] : x;
-        asm("" : "+v"(x));
-    }
-    return x;
-}
-
 // Whether any lane of the wave has it, in a branch that the whole wave takes: what it leads to is out of the way of the
 // straight line (a branch for some lanes would be jumped over by all others, at the cost of a fetch).
 __device__ __forceinline__ bool lp_rare(bool mine)
@@ -1128,7 +1115,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                 const int j = __builtin_ctz(special), v = v0 + offset_of(j);
                 special &= special - 1u;
                 if constexpr (!WORD16) {
-                    float x = lp_pick<N>(y, j);
+                    float x = register_pick<N>(y, j);
                     x       = (flags >> j) & 1u ? rowctx.flagged(x, v) : x;
                     x       = to_end == (uint32_t)offset_of(j) ? -S::max_t() : x;
 #pragma unroll
@@ -1137,7 +1124,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                     }
                 }
                 else {
-                    const uint32_t pair  = lp_pick<NY>(y, j >> 1);
+                    const uint32_t pair  = register_pick<NY>(y, j >> 1);
                     const int      shift = 16 * (j & 1);
                     float          x     = S::ld((T)(pair >> shift));
                     x                    = (flags >> j) & 1u ? rowctx.flagged(x, v) : x;
