@@ -575,6 +575,14 @@ __device__ __forceinline__ float lean_raw_max(const uint4& v)
     }
 }
 
+// a 16-byte load that is read once: it does not displace what the caches hold for others
+__device__ __forceinline__ uint4 stream_load(const uint4* p)
+{
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    const u4             v = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 // element i of an array in registers (the empty asm keeps the compiler from making it an array in memory)
 template<int N, class V>
 __device__ __forceinline__ V register_pick(const V* from, int i)

@@ -102,14 +102,6 @@ __device__ __forceinline__ float lean_below_rounding(float x)
     }
 }
 
-// a 16-byte load that is read once: it does not displace what the caches hold for others
-__device__ __forceinline__ uint4 lean_stream_load(const uint4* p)
-{
-    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-    const u4             v = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-
 constexpr int LG_HIST_U = 8;  // history ids a thread requests before the logits (2048 positions per workgroup)
 
 // What a launch of lean_gather_kernel does.
@@ -214,7 +206,7 @@ __global__ void __launch_bounds__(LG_THREADS, OCC) lean_gather_kernel(FusedParam
 #pragma unroll
         for (int j = 0; j < LG_NV; ++j) {
             const int vi = min(vb + q * LG_SUB_VECS + j * LG_THREADS + t, ve - 1);  // past the end: a harmless vector
-            raw[slot][j] = lean_stream_load(base + vi);
+            raw[slot][j] = stream_load(base + vi);
             if constexpr (BIAS) {
                 rawb[slot][j] = bias_base[vi];
             }

@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(LG_THREADS, LG_OCCUPANCY) lp_rowmax_kernel(Fus
 #pragma unroll
         for (int j = 0; j < LG_NV; ++j) {
             const int vi = min(vb + q * LG_SUB_VECS + j * LG_THREADS + t, ve - 1);
-            raw[slot][j] = lean_stream_load(base + vi);
+            raw[slot][j] = stream_load(base + vi);
         }
     };
 #pragma unroll

@@ -866,7 +866,7 @@ read_yardstick_kernel(const uint4* __restrict__ data, size_t nvec, size_t vec_pe
         for (int j = 0; j < LG_NV; ++j) {
             size_t vi = vb + (size_t)q * LG_SUB_VECS + j * LG_THREADS + t;
             vi        = vi < ve ? vi : ve - 1;
-            raw[slot][j] = lean_stream_load(data + vi);
+            raw[slot][j] = stream_load(data + vi);
         }
     };
 #pragma unroll

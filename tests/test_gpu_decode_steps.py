@@ -58,6 +58,12 @@ def test_log_prob_from_logits(dt, batch_first, shape):
                                                batch_first) == ops.FTK_ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("V", [131072, 131068])  # exactly 64 MB, from where the logits go past the caches, and just below
+def test_log_prob_from_large_logits(dt, V):
+    test_log_prob_from_logits(dt, V == 131068, (8, 32, V))
+
+
 def test_log_prob_masked_logits():
     """rows holding -inf entries (banned tokens) and one row that is -inf everywhere except the target"""
     import torch
