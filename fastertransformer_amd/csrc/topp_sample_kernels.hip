@@ -1857,8 +1857,8 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     prob = sc.fmisc[1];
     // ---- the column: the sh_nth one in order of ids whose value lies in that range. Blocks whose maximum lies below it
     // cannot hold one: a draw near the head of the distribution reads a few blocks only.
-    // (no value lies above the maximum)
-    const uint32_t klo = key_lo, khi = min(key_hi, topp_key16((uint32_t)S::st(r.mx)) + 1u);
+    // (no value lies above the maximum; of zeros the positive one counts as the larger here, whichever the maximum is)
+    const uint32_t klo = key_lo, khi = min(key_hi, topp_key16((uint32_t)S::st(r.mx + 0.0f)) + 1u);
     const int      nth = sh_nth;
     auto match = [&](uint32_t bits) -> bool {
         const uint32_t k = topp_key16(bits);

@@ -115,6 +115,26 @@ def test_deep_draws_into_long_runs(dt, V, kind):
     _same(_sample_step(dt, x, V, p, end_ids, draws), _oracle_step(dt, x, V, p, end_ids, draws), dt)
 
 
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("V,Vp", [(9001, 9001), (9001, 9008), (2000, 2003)])
+@pytest.mark.parametrize("first", [-0.0, 0.0])
+def test_largest_values_are_zeros_of_both_signs(dt, V, Vp, first):
+    """The largest value of a row is zero: -0 and +0 have one probability, and a draw picks among all of them."""
+    zeros = np.array([0, 100, 513, 1024, V - 1])
+    B = len(zeros) + 2
+    rng = np.random.default_rng(V + dt)
+    x = rng.uniform(-14.0, -11.0, (B, Vp)).astype(np.float32)
+    x[:, zeros] = np.where(np.arange(len(zeros)) % 2 == 0, first, -first)
+    x[-1, zeros[1:]] = first     # a row of one sign
+    x = O.to_storage(x, dt)
+    p = np.full(B, 1.0, np.float32)
+    draws = np.append((np.arange(len(zeros)) + 0.5) / (len(zeros) + 0.2), [0.02, 0.4]).astype(np.float32)
+    end_ids = np.full(B, -1, np.int32)
+    want = _oracle_step(dt, x, V, p, end_ids, draws)
+    assert set(want[0][:len(zeros)]) == set(zeros)
+    _same(_sample_step(dt, x, V, p, end_ids, draws), want, dt)
+
+
 @pytest.mark.parametrize("B,V", [(24, 20011), (256, 14000)])   # sixteen and four workgroups per row
 def test_long_fp32_prefixes(B, V):
     """Draws so deep into flat fp32 rows that the prefix in front of them (most of the row, more than 5632 entries) is
