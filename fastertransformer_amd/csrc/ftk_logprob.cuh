@@ -1389,6 +1389,10 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     int*      parked    = s.sel.idx;
     float     raw_floor = NEG_INF;
     bool      raises    = false;  // the history penalty raises values
+    // (the mask of the end id raises a value of -inf to -MAX_T, which is the largest of rows that are masked throughout: the
+    // end id is considered whatever its raw value)
+    const int end_vector =
+        rowctx.masked_end_id >= 0 && rowctx.masked_end_id < p.V ? vector_of(rowctx.masked_end_id) : -1;
     if (valid && ordered) {
         // an unflagged column with e >= thr_low has at least this raw value (e's rounding, the logarithm's, y's)
         const float rounding = DT == DT_F32 ? 0.99999f : (DT == DT_F16 ? (thr_low < 2.44140625e-04f ? 0.4f : 0.998f) : 0.98f);
@@ -1399,6 +1403,9 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         uint32_t mine        = 0u;
         for (int g = 0; g << glog < turns; ++g) {
             mine |= (group_max[g * THREADS + t] >= raw_floor ? 1u : 0u) << g;
+        }
+        if (end_vector >= 0 && end_vector < nvec && (end_vector & (THREADS - 1)) == t) {
+            mine |= 1u << ((end_vector / THREADS) >> glog);
         }
         // (a penalty that raises values: the columns of the history can reach the bound from any raw value)
         raises = hist && !(p.penalty_type == 0 ? rowctx.penalty >= 0.0f : rowctx.penalty >= 1.0f);
@@ -1553,6 +1560,9 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
 #pragma unroll
                 for (int j = 0; j < EPV; ++j) {
                     hits |= (!(vector_element<DT>(v, j) < raw_floor) ? 1u : 0u) << j;
+                }
+                if (rel == end_vector) {
+                    hits |= 1u << ((rowctx.masked_end_id + a) % EPV);
                 }
                 if (raises) {
                     hits = (1u << EPV) - 1u;

@@ -196,3 +196,32 @@ def test_masked_rows_count_their_pads(dt, B, V, Vp, k):
         o.step(H + i, x, u)
         compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
 
+
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16], ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("B,V,Vp,k", [(8, 1452, 1459, 5), (8, 9001, 9001, 30), (264, 1030, 1041, 20), (1032, 1100, 1101, 8)])
+def test_masked_end_ids_count_in_masked_rows(dt, B, V, Vp, k):
+    """Below the minimum length the end id has the type's lowest number, also where its logit is -inf or NaN: in rows without
+    anything larger it is one of the largest. 1024, 512 and 256 threads per row; end ids in the whole vectors of a row and
+    in front of and behind them."""
+    from decode_harness import Case, OracleRunner, ProductRunner, compare
+    from helpers import uniforms
+    rng = np.random.default_rng(V + dt)
+    H = 4
+    ends = np.where(np.arange(B) % 4 == 3, rng.integers(0, V, B), np.array([0, V - 1, V // 2])[np.arange(B) % 3])
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=3, runtime_top_k=[k], runtime_top_p=[1.0], min_length=[100],
+             end_ids=ends, prompt=rng.integers(0, V, (H, B)).astype(np.int32), with_cum=True, with_out_lp=True)
+    p, o = ProductRunner(c), OracleRunner(c)
+    rows = np.arange(B)
+    for i in range(3):
+        x = np.full((B, Vp), -np.inf, np.float32)
+        for r in rows:
+            some = V // 2 if r % 2 == 0 else 8 * k
+            x[r, rng.integers(0, V, some)] = -O.max_t(dt)
+        x[rows % 5 == 4] = rng.standard_normal((1, Vp))     # ordinary rows among them
+        x[rows, ends] = (-np.inf, np.nan, 3.0)[i]
+        x, u = O.to_storage(x, dt), uniforms(rng, B)
+        u[rows % 3 == 0] = 0.999                            # (the order of ties puts late columns first or last)
+        print("masked end ids", DTYPE_NAMES[dt], B, V, Vp, k, i, flush=True)
+        p.step(H + i, x, u)
+        o.step(H + i, x, u)
+        compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
