@@ -164,7 +164,7 @@ __global__ void test_math_kernel(int kind, const float* __restrict__ in, float* 
 
 // Workgroup b: every pair (y, max) with the value of bits b as the maximum and y not above it, or NaN.
 // wrong[0]: results that are not T(det_expf(y - max)); wrong[1]: pairs of values that took det_expf.
-template<int DT>
+template<int DT, bool WIDE>
 __global__ void test_exp_pairs_kernel(unsigned long long* wrong)
 {
     typedef Storage<DT> S;
@@ -180,9 +180,14 @@ __global__ void test_exp_pairs_kernel(unsigned long long* wrong)
             const uint32_t bits = 2u * i + (uint32_t)h;
             y |= (uint32_t)(S::ld((typename S::T)bits) > max ? S::st(max) : (typename S::T)bits) << (16 * h);
         }
-        uint32_t redo = ex.never;
-        uint32_t e    = ex(y, redo);
-        if (ex.undecided(redo)) {
+        uint32_t redo = ex.never, e;
+        if constexpr (WIDE) {
+            e = ex.wide(y, redo);
+        }
+        else {
+            e = ex(y, redo);
+        }
+        if (ex.undecided(redo, WIDE)) {
             e = ex.exact(y);
             again++;
         }
@@ -388,14 +393,21 @@ int ftk_test_device_math(int kind, const float* in, float* out, size_t n, ftk_st
 int ftk_test_exp_pairs(int dtype, unsigned long long* wrong, ftk_stream_t stream)
 {
     if (dtype == FTK_DTYPE_F16) {
-        test_exp_pairs_kernel<DT_F16><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
+        test_exp_pairs_kernel<DT_F16, false><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
     }
     else if (dtype == FTK_DTYPE_BF16) {
-        test_exp_pairs_kernel<DT_BF16><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
+        test_exp_pairs_kernel<DT_BF16, false><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
     }
     else {
         return FTK_ERR_DTYPE;
     }
+    FTK_LAUNCH_CHECK();
+    return 0;
+}
+
+int ftk_test_exp_pairs_wide(unsigned long long* wrong, ftk_stream_t stream)
+{
+    test_exp_pairs_kernel<DT_BF16, true><<<65536, 256, 0, (hipStream_t)stream>>>(wrong);
     FTK_LAUNCH_CHECK();
     return 0;
 }

@@ -18,19 +18,29 @@ struct ExpPairs {
     typedef _Float16    f16x2 __attribute__((ext_vector_type(2)));
     typedef __bf16      bf16x2 __attribute__((ext_vector_type(2)));
     static constexpr float LOG2E = 1.44269502162933349609375f;
-    // t carries 16 more than the argument: where most columns of a row lie (e^-11 and around it) t is then small and
-    // its rounding finer.
-    static constexpr float SHIFT = 16.0f, UNSHIFT = 1.52587890625e-05f;
-    // How far det_expf can lie above / below the hardware's value: a share of it and an absolute part, which takes over
-    // far from the maximum, where the rounding of y - max in det_expf's argument counts. Largest distances over every
-    // pair of values y <= max of the type: binary16 7.8e-7 / 9.2e-7 down to 2^-20 and 1.3e-6 / 1.7e-6 down to 2^-32,
-    // bfloat16 1.2e-6 / 1.7e-6 down to 2^-32; the factors' own rounding comes on top (a test goes through all pairs).
-    // Wider bounds cost time, not bits: more pairs are evaluated twice.
-    static constexpr float UP    = DT == DT_F16 ? 1.0e-6f : 1.4e-6f;
-    static constexpr float DOWN  = DT == DT_F16 ? 1.1e-6f : 1.9e-6f;
-    static constexpr float FLOOR = DT == DT_F16 ? 8.0e-13f : 1.5e-16f;  // (bfloat16: also what the hardware flushes)
+    // t carries SHIFT more than the argument: its rounding is finest where it is small, SHIFT / log2 e below the maximum.
+    // (bfloat16: with it nothing is flushed either that does not round to zero)
+    static constexpr float SHIFT = DT == DT_F16 ? 13.0f : 24.0f, UNSHIFT = DT == DT_F16 ? 0x1p-13f : 0x1p-24f;
+    // How far det_expf can lie above / below the hardware's value: a share of it and an absolute part, for where the
+    // roundings of t and of det_expf's y - max are larger. Largest distances over every pair of values y <= max of the type:
+    // binary16 6.0e-7 / 8.0e-7 and 7.7e-13; bfloat16 1.34e-6 / 1.75e-6 and 2.4e-19. The factors' own rounding comes on top
+    // (a test goes through all pairs). Wider bounds cost time, not bits: more pairs are evaluated twice. (bfloat16, normal
+    // logits at temperatures of 0.7 to 2: a pair in 12.5 % of the groups of 512 columns, with a SHIFT of 16 in 13.7 %, of 28
+    // in 16.4 %: the e of near columns lie close to where the type rounds more often than by chance, so that t has to be
+    // good there)
+    static constexpr float UP    = DT == DT_F16 ? 6.7e-7f : 1.4e-6f;
+    static constexpr float DOWN  = DT == DT_F16 ? 8.7e-7f : 1.82e-6f;
+    static constexpr float FLOOR = DT == DT_F16 ? 8.0e-13f : 3.0e-19f;
+    // bfloat16, columns more than some 30 below the maximum (e below FAR): there the absolute part tells, and soon is as
+    // large as the value, so that nothing is decided. Bounds that grow with |t| hold everywhere (largest distances beyond the
+    // growing parts 8.6e-7 / 1.31e-6) and need none, apart from the last bits of subnormal numbers. They take three more
+    // operations a column.
+    static constexpr float WIDE_UP = 9.4e-7f, WIDE_UP_T = 8.0e-8f, WIDE_DOWN = 1.38e-6f, WIDE_DOWN_T = 1.0e-7f;
+    static constexpr float WIDE_LAST = 0x1p-147f;
+    static constexpr uint32_t FAR = (127 - 43) << 7;  // 2^-43
     float    max;
     float    c, hi, lo, one;
+    float    wide_hi, wide_lo, wide_hi_t, wide_lo_t;
     uint32_t never;  // redo from the start: a maximum so large that c says little about it
 
     // `row_max` is the same for every lane
@@ -44,8 +54,14 @@ struct ExpPairs {
         const float sum_low = (SHIFT - (sum - part)) + (-m - part);
         const float scale   = __builtin_amdgcn_exp2f(sum_low - m_low) * UNSHIFT;
         c                   = uniform_f(sum);
-        hi                  = uniform_f(scale * (1.0f + UP));
-        lo                  = uniform_f(scale * (1.0f - DOWN));
+        hi                  = uniform_f(fma_rn(scale, UP, scale));
+        lo                  = uniform_f(fma_rn(scale, -DOWN, scale));
+        if constexpr (DT == DT_BF16) {
+            wide_hi   = uniform_f(fma_rn(scale, WIDE_UP, scale));
+            wide_lo   = uniform_f(fma_rn(scale, -WIDE_DOWN, scale));
+            wide_hi_t = uniform_f(scale * WIDE_UP_T);
+            wide_lo_t = uniform_f(scale * -WIDE_DOWN_T);
+        }
         one                 = 1.0f;
         asm("" : "+s"(one));  // (a multiplication by a visible 1 would be taken out, and with it the fused conversion)
     }
@@ -87,10 +103,28 @@ struct ExpPairs {
         redo |= up ^ down;
         return up;
     }
-    // whether what the calls above collected asks for det_expf (binary16: below zero the lower end rounds to -0)
-    static __device__ __forceinline__ bool undecided(uint32_t redo)
+    // the same with the bounds that hold at any distance (bfloat16)
+    __device__ __forceinline__ uint32_t wide(uint32_t y, uint32_t& redo) const
     {
-        return DT == DT_F16 ? (redo & 0x7FFF7FFFu) != 0u : redo != 0u;
+        float up[2], down[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float t = fma_rn(h == 0 ? low(y) : high(y), LOG2E, c);
+            const float a = __builtin_amdgcn_exp2f(t);
+            const float d = __builtin_fminf(__builtin_fabsf(t), 256.0f);  // (zero times infinity)
+            up[h]         = fma_rn(a, fma_rn(d, wide_hi_t, wide_hi), WIDE_LAST);
+            down[h]       = fma_rn(a, fma_rn(d, wide_lo_t, wide_lo), -WIDE_LAST);
+        }
+        const uint32_t e = pack(up[0], up[1]);
+        redo |= e ^ pack(down[0], down[1]);
+        return e;
+    }
+    // Whether what the calls above collected asks for det_expf. Where the absolute part rounds to zero (binary16, and the wide
+    // bounds) the lower end of a value near zero rounds to -0, which is no difference; where it does not, a change of sign is
+    // one.
+    static __device__ __forceinline__ bool undecided(uint32_t redo, bool of_wide = false)
+    {
+        return DT == DT_F16 || of_wide ? (redo & 0x7FFF7FFFu) != 0u : redo != 0u;
     }
     // the same by det_expf
     __device__ __forceinline__ uint32_t exact(uint32_t y) const
@@ -98,9 +132,10 @@ struct ExpPairs {
         return pack(det_expf_nonpos(low(y) - max), det_expf_nonpos(high(y) - max));
     }
     // e of P pairs, exactly: all of them in a straight line, then one look for pairs that are not decided, in a branch that
-    // the whole wave takes, and a closer one at two pairs each.
+    // the whole wave takes, and a closer one at two pairs each. `far`: lanes with a column so far below the maximum that the
+    // wide bounds are the better ones are added.
     template<int P>
-    __device__ __forceinline__ void numerators(const uint32_t* y, uint32_t* e) const
+    __device__ __forceinline__ void numerators(const uint32_t* y, uint32_t* e, unsigned long long& far) const
     {
         static_assert(P % 2 == 0, "two pairs at a time");
         uint32_t redo[P / 2], any = 0u;
@@ -112,27 +147,45 @@ struct ExpPairs {
             any |= redo[i];
         }
         if (__builtin_expect(__ballot(undecided(any)) != 0ull, 0)) {
+            if constexpr (DT == DT_BF16) {
+                typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+                u16x2                  least = {0x7FFF, 0x7FFF};
 #pragma unroll
-            for (int i = 0; i < P / 2; ++i) {
-                if (DT == DT_BF16 && never == 0u) {
-                    // masked columns: -inf has e = 0, whatever the absolute part of the bounds says
-                    const uint32_t a = infinite(y[2 * i]), b = infinite(y[2 * i + 1]);
-                    e[2 * i] &= ~a;
-                    e[2 * i + 1] &= ~b;
-                    redo[i] &= ~(a & b);
+                for (int i = 0; i < P; ++i) {
+                    least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, e[i] & 0x7FFF7FFFu));
                 }
-                if (__ballot(undecided(redo[i])) != 0ull) {
-                    e[2 * i]     = exact(y[2 * i]);
-                    e[2 * i + 1] = exact(y[2 * i + 1]);
-                }
+                far |= __ballot(min(least.x, least.y) < FAR);
             }
+            redone<P>(y, e, redo, false);
         }
     }
-    // all ones in the halves that are -inf
-    static __device__ __forceinline__ uint32_t infinite(uint32_t y)
+    // the same with the wide bounds
+    template<int P>
+    __device__ __forceinline__ void wide_numerators(const uint32_t* y, uint32_t* e) const
     {
-        const uint32_t x = Storage<DT>::st(-__builtin_inff());
-        return ((y & 0xFFFFu) == x ? 0xFFFFu : 0u) | ((y >> 16) == x ? 0xFFFF0000u : 0u);
+        uint32_t redo[P / 2], any = 0u;
+#pragma unroll
+        for (int i = 0; i < P / 2; ++i) {
+            redo[i]      = never;
+            e[2 * i]     = wide(y[2 * i], redo[i]);
+            e[2 * i + 1] = wide(y[2 * i + 1], redo[i]);
+            any |= redo[i];
+        }
+        if (__ballot(undecided(any, true)) != 0ull) {
+            redone<P>(y, e, redo, true);
+        }
+    }
+    // e of the pairs that are not decided, by det_expf
+    template<int P>
+    __device__ __forceinline__ void redone(const uint32_t* y, uint32_t* e, const uint32_t* redo, bool of_wide) const
+    {
+#pragma unroll
+        for (int i = 0; i < P / 2; ++i) {
+            if (__ballot(undecided(redo[i], of_wide)) != 0ull) {
+                e[2 * i]     = exact(y[2 * i]);
+                e[2 * i + 1] = exact(y[2 * i + 1]);
+            }
+        }
     }
     // sum + the first / second value of a pair, rounded once
     __device__ __forceinline__ float add_low(float sum, uint32_t e) const
@@ -144,7 +197,7 @@ struct ExpPairs {
         return fma_rn(high(e), one, sum);
     }
     // y times a T, rounded to T
-    static __device__ __forceinline__ uint32_t scale(uint32_t y, float by)
+    static __device__ __forceinline__ uint32_t times(uint32_t y, float by)
     {
         if constexpr (DT == DT_F16) {
             const _Float16 m = (_Float16)by;

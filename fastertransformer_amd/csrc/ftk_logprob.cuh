@@ -1091,7 +1091,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                 else {
                     pair = raw[i];
                 }
-                y[i] = ExpPairs<DT>::scale(pair, rowctx.fast_mul);
+                y[i] = ExpPairs<DT>::times(pair, rowctx.fast_mul);
             }
         }
         if (lp_rare((own_flags & flag_of(v0)) != 0u)) {
@@ -1435,7 +1435,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     if constexpr (THREADS < LPW_THREADS) {
         __builtin_amdgcn_s_setprio(0);
     }
-    // ---- second pass: the sum chain by chain, candidates on the way
+    // ---- second pass: the sum chain by chain
     float acc[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -1456,9 +1456,10 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             return 0;
         }
     }();
+    unsigned long long far = 0ull;  // bfloat16: lanes that have met columns far below the maximum
     // e of slots [j0, j0 + G) of a batch. 16-bit types: half a batch in a straight line (a wave waits for every branch).
     constexpr int G = WORD16 ? 8 : 4;
-    auto numerators = [&](const Val* y, Val* e, int j0) __attribute__((always_inline)) {
+    auto numerators = [&](auto wide, const Val* y, Val* e, int j0) __attribute__((always_inline)) {
         if constexpr (!WORD16) {
             float d[G];
 #pragma unroll
@@ -1476,16 +1477,19 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                 }
             }
         }
+        else if constexpr (decltype(wide)::value) {
+            ex.template wide_numerators<G / 2>(y + j0 / 2, e + j0 / 2);
+        }
         else {
-            ex.template numerators<G / 2>(y + j0 / 2, e + j0 / 2);
+            ex.template numerators<G / 2>(y + j0 / 2, e + j0 / 2, far);
         }
     };
-    stream([&](const Val* y, int rounds) {
+    auto add_batch = [&](auto wide, const Val* y, int rounds) __attribute__((always_inline)) {
 #pragma unroll
         for (int j0 = 0; j0 < N; j0 += G) {
             if (j0 / CH < rounds) {  // (whole batches: always)
                 Val e[NY];
-                numerators(y, e, j0);
+                numerators(wide, y, e, j0);
                 // (slots of a chain in ascending order of their columns)
 #pragma unroll
                 for (int j = j0; j < j0 + G; ++j) {
@@ -1498,6 +1502,15 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                     }
                 }
             }
+        }
+    };
+    stream([&](const Val* y, int rounds) __attribute__((always_inline)) {
+        // (bfloat16: from the first far column on a wave takes the wide bounds for the rest of its columns)
+        if (DT == DT_BF16 && __builtin_expect(far != 0ull, 0)) {
+            add_batch(std::integral_constant<bool, DT == DT_BF16>(), y, rounds);
+        }
+        else {
+            add_batch(std::false_type(), y, rounds);
         }
     });
     const float pad_e = p.V < p.Vp ? round_t<DT>(det_expf_nonpos(-S::max_t() - row_max)) : 0.0f;

@@ -89,6 +89,7 @@ _HOOK_SIGNATURES = {
     "ftk_host_logf": [_f],
     "ftk_test_device_math": [_i, _vp, _vp, _sz, _vp],
     "ftk_test_exp_pairs": [_i, _vp, _vp],
+    "ftk_test_exp_pairs_wide": [_vp, _vp],
     "ftk_test_rng_uniform": [_vp, _vp, _i, _i, _vp],
     "ftk_test_set_topp_force_deep": [_i],
     "ftk_test_topp_prefix_lengths": [_vp, _i, _i, _sz, _i, _vp],

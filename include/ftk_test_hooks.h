@@ -26,6 +26,8 @@ int ftk_test_device_math(int kind, const float* in, float* out, size_t n, ftk_st
  * T(det_expf(y - max)) and to wrong[1] how many pairs of values the hardware's exponential did not decide; `wrong` is on
  * the device */
 int ftk_test_exp_pairs(int dtype, unsigned long long* wrong, ftk_stream_t stream);
+/* the same for bfloat16 with the bounds that are for columns far below the maximum */
+int ftk_test_exp_pairs_wide(unsigned long long* wrong, ftk_stream_t stream);
 /* draws `n_draws` uniforms per row into out[row*n_draws + i], advancing the states */
 int ftk_test_rng_uniform(ftk_rng_state* states, float* out, int batch_size, int n_draws, ftk_stream_t stream);
 /* non-zero: every top-p row takes the radix-sort fallback (exercises it on small inputs); process-wide */

@@ -119,6 +119,20 @@ def test_rounded_exponentials_of_every_pair(env, dt):
     assert 0 < again < (1 << 31)
 
 
+def test_rounded_exponentials_far_below_the_maximum(env):
+    """bfloat16: the bounds for far columns give the same bits, and they decide nearly all of them. (Bounds with a fixed
+    absolute part decide no value further than some 36 below the maximum, more than half of these pairs.)"""
+    torch, _, ops = env
+    wrong = torch.zeros(2, dtype=torch.int64, device="cuda")
+    ops.check(ops.ftk_hooks().ftk_test_exp_pairs_wide(wrong.data_ptr(), ops.current_stream()))
+    _sync(torch)
+    bad, again = wrong.tolist()
+    assert bad == 0
+    # (maxima from 2^20 on are left to the exact form throughout; below, what lies within a few units of 2^-23 of a tie)
+    maxima = (np.arange(65536, dtype=np.uint32) << 16).view(np.float32)
+    assert again < ((np.abs(maxima) >= 1 << 20).sum() + 0.01 * 65536) * 32768
+
+
 def test_device_division_by_a_shared_reciprocal(env):
     """The softmax divides a row by one denominator with the reciprocal's part of the division computed once:
     bit for bit numpy's IEEE quotient, for numerators over the whole range an exponential can take (zero,

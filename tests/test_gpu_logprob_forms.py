@@ -29,6 +29,12 @@ def _case(torch, dt, B, V, Vp, H, k, seed, kind):
         x[2, 7] = float("inf")
         x[3, :] = float("-inf")
         x[3, 11] = 0.0
+    elif kind == "far":  # columns up to a hundred below the maximum, and masked ones of three kinds
+        x *= 4.0
+        masks = torch.rand((B, Vp), generator=gen, device="cuda") < 0.03
+        lows = torch.tensor([float("-inf"), -1e4, -O.max_t(dt), -60.0], device="cuda")
+        x = torch.where(masks, lows[torch.arange(B, device="cuda") % 4][:, None], x)
+        x[:, 3 * Vp // 4:] -= 25.0
     history = torch.randint(0, V, (H, B), generator=gen, device="cuda", dtype=torch.int32)
     if kind == "edges":  # the largest values in the row's first and last columns, all of them in the history
         x[:, :8] += 20.0
@@ -55,6 +61,10 @@ CASES = [
     (O.BF16, 13, 1024, 1027, 16, 8, "edges"),       # rows off 16-byte boundaries whose maxima lie in the columns in
     (O.F32, 11, 4999, 5001, 16, 30, "edges"),       # front of the first whole vector and behind the last
     (O.F16, 19, 33001, 33003, 16, 64, "edges"),
+    (O.BF16, 12, 50257, 50257, 16, 40, "far"),
+    (O.BF16, 12, 9001, 9001, 16, 40, "far"),        # less than one batch of columns per thread
+    (O.BF16, 300, 33001, 33002, 16, 20, "far"),
+    (O.F16, 12, 50257, 50257, 16, 40, "far"),
 ]
 
 
