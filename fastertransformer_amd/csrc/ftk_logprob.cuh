@@ -877,9 +877,9 @@ __global__ void __launch_bounds__(LP_THREADS) lp_row_kernel(FusedParams p, Fused
 // chains of the reference's 1024, so the sum has the reference's order without any regrouping. First pass: the row's
 // maximum after temperature, penalties and masks, and every thread's own largest value, from which the bound of the
 // candidates follows (the k-th largest of 256 joined thread maxima, each of them a column of its own). Second pass (the
-// row comes from the caches this time): e = T(exp(y - max)) summed chain by chain. Then the candidates, out of the few
-// groups of vectors whose largest raw value reaches the bound. Then
-// all waves but four leave and those finish like lp_row_kernel (lp_finish).
+// row comes from the caches this time): e = T(exp(y - max)) summed chain by chain, of fp32 rows with the candidates on the
+// way; those of 16-bit rows are looked for afterwards, in the few groups of vectors whose largest raw value reaches the
+// bound. Then all waves but four leave and those finish like lp_row_kernel (lp_finish).
 // THREADS = 1024 for launches of at most one row per compute unit; with more rows, workgroups of fewer threads share a
 // compute unit and one's first pass (memory) runs beside another's second (arithmetic).
 constexpr int LPW_THREADS = 1024;
@@ -900,11 +900,11 @@ __device__ __forceinline__ bool lp_rare(bool mine)
 // Bound by the arithmetic of the second pass (vector instructions, and its waits where only eight waves share a compute
 // unit). 1024 x 152064 f16, k = 64: 166 us a step with every column through det_expf, columns one by one and candidates
 // looked for in both passes; 141 us now. 16-bit types hold their values in pairs and take det_expf only where the
-// hardware's exponential leaves the rounding open (ftk_exp16.cuh), the first pass looks at raw values alone, candidates
+// hardware's exponential leaves the rounding open (ftk_exp16.cuh), the first pass looks at raw values alone, 16-bit candidates
 // are looked for in some ninety groups of 64 columns, and flags of the history cost a bit test per sixteen columns. Other
 // sizes, us before / now: 256 x 152064 f16 53.7 / 48.7, 512 x 50257 f16 51.9 / 45.2, 1024 x 32000 bf16 56.6 / 43.5, 256 x
-// 128256 f16 with 2000 ids of history 70.8 / 58.1, 8 x 50257 f32 25.2 / 23.1, 400 x 152064 f32 96.0 / 91.7; rows that
-// exceed the last-level cache lose some of it to the second look at the groups (1024 x 152064 f32 206 / 213).
+// 128256 f16 with 2000 ids of history 70.8 / 58.1, 8 x 50257 f32 24.0 / 22.9, 400 x 152064 f32 89.2 / 85.8, 1024 x 152064
+// f32 203 / 199.
 template<int DT, int BMW, int THREADS>
 __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLaunch l, LogProbLaunch lp)
 {
@@ -914,6 +914,10 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     constexpr int         CH = LP_BLOCK / THREADS;     // neighbouring chains of a thread
     constexpr int         N  = WORD16 ? 16 : 8;        // columns of a thread's batch
     constexpr int         U  = N / CH;                 // ... in rounds of 1024 columns
+    // Candidates are gathered on the way of the sum: two more operations per four columns. fp32 rows looked at again after the
+    // sum are out of the second-level cache by then (us a step, again / on the way: 8 x 50257 23.1 / 22.9, 256 x 128256
+    // 50.4 / 48.5, 400 x 152064 87.2 / 85.8, 512 x 152064 113.6 / 107.5, 2048 x 50257 150.5 / 140.2, 1024 x 152064 212 / 199).
+    constexpr bool        IN_SUM = !WORD16;
     constexpr int         NR = WORD16 && CH > 1 ? N / 2 : N;  // registers a batch is loaded into
     constexpr int         NY = WORD16 ? N / 2 : N;            // ... and its values, 16-bit types in pairs
     static_assert(THREADS * CH == LP_BLOCK && U * CH == N && THREADS % 32 == 0 && THREADS >= TK_THREADS,
@@ -1177,7 +1181,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         }
     };
     // The second pass over the row: whole batches with the next one's loads issued before the current one is used,
-    // then the columns behind them in a batch that ends with -inf. use_batch(y, rounds) takes a batch's values, as
+    // then the columns behind them in a batch that ends with -inf. use_batch(v0, y, rounds) takes a batch's values, as
     // many rounds of them as there are.
     auto stream = [&](auto&& use_batch) {
         if (nfull > 0) {
@@ -1196,7 +1200,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                     Val       y[NY];
                     const int v0 = (b0 + r) * U * LP_BLOCK + CH * t;
                     values(std::true_type(), v0, buf[r], y);
-                    use_batch(y, U);
+                    use_batch(v0, y, U);
                 }
             }
         }
@@ -1205,7 +1209,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             Val       y[NY];
             const int v0 = nfull * U * LP_BLOCK + CH * t;
             some_values(v0, y);
-            use_batch(y, (rest + LP_BLOCK - 1) / LP_BLOCK);
+            use_batch(v0, y, (rest + LP_BLOCK - 1) / LP_BLOCK);
         }
     };
 
@@ -1215,8 +1219,8 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     // maximum itself; instead every history id looks whether its raw value is the largest of the thread that owns its
     // column. Such a thread says nothing about its columns (nothing follows for the candidates' bound), unless its raw
     // maximum lies above everything else: then a wave goes through its vectors with the flags at hand.
-    // The maxima of groups of a thread's vectors stay behind in the candidates' array: once the bound is there they tell
-    // which groups to look into for candidates.
+    // 16-bit types: the maxima of groups of a thread's vectors stay behind in the candidates' array: once the bound is there
+    // they tell which groups to look into for candidates.
     constexpr int GROUPS = 2 * TK_CCAP / THREADS;  // per thread
     const float   mul     = rowctx.fast_mul;
     const bool    ordered = mul > 0.0f && mul < __builtin_inff();  // the plain transform keeps the order
@@ -1257,7 +1261,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             }
             group   = __builtin_fmaxf(group, most);
             raw_own = __builtin_fmaxf(raw_own, most);
-            if (((q0 + R1) & ((1 << glog) - 1)) == 0 || q0 + R1 >= turns) {
+            if (!IN_SUM && (((q0 + R1) & ((1 << glog) - 1)) == 0 || q0 + R1 >= turns)) {
                 group_max[(q0 >> glog) * THREADS + t] = group;
                 group                                 = NEG_INF;
             }
@@ -1384,7 +1388,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
         valid         = true;
     }
 
-    // ---- where the candidates are: groups of vectors with a raw value that the bound does not rule out
+    // ---- where the candidates of a 16-bit row are: groups of vectors with a raw value that the bound does not rule out
     // (the list lies where the selection keeps its own later on)
     int*      parked    = s.sel.idx;
     float     raw_floor = NEG_INF;
@@ -1393,9 +1397,9 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     // end id is considered whatever its raw value)
     const int end_vector =
         rowctx.masked_end_id >= 0 && rowctx.masked_end_id < p.V ? vector_of(rowctx.masked_end_id) : -1;
-    if (valid && ordered) {
+    if (!IN_SUM && valid && ordered) {
         // an unflagged column with e >= thr_low has at least this raw value (e's rounding, the logarithm's, y's)
-        const float rounding = DT == DT_F32 ? 0.99999f : (DT == DT_F16 ? (thr_low < 2.44140625e-04f ? 0.4f : 0.998f) : 0.98f);
+        const float rounding = DT == DT_F16 ? (thr_low < 2.44140625e-04f ? 0.4f : 0.998f) : 0.98f;
         float       y        = row_max + det_logf(thr_low * rounding);
         y                    = lean_below_rounding<DT>(y - __builtin_fabsf(row_max) * 1e-6f - 1e-5f) / mul;
         y                    = y - __builtin_fabsf(y) * 1e-6f;
@@ -1435,7 +1439,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     if constexpr (THREADS < LPW_THREADS) {
         __builtin_amdgcn_s_setprio(0);
     }
-    // ---- second pass: the sum chain by chain
+    // ---- second pass: the sum chain by chain, and the candidates of an fp32 row
     float acc[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -1456,6 +1460,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             return 0;
         }
     }();
+    const float        sum_low = valid ? thr_low : __builtin_inff();  // of a column that the sum keeps as a candidate
     unsigned long long far = 0ull;  // bfloat16: lanes that have met columns far below the maximum
     // e of slots [j0, j0 + G) of a batch. 16-bit types: half a batch in a straight line (a wave waits for every branch).
     constexpr int G = WORD16 ? 8 : 4;
@@ -1484,12 +1489,23 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             ex.template numerators<G / 2>(y + j0 / 2, e + j0 / 2, far);
         }
     };
-    auto add_batch = [&](auto wide, const Val* y, int rounds) __attribute__((always_inline)) {
+    auto add_batch = [&](auto wide, int v0, const Val* y, int rounds) __attribute__((always_inline)) {
 #pragma unroll
         for (int j0 = 0; j0 < N; j0 += G) {
             if (j0 / CH < rounds) {  // (whole batches: always)
                 Val e[NY];
                 numerators(wide, y, e, j0);
+                if constexpr (IN_SUM) {
+                    const float top = __builtin_fmaxf(__builtin_fmaxf(e[j0], e[j0 + 1]), __builtin_fmaxf(e[j0 + 2], e[j0 + 3]));
+                    if (lp_rare(top >= sum_low)) {  // (a NaN is no candidate)
+#pragma unroll
+                        for (int j = j0; j < j0 + G; ++j) {
+                            if (e[j] >= sum_low && v0 + offset_of(j) < p.V) {
+                                push(v0 + offset_of(j), e[j]);
+                            }
+                        }
+                    }
+                }
                 // (slots of a chain in ascending order of their columns)
 #pragma unroll
                 for (int j = j0; j < j0 + G; ++j) {
@@ -1504,13 +1520,13 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
             }
         }
     };
-    stream([&](const Val* y, int rounds) __attribute__((always_inline)) {
+    stream([&](int v0, const Val* y, int rounds) __attribute__((always_inline)) {
         // (bfloat16: from the first far column on a wave takes the wide bounds for the rest of its columns)
         if (DT == DT_BF16 && __builtin_expect(far != 0ull, 0)) {
-            add_batch(std::integral_constant<bool, DT == DT_BF16>(), y, rounds);
+            add_batch(std::integral_constant<bool, DT == DT_BF16>(), v0, y, rounds);
         }
         else {
-            add_batch(std::false_type(), y, rounds);
+            add_batch(std::false_type(), v0, y, rounds);
         }
     });
     const float pad_e = p.V < p.Vp ? round_t<DT>(det_expf_nonpos(-S::max_t() - row_max)) : 0.0f;
@@ -1553,8 +1569,8 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     }
     const float denom = uniform_f(total + 1e-6f);
     const float u     = __int_as_float(s.misc[0]);
-    // the candidates: the columns at or above the bound in the groups kept in mind (the whole row where raw values say
-    // nothing), a vector per thread and turn, and those outside the whole vectors
+    // the candidates of a 16-bit row: the columns at or above the bound in the groups kept in mind (the whole row where raw
+    // values say nothing), a vector per thread and turn, and those outside the whole vectors
     const int n_parked = __builtin_amdgcn_readfirstlane(s.misc[1]);
     if (valid && n_parked <= TK_CCAP) {
         auto consider = [&](int v) {
@@ -1563,7 +1579,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                 push(v, e);
             }
         };
-        const int vectors = ordered ? n_parked << glog : nvec;
+        const int vectors = IN_SUM ? 0 : ordered ? n_parked << glog : nvec;
 #pragma unroll 1
         for (int i = t; i < vectors; i += THREADS) {
             const int rel = ordered ? parked[i >> glog] + (i & ((1 << glog) - 1)) * THREADS : i;
@@ -1586,7 +1602,9 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
                 }
             }
         }
-        for_outer(consider);
+        if (!IN_SUM) {
+            for_outer(consider);
+        }
         if (pad_e > 0.0f && pad_e >= thr_low) {
             for (int v = p.V + t; v < p.Vp; v += THREADS) {
                 push(v, pad_e);
