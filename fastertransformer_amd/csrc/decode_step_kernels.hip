@@ -31,8 +31,20 @@ __device__ __forceinline__ MaxSum merge(MaxSum a, MaxSum b)
     return MaxSum{M, a.s * __expf(a.m - M) + b.s * __expf(b.m - M)};
 }
 
-// ONCE: the logits are more than the caches keep, and go past them. 64 x 32 rows of 50257 fp16 (206 MB): 33.7 us, 34.8
-// without (traced), 4.6 TB/s.
+// A 16-byte load of a row that goes past the caches but takes what the last-level cache holds (cache bits nt, sc0 and sc1: with
+// nt alone, 40 x 32 rows of 50257 fp16 that were written just before take 33.5 us a call instead of 28.9).
+__device__ __forceinline__ uint4 once_load(const uint4* row, int n, int i)
+{
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    constexpr int        SC0 = 1, NT = 2, SC1 = 16;
+    const u4             v   = __builtin_amdgcn_raw_buffer_load_b128(
+        __builtin_amdgcn_make_buffer_rsrc((void*)row, 0, n * 16, 0x00027000), i * 16, 0, SC0 | NT | SC1);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// Bound by memory: 64 x 32 rows of 50257 fp16 (206 MB) at 5.1 TB/s. ONCE: the logits are more than the second-level caches
+// keep, and go past them. Then no two waves share a cache line, which would be fetched for each of them: vectors start at a
+// multiple of 128 bytes (rows at any offset: 48 x 32 x 50257 fp16, written just before, 40.9 us a call without, 35.8).
 template<int DT, bool ONCE>
 __global__ void __launch_bounds__(LP_THREADS)
 log_probs_kernel(float* __restrict__ log_probs, const typename Storage<DT>::T* __restrict__ logits,
@@ -73,8 +85,10 @@ log_probs_kernel(float* __restrict__ log_probs, const typename Storage<DT>::T* _
         acc.s += add;
     };
 
-    // columns before the first 16-byte boundary and after the last whole vector go one by one
-    const int a     = (int)(((16u - ((uintptr_t)row & 15u)) & 15u) / sizeof(T));
+    // columns before the first 16-byte (ONCE: 128-byte) boundary and after the last whole vector go one by one
+    constexpr unsigned START = ONCE ? 128 : 16;
+    static_assert(START / sizeof(T) <= LP_THREADS, "a column per thread");
+    const int a     = (int)((-(uintptr_t)row & (START - 1)) / sizeof(T));
     const int head  = a < V ? a : V;
     const int nvec  = (V - head) / EPV;
     const int tail0 = head + nvec * EPV;
@@ -89,7 +103,7 @@ log_probs_kernel(float* __restrict__ log_probs, const typename Storage<DT>::T* _
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = i0 + u * LP_THREADS;
-            raw[u]      = i >= nvec ? make_uint4(0, 0, 0, 0) : ONCE ? stream_load(vec + i) : vec[i];
+            raw[u]      = i >= nvec ? make_uint4(0, 0, 0, 0) : ONCE ? once_load(vec, nvec, i) : vec[i];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -304,22 +318,28 @@ int ftk_invoke_log_prob_from_logits(int dtype, float* cum_log_probs, const void*
         if (rows > 0x7FFFFFFFull) {
             return FTK_ERR_ARGUMENT;
         }
-        // Past the caches where they cannot hold the logits anyway, us a call through them / past them: 64 x 32 x 50257
-        // fp16 39.2 / 35.9, 128 x 32 x 24000 fp16 33.4 / 32.2; fp32 30 x 32 x 50257 30.0 / 30.4, 48 x 8 x 128256 40.2 /
-        // 40.3; what the second-level caches (32 MB) may hold loses: 16 x 8 x 50257 bfloat16 10.8 / 13.2.
-        const size_t bytes = max_input_length * batch_size * vocab_size_padded * (dtype == FTK_DTYPE_F32 ? 4 : 2);
-        const bool   once  = dtype != FTK_DTYPE_F32 && bytes >= ((size_t)64 << 20);
-        auto         run   = [&](auto past) {
-            constexpr bool ONCE = decltype(past)::value;
-            FTK_DISPATCH_DTYPE(dtype, log_probs_kernel<DT, ONCE><<<(unsigned)rows, LP_THREADS, 0, st>>>(
-                                          log_probs, (const Storage<DT>::T*)logits, input_ids, input_lengths,
-                                          (int)max_input_length, (int)batch_size, (int)vocab_size, vocab_size_padded,
-                                          batch_first));
-            return 0;
+        // Past the caches, 16-bit types from 64 MB on. us a call of fp16, through the caches / past them, with logits that
+        // were written just before / that were not: 16 x 16 x 50257 (25 MB) 14.9 / 15.0, 16.5 / 16.8; 40 x 16 x 50257 (64 MB)
+        // 20.5 / 20.2, 21.7 / 21.2; 64 x 16 x 50257 24.7 / 24.5, 27.8 / 25.8; 40 x 32 x 50257 29.0 / 29.9, 32.8 / 30.1; 48 x
+        // 32 x 50257 33.0 / 35.8, 37.1 / 34.9; 64 x 32 x 50257 40.0 / 44.6, 45.3 / 40.7; 96 x 32 x 50257 (more than the
+        // last-level cache) 71.1 / 61.2, 63.2 / 55.4. (the descriptor of a row holds its bytes in 32 bits)
+        const bool once = dtype != FTK_DTYPE_F32 && vocab_size_padded < ((size_t)1 << 30)
+                          && max_input_length * batch_size * vocab_size_padded * 2 >= ((size_t)64 << 20);
+        auto       run  = [&](auto dt, auto past) {
+            constexpr int DT = decltype(dt)::value;
+            log_probs_kernel<DT, decltype(past)::value><<<(unsigned)rows, LP_THREADS, 0, st>>>(
+                log_probs, (const typename Storage<DT>::T*)logits, input_ids, input_lengths, (int)max_input_length, (int)batch_size,
+                (int)vocab_size, vocab_size_padded, batch_first);
         };
-        const int rc = once ? run(std::true_type()) : run(std::false_type());
-        if (rc != 0) {
-            return rc;
+        auto run16 = [&](auto dt) { once ? run(dt, std::true_type()) : run(dt, std::false_type()); };
+        if (dtype == FTK_DTYPE_F32) {
+            run(std::integral_constant<int, DT_F32>(), std::false_type());
+        }
+        else if (dtype == FTK_DTYPE_F16) {
+            run16(std::integral_constant<int, DT_F16>());
+        }
+        else {
+            run16(std::integral_constant<int, DT_BF16>());
         }
         FTK_LAUNCH_CHECK();
     }

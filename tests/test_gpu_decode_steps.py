@@ -64,6 +64,13 @@ def test_log_prob_from_large_logits(dt, V):
     test_log_prob_from_logits(dt, V == 131068, (8, 32, V))
 
 
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("shape", [(1024, 33, 1003), (4096, 256, 33)])
+def test_log_prob_from_large_logits_line_offsets(dt, shape):
+    """Past the caches a row's vectors start at a 128-byte boundary: rows at every offset from one, and rows that end before it."""
+    test_log_prob_from_logits(dt, False, shape)
+
+
 def test_log_prob_masked_logits():
     """rows holding -inf entries (banned tokens) and one row that is -inf everywhere except the target"""
     import torch
