@@ -1329,33 +1329,51 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     if (t == 0) {
         s.misc[0] = __float_as_int(row_uniform(l.rng, l.uniforms, row));  // (read behind the barriers of the sum)
     }
-    seen   = wave_max(seen);
-    unsure = wave_max(unsure);
+    seen                      = wave_max(seen);
+    const float unsure_of_all = wave_max(unsure);
     if (lane_id() == 0) {
         redf[wave_id()]     = seen;
-        warp_sum[wave_id()] = unsure;
+        warp_sum[wave_id()] = unsure_of_all;
     }
     __syncthreads();
     constexpr int NW      = THREADS / WAVE;
     float         row_max = wave_max(lane_id() < NW ? redf[lane_id()] : NEG_INF);
     if (wave_max(lane_id() < NW ? warp_sum[lane_id()] : NEG_INF) > row_max) {  // (the same for every wave)
-        // the vectors of the threads in question, one thread's by a wave (lane i looks at the marks of word i)
-        float          found = NEG_INF;
-        int            n     = 0;
-        const uint32_t marks = lane_id() < THREADS / 32 ? slot_key[lane_id()] : 0u;
-        for (unsigned long long words = __ballot(marks != 0u); words != 0ull; words &= words - 1ull) {
-            const int w = __builtin_ctzll(words);
-            for (uint32_t bits = (uint32_t)__shfl((int)marks, w, WAVE); bits != 0u; bits &= bits - 1u) {
-                const int who = w * 32 + __builtin_ctz(bits);
-                if (!(rowctx.fast(u2f(wide_key[who])) > row_max) || n++ % NW != wave_id()) {
-                    continue;
+        // the vectors of the threads in question again, past the columns that have values of their own: each wave those of its
+        // lanes, two lanes' at a time
+        float found = NEG_INF;
+        for (unsigned long long again = __ballot(unsure > row_max); again != 0ull;) {
+            const int one = __builtin_ctzll(again);
+            again &= again - 1ull;
+            const int other = again != 0ull ? __builtin_ctzll(again) : one;
+            again &= again - 1ull;
+            for (int q = 0; q < turns; q += WAVE) {
+                uint4 v[2];
+                int   rel[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    rel[i] = (q + lane_id()) * THREADS + (t & ~(WAVE - 1)) + (i == 0 ? one : other);
+                    v[i]   = base[vlo + min(rel[i], nvec - 1)];
                 }
-                for (int rel = lane_id() * THREADS + who; rel < nvec; rel += WAVE * THREADS) {
-                    found = __builtin_fmaxf(found, lp_vector_max<DT, BMW>(rowctx, base[vlo + rel], (vlo + rel) * EPV - a,
-                                                                         a, bitsv, ordered));
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int      first = (vlo + rel[i]) * EPV - a;
+                    const uint32_t end   = (uint32_t)(rowctx.masked_end_id - first);
+                    uint32_t       bits  = end < (uint32_t)EPV ? 1u << end : 0u;
+                    if (rel[i] >= nvec) {
+                        bits = (1u << EPV) - 1u;
+                    }
+                    else if (bitsv) {
+                        bits |= rowctx.vector_bits(first, EPV);
+                    }
+#pragma unroll
+                    for (int j = 0; j < EPV; ++j) {
+                        found = __builtin_fmaxf(found, (bits >> j) & 1u ? NEG_INF : vector_element<DT>(v[i], j));
+                    }
                 }
             }
         }
+        found = rowctx.fast(found);
         __syncthreads();
         row_max = __builtin_fmaxf(row_max, block_max<float, NW>(found, redf, NEG_INF));
     }
