@@ -1589,8 +1589,10 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     const float u     = __int_as_float(s.misc[0]);
     // the candidates of a 16-bit row: the columns at or above the bound in the groups kept in mind (the whole row where raw
     // values say nothing), a vector per thread and turn, and those outside the whole vectors
-    const int n_parked = __builtin_amdgcn_readfirstlane(s.misc[1]);
-    if (valid && n_parked <= TK_CCAP) {
+    const int   n_parked = __builtin_amdgcn_readfirstlane(s.misc[1]);
+    const float e_bound  = key_to_float(thr);
+    const bool  covered  = valid && lp_gather_covers<DT>(e_bound, denom);
+    if (covered && n_parked <= TK_CCAP) {
         auto consider = [&](int v) {
             const float e = round_t<DT>(det_expf_nonpos(value(v, rowp[v]) - row_max));
             if (e >= thr_low) {  // (a NaN is no candidate)
@@ -1633,8 +1635,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     int  n     = __builtin_amdgcn_readfirstlane(s.n_cand);
     bool probs = false;
     __syncthreads();
-    const float e_bound = key_to_float(thr);
-    if (n_parked > TK_CCAP || n > TK_CCAP || !valid || !lp_gather_covers<DT>(e_bound, denom)) {
+    if (!covered || n_parked > TK_CCAP || n > TK_CCAP) {
         // (fewer than k columns with e > 0: columns of probability zero are picked too, by the reference's tie rules)
         probs = true;
         n     = lp_regather<DT, THREADS>(
