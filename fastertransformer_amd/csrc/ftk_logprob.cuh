@@ -15,9 +15,10 @@
 //      T(e_v / (sum + 1e-6)), the reference's tie orders are replayed on them and the row is sampled
 //      (topk_select_lds with probabilities in). Rows it cannot bound take the literal replay on probabilities
 //      computed on the fly.
-// Two forms:
+// Three forms:
 //   lp_wide_kernel - the product's: one launch, one workgroup of 1024, 512 or 256 threads per row does both reads
 //                    (the second one comes from the caches), a thread owning 1, 2 or 4 whole summation chains;
+//   lp_short_kernel (ftk_logprob_short.cuh) - the product's for short rows: the same, column by column;
 //   lp_rowmax_kernel + lp_row_kernel - two launches: the first streams the row in the launch shape of the lean
 //                    gather and leaves the maximum of every workgroup's share in the workspace, the second gives
 //                    a row to one 256-thread workgroup whose threads own four neighbouring chains each and walk

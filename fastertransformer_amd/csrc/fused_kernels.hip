@@ -24,7 +24,7 @@
 #include "ftk_fused.cuh"
 #include "ftk_largek.cuh"
 #include "ftk_lean.cuh"
-#include "ftk_logprob.cuh"
+#include "ftk_logprob_short.cuh"
 #include "ftk_rowwide.cuh"
 
 namespace ftk {
@@ -175,6 +175,28 @@ static int lp_threads_per_row(int rows, int vocab_size)
     return rows >= 1024 && vocab_size <= 65536 ? 256 : 512;
 }
 
+// Rows that lp_short_kernel takes, with as many threads: where the arithmetic that lp_wide_kernel saves is less than the
+// latency that it adds, or its batches of 16 columns per thread (16-bit types) are hardly filled. us a step, wide / short,
+// the history drawn at random: f16 256 rows x 12288 18.9 / 18.0, 18000 24.3 / 19.4, 26000 24.1 / 22.3, 28000 23.0 / 22.8,
+// 32000 22.3 / 23.5, 34000 24.8 / 23.8, 36000 23.7 / 24.5; 16 x 16384 22.1 / 23.0, 20000 20.8 / 19.7; 300 x 8192 18.6 / 19.3, 8193
+// 22.3 / 19.4, 11000 22.2 / 21.4, 13000 22.1 / 22.8; 1024 x 2048 20.3 / 18.1, 4096 20.8 / 21.5; f32 256 x 9000 17.3 / 16.2, 18000
+// 19.3 / 19.0, 20000 19.0 / 19.5; 300 x 2048 15.5 / 15.1, 4096 15.8 / 16.5; 1024 x 1100 17.3 / 16.7, 2048 17.2 / 18.0. With the 32
+// largest columns in the history wide takes 2 to 3 us more, short 0.2.
+static bool lp_short_rows(int dtype, int rows, int vocab_size)
+{
+    const bool f32 = dtype == FTK_DTYPE_F32;
+    if (rows >= 1024) {
+        return vocab_size < (f32 ? 2048 : 3072);
+    }
+    if (rows > 256) {
+        return f32 ? vocab_size < 3072 : vocab_size < 12288 && vocab_size % 8192 != 0;
+    }
+    if (f32) {
+        return vocab_size <= 18432;
+    }
+    return vocab_size < 16384 || (vocab_size <= 35840 && vocab_size % 16384 != 0 && vocab_size % 16384 < 11264);
+}
+
 #ifdef FTK_TEST_HOOKS
 // Test hook (hooks build of the library only): non-zero sends every launch through the general stream, so
 // that it can be compared with the lean gather on the shapes the lean gather normally takes.
@@ -184,11 +206,11 @@ extern "C" void ftk_test_set_fused_force_general(int v)
     g_fused_force_general = v;
 }
 // Test hook: the form of the log-prob step. 0: the product's choice, 1: two launches, 1024 / 512 / 256: one launch
-// with that many threads per row.
+// with that many threads per row, -1024 / -512 / -256: lp_short_kernel with that many (not with large windows).
 static int g_lp_form = 0;
 extern "C" void ftk_test_set_lp_form(int v)
 {
-    g_lp_form = (v == 1 || v == 1024 || v == 512 || v == 256) ? v : 0;
+    g_lp_form = (v == 1 || v == 1024 || v == 512 || v == 256 || v == -1024 || v == -512 || v == -256) ? v : 0;
 }
 // Test hook: non-zero keeps launches with a large k on the two launches of the lean gather also where one
 // 1024-thread workgroup per row would make their lists in one.
@@ -427,40 +449,44 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
             lp.partial_max      = (float*)l.headers;  // one float per list header slot: the lists are not used
             lp.splits           = lplan.splits;
             hipEvent_t e0, e1;
-            const int lp_threads = g_lp_form == 0 ? lp_threads_per_row(rows, a->vocab_size) : (g_lp_form == 1 ? 0 : g_lp_form);
-            if (lp_threads != 0) {
+            if (g_lp_form == 1) {
                 take_events(1, &e0, &e1);
                 if (e0 != nullptr) {
                     FTK_HIP_CHECK(hipEventRecord(e0, st));
                 }
-                rc = a->dtype == FTK_DTYPE_F32 ? lp_wide_launch_f32(window, lp_threads, rows, st, p, l, lp) :
-                     a->dtype == FTK_DTYPE_F16 ? lp_wide_launch_f16(window, lp_threads, rows, st, p, l, lp) :
-                                                 lp_wide_launch_bf16(window, lp_threads, rows, st, p, l, lp);
+                rc = a->dtype == FTK_DTYPE_F32 ? lp_rowmax_launch_f32(window, lgrid, st, p, l, lp) :
+                     a->dtype == FTK_DTYPE_F16 ? lp_rowmax_launch_f16(window, lgrid, st, p, l, lp) :
+                                                 lp_rowmax_launch_bf16(window, lgrid, st, p, l, lp);
+                if (rc != 0) {
+                    return rc;
+                }
+                if (e1 != nullptr) {
+                    FTK_HIP_CHECK(hipEventRecord(e1, st));
+                }
+                take_events(2, &e0, &e1);
+                if (e0 != nullptr) {
+                    FTK_HIP_CHECK(hipEventRecord(e0, st));
+                }
+                rc = a->dtype == FTK_DTYPE_F32 ? lp_row_launch_f32(window, rows, st, p, l, lp) :
+                     a->dtype == FTK_DTYPE_F16 ? lp_row_launch_f16(window, rows, st, p, l, lp) :
+                                                 lp_row_launch_bf16(window, rows, st, p, l, lp);
                 if (rc == 0 && e1 != nullptr) {
                     FTK_HIP_CHECK(hipEventRecord(e1, st));
                 }
                 return rc;
             }
+            const bool lp_short   = window != 2 && (g_lp_form == 0 ? lp_short_rows(a->dtype, rows, a->vocab_size) : g_lp_form < 0);
+            const int  lp_threads = g_lp_form != 0 ? abs(g_lp_form) : lp_threads_per_row(rows, a->vocab_size);
             take_events(1, &e0, &e1);
             if (e0 != nullptr) {
                 FTK_HIP_CHECK(hipEventRecord(e0, st));
             }
-            rc = a->dtype == FTK_DTYPE_F32 ? lp_rowmax_launch_f32(window, lgrid, st, p, l, lp) :
-                 a->dtype == FTK_DTYPE_F16 ? lp_rowmax_launch_f16(window, lgrid, st, p, l, lp) :
-                                             lp_rowmax_launch_bf16(window, lgrid, st, p, l, lp);
-            if (rc != 0) {
-                return rc;
-            }
-            if (e1 != nullptr) {
-                FTK_HIP_CHECK(hipEventRecord(e1, st));
-            }
-            take_events(2, &e0, &e1);
-            if (e0 != nullptr) {
-                FTK_HIP_CHECK(hipEventRecord(e0, st));
-            }
-            rc = a->dtype == FTK_DTYPE_F32 ? lp_row_launch_f32(window, rows, st, p, l, lp) :
-                 a->dtype == FTK_DTYPE_F16 ? lp_row_launch_f16(window, rows, st, p, l, lp) :
-                                             lp_row_launch_bf16(window, rows, st, p, l, lp);
+            const auto launch_lp =
+                lp_short ? (a->dtype == FTK_DTYPE_F32 ? lp_short_launch_f32 :
+                            a->dtype == FTK_DTYPE_F16 ? lp_short_launch_f16 : lp_short_launch_bf16) :
+                           (a->dtype == FTK_DTYPE_F32 ? lp_wide_launch_f32 :
+                            a->dtype == FTK_DTYPE_F16 ? lp_wide_launch_f16 : lp_wide_launch_bf16);
+            rc = launch_lp(window, lp_threads, rows, st, p, l, lp);
             if (rc == 0 && e1 != nullptr) {
                 FTK_HIP_CHECK(hipEventRecord(e1, st));
             }

@@ -45,7 +45,8 @@ void ftk_test_set_fused_two_launches(int enable);
    -1 before the first step */
 int ftk_test_last_fused_path(void);
 /* the form of the fused log-prob step: 0 the product's choice, 1 two launches (row maxima, then one 256-thread
-   workgroup per row), 1024 / 512 / 256 one launch with that many threads per row; process-wide */
+   workgroup per row), 1024 / 512 / 256 one launch with that many threads per row, -1024 / -512 / -256 the kernel for short rows with that many
+   threads (where the row's history bitmap fits its LDS window); process-wide */
 void ftk_test_set_lp_form(int form);
 /* non-zero keeps launches with a large k (beyond 192) on the two launches of the lean gather also where one
    1024-thread workgroup per row would make the rows' lists in one launch; process-wide */

@@ -1,5 +1,5 @@
 """The fused top-k step with log-probs has several launch forms (csrc/ftk_logprob.cuh): row maxima and rows in two
-launches, or one launch with 1024, 512 or 256 threads per row. All of them add the row's exponentials in the
+launches, or one launch with 1024, 512 or 256 threads per row, of which short rows have one of their own. All of them add the row's exponentials in the
 reference's order (src/fastertransformer/kernels/sampling_topp_kernels.cu:1308-1344: thread t of 1024 adds columns
 t, t + 1024, ... one after the other, then butterflies), so ids, lengths, finished flags and both log-prob outputs
 must agree bit for bit between the forms, whatever the batch; parity of the product's own choice with the oracle is
@@ -12,7 +12,7 @@ from helpers import DTYPE_NAMES
 
 pytestmark = [pytest.mark.gpu, pytest.mark.timeout(600)]
 
-FORMS = (1, 1024, 512, 256)  # ftk_test_set_lp_form
+FORMS = (1, 1024, 512, 256, -1024, -512, -256)  # ftk_test_set_lp_form
 
 
 def _case(torch, dt, B, V, Vp, H, k, seed, kind):
@@ -95,7 +95,7 @@ def test_forms_of_the_log_prob_step_agree_bit_for_bit(dt, B, V, Vp, H, k, kind):
     for form in FORMS[1:]:
         for name, a, b in zip(("ids", "sequence_length", "finished", "cum_log_probs", "output_log_probs"), ref,
                               results[form]):
-            assert np.array_equal(a, b), "%s differ between the two-launch form and %d threads per row" % (name, form)
+            assert np.array_equal(a, b), "%s differ between the two-launch form and form %d" % (name, form)
 
 
 RAISING = [
@@ -131,7 +131,7 @@ def test_forms_agree_whatever_the_penalty_does_to_the_largest_values(dt, B, V, V
         hooks.ftk_test_set_lp_form(0)
     for form in FORMS[1:]:
         for a, b in zip(results[FORMS[0]], results[form]):
-            assert np.array_equal(a, b), "%d threads per row" % form
+            assert np.array_equal(a, b), "form %d" % form
 
 
 PEAKED = [
