@@ -60,6 +60,10 @@ HIP_FLAGS = [
 HOOK_UNITS = [("fused_kernels.hip", "fused_kernels.o"), ("topp_kernels.hip", "topp_kernels.o"),
               ("topp_sample_kernels.hip", "topp_sample_kernels.o"), ("criteria_kernels.hip", "criteria_kernels.o"),
               ("beam_kernels.hip", "beam_kernels.o")]
+# what only the hooks build has
+HOOK_ONLY_UNITS = [("logprob_two_kernels.hip", "logprob_two_kernels_f32.o", ["-DFTK_LP_DT=0"]),
+                   ("logprob_two_kernels.hip", "logprob_two_kernels_f16.o", ["-DFTK_LP_DT=1"]),
+                   ("logprob_two_kernels.hip", "logprob_two_kernels_bf16.o", ["-DFTK_LP_DT=2"])]
 
 
 def _run(cmd):
@@ -114,6 +118,12 @@ def build(force=True, verbose=True, with_torch=True):
         if force or _newer(obj, [path] + sorted(_includes(path))):
             hook_jobs.append([HIPCC] + HIP_FLAGS + ["-DFTK_TEST_HOOKS", "-c", path, "-o", obj])
         hook_objs[hook_objs.index(os.path.join(LIB, obj_name))] = obj
+    for src, obj_name, extra in HOOK_ONLY_UNITS:
+        path = os.path.join(CSRC, src)
+        obj = os.path.join(LIB, obj_name)
+        if force or _newer(obj, [path] + sorted(_includes(path))):
+            hook_jobs.append([HIPCC] + HIP_FLAGS + extra + ["-c", path, "-o", obj])
+        hook_objs.append(obj)
     with ThreadPoolExecutor(max_workers=4) as pool:
         list(pool.map(_run, hook_jobs))
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", os.path.join(LIB, "libftk_sampling_hooks.so")]

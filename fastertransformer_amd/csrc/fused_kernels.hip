@@ -449,6 +449,7 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
             lp.partial_max      = (float*)l.headers;  // one float per list header slot: the lists are not used
             lp.splits           = lplan.splits;
             hipEvent_t e0, e1;
+#ifdef FTK_TEST_HOOKS
             if (g_lp_form == 1) {
                 take_events(1, &e0, &e1);
                 if (e0 != nullptr) {
@@ -475,6 +476,7 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
                 }
                 return rc;
             }
+#endif
             const bool lp_short   = window != 2 && (g_lp_form == 0 ? lp_short_rows(a->dtype, rows, a->vocab_size) : g_lp_form < 0);
             const int  lp_threads = g_lp_form != 0 ? abs(g_lp_form) : lp_threads_per_row(rows, a->vocab_size);
             take_events(1, &e0, &e1);
