@@ -142,6 +142,13 @@ PEAKED = [
     (O.BF16, 4, 3001, 3001, 128, "level"),
     (O.F32, 4, 2050, 2056, 128, "alone"),   # one column, every other probability exactly zero
     (O.BF16, 4, 2050, 2050, 100, "few"),    # fewer numbers than k
+    (O.F16, 4, 40003, 40003, 64, "sharp"),  # the same in rows that are not short
+    (O.F16, 4, 40003, 40008, 128, "sharper"),
+    (O.F16, 4, 40003, 40003, 40, "plateau"),
+    (O.F32, 3, 20483, 20488, 16, "level"),
+    (O.BF16, 3, 40003, 40003, 128, "level"),
+    (O.F32, 4, 20050, 20056, 128, "alone"),
+    (O.BF16, 4, 40050, 40050, 100, "few"),
 ]
 
 
@@ -183,7 +190,8 @@ def test_rows_whose_candidates_are_gathered_again(dt, B, V, Vp, k, kind):
 
 
 @pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16], ids=lambda d: DTYPE_NAMES[d])
-@pytest.mark.parametrize("B,V,Vp,k", [(6, 1452, 1459, 5), (300, 1030, 1040, 20), (5, 2100, 3200, 130), (4, 9001, 9008, 8)])
+@pytest.mark.parametrize("B,V,Vp,k", [(6, 1452, 1459, 5), (300, 1030, 1040, 20), (5, 2100, 3200, 130), (4, 9001, 9008, 8),
+                                      (6, 40001, 40009, 5), (300, 13001, 13013, 20)])
 def test_masked_rows_count_their_pads(dt, B, V, Vp, k):
     """Rows masked throughout, with -inf or the type's lowest number: the pad columns hold -MAX_T and carry the softmax."""
     from decode_harness import Case, OracleRunner, ProductRunner, compare
@@ -208,11 +216,12 @@ def test_masked_rows_count_their_pads(dt, B, V, Vp, k):
 
 
 @pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16], ids=lambda d: DTYPE_NAMES[d])
-@pytest.mark.parametrize("B,V,Vp,k", [(8, 1452, 1459, 5), (8, 9001, 9001, 30), (264, 1030, 1041, 20), (1032, 1100, 1101, 8)])
+@pytest.mark.parametrize("B,V,Vp,k", [(8, 1452, 1459, 5), (8, 9001, 9001, 30), (264, 1030, 1041, 20), (1032, 1100, 1101, 8),
+                                      (8, 40001, 40003, 30), (264, 13001, 13008, 20), (1032, 4101, 4101, 8)])
 def test_masked_end_ids_count_in_masked_rows(dt, B, V, Vp, k):
     """Below the minimum length the end id has the type's lowest number, also where its logit is -inf or NaN: in rows without
-    anything larger it is one of the largest. 1024, 512 and 256 threads per row; end ids in the whole vectors of a row and
-    in front of and behind them."""
+    anything larger it is one of the largest. Short rows and others, with 1024, 512 and 256 threads per row; end ids in the
+    whole vectors of a row and in front of and behind them."""
     from decode_harness import Case, OracleRunner, ProductRunner, compare
     from helpers import uniforms
     rng = np.random.default_rng(V + dt)
