@@ -318,10 +318,12 @@ __device__ __noinline__ void rowwide_rare(TopkShared& ts, RowwideArgSegment segm
                                                p.end_ids, out);
 }
 
-// Requirements the launcher checks: rows start on 16-byte boundaries (so a vector never straddles a word of the
-// history bitmap and there are no columns in front of the first vector), no embedding bias, the largest k at most
-// LG_MAX_K, at least one whole vector per row, the row's history bitmap fits BMW words, and a history of at most
-// RW_HIST_U * RW_THREADS positions.
+// Requirements the launcher checks: rows start on 16-byte boundaries (ODD: where an element may), no embedding bias,
+// the largest k at most LG_MAX_K, at least 1024 columns, the row's history bitmap fits BMW words, and a history of at
+// most RW_HIST_U * RW_THREADS positions.
+// ODD: the vectors of a row start at its first 128-byte line; what lies in front of it (fewer than 64 columns of a
+// 16-bit type, 32 of fp32) goes the way of the columns behind the last whole vector. Bit 0 of the history bitmap is
+// `lead` columns in front of the row, so that a vector's flags never straddle two words.
 // Keeps a launch argument in a scalar register of its own from here on. Without it the compiler, short of scalar
 // registers, reads arguments again from the kernel-argument segment wherever they are used, and every such read
 // issued after the bulk of the row has been requested queues behind it.
@@ -332,7 +334,7 @@ __device__ __forceinline__ void rowwide_pin(V& v)
                         // such a store are no longer scalar loads)
 }
 
-template<int DT, int BMW>
+template<int DT, int BMW, bool ODD>
 __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideArgs a_in)
 {
     const FusedLaunch& l_in = a_in.l;
@@ -371,8 +373,11 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
     typedef unsigned int                                  u4 __attribute__((ext_vector_type(4)));
     typedef const __attribute__((address_space(1))) u4*   GlobalVec;
     unsigned long long base_addr = (unsigned long long)((const T*)p.logits + (size_t)row * p.Vp);
+    const int head = ODD ? (int)((0ull - base_addr) & 127ull) / (int)sizeof(T) : 0;  // columns in front of the vectors
+    const int lead = ODD ? -head & 31 : 0;
+    base_addr += (unsigned long long)head * sizeof(T);
     rowwide_pin(base_addr);
-    const int nvec = p.V / EPV;  // whole vectors inside columns [0, V)
+    const int nvec = (p.V - head) / EPV;  // whole vectors inside columns [head, V)
     const int    nsub = (nvec + RW_SUB_VECS - 1) / RW_SUB_VECS;
 
     // ---- Everything the row needs from memory is requested at once: the per-row arguments (scalar loads, ahead of
@@ -450,11 +455,17 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
     // issue until data returns and hold up the barriers of the set-up below. The rest of the ring follows once the
     // bitmap is built.
     load(0, 0);
+    // ODD: the columns outside the vectors, one each: the first wave has those in front, the others those behind
+    const int edge_v = !ODD ? p.V : (t < WAVE ? (t < head ? t : p.V) : head + nvec * EPV + t - WAVE);
+    T         edge   = (T)0;
+    if (ODD && edge_v < p.V) {
+        edge = ((const T*)p.logits + (size_t)row * p.Vp)[edge_v];
+    }
     // while all that is on its way: an empty bitmap of the row's history
     uint32_t* window = fused_lds_bitmap<BMW>();
     const bool counting = hist && p.frequencies != nullptr;  // a frequency penalty: the history's ids are counted too
     if (hist) {
-        const int words = min(BMW, (p.V + 31) / 32 + 1);
+        const int words = min(BMW, (p.V + lead + 31) / 32 + 1);
         for (int i = t; i < words; i += RW_THREADS) {
             window[i] = 0u;
         }
@@ -539,14 +550,14 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
             const int pos = t + u * RW_THREADS;
             const int id  = hist_ids[u];
             if (pos < p.step && id >= 0 && id < p.V && rowctx.history_position_counts(pos)) {
-                atomicOr(&window[id >> 5], 1u << (id & 31));
+                atomicOr(&window[(id + lead) >> 5], 1u << ((id + lead) & 31));
                 if (counting) {
                     fused_count_insert(s.count_table, id);
                 }
             }
         }
         rowctx.bm_mode   = 1;
-        rowctx.bm_origin = 0;
+        rowctx.bm_origin = -lead;
         if (counting) {
             rowctx.use_count_table(s.count_table);  // (read after the barrier below)
         }
@@ -604,9 +615,10 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
         return h;
     };
 
-    // flags of the vector that starts at column `first` (a multiple of EPV): one bit per column of the history
+    // flags of the vector that starts at column `first`: one bit per column of the history
     auto vector_flags = [&](int first) -> uint32_t {
-        return bitsv ? (window[first >> 5] >> (first & 31)) & ((1u << EPV) - 1u) : 0u;
+        const int bit = first + lead;  // (a multiple of EPV)
+        return bitsv ? (window[bit >> 5] >> (bit & 31)) & ((1u << EPV) - 1u) : 0u;
     };
 
     // ---- first bound: the k-th largest of 256 maxima over the first sub-tile (the first of the row to arrive).
@@ -616,12 +628,12 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
         uint32_t word[RW_NV];
 #pragma unroll
         for (int j = 0; j < RW_NV; ++j) {
-            word[j] = bitsv ? window[(min(j * RW_THREADS + t, nvec - 1) * EPV) >> 5] : 0u;
+            word[j] = bitsv ? window[(min(j * RW_THREADS + t, nvec - 1) * EPV + head + lead) >> 5] : 0u;
         }
         float tmax = NEG_INF;
 #pragma unroll
         for (int j = 0; j < RW_NV; ++j) {
-            const int   first = (j * RW_THREADS + t) * EPV;
+            const int   first = (j * RW_THREADS + t) * EPV + head;
             const bool  clean = j * RW_THREADS + t < nvec && word[j] == 0u && rowctx.interior_vector(first, EPV);
             const float vm    = lean_raw_max<DT>(raw[0][j]);
             tmax              = __builtin_fmaxf(tmax, clean ? vm : NEG_INF);
@@ -736,7 +748,8 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
                 for (int j = 0; j < RW_NV; ++j) {
                     const int   rel = q * RW_SUB_VECS + j * RW_THREADS + t;
                     const float m   = lean_raw_max<DT>(raw[r][j]) * mul;
-                    park((all_hit || m >= thr_hot) && rel < nvec, raw[r][j], rel * EPV);
+                    park((all_hit || m >= thr_hot) && rel < nvec, raw[r][j],
+                         rel * EPV + head);
                     if ((j + 1) % RW_PARK_GROUP == 0 && j + 1 < RW_NV && wcount >= LG_DRAIN_AT) {
                         drain();
                     }
@@ -797,11 +810,12 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
     }
 
     RW_STAMP(3)
-    // ---- the columns behind the last whole vector, one by one (fewer than a vector's worth)
+    // ---- the columns outside the whole vectors, one by one (without ODD: fewer than a vector's worth at the end)
     {
-        const int v = nvec * EPV + t;
+        const int v = ODD ? edge_v : nvec * EPV + t;
         if (v < p.V && !rowctx.never_selected(v)) {
-            const float xv = topk_value_at<DT>(rowctx, v);
+            const float xv =
+                ODD ? rowctx.slow(v, S::ld(edge), rowctx.vector_bits(v, 1)) : topk_value_at<DT>(rowctx, v);
             if (xv >= thr_f) {
                 const int slot = atomicAdd(&s.n_list[cur], 1);
                 if (slot < TK_CCAP) {
@@ -888,12 +902,12 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
 }
 
 // Launchers, one per element type (lean_kernels.hip). window: 1 = the row's bitmap fits the small LDS window,
-// 2 = the large one. start / stop: optional events carried by the launch.
-int rowwide_launch_f32(int window, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l, hipEvent_t start,
-                       hipEvent_t stop);
-int rowwide_launch_f16(int window, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l, hipEvent_t start,
-                       hipEvent_t stop);
-int rowwide_launch_bf16(int window, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l,
+// 2 = the large one; odd: rows that do not start on 16-byte boundaries. start / stop: optional events carried by the launch.
+int rowwide_launch_f32(int window, bool odd, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l,
+                       hipEvent_t start, hipEvent_t stop);
+int rowwide_launch_f16(int window, bool odd, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l,
+                       hipEvent_t start, hipEvent_t stop);
+int rowwide_launch_bf16(int window, bool odd, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l,
                         hipEvent_t start, hipEvent_t stop);
 
 }  // namespace ftk

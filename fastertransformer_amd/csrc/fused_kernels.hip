@@ -292,10 +292,19 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
     const bool rw_full   = rows * 5 >= rw_rounds * 256 * 4
                          && (size_t)a->vocab_size / (16 / elem) >= (size_t)RW_MIN_SUBS * RW_SUB_VECS;
     const bool rw_small  = rows <= 256 && a->vocab_size >= 1024;
-    const bool rowwide   = lean_mode == 1 && !want_log_probs && a->embedding_bias == nullptr && lplan.splits > 1
+    // Rows off the 16-byte grid (every row of an odd vocabulary) go the same way, except a few very long ones, which
+    // several workgroups each read sooner. us a step, one launch / gather + select: 77 x 50257 f16 15.4 / 21.4, 1 x 50257
+    // f16 14.0 / 18.3, 256 x 50257 f32 20.0 / 27.7, 256 x 128255 f32 30.4 / 38.5, 420 x 151643 f16 46.8 / 49.5, 256 x 9001
+    // f16 17.3 / 17.3; 8 x 128255 f32 19.8 / 21.2, f16 19.7 / 20.1; 8 x 152063 f32 23.4 / 22.0, bf16 22.1 / 21.3, 32 x 152063
+    // f32 23.9 / 25.0. (With a frequency penalty such rows stay FTK_ERR_UNSUPPORTED: callers rely on which they are.)
+    const bool rw_odd     = ((uintptr_t)a->logits & 15u) != 0 || ((size_t)a->vocab_size_padded * elem) % 16 != 0;
+    const bool rw_odd_ok  = (uintptr_t)a->logits % (uintptr_t)elem == 0 && a->frequency_penalties == nullptr
+                           && (rows >= 24 || a->vocab_size <= 131072);
+    const bool rowwide   = lean_mode == 1 && !want_log_probs && a->embedding_bias == nullptr
                          && g_fused_two_launches == 0 && (rw_full || rw_small)
+                         && lplan.splits > 1
                          && (size_t)a->vocab_size / 32 + 4 <= (size_t)FUSED_BITMAP_WORDS_LARGE
-                         && ((uintptr_t)a->logits & 15u) == 0 && ((size_t)a->vocab_size_padded * elem) % 16 == 0
+                         && (!rw_odd || rw_odd_ok)
                          && (a->penalty_type == FTK_PENALTY_NONE || a->penalties == nullptr
                              || a->step <= RW_HIST_U * RW_THREADS);
     // A large k (the launch reads twice) on up to one row per compute unit: one 1024-thread workgroup per row makes
@@ -499,9 +508,9 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
             hipEvent_t e0, e1;
             take_events(1, &e0, &e1);
             const int w = p.lds_window == 2 ? 2 : 1;
-            return a->dtype == FTK_DTYPE_F32 ? rowwide_launch_f32(w, rows, st, p, l, e0, e1) :
-                   a->dtype == FTK_DTYPE_F16 ? rowwide_launch_f16(w, rows, st, p, l, e0, e1) :
-                                               rowwide_launch_bf16(w, rows, st, p, l, e0, e1);
+            return a->dtype == FTK_DTYPE_F32 ? rowwide_launch_f32(w, rw_odd, rows, st, p, l, e0, e1) :
+                   a->dtype == FTK_DTYPE_F16 ? rowwide_launch_f16(w, rw_odd, rows, st, p, l, e0, e1) :
+                                               rowwide_launch_bf16(w, rw_odd, rows, st, p, l, e0, e1);
         }
         if (largek) {
             // one list per row from one launch, then the selection

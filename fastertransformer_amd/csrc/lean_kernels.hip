@@ -94,7 +94,8 @@ int rowwide_launch_f16
 #else
 int rowwide_launch_bf16
 #endif
-    (int window, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l, hipEvent_t start, hipEvent_t stop)
+    (int window, bool odd, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l, hipEvent_t start,
+     hipEvent_t stop)
 {
     RowwideArgs a;
     a.p = p;
@@ -108,10 +109,12 @@ int rowwide_launch_bf16
         }
     };
     if (window == 2) {
-        launch(rowwide_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_LARGE>);
+        odd ? launch(rowwide_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_LARGE, true>) :
+              launch(rowwide_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_LARGE, false>);
     }
     else {
-        launch(rowwide_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_SMALL>);
+        odd ? launch(rowwide_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_SMALL, true>) :
+              launch(rowwide_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_SMALL, false>);
     }
     return (int)hipGetLastError();
 }

@@ -215,3 +215,42 @@ def test_large_k_lists_in_one_launch_agree_with_the_two_launches():
         for name, a, b in zip(("ids", "sequence_length", "finished"), one[:3], two[:3]):
             assert np.array_equal(a, b), (name, DTYPE_NAMES[dt], B, V, kind)
         assert ((one[0] >= 0) & (one[0] < V)).all()
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("B,V,Vp,offset,k", [(3, 1025, 1025, 1, 64), (9, 8193, 8193, 0, 192), (77, 50257, 50257, 3, 50),
+                                             (33, 131069, 131071, 1, 40), (24, 152063, 152063, 0, 64), (5, 4097, 4099, 5, 1)])
+def test_rowwide_rows_off_the_vector_grid(dt, B, V, Vp, offset, k):
+    """Rows that start anywhere: the vectors begin at a row's first 128-byte line. Every row has its largest values in
+    the columns in front of that line, behind the last whole vector, in the first and last vectors or anywhere, some
+    of them in the history (so the penalty decides). Same ids, lengths and flags as gather and selection."""
+    import torch
+    from fastertransformer_amd import ops
+    from helpers import run_fused_step
+    hooks = ops.ftk_hooks()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(31 * V + dt)
+    tdt = {O.F32: torch.float32, O.F16: torch.float16, O.BF16: torch.bfloat16}[dt]
+    H = 40
+    buf = (torch.randn(offset + B * Vp, generator=gen, device="cuda") * 2.0).to(tdt)
+    logits = buf[offset:].view(B, Vp)
+    history = torch.randint(0, V, (H, B), generator=gen, device="cuda", dtype=torch.int32)
+    edges = [0, 1, 5, 20, 62, 63, 64, 65, 72, V - 70, V - 9, V - 8, V - 3, V - 2]
+    for b in range(B):
+        for i, v in enumerate(edges[b % 3::2] if b % 4 else []):
+            logits[b, v] = 9.0 + 0.25 * ((i * 5 + b) % 7)
+            if (i + b) % 3 == 0:
+                history[i, b] = v
+    draws = torch.rand(B, generator=gen, device="cuda").clamp_(min=1e-6)
+    finished0 = torch.zeros(B, dtype=torch.bool, device="cuda")
+    seqlen0 = torch.full((B,), H - 1, dtype=torch.int32, device="cuda")
+    one = run_fused_step("caller", torch, dt, B, V, H, k, logits, history, draws, finished0, seqlen0, lib=hooks, Vp=Vp)
+    assert one[3] == 0 and hooks.ftk_test_last_fused_path() == (3 if V > 50000 else 2)
+    hooks.ftk_test_set_fused_two_launches(1)
+    try:
+        two = run_fused_step("caller", torch, dt, B, V, H, k, logits, history, draws, finished0, seqlen0, lib=hooks, Vp=Vp)
+        assert two[3] == 0 and hooks.ftk_test_last_fused_path() == 1
+    finally:
+        hooks.ftk_test_set_fused_two_launches(0)
+    for a, b in zip(one[:3], two[:3]):
+        assert np.array_equal(a, b)
