@@ -288,6 +288,9 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
     // launch / gather + select in us: 96 x 128256 f32 24.5 / 33.1, 192 x 128256 f32 27.8 / 41.4, 160 x 152064 f16
     // 25.7 / 33.7, 192 x 50264 f32 20.5 / 26.9; 16 to 64 rows, bound by latency either way, within 1 us); with more,
     // it pays when the rounds of 256 workgroups are nearly full and the rows are long.
+    // Up to 256 short rows as well, which one 256-thread workgroup each would take too (that one / this, k = 50): f32 64 x
+    // 1024 14.2 / 11.2, 64 x 9001 17.4 / 10.7, 256 x 12000 17.9 / 11.3; f16 64 x 1024 16.0 / 13.9, 16 x 8192 15.0 / 13.3, 256 x
+    // 20001 19.6 / 14.3. (Short rows with a frequency penalty stay FTK_ERR_UNSUPPORTED, see below.)
     const int  rw_rounds = (rows + 255) / 256;
     const bool rw_full   = rows * 5 >= rw_rounds * 256 * 4
                          && (size_t)a->vocab_size / (16 / elem) >= (size_t)RW_MIN_SUBS * RW_SUB_VECS;
@@ -302,7 +305,7 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
                            && (rows >= 24 || a->vocab_size <= 131072);
     const bool rowwide   = lean_mode == 1 && !want_log_probs && a->embedding_bias == nullptr
                          && g_fused_two_launches == 0 && (rw_full || rw_small)
-                         && lplan.splits > 1
+                         && (lplan.splits > 1 || (rows <= 256 && a->frequency_penalties == nullptr))
                          && (size_t)a->vocab_size / 32 + 4 <= (size_t)FUSED_BITMAP_WORDS_LARGE
                          && (!rw_odd || rw_odd_ok)
                          && (a->penalty_type == FTK_PENALTY_NONE || a->penalties == nullptr

@@ -245,7 +245,7 @@ def test_rowwide_rows_off_the_vector_grid(dt, B, V, Vp, offset, k):
     finished0 = torch.zeros(B, dtype=torch.bool, device="cuda")
     seqlen0 = torch.full((B,), H - 1, dtype=torch.int32, device="cuda")
     one = run_fused_step("caller", torch, dt, B, V, H, k, logits, history, draws, finished0, seqlen0, lib=hooks, Vp=Vp)
-    assert one[3] == 0 and hooks.ftk_test_last_fused_path() == (3 if V > 50000 else 2)
+    assert one[3] == 0 and hooks.ftk_test_last_fused_path() == 3
     hooks.ftk_test_set_fused_two_launches(1)
     try:
         two = run_fused_step("caller", torch, dt, B, V, H, k, logits, history, draws, finished0, seqlen0, lib=hooks, Vp=Vp)
