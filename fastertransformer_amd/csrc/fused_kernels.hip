@@ -212,8 +212,7 @@ extern "C" void ftk_test_set_lp_form(int v)
 {
     g_lp_form = (v == 1 || v == 1024 || v == 512 || v == 256 || v == -1024 || v == -512 || v == -256) ? v : 0;
 }
-// Test hook: non-zero keeps launches with a large k on the two launches of the lean gather also where one
-// 1024-thread workgroup per row would make their lists in one.
+// Test hook: non-zero keeps launches with a large k off largek_step_kernel.
 static int g_largek_two_launches = 0;
 extern "C" void ftk_test_set_largek_two_launches(int v)
 {
@@ -227,7 +226,7 @@ extern "C" void ftk_test_set_fused_two_launches(int v)
 }
 // Test hook: which kernels the last fused step launched. 0: general stream, 1: lean gather + select, 2: lean gather
 // that also selects (one 256-thread workgroup per row), 3: one 1024-thread workgroup per row, 4: log-prob step,
-// 5: large-k lists in one launch + select.
+// 5: large k, one 1024-thread workgroup per row.
 static int g_fused_last_path = -1;
 extern "C" int ftk_test_last_fused_path(void)
 {
@@ -310,18 +309,18 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
                          && (!rw_odd || rw_odd_ok)
                          && (a->penalty_type == FTK_PENALTY_NONE || a->penalties == nullptr
                              || a->step <= RW_HIST_U * RW_THREADS);
-    // A large k (the launch reads twice) on up to one row per compute unit: one 1024-thread workgroup per row makes
-    // the row's list in one launch (ftk_largek.cuh) where the lean gather takes two launches of small workgroups.
-    // Measured on MI355X with k = 1024 in every row, us per step, one launch / two: 256 x 51200 f16 70.7 / 79.3, 16 x
-    // 51200 f16 65 / 67, 256 x 128256 f32 94 / 100, 128 x 128256 f32 83 / 85, 160 x 152064 f16 87 / 96; a few long
-    // rows are better spread over several workgroups each (16 x 128256 f32 78 / 58, 96 x 152064 f16 85 / 78), and
-    // so is more than one round of rows (320 x 51200 f16 93 / 90, 320 x 152064 f16 130 / 116).
-    const bool largek = lean_mode == 2 && !want_log_probs && a->embedding_bias == nullptr && rows <= 256
-                        && (rows >= 128 || (size_t)a->vocab_size * elem <= ((size_t)128 << 10))
-                        && g_largek_two_launches == 0 && a->max_top_k <= 1024
-                        && (size_t)a->vocab_size / (16 / elem) >= (size_t)LK_GROUPS * LK_THREADS
+    // A large k: one 1024-thread workgroup per row does the step in one launch (ftk_largek.cuh), where the lean gather takes
+    // three and its selection has four waves. us a step with k = 1024 in every row, one launch / three: 256 x 51200 f16 31.4 /
+    // 65.4, 256 x 128256 f32 62.8 / 91.5, 16 x 128256 f32 41.4 / 56.5, 1 x 152064 f16 36.5 / 60.7, 257 x 51200 f16 51.6 / 81.8,
+    // 1024 x 152064 f16 176 / 432, 77 x 50257 f16 28.6 / 68.0; with k = 300 25.1 / 54.3, 55.2 / 80.9, 36.1 / 51.6, 31.8 / 54.0,
+    // 41.9 / 69.8, 156 / 204, 22.4 / 57.0; of shorter rows (general stream, two launches) 16 x 12001 f16 24.4 / 83.2 and 19.5 / 55.4.
+    // The bound is the k-th of at most 3072 maxima of whole vectors: with fewer than 3/2 k vectors it is so loose that lists
+    // outgrow LDS (16 x 8192 f16, k = 1024: 150 / 76).
+    const bool largek = lean_ok && !one_read && !want_log_probs && a->embedding_bias == nullptr
+                        && g_largek_two_launches == 0
+                        && (size_t)a->vocab_size / (16 / elem) * 2 >= (size_t)a->max_top_k * 3
                         && (size_t)a->vocab_size / 32 + 4 <= (size_t)FUSED_BITMAP_WORDS_LARGE
-                        && ((uintptr_t)a->logits & 15u) == 0 && ((size_t)a->vocab_size_padded * elem) % 16 == 0;
+                        && (uintptr_t)a->logits % (uintptr_t)elem == 0;
     // A frequency penalty needs the counts of the history's ids, which only that kernel keeps (a table in LDS).
     if (a->frequency_penalties != nullptr
         && (a->penalties == nullptr || a->penalty_type != FTK_PENALTY_ADDITIVE || a->output_ids == nullptr)) {
@@ -447,6 +446,15 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
     };
     const int window = p.bitmaps_ready ? 0 : (p.lds_window == 2 ? 2 : 1);
     int       rc;
+    if (largek) {
+        FTK_NOTE_PATH(5);
+        hipEvent_t e0, e1;
+        take_events(1, &e0, &e1);
+        const int w = p.lds_window == 2 ? 2 : 1;
+        return a->dtype == FTK_DTYPE_F32 ? largek_launch_f32(w, rows, st, p, l, e0, e1) :
+               a->dtype == FTK_DTYPE_F16 ? largek_launch_f16(w, rows, st, p, l, e0, e1) :
+                                           largek_launch_bf16(w, rows, st, p, l, e0, e1);
+    }
     if (lean_mode != 0) {
         l.splits       = lplan.splits;
         l.subs_per_wg  = lplan.subs_per_wg;
@@ -514,24 +522,6 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
             return a->dtype == FTK_DTYPE_F32 ? rowwide_launch_f32(w, rw_odd, rows, st, p, l, e0, e1) :
                    a->dtype == FTK_DTYPE_F16 ? rowwide_launch_f16(w, rw_odd, rows, st, p, l, e0, e1) :
                                                rowwide_launch_bf16(w, rw_odd, rows, st, p, l, e0, e1);
-        }
-        if (largek) {
-            // one list per row from one launch, then the selection
-            FTK_NOTE_PATH(5);
-            l.splits = 1;
-            hipEvent_t e0, e1;
-            take_events(1, &e0, &e1);
-            const int w = p.lds_window == 2 ? 2 : 1;
-            rc = a->dtype == FTK_DTYPE_F32 ? largek_gather_launch_f32(w, rows, st, p, l, e0, e1) :
-                 a->dtype == FTK_DTYPE_F16 ? largek_gather_launch_f16(w, rows, st, p, l, e0, e1) :
-                                             largek_gather_launch_bf16(w, rows, st, p, l, e0, e1);
-            if (rc != 0) {
-                return rc;
-            }
-            take_events(2, &e0, &e1);
-            return a->dtype == FTK_DTYPE_F32 ? lean_select_launch_f32(rows, st, p, l, e0, e1) :
-                   a->dtype == FTK_DTYPE_F16 ? lean_select_launch_f16(rows, st, p, l, e0, e1) :
-                                               lean_select_launch_bf16(rows, st, p, l, e0, e1);
         }
         // one workgroup per row: it also orders and samples, the step is one launch
         const bool row_select =

@@ -120,27 +120,30 @@ int rowwide_launch_bf16
 }
 
 #if FTK_LEAN_DT == 0
-int largek_gather_launch_f32
+int largek_launch_f32
 #elif FTK_LEAN_DT == 1
-int largek_gather_launch_f16
+int largek_launch_f16
 #else
-int largek_gather_launch_bf16
+int largek_launch_bf16
 #endif
     (int window, int rows, hipStream_t st, const FusedParams& p, const FusedLaunch& l, hipEvent_t start, hipEvent_t stop)
 {
+    RowwideArgs a;
+    a.p = p;
+    a.l = l;
     auto launch = [&](auto kernel) {
         if (start != nullptr) {
-            hipExtLaunchKernelGGL(kernel, dim3(rows), dim3(LK_THREADS), 0, st, start, stop, 0, p, l);
+            hipExtLaunchKernelGGL(kernel, dim3(rows), dim3(LK_THREADS), 0, st, start, stop, 0, a);
         }
         else {
-            hipLaunchKernelGGL(kernel, dim3(rows), dim3(LK_THREADS), 0, st, p, l);
+            hipLaunchKernelGGL(kernel, dim3(rows), dim3(LK_THREADS), 0, st, a);
         }
     };
     if (window == 2) {
-        launch(largek_gather_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_LARGE>);
+        launch(largek_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_LARGE>);
     }
     else {
-        launch(largek_gather_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_SMALL>);
+        launch(largek_step_kernel<FTK_LEAN_DT, FUSED_BITMAP_WORDS_SMALL>);
     }
     return (int)hipGetLastError();
 }

@@ -171,9 +171,8 @@ def test_rowwide_rows_walked_again_do_not_depend_on_the_workspace():
 
 
 def test_large_k_lists_in_one_launch_agree_with_the_two_launches():
-    """With a largest k beyond 192 and at most one row per compute unit, one 1024-thread workgroup per row makes the
-    row's candidate list in one launch (csrc/ftk_largek.cuh; path 5) where the lean gather takes two (maxima, then
-    gather); the test build can keep the two launches (path 1). Same ids, lengths and flags on rows of three types:
+    """With a largest k beyond 192 one 1024-thread workgroup per row does the step in one launch (csrc/ftk_largek.cuh; path
+    5) where the lean gather takes three (maxima, gather, selection); the test build can keep those (path 1). Same ids, lengths and flags on rows of three types:
     vocabularies that end inside a 16-byte vector, histories, rows with fewer valid columns than k, constant rows
     (lists that overflow and send the row to the exact replay)."""
     import torch
@@ -254,3 +253,85 @@ def test_rowwide_rows_off_the_vector_grid(dt, B, V, Vp, offset, k):
         hooks.ftk_test_set_fused_two_launches(0)
     for a, b in zip(one[:3], two[:3]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dt,B,V,Vp,offset,H,k,kind", [
+    (O.F32, 5, 1161, 1161, 1, 8, 193, "normal"),        # as few vectors as the rule allows
+    (O.F16, 9, 12289, 12289, 3, 40, 1024, "normal"),
+    (O.BF16, 7, 73729, 73729, 0, 40, 600, "normal"),    # one column more than the registers of a row hold
+    (O.F32, 6, 36864, 36864, 0, 40, 1000, "normal"),
+    (O.F16, 3, 20001, 20003, 1, 5000, 257, "normal"),   # a history longer than one request
+    (O.BF16, 6, 50257, 50257, 1, 40, 1024, "grid"),     # many equal values in a bucket
+    (O.F16, 6, 50257, 50257, 0, 40, 700, "few values"),
+    (O.F32, 6, 50257, 50257, 0, 40, 500, "one slice"),  # more than k of the best in one of the eight slices
+    (O.F32, 6, 50257, 50257, 0, 40, 1024, "outlier"),
+    (O.F16, 6, 50257, 50257, 0, 40, 300, "not finite"),
+    (O.F16, 300, 16385, 16385, 0, 40, 400, "edges"),
+])
+def test_large_k_in_one_launch(dt, B, V, Vp, offset, H, k, kind):
+    """largek_step_kernel (path 5) against the launches that shapes outside its rule take, whose selection orders slices and
+    merges them: every k from 1 on in one batch, rows that start anywhere, values that the buckets of the order separate
+    badly or not at all, maxima in the columns outside the vectors, a masked end id."""
+    import ctypes as C
+    import torch
+    from fastertransformer_amd import ops
+    hooks = ops.ftk_hooks()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(V + k)
+    x = torch.randn(offset + B * Vp, generator=gen, device="cuda") * 2.5
+    rows = x[offset:].view(B, Vp)
+    if kind == "grid":
+        rows.copy_(torch.round(rows * 4.0) / 4.0)
+    elif kind == "few values":
+        rows[::2] = torch.randint(0, 30, (len(rows[::2]), Vp), generator=gen, device="cuda").float() ** 2 * 0.01
+    elif kind == "one slice":
+        rows[::2] += 20.0 * ((torch.arange(Vp, device="cuda") // 256) % 8 == 3)
+    elif kind == "outlier":
+        rows[::2, 777] = 3.0e4
+        rows[1::2, 778] = 60.0
+    elif kind == "not finite":
+        rows[0, ::3] = float("nan")
+        rows[1, 5] = float("inf")
+        rows[2] = float("-inf")
+        rows[3, 200:] = float("-inf")
+        rows[4] = -65504.0
+    elif kind == "edges":
+        for i, v in enumerate([0, 1, 30, 63, 64, V - 65, V - 8, V - 2, V - 1]):
+            rows[i % 3::3, v] = 20.0 + i
+    logits = x.to({O.F32: torch.float32, O.F16: torch.float16, O.BF16: torch.bfloat16}[dt])
+    dev = dict(device="cuda")
+    top_ks = torch.randint(1, k + 1, (B,), generator=gen, dtype=torch.int32, **dev)
+    top_ks[::2] = k
+    history = torch.randint(0, V, (H, B), generator=gen, dtype=torch.int32, **dev)
+    draws = torch.rand(B, generator=gen, **dev).clamp_(min=1e-6)
+    top_ps, temps, pens = torch.full((B,), 0.97, **dev), torch.full((B,), 0.9, **dev), torch.full((B,), 1.15, **dev)
+    end_ids = torch.randint(0, V, (B,), generator=gen, dtype=torch.int32, **dev)
+    min_lengths = torch.full((B,), H + 9, dtype=torch.int32, **dev)
+    results = []
+    for two_launches in (0, 1):
+        ids = torch.full((B,), -7, dtype=torch.int32, **dev)
+        seq, finished = torch.full((B,), H, dtype=torch.int32, **dev), torch.zeros(B, dtype=torch.bool, **dev)
+        finished[1] = B > 5
+        a = ops.FusedTopkArgs()
+        a.dtype, a.logits, a.embedding_bias = dt, logits.data_ptr() + offset * logits.element_size(), None
+        a.vocab_size, a.vocab_size_padded, a.batch_size, a.local_batch_size = V, Vp, B, B
+        a.step, a.max_input_length = H, H
+        a.temperatures, a.penalties, a.penalty_type = temps.data_ptr(), pens.data_ptr(), ops.PENALTY_MULTIPLICATIVE
+        a.end_ids, a.output_ids, a.min_lengths = end_ids.data_ptr(), history.data_ptr(), min_lengths.data_ptr()
+        a.top_ks, a.top_ps, a.max_top_k, a.uniform_draws = top_ks.data_ptr(), top_ps.data_ptr(), k, draws.data_ptr()
+        a.ids, a.sequence_length, a.finished = ids.data_ptr(), seq.data_ptr(), finished.data_ptr()
+        hooks.ftk_test_set_largek_two_launches(two_launches)
+        try:
+            a.workspace = None
+            ops.check(hooks.ftk_fused_topk_step(C.addressof(a), ops.current_stream()))
+            ws = torch.full((a.workspace_size,), 0xFF, dtype=torch.uint8, **dev)
+            a.workspace = ws.data_ptr()
+            ops.check(hooks.ftk_fused_topk_step(C.addressof(a), ops.current_stream()))
+            assert (hooks.ftk_test_last_fused_path() == 5) == (two_launches == 0)
+        finally:
+            hooks.ftk_test_set_largek_two_launches(0)
+        torch.cuda.synchronize()
+        results.append([v.cpu().numpy() for v in (ids, seq, finished)])
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
+    assert ((results[0][0] >= 0) & (results[0][0] < V)).all()
