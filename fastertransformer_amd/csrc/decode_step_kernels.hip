@@ -318,28 +318,32 @@ int ftk_invoke_log_prob_from_logits(int dtype, float* cum_log_probs, const void*
         if (rows > 0x7FFFFFFFull) {
             return FTK_ERR_ARGUMENT;
         }
-        // Past the caches, 16-bit types from 64 MB on. us a call of fp16, through the caches / past them, with logits that
+        // Past the caches. 16-bit types from 64 MB on: us a call of fp16, through the caches / past them, with logits that
         // were written just before / that were not: 16 x 16 x 50257 (25 MB) 14.9 / 15.0, 16.5 / 16.8; 40 x 16 x 50257 (64 MB)
         // 20.5 / 20.2, 21.7 / 21.2; 64 x 16 x 50257 24.7 / 24.5, 27.8 / 25.8; 40 x 32 x 50257 29.0 / 29.9, 32.8 / 30.1; 48 x
         // 32 x 50257 33.0 / 35.8, 37.1 / 34.9; 64 x 32 x 50257 40.0 / 44.6, 45.3 / 40.7; 96 x 32 x 50257 (more than the
-        // last-level cache) 71.1 / 61.2, 63.2 / 55.4. (the descriptor of a row holds its bytes in 32 bits)
-        const bool once = dtype != FTK_DTYPE_F32 && vocab_size_padded < ((size_t)1 << 30)
-                          && max_input_length * batch_size * vocab_size_padded * 2 >= ((size_t)64 << 20);
+        // last-level cache) 71.1 / 61.2, 63.2 / 55.4. fp32 from 128 MB on, also with the same logits in every call: 32 x 16 x
+        // 50257 (103 MB) 21.7 / 21.8, 17.7 / 20.4, 17.7 / 20.8; 32 x 24 x 50257 24.1 / 23.8, 26.7 / 23.9, 23.1 / 24.1; 16 x 64 x
+        // 50257 33.1 / 31.0, 35.4 / 31.3, 29.7 / 30.8; 32 x 40 x 50257 46.7 / 40.7, 44.3 / 38.2, 36.1 / 38.2; 32 x 64 x 50257
+        // 78.3 / 65.6, 63.3 / 55.8, 54.9 / 55.1. (the descriptor of a row holds its bytes in 32 bits)
+        const size_t elem = dtype == FTK_DTYPE_F32 ? 4 : 2;
+        const bool   once = vocab_size_padded * elem < ((size_t)1 << 31)
+                          && max_input_length * batch_size * vocab_size_padded * elem >= (size_t)(elem == 4 ? 128 : 64) << 20;
         auto       run  = [&](auto dt, auto past) {
             constexpr int DT = decltype(dt)::value;
             log_probs_kernel<DT, decltype(past)::value><<<(unsigned)rows, LP_THREADS, 0, st>>>(
                 log_probs, (const typename Storage<DT>::T*)logits, input_ids, input_lengths, (int)max_input_length, (int)batch_size,
                 (int)vocab_size, vocab_size_padded, batch_first);
         };
-        auto run16 = [&](auto dt) { once ? run(dt, std::true_type()) : run(dt, std::false_type()); };
+        auto run_type = [&](auto dt) { once ? run(dt, std::true_type()) : run(dt, std::false_type()); };
         if (dtype == FTK_DTYPE_F32) {
-            run(std::integral_constant<int, DT_F32>(), std::false_type());
+            run_type(std::integral_constant<int, DT_F32>());
         }
         else if (dtype == FTK_DTYPE_F16) {
-            run16(std::integral_constant<int, DT_F16>());
+            run_type(std::integral_constant<int, DT_F16>());
         }
         else {
-            run16(std::integral_constant<int, DT_BF16>());
+            run_type(std::integral_constant<int, DT_BF16>());
         }
         FTK_LAUNCH_CHECK();
     }

@@ -71,6 +71,12 @@ def test_log_prob_from_large_logits_line_offsets(dt, shape):
     test_log_prob_from_logits(dt, False, shape)
 
 
+@pytest.mark.parametrize("shape", [(64, 32, 16384), (64, 32, 16376), (1024, 33, 1003), (4096, 256, 33)])
+def test_log_prob_from_large_fp32_logits(shape):
+    """fp32 goes past the caches from exactly 128 MB on: that size, just below it, rows at every offset from a 128-byte boundary."""
+    test_log_prob_from_logits(O.F32, False, shape)
+
+
 def test_log_prob_masked_logits():
     """rows holding -inf entries (banned tokens) and one row that is -inf everywhere except the target"""
     import torch
