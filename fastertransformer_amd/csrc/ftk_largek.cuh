@@ -718,10 +718,7 @@ __global__ void __launch_bounds__(LK_THREADS) largek_step_kernel(const RowwideAr
         return;  // the first four waves, one per SIMD, do the rest
     }
     if (n <= 256) {
-        int n_list = rowwide_rank_distinct(ts, n, k, p.max_top_k);
-        if (n_list < 0) {
-            n_list = rowwide_rank(ts, n, k, p.max_top_k);
-        }
+        const int n_list = topk_rank_few<DT>(ts, n, k, p.max_top_k);
         topk_finish_list<DT>(ts, n_list, row, p.Vp, tp, false, u, p.end_ids, out);
     }
     else {

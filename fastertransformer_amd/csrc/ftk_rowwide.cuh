@@ -69,7 +69,7 @@ __device__ __forceinline__ uint32_t rowwide_bound(RowwideShared& s, uint32_t my_
             kk[g]       = max(max(s.slot_key[i], s.slot_key[i + 256]), max(s.slot_key[i + 512], s.slot_key[i + 768]));
         }
         uint32_t P = 0u;
-#pragma unroll
+#pragma unroll 1
         for (int bit = 31; bit >= 16; --bit) {
             const uint32_t cand = P | (1u << bit);
             int            c    = 0;
@@ -88,187 +88,6 @@ __device__ __forceinline__ uint32_t rowwide_bound(RowwideShared& s, uint32_t my_
     lds_barrier();
     hot = uniform_f(s.bound_hot);
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)s.bound);
-}
-
-// Both tie orders of the reference by counting, for a list of at most 256 candidates, by the first TK_THREADS threads
-// of the workgroup (the others have left): the composite keys and the counting of the small case of topk_select_lds.
-// Candidates are in s.cand; on return the ordered list is in s.sel (values in w, columns in idx); returns its length.
-__device__ __forceinline__ int rowwide_rank(TopkShared& s, int n, int k, int max_top_k)
-{
-    const int t       = threadIdx.x;
-    const int bs1_log = max_top_k <= 16 ? 7 : 8;
-    const int BS1     = 1 << bs1_log;
-    const int BS2     = max_top_k <= 32 ? 128 : 256;
-    constexpr int CAP = 256;
-    const uint32_t      my_key = t < n ? s.cand.key[t] : 0u;
-    const uint32_t      my_idx = t < n ? s.cand.idx[t] : 0u;
-    unsigned long long* A      = s.keys;                                    // stage-1 keys  [0, 256)
-    unsigned long long* B      = s.keys + CAP;                              // stage-2 keys  [256, 512)
-    int*                cnt    = reinterpret_cast<int*>(s.keys + 2 * CAP);  // 3 x 256 counts
-    const int           n2     = (n + 1) & ~1;
-    int                 CP     = 2;
-    while (CP < n) {
-        CP <<= 1;
-    }
-    const int parts = TK_THREADS / CP;  // CP <= 256
-    const int c     = t & (CP - 1);
-    const int part  = t / CP;
-    const int pairs = n2 >> 1;
-    const int per   = (pairs + parts - 1) / parts;
-    const int jlo   = min(pairs, part * per) * 2;
-    const int jhi   = min(pairs, part * per + per) * 2;
-    lds_barrier();  // every candidate is in registers: the list's memory can be reused
-    unsigned long long mine = ~0ull;
-    if (t < n) {
-        const int blk   = (int)(my_idx >> bs1_log);
-        const int tt    = (int)(my_idx & (uint32_t)(BS1 - 1));
-        const int slice = blk & 7;
-        mine = ((unsigned long long)slice << 61) | ((unsigned long long)(~my_key) << 29)
-               | ((unsigned long long)(BS1 - 1 - tt) << 21) | (unsigned long long)(blk >> 3);
-    }
-    if (t < n2) {
-        A[t] = mine;  // (an odd list is padded with a key that never counts)
-    }
-    cnt[t]           = 0;
-    cnt[CAP + t]     = 0;
-    cnt[2 * CAP + t] = 0;
-    if (t == 0) {
-        s.misc[1] = 0;
-    }
-    lds_barrier();
-    {
-        const unsigned long long key  = c < n ? A[c] : ~0ull;
-        const unsigned long long base = key & (7ull << 61);  // below it: the keys of lower slices
-        int                      q = 0, qs = 0;
-#pragma unroll 4
-        for (int j = jlo; j < jhi; j += 2) {
-            const ulonglong2 kk = *reinterpret_cast<const ulonglong2*>(&A[j]);
-            q += kk.x < key ? 1 : 0;
-            q += kk.y < key ? 1 : 0;
-            qs += kk.x < base ? 1 : 0;
-            qs += kk.y < base ? 1 : 0;
-        }
-        if (c < n && jhi > jlo) {
-            atomicAdd(&cnt[c], q);
-            atomicAdd(&cnt[CAP + c], qs);
-        }
-    }
-    lds_barrier();
-    unsigned long long k2 = ~0ull;
-    if (t < n) {
-        const int slice = (int)(mine >> 61);
-        const int r     = cnt[t] - cnt[CAP + t];  // rank inside the slice
-        if (r < k) {
-            const int pos = slice * k + r;
-            k2 = ((unsigned long long)(uint32_t)(mine >> 29) << 32) | ((unsigned long long)(BS2 - 1 - pos % BS2) << 24)
-                 | ((unsigned long long)(pos / BS2) << 12);
-        }
-    }
-    if (t < n2) {
-        B[t] = k2;
-    }
-    lds_barrier();
-    {
-        const unsigned long long key = c < n ? B[c] : ~0ull;
-        int                      q = 0, kept = 0;
-#pragma unroll 4
-        for (int j = jlo; j < jhi; j += 2) {
-            const ulonglong2 kk = *reinterpret_cast<const ulonglong2*>(&B[j]);
-            q += kk.x < key ? 1 : 0;
-            q += kk.y < key ? 1 : 0;
-            kept += kk.x != ~0ull ? 1 : 0;
-            kept += kk.y != ~0ull ? 1 : 0;
-        }
-        if (c < n && jhi > jlo) {
-            atomicAdd(&cnt[2 * CAP + c], q);
-        }
-        if (c == 0 && jhi > jlo) {
-            atomicAdd(&s.misc[1], kept);  // entries that stage 1 kept, over all parts
-        }
-    }
-    lds_barrier();
-    const int n_list = min(k, s.misc[1]);
-    if (t < n && k2 != ~0ull) {
-        const int q2 = cnt[2 * CAP + t];
-        if (q2 < n_list) {
-            s.sel.w[q2]   = key_to_float(~(uint32_t)(k2 >> 32));
-            s.sel.idx[q2] = (int)my_idx;
-        }
-    }
-    lds_barrier();
-    return n_list;
-}
-
-// The usual case of rowwide_rank in one counting pass over 32-bit keys: when the candidates' keys are all different
-// and no stage-1 slice holds more than k of them, stage 1 drops none of them and both tie rules are idle, so the
-// reference's list is the candidates in descending order of value, cut at k. Returns the length of the list (in
-// s.sel, like rowwide_rank), or -1 when one of the two conditions fails (s.cand is left as it was). Called by the
-// first TK_THREADS threads; n <= 256.
-__device__ __forceinline__ int rowwide_rank_distinct(TopkShared& s, int n, int k, int max_top_k)
-{
-    const int      t       = threadIdx.x;
-    const int      bs1_log = max_top_k <= 16 ? 7 : 8;
-    const uint32_t my_key  = t < n ? s.cand.key[t] : 0u;
-    const uint32_t my_idx  = t < n ? s.cand.idx[t] : 0u;
-    int*           cnt     = s.sel.idx + 1024;  // 256 counts and 256 marks, clear of the list this function writes
-    int            CP      = 4;
-    while (CP < n) {
-        CP <<= 1;
-    }
-    const int parts = TK_THREADS / CP;
-    const int c     = t & (CP - 1);
-    const int part  = t / CP;
-    const int quads = (n + 3) >> 2;
-    const int per   = (quads + parts - 1) / parts;
-    const int jlo   = min(quads, part * per) * 4;
-    const int jhi   = min(quads, part * per + per) * 4;
-    if (t < 4) {
-        s.cand.key[n + t] = 0u;  // the last four keys read may lie past the list: a key that is above nothing
-    }
-    if (t < 8) {
-        s.slice_count[t] = 0;
-    }
-    cnt[t]              = 0;
-    cnt[TK_THREADS + t] = 0;
-    if (t == 0) {
-        s.misc[1] = 0;
-    }
-    lds_barrier();
-    if (t < n) {
-        atomicAdd(&s.slice_count[(my_idx >> bs1_log) & 7u], 1);
-    }
-    {
-        const uint32_t key   = c < n ? s.cand.key[c] : 0xFFFFFFFFu;
-        int            above = 0;
-#pragma unroll 2
-        for (int j = jlo; j < jhi; j += 4) {
-            const uint4 kk = *reinterpret_cast<const uint4*>(&s.cand.key[j]);
-            above += (kk.x > key ? 1 : 0) + (kk.y > key ? 1 : 0) + (kk.z > key ? 1 : 0) + (kk.w > key ? 1 : 0);
-        }
-        if (c < n && jhi > jlo) {
-            atomicAdd(&cnt[c], above);
-        }
-    }
-    lds_barrier();
-    // Keys that are all different give n different counts: two candidates with the same count have the same key.
-    int rank = 0;
-    if (t < n) {
-        rank = cnt[t];
-        if (atomicAdd(&cnt[TK_THREADS + rank], 1) != 0 || s.slice_count[(my_idx >> bs1_log) & 7u] > k) {
-            s.misc[1] = 1;
-        }
-    }
-    lds_barrier();
-    if (s.misc[1] != 0) {
-        return -1;
-    }
-    const int n_list = min(k, n);
-    if (t < n && rank < n_list) {
-        s.sel.w[rank]   = key_to_float(my_key);
-        s.sel.idx[rank] = (int)my_idx;
-    }
-    lds_barrier();
-    return n_list;
 }
 
 // The kernel's arguments as one block, so that code that is rarely reached can read them again from the
@@ -842,7 +661,9 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
     const float tp_late    = uniform_f(__int_as_float(s.setup[12]));
     int         n = s.n_list[cur];
     const float u = __int_as_float(ts.misc[0]);
-    if (n > k + k / 2 && n > 96 && n <= 4 * TK_THREADS) {
+    // (the ranking of 16-bit rows compares more per pair, but two lists of 64 cost it less than this: 64 x 50257 f16, k = 80,
+    // 15.4 us a step with 128 here, 16.9 with 96; 128 x 32000 f32, k = 50, 13.9 and 13.3)
+    if (n > k + k / 2 && n > (DT == DT_F32 ? 96 : 128) && n <= 4 * TK_THREADS) {
         // Far more candidates than needed: raise the bound once more, to the k-th largest of 256 disjoint groups of
         // the list's own entries (at least k entries reach it), and keep what reaches it. The ranking compares every
         // candidate with every other one; this keeps it short.
@@ -884,10 +705,7 @@ __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideA
     }
     if (n <= 256) {
         RW_STAMP(5)
-        int n_list = rowwide_rank_distinct(ts, n, k, p.max_top_k);
-        if (n_list < 0) {
-            n_list = rowwide_rank(ts, n, k, p.max_top_k);
-        }
+        const int n_list = topk_rank_few<DT>(ts, n, k, p.max_top_k);
         RW_STAMP(7)
 #ifdef FTK_RW_STAMPS
         if (threadIdx.x == 0) { stamps[9] = (unsigned long long)n; }

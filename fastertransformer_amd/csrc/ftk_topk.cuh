@@ -1077,6 +1077,7 @@ __device__ __forceinline__ int topk_sample_walk(const float* w, int n, float u, 
     const float4* w4    = reinterpret_cast<const float4*>(w);
     const int     n4    = (n + 3) >> 2;
     float         s_sum = 0.0f;
+#pragma unroll 1
     for (int i0 = 0; i0 < n4; i0 += 8) {
         float4 v[8];
 #pragma unroll
@@ -1093,12 +1094,13 @@ __device__ __forceinline__ int topk_sample_walk(const float* w, int n, float u, 
     }
     // The running difference never rises again (the weights are non-negative), so the first position where it
     // is <= 0 is the number of positions in front of it, where it is still > 0 (or not a number, as in the
-    // reference, whose `<= 0` test a NaN never passes). A batch of 32 whose last difference is still positive has
-    // no such position: only the subtractions, one dependent chain, are paid for it. The batch where the walk
-    // ends is looked at position by position.
+    // reference, whose `<= 0` test a NaN never passes; all differences are NaN then). A batch of 32 whose last difference
+    // is not <= 0 has no such position: only the subtractions, one dependent chain, are paid for it. In the batch
+    // where the walk ends the position is found by halves: straight code that runs once costs its own fetch.
     float rand_num = u * p * s_sum;
     int   ahead    = 0;
     bool  walking  = true;
+#pragma unroll 1
     for (int i0 = 0; i0 < n4 && walking; i0 += 8) {
         float4 v[8];
 #pragma unroll
@@ -1113,15 +1115,28 @@ __device__ __forceinline__ int topk_sample_walk(const float* w, int n, float u, 
             r[4 * b + 2] = rand_num = rand_num - v[b].z;
             r[4 * b + 3] = rand_num = rand_num - v[b].w;
         }
-        if (r[31] > 0.0f) {
+        if (!(r[31] <= 0.0f)) {
             ahead += 32;
         }
         else {
+            // (vectors, not elements of an array chosen by a condition: those become a search through all registers)
+            typedef float f16v __attribute__((ext_vector_type(16)));
+            f16v lo, hi;
 #pragma unroll
-            for (int e = 0; e < 32; ++e) {
-                walking = walking && !(r[e] <= 0.0f);
-                ahead += walking ? 1 : 0;
+            for (int e = 0; e < 16; ++e) {
+                lo[e] = r[e];
+                hi[e] = r[16 + e];
             }
+            const bool b16 = !(lo[15] <= 0.0f);
+            const auto x16 = b16 ? hi : lo;
+            const bool b8  = !(x16[7] <= 0.0f);
+            const auto x8  = b8 ? x16.hi : x16.lo;
+            const bool b4  = !(x8[3] <= 0.0f);
+            const auto x4  = b4 ? x8.hi : x8.lo;
+            const bool b2  = !(x4[1] <= 0.0f);
+            const bool b1  = !((b2 ? x4[2] : x4[0]) <= 0.0f);
+            ahead += (b16 ? 16 : 0) + (b8 ? 8 : 0) + (b4 ? 4 : 0) + (b2 ? 2 : 0) + (b1 ? 1 : 0);
+            walking = false;
         }
     }
     const int pick = ahead < n - 1 ? ahead : n - 1;
@@ -1268,6 +1283,193 @@ __device__ void topk_literal(Row& rowctx, TopkShared& s, int vocab, int k, int B
     *n_list_out = n_list;
 }
 
+// Both tie orders of the reference by counting, for a list of at most 256 candidates, by the first TK_THREADS threads
+// of the workgroup (the others may have left):
+//   stage 1: slice(3) | ~key(32) | BS1-1-t (8) | j (21),   column = (j*8 + slice)*BS1 + t
+//   stage 2: ~key(32) | BS2-1-pos%BS2 (8) | pos/BS2 (12) | 0,   pos = slice*k + rank in slice
+// Composite keys are unique, so "number of smaller keys" is the sorted position. The all-pairs counting is spread over all
+// threads: with CP = n rounded up to a power of two, thread t counts for candidate t % CP over part t / CP of the list, and
+// the partial counts meet in LDS. What is counted per
+// slice (entries in lower slices, entries that stage 1 keeps) comes from the slices' sizes, so that each of the two passes
+// is a comparison and an addition per pair (16-bit rows, 60 candidates: 1.3 us; 2.5 with those counted as well, after
+// topk_rank_distinct had failed). Candidates are in s.cand; on return the ordered list is in s.sel (values in w, columns
+// in idx); returns its length.
+__device__ __forceinline__ int topk_rank(TopkShared& s, int n, int k, int max_top_k)
+{
+    const int t       = threadIdx.x;
+    const int bs1_log = max_top_k <= 16 ? 7 : 8;
+    const int BS1     = 1 << bs1_log;
+    const int bs2_log = max_top_k <= 32 ? 7 : 8;
+    constexpr int CAP = 256;
+    const uint32_t      my_key = t < n ? s.cand.key[t] : 0u;
+    const uint32_t      my_idx = t < n ? s.cand.idx[t] : 0u;
+    unsigned long long* A      = s.keys;                                    // stage-1 keys  [0, 256)
+    unsigned long long* B      = s.keys + CAP;                              // stage-2 keys  [256, 512)
+    int*                cnt    = reinterpret_cast<int*>(s.keys + 2 * CAP);  // 2 x 256 counts
+    const int           n2     = (n + 1) & ~1;
+    int                 CP     = 2;
+    while (CP < n) {
+        CP <<= 1;
+    }
+    const int parts = TK_THREADS / CP;  // CP <= 256
+    const int c     = t & (CP - 1);
+    const int part  = t / CP;
+    const int pairs = n2 >> 1;
+    const int per   = (pairs + parts - 1) / parts;
+    const int jlo   = min(pairs, part * per) * 2;
+    const int jhi   = min(pairs, part * per + per) * 2;
+    if (t < 8) {
+        s.slice_count[t] = 0;
+    }
+    lds_barrier();  // every candidate is in registers: the list's memory can be reused
+    unsigned long long mine  = ~0ull;
+    const int          slice = (int)(my_idx >> bs1_log) & 7;
+    if (t < n) {
+        const int blk = (int)(my_idx >> bs1_log);
+        const int tt  = (int)(my_idx & (uint32_t)(BS1 - 1));
+        mine = ((unsigned long long)slice << 61) | ((unsigned long long)(~my_key) << 29)
+               | ((unsigned long long)(BS1 - 1 - tt) << 21) | (unsigned long long)(blk >> 3);
+        atomicAdd(&s.slice_count[slice], 1);
+    }
+    if (t < n2) {
+        A[t] = mine;  // (an odd list is padded with a key that never counts)
+    }
+    cnt[t]       = 0;
+    cnt[CAP + t] = 0;
+    lds_barrier();
+    // (entries smaller than that of thread c, in this thread's part of the list)
+    auto count = [&](const unsigned long long* keys, int* into) {
+        const unsigned long long key = c < n ? keys[c] : ~0ull;
+        int                      q   = 0;
+#pragma unroll 4
+        for (int j = jlo; j < jhi; j += 2) {
+            const ulonglong2 kk = *reinterpret_cast<const ulonglong2*>(&keys[j]);
+            q += kk.x < key ? 1 : 0;
+            q += kk.y < key ? 1 : 0;
+        }
+        if (c < n && jhi > jlo) {
+            atomicAdd(&into[c], q);
+        }
+    };
+    count(A, cnt);
+    int kept = 0, below = 0;
+#pragma unroll
+    for (int sl = 0; sl < 8; ++sl) {
+        const int size = s.slice_count[sl];
+        kept += min(size, k);
+        below += sl < slice ? size : 0;
+    }
+    lds_barrier();
+    unsigned long long k2 = ~0ull;
+    if (t < n) {
+        const int r = cnt[t] - below;  // rank inside the slice
+        if (r < k) {
+            const int pos = slice * k + r;
+            k2 = ((unsigned long long)(~my_key) << 32)
+                 | ((unsigned long long)((1 << bs2_log) - 1 - (pos & ((1 << bs2_log) - 1))) << 24)
+                 | ((unsigned long long)(pos >> bs2_log) << 12);
+        }
+    }
+    if (t < n2) {
+        B[t] = k2;
+    }
+    lds_barrier();
+    count(B, cnt + CAP);
+    lds_barrier();
+    const int n_list = min(k, kept);
+    if (t < n && k2 != ~0ull) {
+        const int q2 = cnt[CAP + t];
+        if (q2 < n_list) {
+            s.sel.w[q2]   = key_to_float(my_key);
+            s.sel.idx[q2] = (int)my_idx;
+        }
+    }
+    lds_barrier();
+    return n_list;
+}
+
+// The usual case of topk_rank in one counting pass over 32-bit keys: when the candidates' keys are all different
+// and no stage-1 slice holds more than k of them, stage 1 drops none of them and both tie rules are idle, so the
+// reference's list is the candidates in descending order of value, cut at k. Returns the length of the list (in
+// s.sel, like topk_rank), or -1 when one of the two conditions fails (s.cand is left as it was). Called by the
+// first TK_THREADS threads; n <= 256.
+__device__ __forceinline__ int topk_rank_distinct(TopkShared& s, int n, int k, int max_top_k)
+{
+    const int      t       = threadIdx.x;
+    const int      bs1_log = max_top_k <= 16 ? 7 : 8;
+    const uint32_t my_key  = t < n ? s.cand.key[t] : 0u;
+    const uint32_t my_idx  = t < n ? s.cand.idx[t] : 0u;
+    int*           cnt     = s.sel.idx + 1024;  // 256 counts and 256 marks, clear of the list this function writes
+    int            CP      = 4;
+    while (CP < n) {
+        CP <<= 1;
+    }
+    const int parts = TK_THREADS / CP;
+    const int c     = t & (CP - 1);
+    const int part  = t / CP;
+    const int quads = (n + 3) >> 2;
+    const int per   = (quads + parts - 1) / parts;
+    const int jlo   = min(quads, part * per) * 4;
+    const int jhi   = min(quads, part * per + per) * 4;
+    if (t < 4) {
+        s.cand.key[n + t] = 0u;  // the last four keys read may lie past the list: a key that is above nothing
+    }
+    if (t < 8) {
+        s.slice_count[t] = 0;
+    }
+    cnt[t]              = 0;
+    cnt[TK_THREADS + t] = 0;
+    if (t == 0) {
+        s.misc[1] = 0;
+    }
+    lds_barrier();
+    if (t < n) {
+        atomicAdd(&s.slice_count[(my_idx >> bs1_log) & 7u], 1);
+    }
+    {
+        const uint32_t key   = c < n ? s.cand.key[c] : 0xFFFFFFFFu;
+        int            above = 0;
+#pragma unroll 2
+        for (int j = jlo; j < jhi; j += 4) {
+            const uint4 kk = *reinterpret_cast<const uint4*>(&s.cand.key[j]);
+            above += (kk.x > key ? 1 : 0) + (kk.y > key ? 1 : 0) + (kk.z > key ? 1 : 0) + (kk.w > key ? 1 : 0);
+        }
+        if (c < n && jhi > jlo) {
+            atomicAdd(&cnt[c], above);
+        }
+    }
+    lds_barrier();
+    // Keys that are all different give n different counts: two candidates with the same count have the same key.
+    int rank = 0;
+    if (t < n) {
+        rank = cnt[t];
+        if (atomicAdd(&cnt[TK_THREADS + rank], 1) != 0 || s.slice_count[(my_idx >> bs1_log) & 7u] > k) {
+            s.misc[1] = 1;
+        }
+    }
+    lds_barrier();
+    if (s.misc[1] != 0) {
+        return -1;
+    }
+    const int n_list = min(k, n);
+    if (t < n && rank < n_list) {
+        s.sel.w[rank]   = key_to_float(my_key);
+        s.sel.idx[rank] = (int)my_idx;
+    }
+    lds_barrier();
+    return n_list;
+}
+
+// The list of at most 256 candidates in s.cand in the reference's order, by whichever of the two is the shorter as a rule:
+// the candidates of a 16-bit row nearly always hold equal values, a few of binary16 mostly do not.
+template<int DT>
+__device__ __forceinline__ int topk_rank_few(TopkShared& s, int n, int k, int max_top_k)
+{
+    const int few    = DT == DT_F32 ? 256 : DT == DT_F16 ? 16 : 1;
+    const int n_list = n <= few ? topk_rank_distinct(s, n, k, max_top_k) : -1;
+    return n_list >= 0 ? n_list : topk_rank(s, n, k, max_top_k);
+}
+
 // -------------------------------------------------------------------------------------------
 // select: replay the reference's two tie orders on the candidates in s.cand, sample, emit.
 // `n` < 0 asks for the literal replay.
@@ -1289,110 +1491,7 @@ __device__ __forceinline__ void topk_select_lds(Row& rowctx, TopkShared& s, int 
             n = topk_tighten<DEEP>(s, n, k, &thr);  // (a larger k goes to the sorts below, which take any n)
         }
         if (n <= TK_THREADS) {
-            // ---- small candidate sets (the usual case): both tie orders by counting, no sort.
-            //   stage 1: slice(3) | ~key(32) | BS1-1-t (8) | j (21),   i = (j*8 + slice)*BS1 + t
-            //   stage 2: ~key(32) | BS2-1-pos%BS2 (8) | pos/BS2 (12) | 0,   pos = slice*k + rank in slice
-            // Composite keys are unique, so "number of smaller keys" is the sorted position, and the rank inside
-            // a slice is that minus the number of keys of lower slices. The all-pairs counting is spread over
-            // all threads: with CP = n rounded up to a power of two, thread t counts for candidate t % CP over
-            // part t / CP of the list, and the partial counts meet in LDS.
-            const uint32_t my_key = t < n ? s.cand.key[t] : 0u;
-            const uint32_t my_idx = t < n ? s.cand.idx[t] : 0u;
-            unsigned long long* A   = s.keys;                        // stage-1 keys  [0, 256)
-            unsigned long long* B   = s.keys + TK_THREADS;           // stage-2 keys  [256, 512)
-            int*                cnt = reinterpret_cast<int*>(s.keys + 2 * TK_THREADS);  // 3 x 256 partial counts
-            const int           n2  = (n + 1) & ~1;
-            int                 CP  = 2;
-            while (CP < n) {
-                CP <<= 1;
-            }
-            const int parts = TK_THREADS / CP;  // CP <= 256
-            const int c     = t & (CP - 1);
-            const int part  = t / CP;
-            // pairs of list entries [jlo, jhi) belong to this thread's part
-            const int pairs = n2 >> 1;
-            const int per   = (pairs + parts - 1) / parts;
-            const int jlo   = min(pairs, part * per) * 2;
-            const int jhi   = min(pairs, part * per + per) * 2;
-            lds_barrier();  // every candidate is in registers: the list's memory can be reused
-            unsigned long long mine = ~0ull;
-            if (t < n) {
-                const int blk   = (int)(my_idx >> bs1_log);
-                const int tt    = (int)(my_idx & (uint32_t)(BS1 - 1));
-                const int slice = blk & 7;
-                mine = ((unsigned long long)slice << 61) | ((unsigned long long)(~my_key) << 29)
-                       | ((unsigned long long)(BS1 - 1 - tt) << 21) | (unsigned long long)(blk >> 3);
-            }
-            if (t < n2) {
-                A[t] = mine;  // (an odd list is padded with a key that never counts)
-            }
-            cnt[t]                  = 0;
-            cnt[TK_THREADS + t]     = 0;
-            cnt[2 * TK_THREADS + t] = 0;
-            if (t == 0) {
-                s.misc[1] = 0;
-            }
-            lds_barrier();
-            {
-                const unsigned long long key  = c < n ? A[c] : ~0ull;
-                const unsigned long long base = key & (7ull << 61);  // below it: the keys of lower slices
-                int                      q = 0, qs = 0;
-#pragma unroll 4
-                for (int j = jlo; j < jhi; j += 2) {
-                    const ulonglong2 kk = *reinterpret_cast<const ulonglong2*>(&A[j]);
-                    q += kk.x < key ? 1 : 0;
-                    q += kk.y < key ? 1 : 0;
-                    qs += kk.x < base ? 1 : 0;
-                    qs += kk.y < base ? 1 : 0;
-                }
-                if (c < n && jhi > jlo) {
-                    atomicAdd(&cnt[c], q);
-                    atomicAdd(&cnt[TK_THREADS + c], qs);
-                }
-            }
-            lds_barrier();
-            unsigned long long k2 = ~0ull;
-            if (t < n) {
-                const int slice = (int)(mine >> 61);
-                const int r     = cnt[t] - cnt[TK_THREADS + t];  // rank inside the slice
-                if (r < k) {
-                    const int pos = slice * k + r;
-                    k2 = ((unsigned long long)(uint32_t)(mine >> 29) << 32)
-                         | ((unsigned long long)(BS2 - 1 - pos % BS2) << 24) | ((unsigned long long)(pos / BS2) << 12);
-                }
-            }
-            if (t < n2) {
-                B[t] = k2;
-            }
-            lds_barrier();
-            {
-                const unsigned long long key = c < n ? B[c] : ~0ull;
-                int                      q = 0, kept = 0;
-#pragma unroll 4
-                for (int j = jlo; j < jhi; j += 2) {
-                    const ulonglong2 kk = *reinterpret_cast<const ulonglong2*>(&B[j]);
-                    q += kk.x < key ? 1 : 0;
-                    q += kk.y < key ? 1 : 0;
-                    kept += kk.x != ~0ull ? 1 : 0;
-                    kept += kk.y != ~0ull ? 1 : 0;
-                }
-                if (c < n && jhi > jlo) {
-                    atomicAdd(&cnt[2 * TK_THREADS + c], q);
-                }
-                if (c == 0 && jhi > jlo) {
-                    atomicAdd(&s.misc[1], kept);  // entries that stage 1 kept, over all parts
-                }
-            }
-            lds_barrier();
-            n_list = min(k, s.misc[1]);
-            if (t < n && k2 != ~0ull) {
-                const int q2 = cnt[2 * TK_THREADS + t];
-                if (q2 < n_list) {
-                    s.sel.w[q2]   = key_to_float(~(uint32_t)(k2 >> 32));
-                    s.sel.idx[q2] = (int)my_idx;
-                }
-            }
-            __syncthreads();
+            n_list = topk_rank_few<DT>(s, n, k, max_top_k);
         }
         else {
             // candidates -> stage-1 composite keys, in place

@@ -335,3 +335,23 @@ def test_large_k_in_one_launch(dt, B, V, Vp, offset, H, k, kind):
     for a, b in zip(*results):
         assert np.array_equal(a, b)
     assert ((results[0][0] >= 0) & (results[0][0] < V)).all()
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("log_probs", [False, True], ids=["ids", "log_probs"])
+def test_short_lists_of_equal_values_in_the_reference_order(dt, log_probs):
+    """Lists of 1 to 300 candidates (around the sizes at which the ranking is split differently or gives way to another)
+    of a few distinct values, spread over the eight slices or all in one of them, which then keeps k of its entries only."""
+    rng = np.random.default_rng(77 + dt)
+    sizes = [1, 2, 3, 15, 16, 17, 63, 64, 65, 127, 128, 129, 200, 255, 256, 257, 300]
+    B, V = 2 * len(sizes), 17000
+    x = np.full((B, V), -np.inf, np.float32)
+    for b in range(B):
+        n = sizes[b // 2]
+        columns = np.arange(V) if b % 2 == 0 else np.flatnonzero((np.arange(V) // 256) % 8 == 3)
+        at = rng.choice(columns, n, replace=False)
+        x[b, at] = rng.choice([2.0, 2.5, 3.0, 3.25, 6.0], n)
+    x = O.to_storage(x, dt)
+    for k in (1, 5, 30, 64, 100):
+        c = Case(dt, B, V, V, gen_len=1, runtime_top_k=[k], runtime_top_p=[0.95], with_cum=log_probs, with_out_lp=log_probs)
+        _run(c, rng, 1, lambda i: x)
