@@ -30,10 +30,12 @@
 
 namespace ftk {
 
-constexpr int   TSP_STAGE   = 256;        // threads of a stage workgroup
+constexpr int   TSP_STAGE   = 256;        // threads of a stage workgroup, fp32
+constexpr int   TSP_STAGE16 = 512;        // 16-bit types
 constexpr int   TSP_SUM16   = 1024;       // threads of a sum workgroup, 16-bit types
 constexpr int   TSP_SUM32   = 256;        // fp32
 constexpr int   TSP_CHAINS  = 1024;       // summation chains of a row (the reference's block)
+constexpr int   TSP_STAGE_WAVES = 4096;   // waves of a stage launch, 16-bit types
 constexpr int   TSP_SPLITS  = 64;         // most workgroups per row of the 16-bit stage
 constexpr int   TSP_BLOCK   = 512;        // columns whose maximum the 16-bit stage keeps: one 16-byte vector per lane
 constexpr int   TSP_WINDOW  = 5120 + 4;   // words of the history bitmap of a workgroup
@@ -48,6 +50,7 @@ struct ToppStep {
     int          n, Vp, rows;  // columns of the vocabulary, pitch of a row
     void*        y;            // [rows][y_pitch], or null: y is the logits themselves
     int          y_pitch;
+    bool         y_stream;     // 16-bit: y leaves the L2 as it is written
     const float* temperatures;
     const float* penalties;
     int          penalty_type;  // 2: none
@@ -139,27 +142,42 @@ public:
     }
 };
 
-// Calls mark(id) for the tokens of a row's history that the penalty counts. Every id is a cache line of its own: eight
-// in flight per thread.
-template<class Mark>
-__device__ __forceinline__ void topp_walk_history(const ToppStep& s, int row, Mark&& mark)
-{
-    constexpr int H   = 8;
-    const int     len = s.input_lengths != nullptr ? s.input_lengths[row] : s.max_input_length;
-    for (int t0 = threadIdx.x; t0 < s.step; t0 += H * TSP_STAGE) {
-        int ids[H];
+// The tokens of a row's history that the penalty counts. Every id is a cache line of its own: eight in flight per thread.
+// The first eight are requested ahead of everything else that a workgroup reads: vector loads complete in order, and what
+// the history marks is needed first.
+template<int THREADS>
+struct ToppHistory {
+    static constexpr int H = 8;
+    int                  ids[H];
+    __device__ __forceinline__ void request(const ToppStep& s, int row, int first)
+    {
 #pragma unroll
         for (int u = 0; u < H; ++u) {
-            const int at = t0 + u * TSP_STAGE;
-            // (the padding between a short prompt and max_input_length does not count)
-            ids[u] = at < s.step && !(at >= len && at < s.max_input_length) ? s.history[(size_t)at * s.batch_size + row] : -1;
-        }
-#pragma unroll
-        for (int u = 0; u < H; ++u) {
-            mark(ids[u]);
+            if (first + u * THREADS < s.step) {  // (the same for the workgroup)
+                ids[u] = s.history[(size_t)min(first + u * THREADS + (int)threadIdx.x, s.step - 1) * s.batch_size + row];
+            }
         }
     }
-}
+    // Calls mark(id) for all of them; `request(s, row, 0)` came before.
+    template<class Mark>
+    __device__ __forceinline__ void walk(const ToppStep& s, int row, Mark&& mark)
+    {
+        const int len = s.input_lengths != nullptr ? s.input_lengths[row] : s.max_input_length;
+        for (int first = 0; first < s.step; first += H * THREADS) {
+            if (first > 0) {
+                request(s, row, first);
+            }
+#pragma unroll
+            for (int u = 0; u < H; ++u) {
+                const int at = first + u * THREADS + (int)threadIdx.x;
+                // (the padding between a short prompt and max_input_length does not count)
+                if (at < s.step && !(at >= len && at < s.max_input_length)) {
+                    mark(ids[u]);
+                }
+            }
+        }
+    }
+};
 
 __device__ __forceinline__ bool topp_row_idle(const ToppStep& s, int row)
 {
@@ -178,16 +196,18 @@ __device__ __forceinline__ uint4 topp_load8(const uint16_t* from)
 }
 
 // ---- stage, 16-bit types ------------------------------------------------------------------------------------------
-// (rows x splits) workgroups, each over a run of blocks of 512 columns, a block per wave at a time. Memory-bound. The
-// counters that several workgroups of the sum add to are cleared on the way. 64 x 128256 bfloat16 with temperature and
-// penalty: 14.7 us, bound by latency (flags, history, rows); 128 x 152064: 18 us for 39 MB read and 39 MB written.
+// (rows x splits) workgroups, each over a run of blocks of 512 columns, a block per wave at a time. The counters that
+// several workgroups of the sum add to are cleared on the way. Bound by latency where there are few rows: flags and
+// history (2 us), then a few blocks per wave. Requesting the history first and a short loop instead of 25 KB of
+// straight-line code, which every wave fetched to run it once: 64 x 128256 bfloat16 with temperature and penalty
+// 15.1 -> 12.4 us (16 MB read, 16 MB written; 0.2 of the copy rate), 128 x 152064 with 51 rows of its own 17.9 -> 15.7.
 template<int DT, bool TRANSFORM>
-__global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
+__global__ void __launch_bounds__(TSP_STAGE16) topp_stage_kernel(ToppStep s)
 {
     typedef Storage<DT>   S;
     typedef typename S::T T;
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    constexpr int         EPV = 8, U = 4, NW = TSP_STAGE / WAVE;
+    constexpr int         EPV = 8, NW = TSP_STAGE16 / WAVE;
     constexpr uint32_t    INF16 = DT == DT_F16 ? 0x7C00u : 0x7F80u;
     __shared__ uint32_t   window[TRANSFORM ? TSP_WINDOW : 1];
     __shared__ float      red[16];
@@ -197,20 +217,19 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
     const int hi   = min(s.n, lo + s.chunk);
     const int nblk = (hi - lo + TSP_BLOCK - 1) / TSP_BLOCK;
     const T*  rowp = (const T*)s.logits + (size_t)row * s.Vp;
-    // the first blocks and everything about the row are requested together
-    uint4 raw[U];
-    auto  load = [&](int b0) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            // (a vector that runs over the end is put right when it is used)
-            const int v = lo + (b0 + u * NW) * TSP_BLOCK + lane_id() * EPV;
-            raw[u]      = topp_load8(rowp + max(0, min(v, s.n - EPV)));
-        }
+    // the history, the first blocks and everything about the row are requested together
+    const bool  hist = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
+    ToppHistory<TSP_STAGE16> history;
+    if (hist) {
+        history.request(s, row, 0);
+    }
+    auto load = [&](int b) {
+        // (a vector that runs over the end is put right when it is used)
+        return topp_load8(rowp + max(0, min(lo + b * TSP_BLOCK + lane_id() * EPV, s.n - EPV)));
     };
-    load(wave_id());
+    uint4 r0 = load(wave_id()), r1 = load(wave_id() + NW), r2 = load(wave_id() + 2 * NW), r3 = load(wave_id() + 3 * NW);
     const bool              idle = topp_row_idle(s, row);
     const ToppTransform<DT> f(s, row);
-    const bool              hist = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
     if (idle) {
         return;
     }
@@ -219,7 +238,7 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
     const float mul = f.temperature_active ? f.temperature.inv : 1.0f;
     if (s.parts > 1) {
         uint4* counters = reinterpret_cast<uint4*>(s.counts + (size_t)row * ToppCode<DT>::COUNTERS);
-        for (int i = j * TSP_STAGE + t; i < ToppCode<DT>::COUNTERS / 4; i += s.splits * TSP_STAGE) {
+        for (int i = j * TSP_STAGE16 + t; i < ToppCode<DT>::COUNTERS / 4; i += s.splits * TSP_STAGE16) {
             counters[i] = make_uint4(0u, 0u, 0u, 0u);
         }
     }
@@ -228,11 +247,11 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
     }
     if (hist) {
         const int words = (hi - lo + 31) / 32 + 1;
-        for (int i = t; i < words; i += TSP_STAGE) {
+        for (int i = t; i < words; i += TSP_STAGE16) {
             window[i] = 0u;
         }
         lds_barrier();
-        topp_walk_history(s, row, [&](int id) {
+        history.walk(s, row, [&](int id) {
             if (id >= lo && id < hi) {
                 atomicOr(&window[(id - lo) >> 5], 1u << ((id - lo) & 31));
             }
@@ -241,76 +260,95 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_kernel(ToppStep s)
     lds_barrier();
     float mx   = TSP_LOWEST;
     u16x2 seen = {0, 0};  // largest magnitude bits (a NaN has the largest)
-    for (int b0 = wave_id(); b0 < nblk; b0 += U * NW) {
+    // Four vectors of the lane are in flight. The loop stays a loop, and what few columns need are loops in it: a wave goes
+    // through it a few times only, so that straight-line code waits for its own fetch.
+#pragma unroll 1
+    for (int b = wave_id(); b < nblk; b += NW) {
+        uint4 raw = r0;
+        r0        = r1;
+        r1        = r2;
+        r2        = r3;
+        r3        = load(b + 4 * NW);
+        const int      v    = lo + b * TSP_BLOCK + lane_id() * EPV;
+        const int      rel  = v - lo;
+        const uint32_t bits = TRANSFORM && hist && v < hi ? (window[rel >> 5] >> (rel & 31)) & 0xFFu : 0u;
+        float          vm   = TSP_LOWEST;
+        if (v + EPV > s.n || (TRANSFORM && f.bias != nullptr)) {
+            // two columns at a time; the words of the vector take turns in `raw.x`
+#pragma unroll 1
+            for (int k = 0; k < EPV / 2; ++k) {
+                uint32_t word = 0u;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int b = b0 + u * NW;
-            if (b < nblk) {
-                const int v  = lo + b * TSP_BLOCK + lane_id() * EPV;
-                float     vm = TSP_LOWEST;
-                T*        e  = reinterpret_cast<T*>(&raw[u]);
-                if (v + EPV > s.n) {
-                    for (int c = 0; c < EPV; ++c) {
-                        e[c] = v + c < s.n ? rowp[v + c] : (T)0;
+                for (int c = 0; c < 2; ++c) {
+                    const int col = v + 2 * k + c;
+                    if (col < s.n) {
+                        T e = rowp[col];
+                        if constexpr (TRANSFORM) {
+                            e = S::st(f(col, S::ld(e), ((bits >> (2 * k + c)) & 1u) != 0u));
+                        }
+                        vm = __builtin_fmaxf(vm, S::ld(e));
+                        word |= (uint32_t)e << (16 * c);
                     }
                 }
-                if constexpr (TRANSFORM) {
-                    const int      rel  = v - lo;
-                    const uint32_t bits = hist && v < hi ? (window[rel >> 5] >> (rel & 31)) & 0xFFu : 0u;
-                    const uint32_t end  = (uint32_t)(f.masked_end - v);
-                    if (f.bias != nullptr) {
+                raw = make_uint4(raw.y, raw.z, raw.w, word);
+            }
+        }
+        else {
+            if constexpr (TRANSFORM) {
+                T* e = reinterpret_cast<T*>(&raw);
 #pragma unroll
-                        for (int c = 0; c < EPV; ++c) {
-                            e[c] = v + c < hi ? S::st(f(v + c, S::ld(e[c]), ((bits >> c) & 1u) != 0u)) : (T)0;
-                        }
-                    }
-                    else {
-#pragma unroll
-                        for (int c = 0; c < EPV; ++c) {
-                            e[c] = S::st(S::ld(e[c]) * mul);
-                        }
-                        // columns of the history and a masked end id: few lanes
-                        if (bits != 0u || end < (uint32_t)EPV) {
-#pragma unroll
-                            for (int c = 0; c < EPV; ++c) {
-                                if ((bits >> c) & 1u) {
-                                    e[c] = S::st(repetition_value(S::ld(e[c]), f.penalty, f.penalty_type));
-                                }
-                                if (end == (uint32_t)c) {
-                                    e[c] = S::st(-S::max_t());
-                                }
-                            }
-                        }
-                    }
-                    if (v < hi) {
-                        *reinterpret_cast<uint4*>(y + v) = raw[u];  // (rows of y are padded to whole vectors)
-                    }
+                for (int c = 0; c < EPV; ++c) {
+                    e[c] = S::st(S::ld(e[c]) * mul);
                 }
-                const uint32_t* w = reinterpret_cast<const uint32_t*>(&raw[u]);
-#pragma unroll
-                for (int c = 0; c < EPV / 2; ++c) {
-                    seen = __builtin_elementwise_max(seen, __builtin_bit_cast(u16x2, w[c] & 0x7FFF7FFFu));
-                }
-                if (v + EPV <= hi) {
-#pragma unroll
-                    for (int c = 0; c < EPV; ++c) {
-                        vm = __builtin_fmaxf(vm, S::ld(e[c]));
+                // columns of the history and a masked end id: few lanes, a column of each at a time
+                const uint32_t end  = (uint32_t)(f.masked_end - v);
+                uint32_t       todo = bits | (end < (uint32_t)EPV ? 1u << end : 0u);
+                while (todo != 0u) {
+                    const uint32_t c = (uint32_t)__builtin_ctz(todo);
+                    todo &= todo - 1u;
+                    const uint32_t word = c < 4u ? (c < 2u ? raw.x : raw.y) : (c < 6u ? raw.z : raw.w);
+                    const uint32_t sh   = (c & 1u) * 16u;
+                    T              x    = (T)(word >> sh);
+                    if ((bits >> c) & 1u) {
+                        x = S::st(repetition_value(S::ld(x), f.penalty, f.penalty_type));
                     }
+                    if (c == end) {
+                        x = S::st(-S::max_t());
+                    }
+                    const uint32_t put = (word & ~(0xFFFFu << sh)) | ((uint32_t)x << sh);
+                    raw.x              = c >> 1 == 0u ? put : raw.x;
+                    raw.y              = c >> 1 == 1u ? put : raw.y;
+                    raw.z              = c >> 1 == 2u ? put : raw.z;
+                    raw.w              = c >> 1 == 3u ? put : raw.w;
+                }
+            }
+            const T* e = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+            for (int c = 0; c < EPV; ++c) {
+                vm = __builtin_fmaxf(vm, S::ld(e[c]));
+            }
+        }
+        if constexpr (TRANSFORM) {
+            if (v < hi) {  // (rows of y are padded to whole vectors)
+                uint4* to = reinterpret_cast<uint4*>(y + v);
+                if (s.y_stream) {
+                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+                    __builtin_nontemporal_store(__builtin_bit_cast(u32x4, raw), reinterpret_cast<u32x4*>(to));
                 }
                 else {
-                    for (int c = 0; c < EPV; ++c) {
-                        vm = __builtin_fmaxf(vm, v + c < hi ? S::ld(e[c]) : TSP_LOWEST);
-                    }
-                }
-                mx = __builtin_fmaxf(mx, vm);
-                vm = wave_reduce_unordered(vm, [](float a, float c) { return __builtin_fmaxf(a, c); });
-                if (lane_id() == 0) {
-                    bmax[lo / TSP_BLOCK + b] = vm;
+                    *to = raw;
                 }
             }
         }
-        if (b0 + U * NW < nblk) {
-            load(b0 + U * NW);
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+        for (int c = 0; c < EPV / 2; ++c) {
+            seen = __builtin_elementwise_max(seen, __builtin_bit_cast(u16x2, w[c] & 0x7FFF7FFFu));
+        }
+        mx = __builtin_fmaxf(mx, vm);
+        vm = wave_reduce_unordered(vm, [](float a, float c) { return __builtin_fmaxf(a, c); });
+        if (lane_id() == 0) {
+            bmax[lo / TSP_BLOCK + b] = vm;
         }
     }
     if (max((uint32_t)seen.x, (uint32_t)seen.y) > INF16) {
@@ -364,6 +402,11 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     // 0.12 ms). More and shorter stretches cost time on every row: 64 of 16, 0.7 us.
     constexpr int U0 = TSP_CHAINS / TSP_STAGE;
     auto  sample = [&](int u) { return (u * (TSP_STAGE / 32) + (t >> 5)) * ((s.n / 32) & ~31) + (t & 31); };
+    const bool  marks = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
+    ToppHistory<TSP_STAGE> history;
+    if (marks) {
+        history.request(s, row, 0);
+    }
     float plain[U0];
 #pragma unroll
     for (int u = 0; u < U0; ++u) {
@@ -392,7 +435,6 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     if (t == 0) {
         any_nan = 0u;
     }
-    const bool                  marks = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
     const ToppTransform<DT_F32> f(s, row);
     if (TRANSFORM && marks) {
         const int words = (nit * C + 31) / 32 + 1;
@@ -411,7 +453,7 @@ __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
     }
     const float top = first + TSP_ABOVE;
     if (TRANSFORM && marks) {
-        topp_walk_history(s, row, [&](int id) {
+        history.walk(s, row, [&](int id) {
             const int c = (id & (TSP_CHAINS - 1)) - c0;
             if (id >= 0 && id < s.n && c >= 0 && c < C) {
                 const int at = ((id / TSP_CHAINS) << shift) + c;
@@ -684,11 +726,11 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
         __builtin_memcpy(&x, y + max(0, min(v, s.n - 4)), 8);
         return x;
     };
-    uint2 r0 = load(0), r1 = load(1), r2 = load(2), r3 = load(3);
+    const ToppRowMax rm(s, row, s.splits);
+    uint2            r0 = load(0), r1 = load(1), r2 = load(2), r3 = load(3);
     if (topp_row_idle(s, row)) {
         return;
     }
-    const ToppRowMax rm(s, row, s.splits);
     for (int i = t; i < Code::USED; i += TSP_SUM16) {
         cnt[i] = 0u;
     }
@@ -2057,11 +2099,13 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     if (dtype == DT_F32 && keeps_y && topp_part_columns(vocab, p.parts) > TSP_WINDOW_BITS) {
         p.parts = 16;
     }
-    // 16-bit stage: about four workgroups per compute unit, each with at least four blocks of columns (one per wave), and
-    // no more columns than its bitmap of the history covers
+    // 16-bit stage: about sixteen waves per compute unit, at least a block of columns for each, and no more columns than a
+    // workgroup's bitmap of the history covers. Workgroups of 512 threads: each walks the row's whole history (us of the
+    // stage with 256 / 512 / 1024 threads: 64 x 128256 13.9 / 13.7 / 13.4, 128 x 152064, 51 rows of its own 16.1 / 15.6 / 16.0;
+    // twice the waves 14.1 and 15.7).
     p.blocks = (vocab + TSP_BLOCK - 1) / TSP_BLOCK;
-    int s    = (1024 + rows - 1) / rows;
-    s        = std::min(s, std::max(1, p.blocks / 4));
+    int s    = (TSP_STAGE_WAVES / (TSP_STAGE16 / WAVE) + rows - 1) / rows;
+    s        = std::min(s, std::max(1, p.blocks / (TSP_STAGE16 / WAVE)));
     s        = std::max(s, (p.blocks + TSP_WINDOW_BITS / TSP_BLOCK - 1) / (TSP_WINDOW_BITS / TSP_BLOCK));
     p.splits = std::min(s, TSP_SPLITS);
     p.chunk  = (p.blocks + p.splits - 1) / p.splits * TSP_BLOCK;
@@ -2125,6 +2169,10 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
     s.rows   = c.rows;
     s.y      = keeps_y ? ws + p.off_y : nullptr;
     s.y_pitch          = p.y_pitch;
+    // What the L2s (32 MB) hold of y at the end of the stage they write back before the sum may start; y that streams out
+    // while the stage runs does without that wait, and more than that leaves by itself. us, through L2 / streamed: stage
+    // kernel of 64 x 128256 13.8 / 12.4; whole steps 256 x 128256 100.6 / 101.1, 512 x 152064 290 / 303.
+    s.y_stream         = (size_t)c.rows * p.y_pitch * sizeof(uint16_t) <= ((size_t)32 << 20);
     s.temperatures     = c.temperatures;
     s.penalties        = c.penalties;
     s.penalty_type     = c.penalty_type;
@@ -2192,10 +2240,10 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
     auto run = [&](auto type) -> int {
         constexpr int DT = decltype(type)::value;
         if (keeps_y) {
-            topp_stage_kernel<DT, true><<<splits, TSP_STAGE, 0, st>>>(s);
+            topp_stage_kernel<DT, true><<<splits, TSP_STAGE16, 0, st>>>(s);
         }
         else {
-            topp_stage_kernel<DT, false><<<splits, TSP_STAGE, 0, st>>>(s);
+            topp_stage_kernel<DT, false><<<splits, TSP_STAGE16, 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
         if (p.parts == 1) {

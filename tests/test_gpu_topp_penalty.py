@@ -51,6 +51,30 @@ def test_penalised_nucleus_rows(dt, shape):
         compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
 
 
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("H", [1, 511, 2049, 4096, 4097, 9000])
+def test_long_histories_of_nucleus_rows(dt, H):
+    """Histories around the number of ids that a stage requests at once, with vectors whose columns are all in the history,
+    the masked end id among them, and ids on both sides of where workgroups share a row out."""
+    B, V, Vp = 3, 20011, 20016
+    rng = np.random.default_rng(H + dt)
+    prompt = rng.integers(0, V, (H, B)).astype(np.int32)
+    near = rng.random((H, B)) < 0.5
+    prompt[near] = (4090 + rng.integers(0, 24, int(near.sum()))).astype(np.int32)
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=2, runtime_top_k=np.zeros(B, np.uint32),
+             runtime_top_p=rng.uniform(0.5, 1.0, B), temperature=rng.uniform(0.5, 1.5, B), min_length=np.full(B, H + 9),
+             end_ids=np.array([4095, V - 1, 4100]), input_lengths=np.array([H, max(1, H // 2), 1]), prompt=prompt,
+             repetition_penalty=rng.uniform(0.8, 1.5, B), with_cum=True, with_out_lp=True)
+    p, o = ProductRunner(c), OracleRunner(c)
+    for i in range(2):
+        print("long history", DTYPE_NAMES[dt], H, i, flush=True)
+        x = _zipf(rng, dt, B, V, Vp, 0.0)
+        u = uniforms(rng, B)
+        p.step(H + i, x, u)
+        o.step(H + i, x, u)
+        compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d" % i)
+
+
 def _sample_step(dt, x, V, p_arr, end_ids, draws=None, states=None, gathered=None, finished=None, hooks=False):
     """One ftk_fused_topp_sample_step over rows of `x`: (ids, finished, lengths, cumulative log-probs). The draws are
     `draws`, or generated from `states` (advanced in place). `gathered` (fp32; an int32 array) gets the number of entries
