@@ -1564,6 +1564,9 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     constexpr int                 FEW  = 256;                   // threads of the short scan: eight tiles
     __shared__ TopPScan           sc;
     __shared__ ToppRunsShared<DT> rs;
+    // the values of the row's first positions one by one: what the scan reads there
+    constexpr int                 FLAT = DT == DT_F16 ? 8192 : 16384;
+    __shared__ __align__(16) uint16_t flat[FLAT];
     __shared__ uint32_t           wcnt[TW], wrun[TW], wpick[NW];
     __shared__ float              wmass[TW];
     __shared__ uint32_t           sh_enough, key_lo, key_hi;
@@ -1750,31 +1753,83 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
                     }
                 }
             };
+            // Near the head of a row runs are short, and a tile taken out of them is a chain of look-ups (1.6 us per 32 tiles).
+            // Sixteen threads write a run's value to its positions, and a lane's eight values are one read (128 x 152064
+            // bf16: the scan for a draw behind 15000 entries 8.8 -> 5.2 us, behind 77000, with what follows, 20 -> 10).
+            const int flat_n = min(FLAT, (enough + TP_TILE - 1) / TP_TILE * TP_TILE);
+            for (int k = t >> 4; k < (int)nruns; k += TP_THREADS / 16) {
+                const int begin = (int)rs.start[k], end = min((int)rs.start[k + 1], flat_n);
+                if (begin >= flat_n) {
+                    break;
+                }
+                const uint16_t v = rs.prob[k];
+                for (int i = begin + (t & 15); i < end; i += 16) {
+                    flat[i] = v;
+                }
+            }
+            if ((int)n + t < flat_n) {  // (fewer than a tile's)
+                flat[n + t] = 0;
+            }
+            __syncthreads();
+            auto flat_load = [&](int i0, float* x) {
+                const uint4    q    = *reinterpret_cast<const uint4*>(flat + i0);
+                const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    x[2 * k]     = S::ld((T)w[k]);
+                    x[2 * k + 1] = S::ld((T)(w[k] >> 16));
+                }
+            };
             auto load = [&](int tile, int l, float* x) {
                 const int i0 = tile * TP_TILE + l * 8;
-                int       lo = run_at(min(i0, (int)n - 1));
-                values_from(i0, lo, x);
+                if (i0 < flat_n) {
+                    flat_load(i0, x);
+                }
+                else {
+                    int lo = run_at(min(i0, (int)n - 1));
+                    values_from(i0, lo, x);
+                }
             };
-            // Tiles inside one run first, a thread each: the scan of 256 equal values ends with 32 times what a lane adds up
-            // (every step of the raking doubles). The others go to 32-lane groups. (128 x 152064 bf16, a draw behind 62437 entries: 29 us
-            // for the scan with tiles dealt out in order and runs walked one by one, 16 us.)
+            // Behind them: tiles of a few runs first, a thread each. All values of a tile are multiples of the last place of
+            // its smallest one; where the largest is so near that 256 of it stay below 2^24 such places, no addition inside
+            // the tile rounds, and its total is the sum of counts times values in any order. Other tiles go to 32-lane groups.
             auto totals = [&](int base, int count) {
-                const int l = t & 31;
+                constexpr int RUNS = 8, SPREAD = 15 - (DT == DT_F16 ? 10 : 7);  // (of exponents)
+                const int l  = t & 31;
+                const int nf = max(0, min(count, flat_n / TP_TILE - base));
                 if (t == 0) {
                     sh_mixed = 0;
                 }
+                for (int g = t >> 5; g < nf; g += TP_THREADS / 32) {
+                    float x[8];
+                    flat_load((base + g) * TP_TILE + l * 8, x);
+                    const float total = tile_scan(x, l);
+                    if (l == 31) {
+                        sc.agg[g] = total;
+                    }
+                }
+                if (nf == count) {
+                    return;
+                }
                 __syncthreads();
-                if (t < count) {
+                if (t >= nf && t < count) {
                     const int i0    = (base + t) * TP_TILE;
+                    const int end   = min(i0 + TP_TILE, (int)n);
                     const int first = run_at(i0);
-                    if ((int)rs.start[first + 1] >= i0 + TP_TILE) {
-                        const float v   = S::ld(rs.prob[first]);
-                        float       seg = v;
-#pragma unroll
-                        for (int k = 1; k < 8; ++k) {
-                            seg = seg + v;
-                        }
-                        sc.agg[t] = seg * 32.0f;
+                    float     v     = S::ld(rs.prob[first]), sum = 0.0f;
+                    const int top   = __float_as_int(v) >> 23;
+                    int       from = i0, q = first;
+                    bool      exact = true;
+#pragma unroll 1
+                    for (int k = 0; k < RUNS && from < end; ++k) {
+                        const int to = min(end, (int)rs.start[++q]);
+                        exact        = exact && top - (__float_as_int(v) >> 23) <= SPREAD;
+                        sum          = sum + (float)(to - from) * v;
+                        from         = to;
+                        v            = S::ld(rs.prob[min(q, (int)nruns - 1)]);
+                    }
+                    if (exact && from == end) {
+                        sc.agg[t] = sum;
                     }
                     else {
                         sc.carry[atomicAdd(&sh_mixed, 1)] = __int_as_float((t << 16) | first);
@@ -1915,34 +1970,49 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     const unsigned short origin   = (unsigned short)(!one_sign ? klo : positive ? klo - 0x8000u : 0x10000u - khi);
     const unsigned short length   = (unsigned short)min(khi - klo, 0xFFFFu);  // (all 65536: a row of one value ends above)
     const u16x2          from = {origin, origin}, size = {length, length}, unit = {1, 1};
-    auto mask_of = [&](int blk) -> uint32_t {
-        const int b0 = __builtin_amdgcn_readfirstlane(blk) * TSP_BLOCK;  // (the same for the wave)
-        uint32_t  m  = 0u;
-        if (b0 + TSP_BLOCK <= s.n) {
-            const uint4    raw  = topp_load8(r.y + b0 + lane_id() * 8);
-            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+    const int whole_blocks = s.n / TSP_BLOCK;
+    auto vector_of = [&](int blk) -> uint4 {
+        return topp_load8(r.y + __builtin_amdgcn_readfirstlane(blk) * TSP_BLOCK + lane_id() * 8);
+    };
+    auto mask_whole = [&](const uint4& raw, auto same_sign) -> uint32_t {
+        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+        uint32_t       m    = 0u;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                u16x2 x = __builtin_bit_cast(u16x2, w[k]);
-                if (!one_sign) {
-                    const i16x2 sign = __builtin_bit_cast(i16x2, w[k]) >> 15;
-                    x = __builtin_bit_cast(u16x2, w[k] ^ (__builtin_bit_cast(uint32_t, sign) | 0x80008000u));
-                }
-                const u16x2 in = __builtin_elementwise_min(__builtin_elementwise_sub_sat(size, (u16x2)(x - from)), unit);
-                m |= __builtin_bit_cast(uint32_t, in) << k;
+        for (int k = 0; k < 4; ++k) {
+            u16x2 x = __builtin_bit_cast(u16x2, w[k]);
+            if constexpr (!decltype(same_sign)::value) {
+                const i16x2 sign = __builtin_bit_cast(i16x2, w[k]) >> 15;
+                x = __builtin_bit_cast(u16x2, w[k] ^ (__builtin_bit_cast(uint32_t, sign) | 0x80008000u));
             }
-            m = (m | (m >> 12)) & 0xFFu;
+            // (left to itself the compiler makes two comparisons and two selects of this minimum)
+            uint32_t in = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(size, (u16x2)(x - from)));
+            asm("v_pk_min_u16 %0, %0, %1" : "+v"(in) : "v"(0x00010001u));
+            m |= in << k;
         }
-        else {
-            const int v0 = b0 + lane_id() * 8;
-#pragma unroll 1
-            for (int k = 0; k < 8; ++k) {
-                if (v0 + k < s.n && match((uint32_t)r.y[v0 + k])) {
-                    m |= 1u << ((k >> 1) + 4 * (k & 1));
-                }
+        return (m | (m >> 12)) & 0xFFu;
+    };
+    auto mask_part = [&]() -> uint32_t {  // of the block that runs over the end
+        const int v0 = whole_blocks * TSP_BLOCK + lane_id() * 8;
+        T         x[8];
+        uint32_t  m = 0u;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            x[k] = r.y[min(v0 + k, s.n - 1)];  // (all of them requested before the first is looked at)
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (v0 + k < s.n && match((uint32_t)x[k])) {
+                m |= 1u << ((k >> 1) + 4 * (k & 1));
             }
         }
         return m;
+    };
+    auto mask_of = [&](int blk) -> uint32_t {
+        if (blk == whole_blocks) {
+            return mask_part();
+        }
+        const uint4 raw = vector_of(blk);
+        return one_sign ? mask_whole(raw, std::true_type()) : mask_whole(raw, std::false_type());
     };
     const bool kept = s.blocks <= (int)sizeof(rs.masks) / WAVE;  // the matches of every block fit LDS
     int        mine = 0;
@@ -1954,28 +2024,52 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
             z[0] = z[1] = z[2] = z[3] = make_uint4(0u, 0u, 0u, 0u);
         }
         unsigned long long todo = __ballot(may);
-        while (todo != 0ull) {
-            constexpr int U = 4;  // (eight: a microsecond more on rows with one block, nothing gained on long ones)
+        auto count = [&](int blk, uint32_t m) {
+            mine += __popc(m);
+            if (kept) {
+                rs.masks[blk * WAVE + lane_id()] = (uint8_t)m;
+            }
+        };
+        if (whole_blocks >= g && whole_blocks < g + WAVE && ((todo >> (whole_blocks - g)) & 1ull) != 0ull) {
+            todo &= ~(1ull << (whole_blocks - g));
+            count(whole_blocks, mask_part());
+        }
+        // U blocks in flight, the next one requested as soon as one has been looked at (requested where they were looked at,
+        // which kept one in flight, and with two comparisons per pair of columns: 10.1 us for the 297 blocks of 152064
+        // columns; so: 6.1, the 43 KB/us that a compute unit gets from the last-level cache)
+        auto look = [&](auto same_sign) {
+            constexpr int U = 4;
             int           blk[U];
-            uint32_t      m[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                blk[u] = todo != 0ull ? g + __builtin_ctzll(todo) : -1;
+            uint4         raw[U];
+            auto          next = [&]() -> int {
+                const int b = todo != 0ull ? g + (int)__builtin_ctzll(todo) : -1;
                 todo &= todo - 1ull;
-            }
+                return __builtin_amdgcn_readfirstlane(b);
+            };
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                m[u] = mask_of(max(blk[u], 0));
+                blk[u] = next();
+                raw[u] = vector_of(max(blk[u], 0));
             }
+#pragma unroll 1
+            while (blk[0] >= 0) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (blk[u] >= 0) {
-                    mine += __popc(m[u]);
-                    if (kept) {
-                        rs.masks[blk[u] * WAVE + lane_id()] = (uint8_t)m[u];
+                for (int u = 0; u < U; ++u) {
+                    const int      now = blk[u];
+                    const uint32_t m   = mask_whole(raw[u], same_sign);
+                    blk[u]             = next();
+                    raw[u]             = vector_of(max(blk[u], 0));
+                    if (now >= 0) {
+                        count(now, m);
                     }
                 }
             }
+        };
+        if (one_sign) {
+            look(std::true_type());
+        }
+        else {
+            look(std::false_type());
         }
     }
     mine = wave_sum_i(mine);

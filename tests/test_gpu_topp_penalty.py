@@ -140,6 +140,29 @@ def test_deep_draws_into_long_runs(dt, V, kind):
 
 
 @pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("head", [600, 2048, 2049, 8191, 8193, 16384, 16640])
+@pytest.mark.parametrize("V", [20011, 19969])
+def test_draws_around_the_end_of_the_short_runs(dt, head, V):
+    """16-bit rows of `head` columns of hundreds of values in front of long runs whose probabilities are half a last place
+    of the running sum and less: draws on both sides of where the scan's values lie position by position, and picks in the
+    last columns, of which 43 or one fill no block."""
+    B = 8
+    rng = np.random.default_rng(V + head + dt)
+    x = np.full((B, V), -6.0, np.float32) + rng.choice(np.array([0.0, 0.03125, 0.0625], np.float32), (B, V))
+    for row in x:
+        at = rng.permutation(V)[:head]
+        row[at] = rng.standard_normal(head) * 1.2 - 0.5
+    x[6:, :] = -9.0
+    x[6:, -30:] = rng.standard_normal((2, 30))
+    x[7, -1] = 5.0
+    x = O.to_storage(x, dt)
+    p = np.ones(B, np.float32)
+    draws = np.array([0.02, 0.6, 0.9, 0.97, 0.995, 0.9999, 0.7, 0.3], np.float32)
+    end_ids = np.full(B, -1, np.int32)
+    _same(_sample_step(dt, x, V, p, end_ids, draws), _oracle_step(dt, x, V, p, end_ids, draws), dt)
+
+
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("V,Vp", [(9001, 9001), (9001, 9008), (2000, 2003)])
 @pytest.mark.parametrize("first", [-0.0, 0.0])
 def test_largest_values_are_zeros_of_both_signs(dt, V, Vp, first):
