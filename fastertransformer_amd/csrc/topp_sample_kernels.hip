@@ -31,7 +31,8 @@
 namespace ftk {
 
 constexpr int   TSP_STAGE   = 256;        // threads of a stage workgroup, fp32
-constexpr int   TSP_STAGE16 = 512;        // 16-bit types
+// 16-bit types: of a workgroup with and without penalties
+constexpr int   topp_stage16_threads(bool penalties) { return penalties ? 512 : 256; }
 constexpr int   TSP_SUM16   = 1024;       // threads of a sum workgroup, 16-bit types
 constexpr int   TSP_SUM32   = 256;        // fp32
 constexpr int   TSP_CHAINS  = 1024;       // summation chains of a row (the reference's block)
@@ -202,12 +203,12 @@ __device__ __forceinline__ uint4 topp_load8(const uint16_t* from)
 // straight-line code, which every wave fetched to run it once: 64 x 128256 bfloat16 with temperature and penalty
 // 15.1 -> 12.4 us (16 MB read, 16 MB written; 0.2 of the copy rate), 128 x 152064 with 51 rows of its own 17.9 -> 15.7.
 template<int DT, bool TRANSFORM>
-__global__ void __launch_bounds__(TSP_STAGE16) topp_stage_kernel(ToppStep s)
+__global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_kernel(ToppStep s)
 {
     typedef Storage<DT>   S;
     typedef typename S::T T;
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    constexpr int         EPV = 8, NW = TSP_STAGE16 / WAVE;
+    constexpr int         EPV = 8, THREADS = topp_stage16_threads(TRANSFORM), NW = THREADS / WAVE;
     constexpr uint32_t    INF16 = DT == DT_F16 ? 0x7C00u : 0x7F80u;
     __shared__ uint32_t   window[TRANSFORM ? TSP_WINDOW : 1];
     __shared__ float      red[16];
@@ -219,7 +220,7 @@ __global__ void __launch_bounds__(TSP_STAGE16) topp_stage_kernel(ToppStep s)
     const T*  rowp = (const T*)s.logits + (size_t)row * s.Vp;
     // the history, the first blocks and everything about the row are requested together
     const bool  hist = TRANSFORM && s.penalties != nullptr && s.penalty_type != 2;
-    ToppHistory<TSP_STAGE16> history;
+    ToppHistory<THREADS> history;
     if (hist) {
         history.request(s, row, 0);
     }
@@ -238,7 +239,7 @@ __global__ void __launch_bounds__(TSP_STAGE16) topp_stage_kernel(ToppStep s)
     const float mul = f.temperature_active ? f.temperature.inv : 1.0f;
     if (s.parts > 1) {
         uint4* counters = reinterpret_cast<uint4*>(s.counts + (size_t)row * ToppCode<DT>::COUNTERS);
-        for (int i = j * TSP_STAGE16 + t; i < ToppCode<DT>::COUNTERS / 4; i += s.splits * TSP_STAGE16) {
+        for (int i = j * THREADS + t; i < ToppCode<DT>::COUNTERS / 4; i += s.splits * THREADS) {
             counters[i] = make_uint4(0u, 0u, 0u, 0u);
         }
     }
@@ -247,7 +248,7 @@ __global__ void __launch_bounds__(TSP_STAGE16) topp_stage_kernel(ToppStep s)
     }
     if (hist) {
         const int words = (hi - lo + 31) / 32 + 1;
-        for (int i = t; i < words; i += TSP_STAGE16) {
+        for (int i = t; i < words; i += THREADS) {
             window[i] = 0u;
         }
         lds_barrier();
@@ -2193,13 +2194,14 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     if (dtype == DT_F32 && keeps_y && topp_part_columns(vocab, p.parts) > TSP_WINDOW_BITS) {
         p.parts = 16;
     }
-    // 16-bit stage: about sixteen waves per compute unit, at least a block of columns for each, and no more columns than a
-    // workgroup's bitmap of the history covers. Workgroups of 512 threads: each walks the row's whole history (us of the
-    // stage with 256 / 512 / 1024 threads: 64 x 128256 13.9 / 13.7 / 13.4, 128 x 152064, 51 rows of its own 16.1 / 15.6 / 16.0;
-    // twice the waves 14.1 and 15.7).
+    // 16-bit stage: about sixteen waves per compute unit, workgroups of at least four blocks of columns, no more columns than
+    // a bitmap of the history covers. Workgroups of 512 threads where each walks the row's whole history (us of the stage
+    // with 256 / 512 / 1024: 64 x 128256 13.9 / 13.7 / 13.4, 128 x 152064 with 51 rows of its own 16.1 / 15.6 / 16.0; twice
+    // the waves 14.1 and 15.7), of 256 where there are no penalties (a step of 8 x 50257 29.5, with 512 30.2). Eight blocks
+    // per workgroup, one for each wave, instead of four: a step of 1 x 32000 with penalties 25.8 / 26.4.
     p.blocks = (vocab + TSP_BLOCK - 1) / TSP_BLOCK;
-    int s    = (TSP_STAGE_WAVES / (TSP_STAGE16 / WAVE) + rows - 1) / rows;
-    s        = std::min(s, std::max(1, p.blocks / (TSP_STAGE16 / WAVE)));
+    int s    = (TSP_STAGE_WAVES / (topp_stage16_threads(keeps_y) / WAVE) + rows - 1) / rows;
+    s        = std::min(s, std::max(1, p.blocks / 4));
     s        = std::max(s, (p.blocks + TSP_WINDOW_BITS / TSP_BLOCK - 1) / (TSP_WINDOW_BITS / TSP_BLOCK));
     p.splits = std::min(s, TSP_SPLITS);
     p.chunk  = (p.blocks + p.splits - 1) / p.splits * TSP_BLOCK;
@@ -2334,10 +2336,10 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
     auto run = [&](auto type) -> int {
         constexpr int DT = decltype(type)::value;
         if (keeps_y) {
-            topp_stage_kernel<DT, true><<<splits, TSP_STAGE16, 0, st>>>(s);
+            topp_stage_kernel<DT, true><<<splits, topp_stage16_threads(true), 0, st>>>(s);
         }
         else {
-            topp_stage_kernel<DT, false><<<splits, TSP_STAGE16, 0, st>>>(s);
+            topp_stage_kernel<DT, false><<<splits, topp_stage16_threads(false), 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
         if (p.parts == 1) {
