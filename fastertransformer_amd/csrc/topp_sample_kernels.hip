@@ -705,7 +705,9 @@ __device__ __forceinline__ void topp_group_sums(const ToppStep& s, int row, int 
 // A workgroup owns C summation chains: C neighbouring columns out of every 1024 (a "stretch"). Its waves share the
 // stretches out, read eight bytes - four chains - per lane and leave the e of a chunk of stretches in LDS, from where
 // one thread per chain adds them up in the reference's order. (One chain per thread straight from memory would mean
-// two-byte loads and a dependent addition per load.) 64 x 128256 bfloat16: 14 us, vector instructions in 0.55 of it.
+// two-byte loads and a dependent addition per load.) Where a quarter of the threads adds, the others go on with the next
+// chunk in a second buffer: 64 x 128256 bfloat16 13.0 -> 12.0 us, vector instructions in 0.6 of it; 51 rows of 152064 18.3 ->
+// 17.7. Where all of them add, two buffers of half the size only cost barriers (a step of 256 x 128256 bfloat16 93.8 -> 95.4).
 // e is a function of the 16 bits of y once the maximum is known, but a table of it in LDS, made by every workgroup, does
 // not pay: gathers from it cost as much as the exponential (256 x 128256, us a step with a table / so: binary16 95 / 92,
 // bfloat16 76 / 76; every second column masked 98 / 84 and 85 / 72).
@@ -715,12 +717,13 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
     typedef Storage<DT>   S;
     typedef typename S::T T;
     typedef ToppCode<DT>  Code;
-    constexpr int         KI  = 16384 / C;                 // stretches of a chunk: 32 KB of e
+    constexpr int         HALVES = C < TSP_SUM16 ? 2 : 1;  // buffers of e, 32 KB in all
+    constexpr int         KI  = 16384 / HALVES / C;        // stretches of a chunk
     constexpr int         WS  = C / 4 / WAVE;              // waves side by side in a stretch
     constexpr int         PAR = TSP_SUM16 / WAVE / WS;     // stretches taken at a time
     constexpr int         U   = KI / PAR;                  // vectors per lane and chunk
     __shared__ uint32_t   cnt[Code::USED + WAVE];
-    __shared__ uint2      e_of[KI * C / 4];
+    __shared__ uint2      e_of[HALVES][KI * C / 4];
     const int             row = blockIdx.x, part = blockIdx.y, t = threadIdx.x;
     const T* y = s.y != nullptr ? (const T*)s.y + (size_t)row * s.y_pitch : (const T*)s.logits + (size_t)row * s.Vp;
     const int q    = (t & (C / 4 - 1)) * 4 + part * C;  // first of this lane's four chains
@@ -765,7 +768,8 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
     const uint32_t pad = S::st(-S::max_t());
     float          sum = 0.0f;
     int            at  = 0;
-    for (int i0 = 0; i0 < nst; i0 += KI) {
+    int            half = 0;
+    for (int i0 = 0; i0 < nst; i0 += KI, half ^= HALVES - 1) {
 #pragma unroll 1
         for (int u = 0; u < U; ++u, ++at) {
             const int i = mine + u * PAR;
@@ -799,18 +803,22 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
                     b[3] = c == 3 ? e : b[3];
                 }
             }
-            e_of[i * (C / 4) + (t & (C / 4 - 1))] = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+            e_of[half][i * (C / 4) + (t & (C / 4 - 1))] = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
         }
         lds_barrier();
         if (t < C) {
-            const T*  e = reinterpret_cast<const T*>(e_of) + t;
+            const T*  e = reinterpret_cast<const T*>(e_of[half]) + t;
             const int k = min(KI, nst - i0);
 #pragma unroll 8
             for (int i = 0; i < k; ++i) {
                 sum += S::ld(e[i * C]);
             }
         }
-        lds_barrier();
+        // (with two buffers the waves that add nothing go on with the other one; what is added here is overwritten behind the
+        // next barrier only)
+        if constexpr (HALVES == 1) {
+            lds_barrier();
+        }
     }
     if (t < C) {
 #pragma unroll
