@@ -163,6 +163,23 @@ def test_draws_around_the_end_of_the_short_runs(dt, head, V):
 
 
 @pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("runs", [[1, 127, 128, 129, 130, 135, 136, 137, 143, 144, 145, 301, 1001], [5000, 5003, 5001], [3, 16379, 9],
+                                  [8191, 127, 140], [16384, 1, 133], [129] * 140, [1]], ids=lambda r: "%dx%d" % (len(r), r[0]))
+def test_draws_from_long_runs_at_the_head(dt, runs):
+    """16-bit rows of few distinct values, whose first runs are around the lengths at which their positions are written by
+    different threads, end anywhere in a vector of eight and reach over the end of the array; draws from all over the row."""
+    V, B = 20011, 24
+    rng = np.random.default_rng(sum(runs) + dt)
+    value = np.concatenate([np.full(n, -0.0625 * i) for i, n in enumerate(runs)] + [np.full(V - sum(runs), -0.0625 * len(runs))])
+    x = O.to_storage(np.stack([value[rng.permutation(V)] for _ in range(B)]).astype(np.float32), dt)
+    p = np.ones(B, np.float32)
+    draws = rng.uniform(0.0, 1.0, B).astype(np.float32)
+    draws[:4] = [1e-7, 0.9999, 0.01, 0.02]
+    end_ids = np.full(B, -1, np.int32)
+    _same(_sample_step(dt, x, V, p, end_ids, draws), _oracle_step(dt, x, V, p, end_ids, draws), dt)
+
+
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("V,Vp", [(9001, 9001), (9001, 9008), (2000, 2003)])
 @pytest.mark.parametrize("first", [-0.0, 0.0])
 def test_largest_values_are_zeros_of_both_signs(dt, V, Vp, first):
