@@ -1619,7 +1619,6 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     if (t == 0) {
         sh_enough = 0xFFFFFFFFu;
         sh_found  = 0x7FFFFFFF;
-        sh_mixed  = 0;
     }
     if (r.skip) {
         if (t == 0) {
@@ -1781,45 +1780,50 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
             // Near the head of a row runs are short, and a tile taken out of them is a chain of look-ups (1.6 us per 32 tiles).
             // Sixteen threads write a run's value to its positions, and a lane's eight values are one read (128 x 152064
             // bf16: the scan for a draw behind 15000 entries 8.8 -> 5.2 us, behind 77000, with what follows, 20 -> 10). A row of
-            // few distinct values has long runs at its head: what they have beyond SHORT positions is left to a wave each, eight
-            // positions per lane. us a step of 64 x 128256, sixteen threads for a run of any length / so: bf16 of four values
-            // 72.4 / 45.6 (binary16 61.4 / 48.3), 16000 equal ones at the head 63.3 / 36.9 (57.8 / 44.7), Zipf 37.0 / 36.5
-            // (44.1 / 44.6); 8 x 32000 bf16 of four values 45.5 / 28.1. SHORT of 64 and 256: within 0.5 of it.
+            // few distinct values has long runs at its head: sixteen bytes per store beyond SHORT positions. us a step of 64 x
+            // 128256, two bytes per store throughout / so: bf16 of four values 72.5 / 46.1 (binary16 61.4 / 48.4), 16000 equal ones
+            // at the head 63.0 / 37.3 (57.6 / 44.6), Zipf 37.0 / 36.0 (44.7 / 44.8); 8 x 32000 bf16 of four values 45.3 / 28.4. The
+            // next run is requested ahead of the stores: without that binary16 lost 0.4 on rows of short runs.
             constexpr int SHORT  = 128;
             const int     flat_n = min(FLAT, (enough + TP_TILE - 1) / TP_TILE * TP_TILE);
-            for (int k = t >> 4; k < (int)nruns; k += TP_THREADS / 16) {
-                const int begin = (int)rs.start[k], end = min((int)rs.start[k + 1], flat_n);
-                if (begin >= flat_n) {
-                    break;
-                }
-                const uint16_t v    = rs.prob[k];
-                const int      some = min(end, (begin + SHORT + 7) & ~7);
-                for (int i = begin + (t & 15); i < some; i += 16) {
-                    flat[i] = v;
-                }
-                if (some < end && (t & 15) == 0) {
-                    sc.carry[atomicAdd(&sh_mixed, 1)] = __int_as_float(k);
+            {
+                const int lane = t & 15, last = (int)nruns;
+                int       k = t >> 4, begin = (int)rs.start[min(k, last)], end = (int)rs.start[min(k + 1, last)];
+                uint32_t  v = rs.prob[min(k, last)];
+                while (k < last && begin < flat_n) {
+                    k += TP_THREADS / 16;
+                    const int      begin_next = (int)rs.start[min(k, last)], end_next = (int)rs.start[min(k + 1, last)];
+                    const uint32_t v_next     = rs.prob[min(k, last)];
+                    end                       = min(end, flat_n);
+                    if (end - begin <= SHORT) {
+#pragma unroll 1
+                        for (int i = begin + lane; i < end; i += 16) {
+                            flat[i] = (uint16_t)v;
+                        }
+                    }
+                    else {
+                        const int      lo = (begin + 7) & ~7, hi = end & ~7;
+                        const uint32_t vv = v * 0x00010001u;
+                        if (begin + lane < lo) {
+                            flat[begin + lane] = (uint16_t)v;
+                        }
+                        if (hi + lane < end) {
+                            flat[hi + lane] = (uint16_t)v;
+                        }
+#pragma unroll 4
+                        for (int i = lo + lane * 8; i < hi; i += 128) {
+                            *reinterpret_cast<uint4*>(flat + i) = make_uint4(vv, vv, vv, vv);
+                        }
+                    }
+                    begin = begin_next;
+                    end   = end_next;
+                    v     = v_next;
                 }
             }
             if ((int)n + t < flat_n) {  // (fewer than a tile's)
                 flat[n + t] = 0;
             }
             __syncthreads();
-            const int longer = sh_mixed;
-            if (longer != 0) {
-                for (int m = wave_id(); m < longer; m += NW) {
-                    const int      k   = __float_as_int(sc.carry[m]);
-                    const int      end = min((int)rs.start[k + 1], flat_n);
-                    const uint32_t vv  = (uint32_t)rs.prob[k] * 0x00010001u;
-                    for (int i = (((int)rs.start[k] + SHORT + 7) & ~7) + lane_id() * 8; i + 8 <= end; i += WAVE * 8) {
-                        *reinterpret_cast<uint4*>(flat + i) = make_uint4(vv, vv, vv, vv);
-                    }
-                    if (lane_id() < (end & 7)) {
-                        flat[(end & ~7) + lane_id()] = (uint16_t)vv;
-                    }
-                }
-                __syncthreads();
-            }
             auto flat_load = [&](int i0, float* x) {
                 const uint4    q    = *reinterpret_cast<const uint4*>(flat + i0);
                 const uint32_t w[4] = {q.x, q.y, q.z, q.w};
