@@ -202,7 +202,10 @@ __device__ __forceinline__ uint4 topp_load8(const uint16_t* from)
 // history (2 us), then a few blocks per wave. Requesting the history first and a short loop instead of 25 KB of
 // straight-line code, which every wave fetched to run it once: 64 x 128256 bfloat16 with temperature and penalty
 // 15.1 -> 12.4 us (16 MB read, 16 MB written; 0.2 of the copy rate), 128 x 152064 with 51 rows of its own 17.9 -> 15.7.
-template<int DT, bool TRANSFORM>
+// An embedding bias has an instantiation of its own and is read like the row, sixteen bytes from any column on. us a step with
+// a bias, its columns through the loop of the row's end / one two-byte load each / so: 256 x 128256 bfloat16 128.5 / 108.6 /
+// 75.5, binary16 143.2 / 124.4 / 91.3; 64 x 128256 52.4 / 53.3 / 40.2; 1 x 32000 with penalties 27.0 / 29.4 / 26.1.
+template<int DT, bool TRANSFORM, bool BIASED>
 __global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_kernel(ToppStep s)
 {
     typedef Storage<DT>   S;
@@ -265,7 +268,10 @@ __global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_ke
     // through it a few times only, so that straight-line code waits for its own fetch.
 #pragma unroll 1
     for (int b = wave_id(); b < nblk; b += NW) {
-        uint4 raw = r0;
+        uint4 raw = r0, add = {};
+        if constexpr (BIASED) {  // (in front of the next block's load: what is waited for first)
+            add = topp_load8(f.bias + max(0, min(lo + b * TSP_BLOCK + lane_id() * EPV, s.n - EPV)));
+        }
         r0        = r1;
         r1        = r2;
         r2        = r3;
@@ -274,7 +280,7 @@ __global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_ke
         const int      rel  = v - lo;
         const uint32_t bits = TRANSFORM && hist && v < hi ? (window[rel >> 5] >> (rel & 31)) & 0xFFu : 0u;
         float          vm   = TSP_LOWEST;
-        if (v + EPV > s.n || (TRANSFORM && f.bias != nullptr)) {
+        if (v + EPV > s.n) {
             // two columns at a time; the words of the vector take turns in `raw.x`
 #pragma unroll 1
             for (int k = 0; k < EPV / 2; ++k) {
@@ -297,6 +303,13 @@ __global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_ke
         else {
             if constexpr (TRANSFORM) {
                 T* e = reinterpret_cast<T*>(&raw);
+                if constexpr (BIASED) {
+                    const T* a = reinterpret_cast<const T*>(&add);
+#pragma unroll
+                    for (int c = 0; c < EPV; ++c) {
+                        e[c] = S::st(S::ld(e[c]) + S::ld(a[c]));
+                    }
+                }
 #pragma unroll
                 for (int c = 0; c < EPV; ++c) {
                     e[c] = S::st(S::ld(e[c]) * mul);
@@ -2387,11 +2400,14 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
     }
     auto run = [&](auto type) -> int {
         constexpr int DT = decltype(type)::value;
-        if (keeps_y) {
-            topp_stage_kernel<DT, true><<<splits, topp_stage16_threads(true), 0, st>>>(s);
+        if (keeps_y && s.temperatures != nullptr && s.bias != nullptr) {  // (the bias comes with the temperature)
+            topp_stage_kernel<DT, true, true><<<splits, topp_stage16_threads(true), 0, st>>>(s);
+        }
+        else if (keeps_y) {
+            topp_stage_kernel<DT, true, false><<<splits, topp_stage16_threads(true), 0, st>>>(s);
         }
         else {
-            topp_stage_kernel<DT, false><<<splits, topp_stage16_threads(false), 0, st>>>(s);
+            topp_stage_kernel<DT, false, false><<<splits, topp_stage16_threads(false), 0, st>>>(s);
         }
         FTK_LAUNCH_CHECK();
         if (p.parts == 1) {

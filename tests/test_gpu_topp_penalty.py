@@ -316,6 +316,28 @@ def test_biased_nucleus_rows(dt, B, window, V, Vp):
                 compare(p.snapshot(), o.snapshot(), dt, check_logits=False, where="step %d window %d" % (i, ite))
 
 
+@pytest.mark.parametrize("dt", [O.F16, O.BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("V,Vp,offset", [(1025, 1025, 1), (4103, 4104, 3), (20011, 20011, 0)])
+def test_bias_anywhere_in_memory(dt, V, Vp, offset):
+    """A bias that starts off the 16-byte grid, under rows whose last vector runs over the end, with a history and a masked
+    end id in whole vectors and in that one."""
+    import torch
+    B, H = 4, 40
+    rng = np.random.default_rng(V + dt)
+    prompt = rng.integers(0, V, (H, B)).astype(np.int32)
+    prompt[:8] = V - 1 - np.arange(8)[:, None]
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=1, runtime_top_k=np.zeros(B, np.uint32), runtime_top_p=np.full(B, 0.9),
+             temperature=rng.uniform(0.5, 1.5, B), min_length=np.full(B, H + 9), end_ids=np.array([V - 1, V - 9, 8, 0]),
+             prompt=prompt, embedding_bias=O.to_storage(rng.standard_normal(Vp).astype(np.float32) * 2, dt),
+             repetition_penalty=rng.uniform(1.1, 1.5, B), with_cum=True, with_out_lp=True)
+    p, o = ProductRunner(c), OracleRunner(c)
+    p.bias = torch.cat([torch.zeros(offset, dtype=p.bias.dtype, device="cuda"), p.bias])[offset:]
+    x, u = make_logits(rng, dt, B, V, Vp, 2.0), uniforms(rng, B)
+    p.step(H, x, u)
+    o.step(H, x, u)
+    compare(p.snapshot(), o.snapshot(), dt, check_logits=False)
+
+
 def _penalty_step(dt, x, V, p_arr, end_ids, draws, finished, temps, penalties, history):
     """_sample_step with a temperature and a repetition penalty over `history` [steps, rows]"""
     import torch
