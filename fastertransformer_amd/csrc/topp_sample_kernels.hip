@@ -51,7 +51,6 @@ struct ToppStep {
     int          n, Vp, rows;  // columns of the vocabulary, pitch of a row
     void*        y;            // [rows][y_pitch], or null: y is the logits themselves
     int          y_pitch;
-    bool         y_stream;     // 16-bit: y leaves the L2 as it is written
     const float* temperatures;
     const float* penalties;
     int          penalty_type;  // 2: none
@@ -276,6 +275,13 @@ __global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_ke
         r1        = r2;
         r2        = r3;
         r3        = load(b + 4 * NW);
+        {   // One vector from here on. Left to itself the compiler takes it apart: loads of 12 and 8 bytes in binary16 (the kernel
+            // at 160 x 50257 14.2 -> 15.3 us), a conversion per column instead of one per two in bfloat16 (64 x 128256 12.6 -> 13.2).
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            u32x4 whole = __builtin_bit_cast(u32x4, raw);
+            asm("" : "+v"(whole));
+            raw = __builtin_bit_cast(uint4, whole);
+        }
         const int      v    = lo + b * TSP_BLOCK + lane_id() * EPV;
         const int      rel  = v - lo;
         const uint32_t bits = TRANSFORM && hist && v < hi ? (window[rel >> 5] >> (rel & 31)) & 0xFFu : 0u;
@@ -343,15 +349,11 @@ __global__ void __launch_bounds__(topp_stage16_threads(TRANSFORM)) topp_stage_ke
             }
         }
         if constexpr (TRANSFORM) {
-            if (v < hi) {  // (rows of y are padded to whole vectors)
-                uint4* to = reinterpret_cast<uint4*>(y + v);
-                if (s.y_stream) {
-                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-                    __builtin_nontemporal_store(__builtin_bit_cast(u32x4, raw), reinterpret_cast<u32x4*>(to));
-                }
-                else {
-                    *to = raw;
-                }
+            // (rows of y are padded to whole vectors; y that does not stay in the L2s, which the stage writes back at its end,
+            // makes the stage faster and the sum slower: 64 x 128256 12.6 -> 11.8 and 11.4 -> 12.0 us, a step of 128 x 152064 with
+            // 51 rows of its own 74 -> 75)
+            if (v < hi) {
+                *reinterpret_cast<uint4*>(y + v) = raw;
             }
         }
         const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -2330,10 +2332,6 @@ int topp_sample_launch(const ToppSampleCall& c, hipStream_t st)
     s.rows   = c.rows;
     s.y      = keeps_y ? ws + p.off_y : nullptr;
     s.y_pitch          = p.y_pitch;
-    // What the L2s (32 MB) hold of y at the end of the stage they write back before the sum may start; y that streams out
-    // while the stage runs does without that wait, and more than that leaves by itself. us, through L2 / streamed: stage
-    // kernel of 64 x 128256 13.8 / 12.4; whole steps 256 x 128256 100.6 / 101.1, 512 x 152064 290 / 303.
-    s.y_stream         = (size_t)c.rows * p.y_pitch * sizeof(uint16_t) <= ((size_t)32 << 20);
     s.temperatures     = c.temperatures;
     s.penalties        = c.penalties;
     s.penalty_type     = c.penalty_type;
