@@ -322,13 +322,14 @@ int ftk_invoke_log_prob_from_logits(int dtype, float* cum_log_probs, const void*
         // were written just before / that were not: 16 x 16 x 50257 (25 MB) 14.9 / 15.0, 16.5 / 16.8; 40 x 16 x 50257 (64 MB)
         // 20.5 / 20.2, 21.7 / 21.2; 64 x 16 x 50257 24.7 / 24.5, 27.8 / 25.8; 40 x 32 x 50257 29.0 / 29.9, 32.8 / 30.1; 48 x
         // 32 x 50257 33.0 / 35.8, 37.1 / 34.9; 64 x 32 x 50257 40.0 / 44.6, 45.3 / 40.7; 96 x 32 x 50257 (more than the
-        // last-level cache) 71.1 / 61.2, 63.2 / 55.4. fp32 from 128 MB on, also with the same logits in every call: 32 x 16 x
-        // 50257 (103 MB) 21.7 / 21.8, 17.7 / 20.4, 17.7 / 20.8; 32 x 24 x 50257 24.1 / 23.8, 26.7 / 23.9, 23.1 / 24.1; 16 x 64 x
-        // 50257 33.1 / 31.0, 35.4 / 31.3, 29.7 / 30.8; 32 x 40 x 50257 46.7 / 40.7, 44.3 / 38.2, 36.1 / 38.2; 32 x 64 x 50257
-        // 78.3 / 65.6, 63.3 / 55.8, 54.9 / 55.1. (the descriptor of a row holds its bytes in 32 bits)
+        // last-level cache) 71.1 / 61.2, 63.2 / 55.4. fp32 only from 320 MB on, where even logits that are scored again, as many
+        // of them as the last-level cache holds, lose nothing; written just before / the same logits in every call: 32 x 24 x
+        // 50257 (147 MB) 25.4 / 28.4, 21.8 / 22.4; 8 x 40 x 128256 44.4 / 47.3, 31.3 / 39.0; 8 x 64 x 128256 52.4 / 47.7, 32.9 / 40.8; 32 x
+        // 44 x 50257 (270 MB) 61.3 / 52.3, 39.6 / 42.0; 32 x 56 x 50257 (344 MB) 83.1 / 69.3, 50.3 / 50.1; 8 x 96 x 128256 83.2 /
+        // 69.4, 52.5 / 51.3; 32 x 96 x 50257 122.0 / 90.3, 89.2 / 78.5. (the descriptor of a row holds its bytes in 32 bits)
         const size_t elem = dtype == FTK_DTYPE_F32 ? 4 : 2;
         const bool   once = vocab_size_padded * elem < ((size_t)1 << 31)
-                          && max_input_length * batch_size * vocab_size_padded * elem >= (size_t)(elem == 4 ? 128 : 64) << 20;
+                          && max_input_length * batch_size * vocab_size_padded * elem >= (size_t)(elem == 4 ? 320 : 64) << 20;
         auto       run  = [&](auto dt, auto past) {
             constexpr int DT = decltype(dt)::value;
             log_probs_kernel<DT, decltype(past)::value><<<(unsigned)rows, LP_THREADS, 0, st>>>(

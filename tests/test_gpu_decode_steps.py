@@ -71,9 +71,11 @@ def test_log_prob_from_large_logits_line_offsets(dt, shape):
     test_log_prob_from_logits(dt, False, shape)
 
 
-@pytest.mark.parametrize("shape", [(64, 32, 16384), (64, 32, 16376), (1024, 33, 1003), (4096, 256, 33)])
+@pytest.mark.parametrize("shape", [(64, 32, 16384), (64, 32, 16376), (1024, 33, 1003), (4096, 256, 33), (64, 32, 40960), (64, 32, 40952),
+                                   (2600, 33, 1003), (8192, 256, 33)])
 def test_log_prob_from_large_fp32_logits(shape):
-    """fp32 goes past the caches from exactly 128 MB on: that size, just below it, rows at every offset from a 128-byte boundary."""
+    """fp32 goes past the caches from exactly 320 MB on: that size, just below it, rows at every offset from a 128-byte boundary,
+    and the same below it."""
     test_log_prob_from_logits(O.F32, False, shape)
 
 
