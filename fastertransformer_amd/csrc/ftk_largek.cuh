@@ -3,8 +3,8 @@
 //
 // The lean gather takes three launches for them (lean_gather_kernel in its SLOTS and PRESET modes, lean_select_kernel),
 // bound by the latency of many small workgroups and by a selection on four waves. Here
-//   1. every thread takes the exact maxima of three disjoint groups of its columns (3072 per row, each the final
-//      value of a column of its own, after temperature, history penalty and masks);
+//   1. every thread takes the exact maxima of three disjoint groups of its columns (3072 per row, in short rows
+//      one per vector and edge column, each the final value of a column of its own, after temperature, history penalty and masks);
 //   2. the row's bound: the largest P, to within its low sixteen bits, that at least k of those maxima reach (two
 //      rounds of a 256-bin count over the keys' top bytes) - at least k columns lie at or above it;
 //   3. the vectors that hold something at or above the bound are noted in LDS and evaluated exactly, one per lane, into
@@ -16,7 +16,7 @@
 // What bounds it, 256 x 51200 f16, k = 1024 (us inside a workgroup): set-up 1.9, first pass 2.4, bound 4.4, second pass 7.4
 // with its barrier, order 5.6, draw 4.1; 31 a step, 65 with maxima, gather and selection in launches of their own. With 12
 // instead of 9 vectors in registers the compiler spills 41 of them.
-// Preconditions (checked by the host): no embedding bias, three vectors of a row per unit of k, the row's history bitmap
+// Preconditions (checked by the host): no embedding bias, three vectors of a row for every two of k, the row's history bitmap
 // fits the LDS window, logits on an element's boundary.
 #pragma once
 #include "ftk_rowwide.cuh"
@@ -30,6 +30,7 @@ constexpr int LK_RING       = 9;    // vectors a thread holds
 constexpr int LK_HIST_U     = 4;     // history ids a thread requests at a time
 constexpr int LK_BUCKETS    = 2048;  // of the final order: 256 for each of eight doublings of the distance to the bound
 constexpr int LK_BUCKET_CAP = 512;   // entries of a bucket are compared with each other
+constexpr int LK_BUCKET_FEW = 96;    // a bucket with more of them and most of the list is divided by buckets of its own
 static_assert(LK_RING % LK_GROUPS == 0, "a slot of the ring always belongs to the same group");
 
 struct LargekShared {
@@ -42,7 +43,8 @@ struct LargekShared {
     uint32_t key_max;
     int      slice_count[8];
     int      n_list;
-    int      crowded;
+    uint32_t fullest;         // entries of the fullest bucket << 16 | its number, where it holds more than a few
+    uint32_t key_lo[2], key_hi[2];  // the range of its keys, twice
 };
 
 // The lane of wave 0 that holds bins 4 lane .. 4 lane + 3 of a 256-bin count finds the highest bin b with at least
@@ -92,10 +94,12 @@ __device__ __forceinline__ bool largek_bin_of_rank(const uint32_t* hist, int lan
 // The list in ts.cand (256 < n <= TK_CCAP entries, all at or above thr_f, key_max the largest key) in the order of the
 // reference, by all threads: stage 1 orders a slice by (value, thread, block), which gives every entry its rank in the
 // slice, stage 2 the whole list by (value, what follows from slice and rank). Both need only neighbours of similar value:
-// the entries are counted into 2048 buckets, put down bucket by bucket, and compared inside their bucket;
+// the entries are counted into 2048 buckets, put down bucket by bucket, and compared inside their bucket (counted again where one
+// bucket holds many: us a step of 64 x 50257, k = 1024, counted once / so, a column 3e4 ahead of the others f16 94.0 / 29.2, f32
+// 94.0 / 29.8; 300 valid columns f16 53.5 / 26.1, f32 55.5 / 29.7; 800 f32 53.7 / 33.8; ordinary rows 28.5 / 28.7 and 29.3 / 29.5);
 // what lies in higher buckets is a prefix sum (over all, and per slice). Weights and columns of the first min(k, n) go to
-// ts.sel, padded with zeros to a multiple of 32. False, with ts.cand as it was, where a bucket is crowded (many equal
-// values, or an outlier far ahead) or a slice holds more than k entries.
+// ts.sel, padded with zeros to a multiple of 32. False, with ts.cand as it was, where a bucket stays crowded (many
+// equal values) or a slice holds more than k entries.
 // Bound by the latency of its barriers and by LDS: 5.6 us for 1400 entries, k = 1024, and 4.1 for the draw after it, two
 // chains of 1024 dependent operations; selection and draw took 41 with the per-slice sorts and merges on four waves.
 __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, int n, int k, int max_top_k, float thr_f)
@@ -108,14 +112,15 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
     const int   bs2_log = max_top_k <= 32 ? 7 : 8;
     const float x_max   = key_to_float(s.key_max);
     // 1 at the bound, 257 at the row's maximum: the bits of that number are close to its logarithm, which gives the dense
-    // values near the bound most of the buckets, also where a single value lies far ahead of all others
-    const float scale = 256.0f / (x_max - thr_f);
-    if (!(scale > 0.0f && scale < __builtin_inff())) {
+    // values near the bound most of the buckets, also where a single value lies ahead of all others
+    // (the bound may be the lowest value of the type: the limit keeps the quotient a normal number)
+    float lo = thr_f, scale = 256.0f / __builtin_fminf(x_max - thr_f, 1.0e30f);
+    if (!(x_max < __builtin_inff() && scale < __builtin_inff())) {
         return false;
     }
-    auto bucket_of = [&](uint32_t key) -> int {
-        const uint32_t y = __float_as_uint((key_to_float(key) - thr_f) * scale + 1.0f);
-        return max(LK_BUCKETS - 1 - (int)((y - 0x3F800000u) >> 15), 0);  // (never falls as the value does)
+    auto bucket_of = [&](uint32_t key) -> int {  // (never falls as the value does)
+        const uint32_t y = __float_as_uint(__builtin_fmaxf((key_to_float(key) - lo) * scale + 1.0f, 1.0f));
+        return max(LK_BUCKETS - 1 - (int)((y - 0x3F800000u) >> 15), 0);
     };
     // lanes of the wave whose entry lies in the same slice
     auto same_slice = [&](bool have, int slice) -> unsigned long long {
@@ -140,17 +145,28 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
         const int      blk = (int)(idx >> bs1_log), slice = blk & 7;
         comp[u] = ((unsigned long long)slice << 61) | ((unsigned long long)(~key) << 29)
                   | ((unsigned long long)(BS1 - 1 - (int)(idx & (uint32_t)(BS1 - 1))) << 21) | (unsigned long long)(blk >> 3);
-        bucket[u] = have ? bucket_of(key) : 0;
-        slot[u]   = have ? (int)atomicAdd(&s.count[bucket[u]], 1u) : 0;
-        const unsigned long long m = same_slice(have, slice);
-        if (have && below_lane(m) == 0) {
-            atomicAdd(&s.slice_count[slice], (int)__builtin_popcountll(m));
-        }
     }
-    lds_barrier();
-    {  // bucket counts -> where each bucket starts
-        const uint32_t c0 = s.count[2 * t], c1 = s.count[2 * t + 1];
-        uint32_t       incl = c0 + c1;
+    auto key_of = [&](int u) -> uint32_t { return ~(uint32_t)(comp[u] >> 29); };
+    // the entries' buckets, and the entries in this thread's two buckets and all below them of the wave
+    uint32_t c0, c1, incl, sums, fullest;
+    auto     count = [&](auto slices) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool have = t + u * LK_THREADS < n;
+            bucket[u]       = have ? bucket_of(key_of(u)) : 0;
+            slot[u]         = have ? (int)atomicAdd(&s.count[bucket[u]], 1u) : 0;
+            if constexpr (decltype(slices)::value) {
+                const int                slice = (int)(comp[u] >> 61);
+                const unsigned long long m     = same_slice(have, slice);
+                if (have && below_lane(m) == 0) {
+                    atomicAdd(&s.slice_count[slice], (int)__builtin_popcountll(m));
+                }
+            }
+        }
+        lds_barrier();
+        c0   = s.count[2 * t];
+        c1   = s.count[2 * t + 1];
+        incl = c0 + c1;
 #pragma unroll
         for (int d = 1; d < WAVE; d <<= 1) {
             const uint32_t v = __shfl_up(incl, d, WAVE);
@@ -159,12 +175,50 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
         if (lane == WAVE - 1) {
             s.wave_sum[wv] = incl;
         }
-        if (__ballot(max(c0, c1) > (uint32_t)LK_BUCKET_CAP) != 0ull && lane == 0) {
-            s.crowded = 1;
+        const uint32_t most = max(c0, c1);
+        if (most > (uint32_t)LK_BUCKET_FEW) {
+            atomicMax(&s.fullest, most << 16 | (uint32_t)(2 * t + (c0 == most ? 0 : 1)));
         }
         lds_barrier();
-        const uint32_t sums  = s.wave_sum[lane & (LK_WAVES - 1)];
-        uint32_t       start = incl - c0 - c1;
+        sums    = s.wave_sum[lane & (LK_WAVES - 1)];
+        fullest = s.fullest;
+    };
+    count(std::true_type());
+#pragma unroll 1
+    for (int round = 0; __builtin_expect(fullest != 0u && round < 2, 0); ++round) {
+        // Much of the list in one bucket: the row's maximum is far ahead of it, or the bound is the lowest value of the type
+        // (fewer than k valid columns). Again, with 1 to 17, about half of the buckets, for what that one holds.
+        uint32_t klo = 0xFFFFFFFFu, khi = 0u;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool in = t + u * LK_THREADS < n && bucket[u] == (int)(fullest & 0xFFFFu);
+            klo           = min(klo, in ? key_of(u) : 0xFFFFFFFFu);
+            khi           = max(khi, in ? key_of(u) : 0u);
+        }
+        klo = ~wave_max(~klo);
+        khi = wave_max(khi);
+        if (lane == 0 && khi != 0u) {
+            atomicMin(&s.key_lo[round], klo);
+            atomicMax(&s.key_hi[round], khi);
+        }
+        lds_barrier();
+        const float from = key_to_float(s.key_lo[round]), to = key_to_float(s.key_hi[round]), finer = 16.0f / (to - from);
+        // (not where its values are equal, or equal but for rounding: then finer buckets would crowd all others)
+        if (!(finer > scale && to - from > __builtin_fabsf(to) * 0x1p-9f)) {
+            break;
+        }
+        lo                 = from;
+        scale              = finer;
+        s.count[2 * t]     = 0u;
+        s.count[2 * t + 1] = 0u;
+        if (t == 0) {
+            s.fullest = 0u;
+        }
+        lds_barrier();
+        count(std::false_type());
+    }
+    {
+        uint32_t start = incl - c0 - c1;
 #pragma unroll
         for (int w = 0; w < LK_WAVES; ++w) {
             start += w < wv ? (uint32_t)__builtin_amdgcn_readlane((int)sums, w) : 0u;
@@ -175,7 +229,7 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
             s.count[LK_BUCKETS] = (uint32_t)n;
         }
     }
-    bool one_by_one = s.crowded != 0;
+    bool one_by_one = fullest >> 16 > (uint32_t)LK_BUCKET_CAP;
 #pragma unroll
     for (int sl = 0; sl < 8; ++sl) {
         one_by_one = one_by_one || s.slice_count[sl] > k;
@@ -344,9 +398,13 @@ __global__ void __launch_bounds__(LK_THREADS) largek_step_kernel(const RowwideAr
     if (t < 8) {
         s.slice_count[t] = 0;
     }
+    if (t >= WAVE && t < WAVE + 2) {
+        s.key_lo[t - WAVE] = 0xFFFFFFFFu;
+        s.key_hi[t - WAVE] = 0u;
+    }
     if (t == 0) {
         s.n_list  = 0;
-        s.crowded = 0;
+        s.fullest = 0u;
         s.key_max = 0u;
     }
     uint32_t* window = fused_lds_bitmap<BMW>();
@@ -495,7 +553,7 @@ __global__ void __launch_bounds__(LK_THREADS) largek_step_kernel(const RowwideAr
         const bool mine = largek_bin_of_rank(s.hist, lane, (uint32_t)k, &bin, &above);
         if (__ballot(mine) == 0ull) {
             if (lane == 0) {
-                s.pick[0] = 0xFFFFFFFFu;  // (fewer than k maxima at all: there are 3072 of them)
+                s.pick[0] = 0xFFFFFFFFu;  // (fewer than k maxima at all: there are 3/2 k vectors)
             }
         }
         else if (mine) {

@@ -338,6 +338,46 @@ def test_large_k_in_one_launch(dt, B, V, Vp, offset, H, k, kind):
 
 
 @pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+def test_large_k_in_the_reference_order(dt):
+    """largek_step_kernel against the oracle: lists whose buckets are as they should be, that lie in one bucket of the first
+    count (fewer valid columns than k, a maximum far ahead, a heap in the middle), with buckets that stay full (equal values)
+    and with most candidates in one slice."""
+    rng = np.random.default_rng(91 + dt)
+    kinds = ["plain", "grid", "one slice", "valid 257", "valid 300", "valid 800", "valid 1000", "ahead 60", "ahead 200", "ahead 30000",
+             "heap", "equal 90", "equal 600", "lowest", "both"]
+    V, B = 12345, len(kinds)
+    x = (rng.standard_normal((B, V)) * 2.5).astype(np.float32)
+    for b, kind in enumerate(kinds):
+        if kind == "grid":
+            x[b] = np.round(x[b] * 4.0) / 4.0
+        elif kind == "one slice":
+            x[b, (np.arange(V) // 256) % 8 == 3] += 20.0
+        elif kind.startswith("valid"):
+            x[b, rng.permutation(V)[int(kind[5:]):]] = -np.inf
+        elif kind.startswith("ahead"):
+            x[b, 777] = float(kind[5:])
+        elif kind == "heap":
+            x[b, rng.permutation(V)[:700]] = 30.0 + rng.uniform(0.0, 0.01, 700)
+            x[b, rng.permutation(V)[:3]] = 300.0
+        elif kind.startswith("equal"):
+            x[b, rng.permutation(V)[:int(kind[5:])]] = 4.0
+        elif kind == "lowest":
+            x[b, rng.permutation(V)[500:]] = -65504.0 if dt == O.F16 else -3.3e38
+        elif kind == "both":
+            x[b, rng.permutation(V)[400:]] = -np.inf
+            x[b, :5] = 1.0e4
+    x = O.to_storage(x, dt)
+    for ks in ([1024], [600], [257, 1024, 40]):
+        c = Case(dt, B, V, V, gen_len=1, runtime_top_k=np.resize(np.array(ks, np.uint32), B), runtime_top_p=[0.95], temperature=[0.9])
+        _run(c, rng, 1, lambda i: x)
+    for k, v in ((193, 1161), (1024, 6151)):  # as few vectors as the rule allows
+        if v // (4 if dt == O.F32 else 8) * 2 < 3 * k:
+            continue
+        c = Case(dt, B, v, v, gen_len=1, runtime_top_k=[k], runtime_top_p=[0.95])
+        _run(c, rng, 1, lambda i: np.ascontiguousarray(x[:, :v]))
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
 @pytest.mark.parametrize("log_probs", [False, True], ids=["ids", "log_probs"])
 def test_short_lists_of_equal_values_in_the_reference_order(dt, log_probs):
     """Lists of 1 to 300 candidates (around the sizes at which the ranking is split differently or gives way to another)
