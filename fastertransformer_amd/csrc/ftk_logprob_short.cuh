@@ -209,6 +209,7 @@ __global__ void __launch_bounds__(THREADS) lp_short_kernel(FusedParams p, FusedL
         }
     };
 
+    lp_note_equal<DT>(s, ring[0]);
     // ---- first pass: the maximum (pad columns count as -MAX_T), and the thread's own
     float m = NEG_INF;
     {
@@ -398,7 +399,7 @@ __global__ void __launch_bounds__(THREADS) lp_short_kernel(FusedParams p, FusedL
         return;  // the first four waves select
     }
     LPW_STAMP(6)
-    lp_finish<DT>(s, slot_key, n, probs, denom, row_max, k, tp, u, p, l, row, out);
+    lp_finish<DT>(s, slot_key, n, probs, denom, row_max, k, tp, u, p, l, row, out, DT == DT_F32 && s.misc[3] != 0);
     LPW_STAMP(7)
 }
 

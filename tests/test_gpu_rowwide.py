@@ -395,3 +395,24 @@ def test_short_lists_of_equal_values_in_the_reference_order(dt, log_probs):
     for k in (1, 5, 30, 64, 100):
         c = Case(dt, B, V, V, gen_len=1, runtime_top_k=[k], runtime_top_p=[0.95], with_cum=log_probs, with_out_lp=log_probs)
         _run(c, rng, 1, lambda i: x)
+
+
+@pytest.mark.parametrize("V,Vp", [(4097, 4104), (30011, 30011)])
+def test_fp32_rows_of_16_bit_values_with_log_probs(V, Vp):
+    """fp32 rows that hold binary16 or bfloat16 values (their lists go straight to the ranking that expects equal values), the
+    same with finer values at the row's start or anywhere else, and finer values with equal ones among the candidates."""
+    rng = np.random.default_rng(V)
+    B = 24
+    x = (rng.standard_normal((B, Vp)) * 2.5).astype(np.float32)
+    x[::4] = x[::4].astype(np.float16)
+    x[1::4] = (x[1::4].view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    x[4, 3] = x[5, 200] = x[8, 5] = x[9, 9] = 0.1
+    x[12, 3000] = x[13, 4000] = np.float32(7.1)
+    for b in range(2, B, 4):
+        x[b, rng.permutation(V)[:200]] = rng.choice(np.array([8.1, 8.3, 9.7], np.float32), 200)
+    x[3, :] = np.round(x[3, :])
+    x = np.ascontiguousarray(x)
+    for ks in ([1], [40], [64, 20, 100, 1]):
+        c = Case(O.F32, B, V, Vp, gen_len=1, runtime_top_k=np.resize(np.array(ks, np.uint32), B), runtime_top_p=[0.95],
+                 temperature=[0.8], with_cum=True, with_out_lp=True)
+        _run(c, rng, 1, lambda i: x)
