@@ -445,6 +445,7 @@ struct FusedRow {
         const uint32_t bit = bm_mode != 0 ? (bm_word((v - bm_origin) >> 5) >> ((v - bm_origin) & 31)) & 1u : 0u;
         return order_key(slow(v, S::ld(rowp[v]), bit));
     }
+    static constexpr int IN_FLIGHT = 1;  // columns that the literal replay requests at a time
     // before key_at() may be used over the whole row
     __device__ __forceinline__ void prepare_whole_row()
     {

@@ -231,6 +231,7 @@ struct ProbRow {
     FusedRow<DT, 0>*          base;
     float                     row_max;
     float                     denom;  // sum + 1e-6
+    static constexpr int      IN_FLIGHT = 1;
     __device__ __forceinline__ void prepare_whole_row()
     {
         base->prepare_whole_row();
@@ -268,7 +269,7 @@ __device__ __forceinline__ float lp_chunk_element(const uint2& v, int c)
 // with one likely token get there with ordinary k (a probability below 6e-5). The unit is then 2^-24, so candidates
 // are gathered LP_TIE_DENOM units and a quarter below the bound, which is enough for denominators up to LP_TIE_DENOM
 // (a row whose k-th probability is that small has most of its mass in a few columns, whose e are at most 1). Rows
-// that neither rule covers are gathered again with the denominator at hand (lp_regather).
+// that neither rule covers are gathered again with the denominator at hand (topk_regather).
 template<int DT>
 __device__ __forceinline__ float lp_tie_rel()
 {
@@ -298,176 +299,6 @@ __device__ __forceinline__ bool lp_gather_covers(float e_bound, float denom)
 {
     return lp_ties_bounded<DT>(e_bound, denom)
            || (DT == DT_F16 && denom <= LP_TIE_DENOM && e_bound >= 2.5f * LP_TIE_UNIT * LP_TIE_DENOM);
-}
-
-// One wave: the bin of a descending walk over 64 * `per` counters at which the running count reaches `need`, and what
-// lies above it; bin -1 when all of them together do not. Every lane gets the answer.
-struct LpBin {
-    int bin, above;
-};
-__device__ __forceinline__ LpBin lp_descend(const uint32_t* bins, int per, int need)
-{
-    const int first = WAVE * per - 1 - lane_id() * per;  // this lane's bins: first, first - 1, ...
-    int       mine  = 0;
-    for (int i = 0; i < per; ++i) {
-        mine += (int)bins[first - i];
-    }
-    int incl = mine;
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-        const int up = __shfl_up(incl, o, WAVE);
-        incl += lane_id() >= o ? up : 0;
-    }
-    const unsigned long long reached = __ballot(incl >= need);
-    if (reached == 0ull) {
-        return LpBin{-1, 0};
-    }
-    const int who   = __builtin_ctzll(reached);
-    int       above = incl - mine, bin = first;
-    if (lane_id() == who) {
-        while (above + (int)bins[bin] < need) {
-            above += (int)bins[bin];
-            --bin;
-        }
-    }
-    return LpBin{__shfl(bin, who, WAVE), __shfl(above, who, WAVE)};
-}
-
-// The candidates of a row that one look at e could not bound, now that the denominator is known: the list ends up with
-// everything that can reach the result, as probabilities. All THREADS threads of the workgroup call; key_at(v) is the
-// key of column v's probability, `floor` a key that at least k columns reach (0: none known). Returns the length of the
-// list, or -1 when it does not fit.
-//   1. everything at or above `floor`, if that fits;
-//   2. otherwise the exact k-th largest key (a histogram per digit) and, of the columns that tie with it, those that
-//      the reference's first stage can pick: in each of its eight slices it takes at most k columns, by key, then by
-//      descending thread number (column modulo `1 << bs1_log`), so a tie counts down to the thread number at which
-//      its slice is full.
-// One walk over the row out of the caches for 1., five or six more for 2. Bound by those reads. 1024 x 152064 binary16,
-// one row of which has a subnormal k-th probability: 0.17 ms a step; 20.6 ms with the pick-by-pick replay for that row.
-template<int DT, int THREADS, class KeyAt>
-__device__ __forceinline__ int lp_regather(TopkShared& s, uint32_t* scratch, int vocab, int k, int bs1_log,
-                                           uint32_t floor, KeyAt&& key_at)
-{
-    const int      t    = threadIdx.x;
-    const uint32_t KMIN = min_valid_key<DT>();
-    const uint32_t ZERO = order_key(0.0f);
-    auto           walk = [&](auto&& visit) {
-#pragma unroll 4
-        for (int v = t; v < vocab; v += THREADS) {
-            visit(v, key_at(v));
-        }
-    };
-    auto push = [&](int v, uint32_t key) {
-        const int slot = atomicAdd(&s.n_cand, 1);
-        if (slot < TK_CCAP) {
-            s.cand.key[slot] = key;
-            s.cand.idx[slot] = (uint32_t)v;
-        }
-    };
-    if (floor >= KMIN && floor > ZERO) {
-        __syncthreads();
-        if (t == 0) {
-            s.n_cand = 0;
-        }
-        __syncthreads();
-        walk([&](int v, uint32_t key) {
-            if (key >= floor) {
-                push(v, key);
-            }
-        });
-        __syncthreads();
-        if (s.n_cand <= TK_CCAP) {
-            return s.n_cand;
-        }
-    }
-    static_assert(TK_CCAP == 2048 && THREADS >= TK_THREADS, "2048 counters, a wave for every two slices");
-    uint32_t* bins = s.cand.key;
-    uint32_t* ties = s.cand.idx;
-    int*      res  = reinterpret_cast<int*>(scratch);  // [0], [1]: a descent's answer; [8..15]: a slice's thread number
-    // ---- the k-th largest key. Probabilities of 16-bit types have nothing in the last ten bits.
-    constexpr int DIGITS = DT == DT_F32 ? 3 : 2;
-    uint32_t      q      = 0u;
-    int           need   = k;
-    bool          all    = false;
-#pragma unroll 1
-    for (int d = 0; d < DIGITS; ++d) {
-        const int shift = d == 0 ? 21 : d == 1 ? 10 : 0;
-        const int width = d == 2 ? 10 : 11;
-        __syncthreads();
-        for (int i = t; i < 2048; i += THREADS) {
-            bins[i] = 0u;
-        }
-        __syncthreads();
-        uint32_t zeros = 0u;  // (a whole row of them would queue for one counter)
-        auto     count = [&](uint32_t key, uint32_t n) {
-            if (key >= KMIN && n != 0u && (d == 0 || (key >> (shift + width)) == (q >> (shift + width)))) {
-                atomicAdd(&bins[(key >> shift) & ((1u << width) - 1u)], n);
-            }
-        };
-        walk([&](int, uint32_t key) {
-            zeros += key == ZERO ? 1u : 0u;
-            count(key, key == ZERO ? 0u : 1u);
-        });
-        count(ZERO, zeros);
-        __syncthreads();
-        if (wave_id() == 0) {
-            const LpBin b = lp_descend(bins, 32, need);
-            if (lane_id() == 0) {
-                res[0] = b.bin;
-                res[1] = b.above;
-            }
-        }
-        __syncthreads();
-        const int bin = __builtin_amdgcn_readfirstlane(res[0]);
-        if (bin < 0) {
-            all = true;  // fewer than k columns have a probability that is a number: all of them are picked
-            break;
-        }
-        q |= (uint32_t)bin << shift;
-        need -= __builtin_amdgcn_readfirstlane(res[1]);
-    }
-    // ---- the ties of every slice by thread number, and how many columns of the slice come before them
-    __syncthreads();
-    for (int i = t; i < 2048; i += THREADS) {
-        ties[i] = 0u;
-    }
-    if (t < 8) {
-        s.slice_count[t] = 0;
-        res[8 + t]       = 0;
-    }
-    if (t == 0) {
-        s.n_cand = 0;
-    }
-    __syncthreads();
-    if (!all) {
-        walk([&](int v, uint32_t key) {
-            const int slice = (v >> bs1_log) & 7;
-            if (key == q) {
-                atomicAdd(&ties[(slice << bs1_log) | (v & ((1 << bs1_log) - 1))], 1u);
-            }
-            else if (key > q) {
-                atomicAdd(&s.slice_count[slice], 1);
-            }
-        });
-        __syncthreads();
-        if (wave_id() < TK_WAVES) {
-#pragma unroll 1
-            for (int slice = wave_id(); slice < 8; slice += TK_WAVES) {
-                const LpBin b = lp_descend(ties + (slice << bs1_log), (1 << bs1_log) / WAVE, k - s.slice_count[slice]);
-                if (lane_id() == 0) {
-                    res[8 + slice] = max(b.bin, 0);  // (none: all of its ties)
-                }
-            }
-        }
-        __syncthreads();
-    }
-    walk([&](int v, uint32_t key) {
-        if (all ? key >= KMIN : key > q || (key == q && (v & ((1 << bs1_log) - 1)) >= res[8 + ((v >> bs1_log) & 7)])) {
-            push(v, key);
-        }
-    });
-    __syncthreads();
-    return s.n_cand <= TK_CCAP ? s.n_cand : -1;
 }
 
 // The end of a row, by TK_THREADS threads: the n candidates in s.cand carry e = T(exp(y - max)) as their keys (`probs`:
@@ -1657,7 +1488,7 @@ __global__ void __launch_bounds__(THREADS) lp_wide_kernel(FusedParams p, FusedLa
     if (!covered || n_parked > TK_CCAP || n > TK_CCAP) {
         // (fewer than k columns with e > 0: columns of probability zero are picked too, by the reference's tie rules)
         probs = true;
-        n     = lp_regather<DT, THREADS>(
+        n     = topk_regather<DT, THREADS, true>(
             s, wide_key, p.Vp, k, p.max_top_k <= 16 ? 7 : 8, valid ? order_key(round_t<DT>(e_bound / denom)) : 0u,
             [&](int v) -> uint32_t {
                 const float y = v < p.V ? value(v, rowp[v]) : -S::max_t();

@@ -386,7 +386,7 @@ __global__ void __launch_bounds__(THREADS) lp_short_kernel(FusedParams p, FusedL
     if (n > TK_CCAP || !valid || !lp_gather_covers<DT>(e_bound, denom)) {
         // (fewer than k columns with e > 0: columns of probability zero are picked too, by the reference's tie rules)
         probs = true;
-        n     = lp_regather<DT, THREADS>(
+        n     = topk_regather<DT, THREADS, true>(
             s, wide_key, p.Vp, k, p.max_top_k <= 16 ? 7 : 8, valid ? order_key(round_t<DT>(e_bound / denom)) : 0u,
             [&](int v) -> uint32_t {
                 const float y = v < p.V ? value(v, rowp[v]) : -S::max_t();

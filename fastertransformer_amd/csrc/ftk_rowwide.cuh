@@ -98,6 +98,32 @@ struct RowwideArgs {
 };
 typedef const __attribute__((address_space(4))) void* RowwideArgSegment;
 
+// A row as the rare cases see it: by a quarter of the workgroup, out of the caches.
+template<int DT>
+struct RareRow: FusedRow<DT, 0> {
+    static constexpr int IN_FLIGHT = 8;
+    using FusedRow<DT, 0>::FusedRow;
+    // key_at() of several columns, all of them requested before the first is looked at
+    template<int U>
+    __device__ __forceinline__ void keys_at(const int (&v)[U], uint32_t (&keys)[U]) const
+    {
+        typename Storage<DT>::T raw[U];
+        uint32_t                word[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            raw[u] = this->rowp[v[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            word[u] = this->bm_mode != 0 ? this->bm_word((v[u] - this->bm_origin) >> 5) : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            keys[u] = order_key(this->slow(v[u], Storage<DT>::ld(raw[u]), (word[u] >> ((v[u] - this->bm_origin) & 31)) & 1u));
+        }
+    }
+};
+
 // What is left to the first four waves when a row's list is still longer than 256 entries after the cut (the
 // selection of topk_select_lds for long lists) or outgrew LDS (the whole row is walked again with the stream that
 // recovers from overfull tiles; rows it cannot bound either take the literal replay). Not inlined, so that the
@@ -123,7 +149,7 @@ __device__ __noinline__ void rowwide_rare(TopkShared& ts, RowwideArgSegment segm
     out.cum_log_prob_in    = 0.0f;
     out.end_id_in          = args.end_id;
     TopkEntry*      row_entries = l.entries + (size_t)row * l.row_entries;
-    FusedRow<DT, 0> r0(p, row, args);
+    RareRow<DT>     r0(p, row, args);
     r0.team = TK_THREADS;  // (the other waves of the workgroup have left)
     if (count_table != nullptr) {
         r0.use_count_table(count_table);
@@ -131,10 +157,21 @@ __device__ __noinline__ void rowwide_rare(TopkShared& ts, RowwideArgSegment segm
     if (n > TK_CCAP) {
         r0.prepare_whole_row();
         __syncthreads();
-        n = topk_stream<DT, FusedRow<DT, 0>, 0>(r0, ts, p.Vp, k, 0, topk_row_tiles<DT>(r0.rowp, p.Vp), &thr);
+        n = topk_stream<DT, RareRow<DT>, 0>(r0, ts, p.Vp, k, 0, topk_row_tiles<DT>(r0.rowp, p.Vp), &thr);
+        if (n < 0) {
+            // More columns tie with the k-th than a list holds (flat rows, fewer columns than k above a finite mask). us a step, the
+            // literal replay / so: 77 x 50257, k = 50, bf16 4803 / 1458, f32 4608 / 969; 64 x 50264, k = 192, 15664 / 1598 and 16236 /
+            // 1105. With k > 192 the first stage's picks may not fit a list: the literal replay with eight columns in flight, 4 x
+            // 50257, k = 1024, bf16 67.2 -> 53.3 ms.
+            n   = topk_regather<DT, TK_THREADS, false>(ts, ts.red32, p.Vp, k, p.max_top_k <= 16 ? 7 : 8, 0u,
+                                                       [&](int v) -> uint32_t { return r0.key_at(v); });
+            n   = __builtin_amdgcn_readfirstlane(n);
+            thr = min_valid_key<DT>();
+            __syncthreads();
+        }
     }
-    topk_select_lds<DT, FusedRow<DT, 0>, true>(r0, ts, n, thr, row, p.Vp, k, tp, p.max_top_k, row_entries, false, u,
-                                               p.end_ids, out);
+    topk_select_lds<DT, RareRow<DT>, true>(r0, ts, n, thr, row, p.Vp, k, tp, p.max_top_k, row_entries, false, u,
+                                           p.end_ids, out);
 }
 
 // Requirements the launcher checks: rows start on 16-byte boundaries (ODD: where an element may), no embedding bias,

@@ -1191,7 +1191,188 @@ __device__ __forceinline__ void topk_finish_list(TopkShared& s, int n_list, int 
     }
 }
 
-// Literal replay for rows the gather could not bound. `Row::key_at(v)` re-reads the row.
+// One wave: the bin of a descending walk over 64 * `per` counters at which the running count reaches `need`, and what
+// lies above it; bin -1 when all of them together do not. Every lane gets the answer.
+struct TopkBin {
+    int bin, above;
+};
+__device__ __forceinline__ TopkBin topk_descend(const uint32_t* bins, int per, int need)
+{
+    const int first = WAVE * per - 1 - lane_id() * per;  // this lane's bins: first, first - 1, ...
+    int       mine  = 0;
+    for (int i = 0; i < per; ++i) {
+        mine += (int)bins[first - i];
+    }
+    int incl = mine;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int up = __shfl_up(incl, o, WAVE);
+        incl += lane_id() >= o ? up : 0;
+    }
+    const unsigned long long reached = __ballot(incl >= need);
+    if (reached == 0ull) {
+        return TopkBin{-1, 0};
+    }
+    const int who   = __builtin_ctzll(reached);
+    int       above = incl - mine, bin = first;
+    if (lane_id() == who) {
+        while (above + (int)bins[bin] < need) {
+            above += (int)bins[bin];
+            --bin;
+        }
+    }
+    return TopkBin{__shfl(bin, who, WAVE), __shfl(above, who, WAVE)};
+}
+
+// The candidates of a row that one look could not bound: the list ends up with everything that can reach the result. All
+// THREADS threads of the workgroup call; key_at(v) is the key of column v, `floor` a key that at least k columns reach (0: none
+// known), `scratch` sixteen words. PROBS: the keys are those of probabilities. Returns the length of the list, or -1 when it
+// does not fit.
+//   1. everything at or above `floor`, if that fits;
+//   2. otherwise the exact k-th largest key (a histogram per digit) and, of the columns that tie with it, those that
+//      the reference's first stage can pick: in each of its eight slices it takes at most k columns, by key, then by
+//      descending thread number (column modulo `1 << bs1_log`), so a tie counts down to the thread number at which
+//      its slice is full.
+// One walk over the row out of the caches for 1., five or six more for 2. Bound by those reads. Log-prob step of 1024 x 152064
+// binary16, one row of which has a subnormal k-th probability: 0.17 ms; 20.6 ms with the pick-by-pick replay for that row.
+template<int DT, int THREADS, bool PROBS, class KeyAt>
+__device__ __forceinline__ int topk_regather(TopkShared& s, uint32_t* scratch, int vocab, int k, int bs1_log,
+                                           uint32_t floor, KeyAt&& key_at)
+{
+    const int      t    = threadIdx.x;
+    const uint32_t KMIN = min_valid_key<DT>();
+    const uint32_t ZERO = order_key(0.0f);
+    auto           walk = [&](auto&& visit) {
+#pragma unroll 4
+        for (int v = t; v < vocab; v += THREADS) {
+            visit(v, key_at(v));
+        }
+    };
+    auto push = [&](int v, uint32_t key) {
+        const int slot = atomicAdd(&s.n_cand, 1);
+        if (slot < TK_CCAP) {
+            s.cand.key[slot] = key;
+            s.cand.idx[slot] = (uint32_t)v;
+        }
+    };
+    if (floor >= KMIN && floor > ZERO) {
+        __syncthreads();
+        if (t == 0) {
+            s.n_cand = 0;
+        }
+        __syncthreads();
+        walk([&](int v, uint32_t key) {
+            if (key >= floor) {
+                push(v, key);
+            }
+        });
+        __syncthreads();
+        if (s.n_cand <= TK_CCAP) {
+            return s.n_cand;
+        }
+    }
+    static_assert(TK_CCAP == 2048 && THREADS >= TK_THREADS, "2048 counters, a wave for every two slices");
+    uint32_t* bins = s.cand.key;
+    uint32_t* ties = s.cand.idx;
+    int*      res  = reinterpret_cast<int*>(scratch);  // [0], [1]: a descent's answer; [8..15]: a slice's thread number
+    // ---- the k-th largest key. Probabilities of 16-bit types have nothing in the last ten bits.
+    constexpr int DIGITS = DT == DT_F32 || !PROBS ? 3 : 2;
+    uint32_t      q      = 0u;
+    int           need   = k;
+    bool          all    = false;
+#pragma unroll 1
+    for (int d = 0; d < DIGITS; ++d) {
+        const int shift = d == 0 ? 21 : d == 1 ? 10 : 0;
+        const int width = d == 2 ? 10 : 11;
+        __syncthreads();
+        for (int i = t; i < 2048; i += THREADS) {
+            bins[i] = 0u;
+        }
+        __syncthreads();
+        auto count = [&](uint32_t key, uint32_t n) {
+            if (key >= KMIN && n != 0u && (d == 0 || (key >> (shift + width)) == (q >> (shift + width)))) {
+                atomicAdd(&bins[(key >> shift) & ((1u << width) - 1u)], n);
+            }
+        };
+        // (a whole row of equal values would queue for one counter: zeros, or a thread's runs of them, are added at once)
+        uint32_t held = ZERO, times = 0u;
+        walk([&](int, uint32_t key) {
+            if (key == held) {
+                ++times;
+            }
+            else if constexpr (PROBS) {
+                count(key, 1u);
+            }
+            else {
+                count(held, times);
+                held  = key;
+                times = 1u;
+            }
+        });
+        count(held, times);
+        __syncthreads();
+        if (wave_id() == 0) {
+            const TopkBin b = topk_descend(bins, 32, need);
+            if (lane_id() == 0) {
+                res[0] = b.bin;
+                res[1] = b.above;
+            }
+        }
+        __syncthreads();
+        const int bin = __builtin_amdgcn_readfirstlane(res[0]);
+        if (bin < 0) {
+            all = true;  // fewer than k columns are valid: all of them are picked
+            break;
+        }
+        q |= (uint32_t)bin << shift;
+        need -= __builtin_amdgcn_readfirstlane(res[1]);
+    }
+    // ---- the ties of every slice by thread number, and how many columns of the slice come before them
+    __syncthreads();
+    for (int i = t; i < 2048; i += THREADS) {
+        ties[i] = 0u;
+    }
+    if (t < 8) {
+        s.slice_count[t] = 0;
+        res[8 + t]       = 0;
+    }
+    if (t == 0) {
+        s.n_cand = 0;
+    }
+    __syncthreads();
+    if (!all) {
+        walk([&](int v, uint32_t key) {
+            const int slice = (v >> bs1_log) & 7;
+            if (key == q) {
+                atomicAdd(&ties[(slice << bs1_log) | (v & ((1 << bs1_log) - 1))], 1u);
+            }
+            else if (key > q) {
+                atomicAdd(&s.slice_count[slice], 1);
+            }
+        });
+        __syncthreads();
+        if (wave_id() < TK_WAVES) {
+#pragma unroll 1
+            for (int slice = wave_id(); slice < 8; slice += TK_WAVES) {
+                const TopkBin b = topk_descend(ties + (slice << bs1_log), (1 << bs1_log) / WAVE, k - s.slice_count[slice]);
+                if (lane_id() == 0) {
+                    res[8 + slice] = max(b.bin, 0);  // (none: all of its ties)
+                }
+            }
+        }
+        __syncthreads();
+    }
+    walk([&](int v, uint32_t key) {
+        if (all ? key >= KMIN : key > q || (key == q && (v & ((1 << bs1_log) - 1)) >= res[8 + ((v >> bs1_log) & 7)])) {
+            push(v, key);
+        }
+    });
+    __syncthreads();
+    return s.n_cand <= TK_CCAP ? s.n_cand : -1;
+}
+
+// Literal replay for rows the gather could not bound. `Row::key_at(v)` re-reads the row, `Row::keys_at(v, keys)` IN_FLIGHT
+// columns of it at a time.
 // Every pick is the smallest composite key strictly greater than the previous pick, where the
 // composite encodes the reference's order; picks of stage 1 go to `picks` (8k entries, global).
 template<int DT, class Row>
@@ -1208,18 +1389,36 @@ __device__ void topk_literal(Row& rowctx, TopkShared& s, int vocab, int k, int B
         for (int ite = 0; ite < k; ++ite) {
             unsigned long long best = ~0ull;
             // elements of this slice: i = (j*8 + slice)*BS1 + tt
-            for (int blk = slice; blk * BS1 < vocab; blk += 8) {
+            auto consider = [&](uint32_t kk, int blk, int tt) {
+                if (kk >= KMIN) {
+                    const unsigned long long c = ((unsigned long long)(~kk) << 29)
+                                                 | ((unsigned long long)(BS1 - 1 - tt) << 21)
+                                                 | (unsigned long long)(blk / 8);
+                    if ((!have_last || c > last) && c < best) {
+                        best = c;
+                    }
+                }
+            };
+            constexpr int U = Row::IN_FLIGHT;
+            for (int blk = slice; blk * BS1 < vocab; blk += 8 * U) {
                 for (int tt = t; tt < BS1; tt += TK_THREADS) {
-                    const int i = blk * BS1 + tt;
-                    if (i < vocab) {
-                        const uint32_t kk = rowctx.key_at(i);
-                        if (kk >= KMIN) {
-                            const unsigned long long c = ((unsigned long long)(~kk) << 29)
-                                                         | ((unsigned long long)(BS1 - 1 - tt) << 21)
-                                                         | (unsigned long long)(blk / 8);
-                            if ((!have_last || c > last) && c < best) {
-                                best = c;
-                            }
+                    if constexpr (U == 1) {
+                        const int i = blk * BS1 + tt;
+                        if (i < vocab) {
+                            consider(rowctx.key_at(i), blk, tt);
+                        }
+                    }
+                    else {
+                        int      v[U];
+                        uint32_t kk[U];
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            v[u] = min((blk + 8 * u) * BS1 + tt, vocab - 1);
+                        }
+                        rowctx.template keys_at<U>(v, kk);
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            consider((blk + 8 * u) * BS1 + tt < vocab ? kk[u] : 0u, blk + 8 * u, tt);
                         }
                     }
                 }

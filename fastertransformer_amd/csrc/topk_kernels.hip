@@ -9,6 +9,7 @@ namespace ftk {
 
 template<int DT>
 struct PlainRowAt: PlainRow<DT> {
+    static constexpr int IN_FLIGHT = 1;
     __device__ __forceinline__ uint32_t key_at(int v) const
     {
         return order_key(Storage<DT>::ld(this->rowp[v]));

@@ -416,3 +416,35 @@ def test_fp32_rows_of_16_bit_values_with_log_probs(V, Vp):
         c = Case(O.F32, B, V, Vp, gen_len=1, runtime_top_k=np.resize(np.array(ks, np.uint32), B), runtime_top_p=[0.95],
                  temperature=[0.8], with_cum=True, with_out_lp=True)
         _run(c, rng, 1, lambda i: x)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("V,Vp,ks", [(20011, 20011, [50]), (32000, 32000, [16, 1, 7]), (20011, 20016, [181, 64, 192]), (120001, 120001, [192])])
+def test_more_equal_columns_than_a_list_holds(dt, V, Vp, ks):
+    """Rows whose k-th largest value thousands of columns share, so that the reference's tie orders alone decide: flat rows, fewer
+    columns than k above a finite mask, two values, ties in one slice or above k in some of them, negative and zero ties; with a
+    history that takes columns out of the tie. (192 of 120001 columns: more than a list holds even so, the literal replay.)"""
+    rng = np.random.default_rng(V + dt + ks[0])
+    H, kinds = 30, ["flat", "zero", "mask", "mask few", "two", "one slice", "above", "steps"]
+    B = len(kinds)
+    x = (rng.standard_normal((B, Vp)) * 2.0).astype(np.float32)
+    slices = (np.arange(Vp) // (128 if max(ks) <= 16 else 256)) % 8
+    for b, kind in enumerate(kinds):
+        if kind in ("flat", "zero"):
+            x[b] = 0.7 if kind == "flat" else 0.0
+        elif kind.startswith("mask"):
+            x[b, rng.permutation(Vp)[30 if kind == "mask" else 3:]] = -1.0e4
+        elif kind == "two":
+            x[b] = np.where(rng.uniform(size=Vp) < 0.4, 3.0, -2.5)
+        elif kind == "one slice":
+            x[b] = np.where(slices == 5, 1.25, -np.inf)
+        elif kind == "above":
+            x[b] = 1.0
+            x[b, np.flatnonzero(slices == 2)[:max(ks) // 2]] = 4.0
+        else:
+            x[b] = np.minimum(np.round(x[b]), 1.0)
+    x = O.to_storage(x, dt)
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=2, runtime_top_k=np.resize(np.array(ks, np.uint32), B), runtime_top_p=[0.97],
+             temperature=[0.9], repetition_penalty=[1.2], prompt=rng.integers(0, V, (H, B)).astype(np.int32),
+             end_ids=np.full(B, V - 1, np.int32), min_length=[H + 9])
+    _run(c, rng, 2, lambda i: x)
