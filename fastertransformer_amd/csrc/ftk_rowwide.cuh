@@ -174,12 +174,6 @@ __device__ __noinline__ void rowwide_rare(TopkShared& ts, RowwideArgSegment segm
                                            p.end_ids, out);
 }
 
-// Requirements the launcher checks: rows start on 16-byte boundaries (ODD: where an element may), no embedding bias,
-// the largest k at most LG_MAX_K, at least 1024 columns, the row's history bitmap fits BMW words, and a history of at
-// most RW_HIST_U * RW_THREADS positions.
-// ODD: the vectors of a row start at its first 128-byte line; what lies in front of it (fewer than 64 columns of a
-// 16-bit type, 32 of fp32) goes the way of the columns behind the last whole vector. Bit 0 of the history bitmap is
-// `lead` columns in front of the row, so that a vector's flags never straddle two words.
 // Keeps a launch argument in a scalar register of its own from here on. Without it the compiler, short of scalar
 // registers, reads arguments again from the kernel-argument segment wherever they are used, and every such read
 // issued after the bulk of the row has been requested queues behind it.
@@ -190,6 +184,12 @@ __device__ __forceinline__ void rowwide_pin(V& v)
                         // such a store are no longer scalar loads)
 }
 
+// Requirements the launcher checks: rows start on 16-byte boundaries (ODD: where an element may), no embedding bias,
+// the largest k at most LG_MAX_K, at least 1024 columns, the row's history bitmap fits BMW words, and a history of at
+// most RW_HIST_U * RW_THREADS positions.
+// ODD: the vectors of a row start at its first 128-byte line; what lies in front of it (fewer than 64 columns of a
+// 16-bit type, 32 of fp32) goes the way of the columns behind the last whole vector. Bit 0 of the history bitmap is
+// `lead` columns in front of the row, so that a vector's flags never straddle two words.
 template<int DT, int BMW, bool ODD>
 __global__ void __launch_bounds__(RW_THREADS) rowwide_step_kernel(const RowwideArgs a_in)
 {

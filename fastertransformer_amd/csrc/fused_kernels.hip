@@ -329,6 +329,8 @@ extern "C" int ftk_fused_topk_step(ftk_fused_topk_args* a, ftk_stream_t stream)
     if (a->frequency_penalties != nullptr && (!rowwide || a->vocab_size_padded > FUSED_COUNT_MAX_VOCAB)) {
         return FTK_ERR_UNSUPPORTED;
     }
+    // (also where one launch does the step and needs its history's bitmaps and the replay's picks alone: a caller that asked
+    // for the largest k, or for logits on another boundary, keeps the workspace for all of its steps)
     const size_t   slot_bytes = lean_mode == 2 ? (size_t)lplan.splits * slot_u * LG_THREADS * sizeof(uint32_t) : 0;
     const size_t   lean_bytes =
         (size_t)(rows > 0 ? rows : 0)

@@ -2040,7 +2040,7 @@ __global__ void __launch_bounds__(TP_THREADS) topp_pick_runs_kernel(ToppStep s, 
     const bool           positive = klo >= 0x8000u, one_sign = positive || khi <= 0x8000u;
     const unsigned short origin   = (unsigned short)(!one_sign ? klo : positive ? klo - 0x8000u : 0x10000u - khi);
     const unsigned short length   = (unsigned short)min(khi - klo, 0xFFFFu);  // (all 65536: a row of one value ends above)
-    const u16x2          from = {origin, origin}, size = {length, length}, unit = {1, 1};
+    const u16x2          from = {origin, origin}, size = {length, length};
     const int whole_blocks = s.n / TSP_BLOCK;
     auto vector_of = [&](int blk) -> uint4 {
         return topp_load8(r.y + __builtin_amdgcn_readfirstlane(blk) * TSP_BLOCK + lane_id() * 8);

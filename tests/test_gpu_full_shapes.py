@@ -195,7 +195,7 @@ def test_few_rows_many_lists_per_row(dt, B, k):
     """A handful of rows of a long vocabulary: every row is cut into the largest number of workgroups, each of which
     reports at least k candidates of its own, so the union of a row's lists is longer than the 2048 entries the
     select kernel holds at once (k up to 192, one read of the logits) and the bound is raised before the lists are
-    merged; with k beyond 192 the same geometry goes through the two reads with two maxima per thread."""
+    merged; with k beyond 192 one workgroup per row does the step (csrc/ftk_largek.cuh), its rows from the caches."""
     rng = np.random.default_rng(7000 + 10 * B + dt)
     V, H = 128256, 4
     c = Case(dt, B, V, V, max_input_length=H, gen_len=2, runtime_top_k=[k], runtime_top_p=[0.95],

@@ -1,9 +1,8 @@
-"""The one-launch step for batches of about one row per compute unit (a 1024-thread workgroup per row,
-csrc/ftk_rowwide.cuh) against the CPU oracle, through DynamicDecodeLayer with injected draws: ids / finished /
-sequence_length bit-exact. The shapes are the ones the launcher sends to that kernel (up to 256 rows, or up to 1023
-in nearly full rounds of 256 with rows of at least 16384 16-byte vectors; rows on 16-byte boundaries, k <= 192, no
-bias, no log-probs);
-the last test asks the test build of the library which kernel a launch of such a shape took."""
+"""The one-launch steps (a 1024-thread workgroup per row: csrc/ftk_rowwide.cuh, k <= 192, up to 256 rows, or up to 1023
+in nearly full rounds of 256 with rows of at least 16384 16-byte vectors; csrc/ftk_largek.cuh, larger k; no bias, no
+log-probs) against the CPU oracle, through DynamicDecodeLayer with injected draws: ids / finished / sequence_length
+bit-exact. Where the test build of the library is asked which kernel a launch took, that kernel is compared with
+the launches it replaces. The last tests are of selections that the log-prob step shares."""
 import numpy as np
 import pytest
 
@@ -253,6 +252,29 @@ def test_rowwide_rows_off_the_vector_grid(dt, B, V, Vp, offset, k):
         hooks.ftk_test_set_fused_two_launches(0)
     for a, b in zip(one[:3], two[:3]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dt", DTYPES, ids=lambda d: DTYPE_NAMES[d])
+@pytest.mark.parametrize("B,V,Vp,k", [(9, 1025, 1025, 64), (40, 9001, 9003, 50), (30, 50257, 50257, 192)])
+def test_rows_off_the_vector_grid_in_the_reference_order(dt, B, V, Vp, k):
+    """The same kind of rows against the oracle: the largest values in front of a row's first 128-byte line, behind its last whole
+    vector, in the vectors beside them or anywhere, some of them equal, some in the history, one of them the masked end id."""
+    rng = np.random.default_rng(41 * V + dt)
+    H = 40
+    x = (rng.standard_normal((B, Vp)) * 2.0).astype(np.float32)
+    prompt = rng.integers(0, V, (H, B)).astype(np.int32)
+    end_ids = rng.integers(0, V, B).astype(np.int32)
+    edges = [0, 1, 5, 20, 31, 32, 62, 63, 64, 65, 72, V - 70, V - 9, V - 8, V - 5, V - 4, V - 3, V - 2, V - 1]
+    for b in range(B):
+        for i, v in enumerate(edges[b % 3::2] if b % 4 else []):
+            x[b, v] = 9.0 + 0.25 * ((i * 5 + b) % 7)
+            if (i + b) % 3 == 0:
+                prompt[i, b] = v
+        end_ids[b] = edges[b % len(edges)]
+    x = O.to_storage(x, dt)
+    c = Case(dt, B, V, Vp, max_input_length=H, gen_len=1, runtime_top_k=np.resize(np.array([k, 1, k // 2], np.uint32), B),
+             runtime_top_p=[0.9], temperature=[0.8], repetition_penalty=[1.15], prompt=prompt, end_ids=end_ids, min_length=[H + 5])
+    _run(c, rng, 1, lambda i: x)
 
 
 @pytest.mark.parametrize("dt,B,V,Vp,offset,H,k,kind", [
