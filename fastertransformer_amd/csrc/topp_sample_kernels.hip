@@ -36,6 +36,10 @@ constexpr int   topp_stage16_threads(bool penalties) { return penalties ? 512 : 
 constexpr int   TSP_SUM16   = 1024;       // threads of a sum workgroup, 16-bit types
 constexpr int   TSP_SUM32   = 256;        // fp32
 constexpr int   TSP_CHAINS  = 1024;       // summation chains of a row (the reference's block)
+// Where the code of the large fp32 kernels starts. The same instructions at another multiple of 256 bytes take longer or
+// shorter with every change to the file: 256 x 128256, at 1.5 KB behind a multiple of 2 KB / at one, stage 27.7 / 27.3 and sum 28.7 / 28.25
+// us, a step 71.0 / 70.4.
+constexpr int   TSP_CODE_ALIGN = 2048;
 constexpr int   TSP_STAGE_WAVES = 4096;   // waves of a stage launch, 16-bit types
 constexpr int   TSP_SPLITS  = 64;         // most workgroups per row of the 16-bit stage
 constexpr int   TSP_BLOCK   = 512;        // columns whose maximum the 16-bit stage keeps: one 16-byte vector per lane
@@ -390,7 +394,7 @@ __device__ __forceinline__ int topp_y_bucket(float y, float top, float last = (f
 // 113 / 117). With the parts as the fast index every XCD would see the same quarter of every 4 KB and use a quarter of its
 // L2's channels.
 template<bool TRANSFORM>
-__global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
+__attribute__((aligned(TSP_CODE_ALIGN))) __global__ void __launch_bounds__(TSP_STAGE) topp_stage_f32_kernel(ToppStep s)
 {
     // The last bucket is open below: masked columns, half of a row perhaps, lie there and would queue for its counter. It
     // is spread over a counter per lane (256 x 128256, every second column -inf: 153 -> 114 us a step).
@@ -663,11 +667,9 @@ __device__ __forceinline__ float topp_walk_chains(const T (&first)[U], const T* 
             add(visit((int)lane + (b * U + u) * STRIDE, raw[u]));
         }
     };
-    if (nb > 0) {  // (otherwise nothing was requested)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            buf[0][u] = first[u];
-        }
+    for (int u = 0; u < U; ++u) {
+        buf[0][u] = first[u];
     }
     for (int b = 0; b < nb; b += 2) {
         load(buf[1], min(b + 1, nb - 1));
@@ -868,7 +870,7 @@ __global__ void __launch_bounds__(TSP_SUM16) topp_sum_count_kernel(ToppStep s)
 // draw - and two more, so that all entries which share a probability with the last one that can be drawn are
 // there - goes to its bucket's place in the prefix, keyed by e (the division by the denominator keeps the order).
 template<int LPC>
-__global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
+__attribute__((aligned(TSP_CODE_ALIGN))) __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
 {
     constexpr int       C  = TSP_SUM32 / LPC;
     constexpr int       K  = TSP_BUCKETS / TSP_SUM32;
@@ -912,7 +914,7 @@ __global__ void __launch_bounds__(TSP_SUM32) topp_sum_gather_kernel(ToppStep s)
     }
     // (behind the histograms in the queue, and there when the cut is known: 256 x 128256 29.9 -> 29.0 us, a step 65.5 -> 64.1
     // once p has decayed; with sixteen parts a row, 1 to 71 rows of 32000 to 128256 columns, steps take as long either way)
-    float first_batch[U];
+    float first_batch[U] = {};
     if (s.n >= U * LPC * TSP_CHAINS) {
         topp_chains_load<float, LPC, U>(first_batch, y, 0, part * C + t / LPC, t % LPC);
     }
