@@ -30,7 +30,7 @@ constexpr int LK_RING       = 9;    // vectors a thread holds
 constexpr int LK_HIST_U     = 4;     // history ids a thread requests at a time
 constexpr int LK_BUCKETS    = 2048;  // of the final order: 256 for each of eight doublings of the distance to the bound
 constexpr int LK_BUCKET_CAP = 512;   // entries of a bucket are compared with each other
-constexpr int LK_BUCKET_FEW = 96;    // a bucket with more of them and most of the list is divided by buckets of its own
+constexpr int LK_BUCKET_FEW = 96;    // more, and a quarter of the list: the bucket is divided by buckets of its own
 static_assert(LK_RING % LK_GROUPS == 0, "a slot of the ring always belongs to the same group");
 
 struct LargekShared {
@@ -94,14 +94,26 @@ __device__ __forceinline__ bool largek_bin_of_rank(const uint32_t* hist, int lan
 // The list in ts.cand (256 < n <= TK_CCAP entries, all at or above thr_f, key_max the largest key) in the order of the
 // reference, by all threads: stage 1 orders a slice by (value, thread, block), which gives every entry its rank in the
 // slice, stage 2 the whole list by (value, what follows from slice and rank). Both need only neighbours of similar value:
-// the entries are counted into 2048 buckets, put down bucket by bucket, and compared inside their bucket (counted again where one
-// bucket holds many: us a step of 64 x 50257, k = 1024, counted once / so, a column 3e4 ahead of the others f16 94.0 / 29.2, f32
-// 94.0 / 29.8; 300 valid columns f16 53.5 / 26.1, f32 55.5 / 29.7; 800 f32 53.7 / 33.8; ordinary rows 28.5 / 28.7 and 29.3 / 29.5);
+// the entries are counted into 2048 buckets, put down bucket by bucket, and compared inside their bucket;
 // what lies in higher buckets is a prefix sum (over all, and per slice). Weights and columns of the first min(k, n) go to
 // ts.sel, padded with zeros to a multiple of 32. False, with ts.cand as it was, where a bucket stays crowded (many
 // equal values) or a slice holds more than k entries.
 // Bound by the latency of its barriers and by LDS: 5.6 us for 1400 entries, k = 1024, and 4.1 for the draw after it, two
 // chains of 1024 dependent operations; selection and draw took 41 with the per-slice sorts and merges on four waves.
+// AGAIN: a bucket holds a quarter of the list, or more than are compared, and is counted again in finer ones. A function of its
+// own, out of the way of other lists (inside the kernel it cost those 0.3 to 0.5 us, so 0.2). us a step of 64 x 50257, k = 1024,
+// counted once / so: a column 3e4 ahead of the others f16 94.0 / 31.9, f32 93.8 / 32.4; 300 valid columns f16 53.4 / 28.6, f32 55.5 /
+// 32.3; 800 f32 53.6 / 36.4; whole numbers and quarters up to 3 us more; ordinary rows f16 28.4 / 28.6, f32 29.2 / 29.4.
+template<bool AGAIN>
+__device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, int n, int k, int max_top_k, float thr_f);
+typedef __attribute__((address_space(3))) TopkShared*   TopkSharedPtr;  // (what is behind it is addressed as LDS in a call, too)
+typedef __attribute__((address_space(3))) LargekShared* LargekSharedPtr;
+__device__ __noinline__ bool largek_order_again(TopkSharedPtr ts, LargekSharedPtr s, int n, int k, int max_top_k, float thr_f)
+{
+    return largek_order<true>(*(TopkShared*)ts, *(LargekShared*)s, n, k, max_top_k, thr_f);
+}
+
+template<bool AGAIN>
 __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, int n, int k, int max_top_k, float thr_f)
 {
     const int   t       = threadIdx.x;
@@ -113,13 +125,30 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
     const float x_max   = key_to_float(s.key_max);
     // 1 at the bound, 257 at the row's maximum: the bits of that number are close to its logarithm, which gives the dense
     // values near the bound most of the buckets, also where a single value lies ahead of all others
-    // (the bound may be the lowest value of the type: the limit keeps the quotient a normal number)
-    float lo = thr_f, scale = 256.0f / __builtin_fminf(x_max - thr_f, 1.0e30f);
-    if (!(x_max < __builtin_inff() && scale < __builtin_inff())) {
-        return false;
+    float lo = thr_f, scale = 256.0f / (x_max - thr_f);
+    if constexpr (AGAIN) {
+        // (the bound may be the lowest value of the type: the limit keeps the quotient a normal number)
+        scale = 256.0f / __builtin_fminf(x_max - thr_f, 1.0e30f);
+        if (!(x_max < __builtin_inff() && scale < __builtin_inff())) {
+            return false;
+        }
+        lds_barrier();
+        s.count[2 * t]     = 0u;
+        s.count[2 * t + 1] = 0u;
+        if (t < 8) {
+            s.slice_count[t] = 0;
+        }
+        if (t == 0) {
+            s.fullest = 0u;
+        }
+        lds_barrier();
+    }
+    else if (!(scale > 0.0f && scale < __builtin_inff())) {
+        return largek_order_again((TopkSharedPtr)&ts, (LargekSharedPtr)&s, n, k, max_top_k, thr_f);
     }
     auto bucket_of = [&](uint32_t key) -> int {  // (never falls as the value does)
-        const uint32_t y = __float_as_uint(__builtin_fmaxf((key_to_float(key) - lo) * scale + 1.0f, 1.0f));
+        const float    x = (key_to_float(key) - lo) * scale + 1.0f;
+        const uint32_t y = __float_as_uint(AGAIN ? __builtin_fmaxf(x, 1.0f) : x);
         return max(LK_BUCKETS - 1 - (int)((y - 0x3F800000u) >> 15), 0);
     };
     // lanes of the wave whose entry lies in the same slice
@@ -148,7 +177,7 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
     }
     auto key_of = [&](int u) -> uint32_t { return ~(uint32_t)(comp[u] >> 29); };
     // the entries' buckets, and the entries in this thread's two buckets and all below them of the wave
-    uint32_t c0, c1, incl, sums, fullest;
+    uint32_t c0, c1, incl;
     auto     count = [&](auto slices) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
@@ -176,49 +205,54 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
             s.wave_sum[wv] = incl;
         }
         const uint32_t most = max(c0, c1);
-        if (most > (uint32_t)LK_BUCKET_FEW) {
+        if (most > (uint32_t)LK_BUCKET_CAP || (most > (uint32_t)LK_BUCKET_FEW && 4u * most > (uint32_t)n)) {
             atomicMax(&s.fullest, most << 16 | (uint32_t)(2 * t + (c0 == most ? 0 : 1)));
         }
         lds_barrier();
-        sums    = s.wave_sum[lane & (LK_WAVES - 1)];
-        fullest = s.fullest;
     };
     count(std::true_type());
+    if constexpr (AGAIN) {
 #pragma unroll 1
-    for (int round = 0; __builtin_expect(fullest != 0u && round < 2, 0); ++round) {
-        // Much of the list in one bucket: the row's maximum is far ahead of it, or the bound is the lowest value of the type
-        // (fewer than k valid columns). Again, with 1 to 17, about half of the buckets, for what that one holds.
-        uint32_t klo = 0xFFFFFFFFu, khi = 0u;
+        for (int round = 0; round < 2; ++round) {
+            // The row's maximum is far ahead of the others, or the bound is the lowest value of the type (fewer than k valid
+            // columns). Buckets for what the fullest one holds, with 1 to 17, about half of the buckets.
+            const uint32_t fullest = s.fullest;
+            if (fullest == 0u) {
+                break;
+            }
+            uint32_t klo = 0xFFFFFFFFu, khi = 0u;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const bool in = t + u * LK_THREADS < n && bucket[u] == (int)(fullest & 0xFFFFu);
-            klo           = min(klo, in ? key_of(u) : 0xFFFFFFFFu);
-            khi           = max(khi, in ? key_of(u) : 0u);
+            for (int u = 0; u < 2; ++u) {
+                const bool in = t + u * LK_THREADS < n && bucket[u] == (int)(fullest & 0xFFFFu);
+                klo           = min(klo, in ? key_of(u) : 0xFFFFFFFFu);
+                khi           = max(khi, in ? key_of(u) : 0u);
+            }
+            klo = ~wave_max(~klo);
+            khi = wave_max(khi);
+            if (lane == 0 && khi != 0u) {
+                atomicMin(&s.key_lo[round], klo);
+                atomicMax(&s.key_hi[round], khi);
+            }
+            lds_barrier();
+            const float from = key_to_float(s.key_lo[round]), to = key_to_float(s.key_hi[round]), finer = 16.0f / (to - from);
+            // (not where its values are equal, or equal but for rounding: then finer buckets would crowd all others)
+            if (!(finer > scale && to - from > __builtin_fabsf(to) * 0x1p-9f)) {
+                break;
+            }
+            lo                 = from;
+            scale              = finer;
+            s.count[2 * t]     = 0u;
+            s.count[2 * t + 1] = 0u;
+            if (t == 0) {
+                s.fullest = 0u;
+            }
+            lds_barrier();
+            count(std::false_type());
         }
-        klo = ~wave_max(~klo);
-        khi = wave_max(khi);
-        if (lane == 0 && khi != 0u) {
-            atomicMin(&s.key_lo[round], klo);
-            atomicMax(&s.key_hi[round], khi);
-        }
-        lds_barrier();
-        const float from = key_to_float(s.key_lo[round]), to = key_to_float(s.key_hi[round]), finer = 16.0f / (to - from);
-        // (not where its values are equal, or equal but for rounding: then finer buckets would crowd all others)
-        if (!(finer > scale && to - from > __builtin_fabsf(to) * 0x1p-9f)) {
-            break;
-        }
-        lo                 = from;
-        scale              = finer;
-        s.count[2 * t]     = 0u;
-        s.count[2 * t + 1] = 0u;
-        if (t == 0) {
-            s.fullest = 0u;
-        }
-        lds_barrier();
-        count(std::false_type());
     }
-    {
-        uint32_t start = incl - c0 - c1;
+    {  // bucket counts -> where each bucket starts
+        const uint32_t sums  = s.wave_sum[lane & (LK_WAVES - 1)];
+        uint32_t       start = incl - c0 - c1;
 #pragma unroll
         for (int w = 0; w < LK_WAVES; ++w) {
             start += w < wv ? (uint32_t)__builtin_amdgcn_readlane((int)sums, w) : 0u;
@@ -229,7 +263,8 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
             s.count[LK_BUCKETS] = (uint32_t)n;
         }
     }
-    bool one_by_one = fullest >> 16 > (uint32_t)LK_BUCKET_CAP;
+    const uint32_t fullest    = s.fullest;
+    bool           one_by_one = AGAIN && fullest >> 16 > (uint32_t)LK_BUCKET_CAP;
 #pragma unroll
     for (int sl = 0; sl < 8; ++sl) {
         one_by_one = one_by_one || s.slice_count[sl] > k;
@@ -237,6 +272,9 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
     lds_barrier();
     if (one_by_one) {
         return false;
+    }
+    if (!AGAIN && fullest != 0u) {
+        return largek_order_again((TopkSharedPtr)&ts, (LargekSharedPtr)&s, n, k, max_top_k, thr_f);
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -761,7 +799,7 @@ __global__ void __launch_bounds__(LK_THREADS) largek_step_kernel(const RowwideAr
     // ---- 4. the selection
     const int   n       = s.n_list;
     const float u       = __int_as_float(ts.misc[0]);
-    const bool  ordered_list = n > 256 && n <= TK_CCAP && largek_order(ts, s, n, k, p.max_top_k, thr_f);
+    const bool  ordered_list = n > 256 && n <= TK_CCAP && largek_order<false>(ts, s, n, k, p.max_top_k, thr_f);
     if (ordered_list) {
         LK_STAMP(6)
         if (t == 0) {
