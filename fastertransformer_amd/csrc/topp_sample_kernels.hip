@@ -204,7 +204,7 @@ __device__ __forceinline__ uint4 topp_load8(const uint16_t* from)
 // several workgroups of the sum add to are cleared on the way. Bound by latency where there are few rows: flags and
 // history (2 us), then a few blocks per wave. Requesting the history first and a short loop instead of 25 KB of
 // straight-line code, which every wave fetched to run it once: 64 x 128256 bfloat16 with temperature and penalty
-// 15.1 -> 12.4 us (16 MB read, 16 MB written; 0.2 of the copy rate), 128 x 152064 with 51 rows of its own 17.9 -> 15.7.
+// 15.1 -> 12.8 us (16 MB read, 16 MB written; 0.2 of the copy rate), 128 x 152064 with 51 rows of its own 17.9 -> 14.6.
 // An embedding bias has an instantiation of its own and is read like the row, sixteen bytes from any column on. us a step with
 // a bias, its columns through the loop of the row's end / one two-byte load each / so: 256 x 128256 bfloat16 128.5 / 108.6 /
 // 75.5, binary16 143.2 / 124.4 / 91.3; 64 x 128256 52.4 / 53.3 / 40.2; 1 x 32000 with penalties 27.0 / 29.4 / 26.1.
@@ -2268,8 +2268,8 @@ static ToppSamplePlan topp_sample_plan(int dtype, int rows, int vocab, size_t vo
     }
     // 16-bit stage: about sixteen waves per compute unit, workgroups of at least four blocks of columns, no more columns than
     // a bitmap of the history covers. Workgroups of 512 threads where each walks the row's whole history (us of the stage
-    // with 256 / 512 / 1024: 64 x 128256 13.9 / 13.7 / 13.4, 128 x 152064 with 51 rows of its own 16.1 / 15.6 / 16.0; twice
-    // the waves 14.1 and 15.7), of 256 where there are no penalties (a step of 8 x 50257 29.5, with 512 30.2). Eight blocks
+    // with 256 / 512 / 1024: 64 x 128256 12.9 / 12.8 / 13.2, 128 x 152064 with 51 rows of its own 15.1 / 14.6 / 15.5; twice
+    // the waves, when that was 13.7 and 15.6, 14.1 and 15.7), of 256 where there are no penalties (a step of 8 x 50257 29.5, with 512 30.2). Eight blocks
     // per workgroup, one for each wave, instead of four: a step of 1 x 32000 with penalties 25.8 / 26.4.
     p.blocks = (vocab + TSP_BLOCK - 1) / TSP_BLOCK;
     int s    = (TSP_STAGE_WAVES / (topp_stage16_threads(keeps_y) / WAVE) + rows - 1) / rows;
