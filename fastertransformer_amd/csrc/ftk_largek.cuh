@@ -43,7 +43,7 @@ struct LargekShared {
     uint32_t key_max;
     int      slice_count[8];
     int      n_list;
-    uint32_t fullest;         // entries of the fullest bucket << 16 | its number, where it holds more than a few
+    uint32_t fullest;         // not zero: a bucket is full; the second time its entries << 16 | its number
     uint32_t key_lo[2], key_hi[2];  // the range of its keys, twice
 };
 
@@ -100,10 +100,10 @@ __device__ __forceinline__ bool largek_bin_of_rank(const uint32_t* hist, int lan
 // equal values) or a slice holds more than k entries.
 // Bound by the latency of its barriers and by LDS: 5.6 us for 1400 entries, k = 1024, and 4.1 for the draw after it, two
 // chains of 1024 dependent operations; selection and draw took 41 with the per-slice sorts and merges on four waves.
-// AGAIN: a bucket holds a quarter of the list, or more than are compared, and is counted again in finer ones. A function of its
-// own, out of the way of other lists (inside the kernel it cost those 0.3 to 0.5 us, so 0.2). us a step of 64 x 50257, k = 1024,
-// counted once / so: a column 3e4 ahead of the others f16 94.0 / 31.9, f32 93.8 / 32.4; 300 valid columns f16 53.4 / 28.6, f32 55.5 /
-// 32.3; 800 f32 53.6 / 36.4; whole numbers and quarters up to 3 us more; ordinary rows f16 28.4 / 28.6, f32 29.2 / 29.4.
+// AGAIN: a bucket holds a quarter of the list, or more than are compared, and all are counted once more, then in finer buckets. A
+// function of its own, out of the way of other lists (inside the kernel it cost those 0.3 to 0.5 us). us a step of 64 x 50257, k =
+// 1024, counted once / so: a column 3e4 ahead of the others f16 94.0 / 31.9, f32 94.1 / 32.4; 300 valid columns f16 53.4 / 28.6, f32
+// 55.6 / 32.4; 800 f32 54.0 / 36.5; fp32 multiples of 0.25 78.4 / 80.1; ordinary rows f16 28.5 / 28.5, f32 29.2 / 29.2.
 template<bool AGAIN>
 __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, int n, int k, int max_top_k, float thr_f);
 typedef __attribute__((address_space(3))) TopkShared*   TopkSharedPtr;  // (what is behind it is addressed as LDS in a call, too)
@@ -137,6 +137,10 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
         s.count[2 * t + 1] = 0u;
         if (t < 8) {
             s.slice_count[t] = 0;
+        }
+        if (t < 2) {
+            s.key_lo[t] = 0xFFFFFFFFu;
+            s.key_hi[t] = 0u;
         }
         if (t == 0) {
             s.fullest = 0u;
@@ -174,22 +178,26 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
         const int      blk = (int)(idx >> bs1_log), slice = blk & 7;
         comp[u] = ((unsigned long long)slice << 61) | ((unsigned long long)(~key) << 29)
                   | ((unsigned long long)(BS1 - 1 - (int)(idx & (uint32_t)(BS1 - 1))) << 21) | (unsigned long long)(blk >> 3);
+        if constexpr (!AGAIN) {
+            bucket[u] = have ? bucket_of(key) : 0;
+            slot[u]   = have ? (int)atomicAdd(&s.count[bucket[u]], 1u) : 0;
+        }
+        const unsigned long long m = same_slice(have, slice);
+        if (have && below_lane(m) == 0) {
+            atomicAdd(&s.slice_count[slice], (int)__builtin_popcountll(m));
+        }
     }
     auto key_of = [&](int u) -> uint32_t { return ~(uint32_t)(comp[u] >> 29); };
+    const uint32_t full = (uint32_t)min(max(n >> 2, LK_BUCKET_FEW), LK_BUCKET_CAP);
     // the entries' buckets, and the entries in this thread's two buckets and all below them of the wave
     uint32_t c0, c1, incl;
-    auto     count = [&](auto slices) {
+    auto     count = [&]() {
+        if constexpr (AGAIN) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const bool have = t + u * LK_THREADS < n;
-            bucket[u]       = have ? bucket_of(key_of(u)) : 0;
-            slot[u]         = have ? (int)atomicAdd(&s.count[bucket[u]], 1u) : 0;
-            if constexpr (decltype(slices)::value) {
-                const int                slice = (int)(comp[u] >> 61);
-                const unsigned long long m     = same_slice(have, slice);
-                if (have && below_lane(m) == 0) {
-                    atomicAdd(&s.slice_count[slice], (int)__builtin_popcountll(m));
-                }
+            for (int u = 0; u < 2; ++u) {
+                const bool have = t + u * LK_THREADS < n;
+                bucket[u]       = have ? bucket_of(key_of(u)) : 0;
+                slot[u]         = have ? (int)atomicAdd(&s.count[bucket[u]], 1u) : 0;
             }
         }
         lds_barrier();
@@ -205,12 +213,17 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
             s.wave_sum[wv] = incl;
         }
         const uint32_t most = max(c0, c1);
-        if (most > (uint32_t)LK_BUCKET_CAP || (most > (uint32_t)LK_BUCKET_FEW && 4u * most > (uint32_t)n)) {
-            atomicMax(&s.fullest, most << 16 | (uint32_t)(2 * t + (c0 == most ? 0 : 1)));
+        if constexpr (AGAIN) {
+            if (most > full) {
+                atomicMax(&s.fullest, most << 16 | (uint32_t)(2 * t + (c0 == most ? 0 : 1)));
+            }
+        }
+        else if (__ballot(most > full) != 0ull && lane == 0) {
+            s.fullest = 1u;
         }
         lds_barrier();
     };
-    count(std::true_type());
+    count();
     if constexpr (AGAIN) {
 #pragma unroll 1
         for (int round = 0; round < 2; ++round) {
@@ -247,7 +260,7 @@ __device__ __forceinline__ bool largek_order(TopkShared& ts, LargekShared& s, in
                 s.fullest = 0u;
             }
             lds_barrier();
-            count(std::false_type());
+            count();
         }
     }
     {  // bucket counts -> where each bucket starts
@@ -435,10 +448,6 @@ __global__ void __launch_bounds__(LK_THREADS) largek_step_kernel(const RowwideAr
     }
     if (t < 8) {
         s.slice_count[t] = 0;
-    }
-    if (t >= WAVE && t < WAVE + 2) {
-        s.key_lo[t - WAVE] = 0xFFFFFFFFu;
-        s.key_hi[t - WAVE] = 0u;
     }
     if (t == 0) {
         s.n_list  = 0;
